@@ -315,10 +315,13 @@ int moe_experts_decode_q4k(const void *x_bf16, int T, int H, int I, int I_sh, in
  * sorted pair order; expert_ptr[e] == 0 for an active expert sets *err |= 1 and skips it).
  *   fmt       : MOE_FMT_BF16 (expert image = blocked w13 [2I,H] then blocked w2 [H,I]; bf16 MFMA),
  *               MOE_FMT_INT4_G128 or MOE_FMT_Q4K (nibble tiles dequantised in registers to fp16
- *               operands, activations converted bf16 -> fp16 on the way into LDS; tiles of 192 rows)
+ *               operands, activations converted to fp16 once per call; tiles of 128 rows)
  *   tiles_ws  : device workspace of moe_prefill_workspace_bytes(T, k, max_units) bytes; the
  *               list of row tiles per expert is built there by a kernel, so the host
  *               needs no copy of the dispatch counts.
+ *   phases    : bit 0 = w13 + SwiGLU, bit 1 = w2; bit 2 (nibble formats) = tiles_ws has room for the fp16 copy of
+ *               x behind the list, T*H*2 bytes at the next multiple of 256 (without it the call takes and returns
+ *               stream-ordered memory for the copy); bit 3, with bit 2 = that room already holds the copy of this x.
  * Between the two passes h_r / h_s hold bf16 for MOE_FMT_BF16 and fp16 for the nibble formats (whose matrix-core
  * operands are fp16: the w2 pass then stages them without a conversion); both passes of a batch go through this entry.
  * H % 256 == 0, I % 128 == 0, I_sh % 128 == 0.  The reference leaves this product to the

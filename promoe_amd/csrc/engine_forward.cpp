@@ -190,7 +190,9 @@ extern "C" int moe_forward_prepare(moe_engine *eng, int max_tokens) {
   }
   rc |= dalloc(s, &s->part_s, rows_s * H);
   s->part_s_elems = rows_s * H;
-  rc |= dalloc(s, (unsigned char **)&s->tiles_ws, (size_t)moe_prefill_workspace_bytes(T, k, s->max_units));
+  // the tile list and, for the nibble formats, the fp16 copy of a prefill batch's activations behind it
+  rc |= dalloc(s, (unsigned char **)&s->tiles_ws,
+               (((size_t)moe_prefill_workspace_bytes(T, k, s->max_units) + 255) & ~(size_t)255) + (size_t)T * H * 2);
   s->disp_ws_bytes = moe_dispatch_workspace_bytes(T, k, E);
   if (s->disp_ws_bytes) rc |= dalloc(s, &s->disp_ws, (size_t)s->disp_ws_bytes);
   rc |= halloc(s, &s->units_host, s->max_units);
@@ -279,7 +281,7 @@ static int run_units(moe_engine *eng, const moe_layer_desc &d, LayerState *s, co
     return moe_experts_prefill_pieces(x, T, d.H, d.I, with_shared ? d.I_sh : 0, d.top_k, d.fmt, units_dev, n_units,
                                       s->sorted_tok, table, with_shared ? d.shared : nullptr, s->h_r, s->h_s, s->part_r,
                                       s->part_s, with_shared ? shared_pieces(d, T, s) : 1, s->tiles_ws,
-                                      s->err_host + layer, 3, st);
+                                      s->err_host + layer, d.fmt == MOE_FMT_BF16 ? 3 : 7, st);
   if (d.fmt == MOE_FMT_Q4K)
     return moe_experts_decode_q4k(x, T, d.H, d.I, with_shared ? d.I_sh : 0, d.top_k, units_dev, n_units,
                                   s->sorted_tok, table, with_shared ? d.shared : nullptr, s->h_r, s->h_s,

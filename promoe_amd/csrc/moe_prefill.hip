@@ -334,160 +334,289 @@ __global__ __launch_bounds__(256, 1) void k_prefill_gemm(const PfArgs a) {
     }
 }
 
-// ---- int4-g128 experts ----------------------------------------------------------------
-// Same tiling as the bf16 kernel (8 waves, tile of up to 256 rows, wave w of group g owns 64
-// weight rows and the 32-row blocks g, g+2, ...), K advances one quantisation group (128) at
-// a time.  The int4 tiles of the slot layout are already in the operand order of
-// v_mfma_f32_16x16x32_f16 (lane = row l&15, k quarter l>>4, dword j = 8 consecutive k), so a
-// wave loads them straight into registers and dequantises there: a nibble pair is shifted and masked
-// into the mantissas of two fp16 values 1 + q/16 and one packed fma per pair applies scale and zero
-// (deq8_f16 below).  gfx950 has packed fp16 arithmetic
-// but no packed bf16 arithmetic, hence fp16 operands: activations are converted bf16 -> fp16
-// while they are staged into LDS (exact for |x| < 65504 outside the fp16 subnormal range); the h rows
-// between the two passes are written as fp16 by the w13 epilogue, so the w2 pass stages them as they are.
+// ---- int4-g128 and q4_K experts ---------------------------------------------------------
+// A workgroup of four waves (one per SIMD, two workgroups per compute unit) computes a tile of up to 128 rows x
+// (128 + 128) columns; wave w owns 32 columns of both halves (for w13 the same columns of gate and up, for w2
+// adjacent column blocks) and ALL row blocks of the tile, so every weight is dequantised once per tile.  K advances
+// 64 at a time (half a quantisation group).  A 16-byte piece of a nibble tile is 32 consecutive k of one weight row;
+// lane (n = lane % 32, q = lane / 32) of a fragment takes row n and the slab's k quarter q, so dword j of its piece is
+// the B operand of product j with k = 32 q + 8 j + 0..7 (the order in which the activation rows are read as well: a
+// dot product allows any).  What goes into the loop and why:
+//   * everything from memory goes global -> LDS directly (buffer_load ... lds) into one ring of slabs: the
+//     activation rows (fp16, a converted copy of x or the h rows; 128-byte rows with XOR-swizzled 16-byte chunks),
+//     and, private to each wave, the two fragments' nibbles, the scale section and the zero section of the slab.
+//     All requests are assembly, so that ONE hand-placed counter wait per slab covers them in order and the
+//     compiler, which knows of none, adds no waits of its own;
+//   * a slab's nibbles and scales are read from LDS in the third quarter of the slab before it, and the first
+//     fragments are dequantised in its last quarter: a wave depends on the others only for the activation rows;
+//   * dequantisation (three vector operations per pair, deq8_f16) of product step j + 1 is spread between the
+//     products of step j, in pieces of one pair (order pinned by sched_barrier);
+//   * two workgroups per compute unit cover each other's barriers, prologues and epilogues.
+// h rows leave the w13 pass as fp16, so that the w2 pass brings them into LDS as they are.
+// Measured (one box, w13 / w2 launch; in brackets the kernel before: eight waves, the weights of a tile dequantised
+// by two of them each, activations converted and nibbles loaded through registers one group ahead): DeepSeek shape
+// 2048 tokens 215 / 121 us (305 / 167), 379 tokens 76 / 49 (115 / 65), Mixtral shape 4096 tokens 1733 / 991 (2132 /
+// 1038), Qwen2-57B shape q4_K 512 tokens 408 / 219 (577 / 303).  What bounds it: on the large shapes the power limit
+// (matrix cores busy 78 % of the cycles of the Mixtral w13 launch, at 1.4 GHz); tiles of 256 rows with one workgroup
+// per compute unit halve the dequantisation per product and lose 8 to 15 % on all but that shape (+1 %).
 typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(1))) const uint16_t g_u16;
-typedef __attribute__((address_space(1))) const unsigned char g_u8;
 
-#define PI_LDK 136  // LDS row stride in fp16 (128 + 8 pad = 272 bytes)
-#define PI_BM 192   // most rows of one tile: 6 blocks of 32 (96 accumulator registers per wave)
+#define PN_BM 128                         // most rows of one tile: 4 blocks of 32 (128 accumulator registers)
+#define PN_LDS 81920                      // half of a compute unit's LDS
+template <bool Q4K> struct PnSlab {       // one ring slot: activations, then per wave 2 KiB of nibbles and the scales
+  static constexpr int SB = Q4K ? 512 : 256;                 // scale bytes of one wave
+  static constexpr int bytes(int nb) { return nb * 4096 + 4 * (2048 + SB); }
+  static constexpr int ring(int nb) { return PN_LDS / bytes(nb) < 8 ? PN_LDS / bytes(nb) : 8; }
+};
 
-// buffer resource over [p, p+bytes): loads past the end return 0 instead of faulting
-static __device__ __forceinline__ rsrc_t pf_rsrc(const void *p, unsigned bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc((void *)p, 0, (int)bytes, 0x00020000);
-}
-static __device__ __forceinline__ const unsigned char *pf_uniform(const unsigned char *p) {
+static __device__ __forceinline__ pf_i32x4_t pn_rsrc(const void *p) {
   const unsigned long long v = (unsigned long long)p;
-  const u32 lo = __builtin_amdgcn_readfirstlane((u32)v), hi = __builtin_amdgcn_readfirstlane((u32)(v >> 32));
-  return (const unsigned char *)(((unsigned long long)hi << 32) | lo);
+  pf_i32x4_t r;
+  r.x = __builtin_amdgcn_readfirstlane((int)(unsigned)v);
+  r.y = __builtin_amdgcn_readfirstlane((int)(unsigned)(v >> 32));
+  r.z = 0x7fffffff; r.w = 0x00020000;
+  return r;
+}
+// 64 lanes x 16 (4) bytes from base + voff + soff to LDS address lds + 16 (4) * lane
+static __device__ __forceinline__ void pn_dma16(unsigned lds, int voff, const pf_i32x4_t r, int soff) {
+  __asm__ volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+                   :: "s"(lds), "v"(voff), "s"(r), "s"(soff) : "memory", "m0");
+}
+static __device__ __forceinline__ void pn_dma4(unsigned lds, int voff, const pf_i32x4_t r, int soff) {
+  __asm__ volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds"
+                   :: "s"(lds), "v"(voff), "s"(r), "s"(soff) : "memory", "m0");
+}
+template <typename T>
+static __device__ __forceinline__ T pn_lds(unsigned addr) {
+  typedef __attribute__((address_space(3))) const T lds_t;
+  return *(lds_t *)(uintptr_t)addr;
 }
 
-struct PiMeta { u32 sc[4]; u32 zz[4]; };  // raw fp16 scale bits / zero nibble of the lane's row in the 4 tiles
+// what a wave of a tile reads; offsets in bytes, voff per lane
+struct PnSrc {
+  pf_i32x4_t ra, rw;        // activation matrix; expert image
+  int a_voff[4];            // row block n: the lane's row and chunk
+  int w_voff[2];            // fragment f
+  int s_voff, z_voff;       // scale request; q4_K: (d, dmin) request; int4: s_voff covers scales and zeros
+  int s_step;               // int4: what s_voff advances by per quantisation group (scales and zeros differ)
+};
 
-// ACT16: the activations are fp16 already (the h rows this kernel's w13 pass wrote, or a converted copy of x):
-// staged as they are, without the three vector operations per pair of the bf16 -> fp16 conversion
-// Gt: quantisation groups per weight row in memory; this workgroup reduces over the window [g0, g0 + G) of them
-template <int NBW, bool Q4K, bool ACT16>
-static __device__ __forceinline__ void pi_mainloop(f32x4_t (&acc)[4][6], uint16_t *As, const rsrc_t rx, const u32 (&a_off)[6],
-                                                   const rsrc_t rq, const rsrc_t rs, const rsrc_t rz, int Gt, int g0, int G,
-                                                   int nb, int tid) {
-  const int lane = tid & 63, g = tid >> 8;
-  const int r = lane & 15, qd = lane >> 4;
-  const int ch = tid & 15, r0 = tid >> 4;  // staging: row r0 + 32 i (block i), 16-byte chunk ch of the 128-k group
+// acc[i][f]: row block i, fragment (column half) f; slabs kt0 .. kt0 + nk - 1 (64 k each), nk >= 2 and even
+template <int NB, bool Q4K>
+static __device__ __forceinline__ void pn_mainloop(f32x16_t (&acc)[NB][2], const unsigned lds_base, const PnSrc &m, const int kt0,
+                                                   const int nk, const int tid) {
+  constexpr int SB = PnSlab<Q4K>::SB, SLOT = PnSlab<Q4K>::bytes(NB), R = PnSlab<Q4K>::ring(NB);
+  constexpr int NS_ = Q4K ? 2 : 1;         // scale requests of a slab
+  constexpr int NL = NB + 2 + NS_;         // requests of a slab
+  static_assert(R >= 3 && (R - 2) * NL < 63, "ring depth");
+  constexpr int NG = 4 * NB;               // product groups of a slab (two products each)
+  constexpr int FD = NG < 4 ? NG : 4;      // activation fragments read ahead
+  const int lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n = lane & 31, q = lane >> 5;
   const DeqF16Consts dqc = deq_f16_consts();
-  u32x4_t ra[3], wA[4], wB[4];
-  PiMeta mA, mB;
-  // activations of the next group travel in two halves (row blocks 0..2, then 3..5) through
-  // the same three staging registers
-  auto gloadA = [&](int gi, int half) {
-#pragma unroll
-    for (int i = 0; i < 3; ++i)  // unconditional (blocks past the tile's end re-read its first rows): the same
-      ra[i] = __builtin_amdgcn_raw_buffer_load_b128(rx, a_off[3 * half + i], (g0 + gi) * 256, 0);  // number of loads in every iteration
+  const unsigned wbase = lds_base + (unsigned)(NB * 4096 + w * (2048 + SB));   // this wave's nibbles, then scales
+  // request r of slab kt (clamped: past the end the last slab again, into a slot nobody reads) into slot offset so
+  auto request = [&](int r, int kt_, int so) {
+    const int kt = kt0 + (kt_ < nk ? kt_ : nk - 1);
+    if (r < NB) pn_dma16(lds_base + (unsigned)(so + (32 * r + 8 * w) * 128), m.a_voff[r], m.ra, kt * 128);
+    else if (r < NB + 2) pn_dma16(wbase + (unsigned)(so + 1024 * (r - NB)), m.w_voff[r - NB], m.rw, kt * 512);
+    else if (!Q4K) pn_dma4(wbase + (unsigned)(so + 2048), m.s_voff + (kt >> 1) * m.s_step, m.rw, 0);
+    else if (r == NB + 2) pn_dma4(wbase + (unsigned)(so + 2048), m.s_voff, m.rw, kt * 64);
+    else pn_dma4(wbase + (unsigned)(so + 2048 + 256), m.z_voff, m.rw, (kt >> 2) * 64);
   };
-  auto sstore = [&](int st, int half) {
-    uint16_t *A_ = As + st * PI_BM * PI_LDK;
+  // LDS addresses in slot 0: the lane's activation chunk of product step j, its nibbles, its scale words
+  unsigned fa0[4];
 #pragma unroll
-    for (int i = 0; i < 3; ++i)
-      if (3 * half + i < nb) {
-        u32x4_t v = ra[i];
-        if (!ACT16) {
-          v.x = bf16x2_to_f16x2(ra[i].x); v.y = bf16x2_to_f16x2(ra[i].y);
-          v.z = bf16x2_to_f16x2(ra[i].z); v.w = bf16x2_to_f16x2(ra[i].w);
-        }
-        *(u32x4_t *)(A_ + (r0 + 32 * (3 * half + i)) * PI_LDK + ch * 8) = v;
-      }
-  };
-  auto gloadW = [&](u32x4_t(&wq)[4], PiMeta &m, int gi) {
+  for (int j = 0; j < 4; ++j) fa0[j] = lds_base + (unsigned)(n * 128 + (((4 * q + j) ^ ((n >> 1) & 7)) * 16));
+  const unsigned na0 = wbase + (unsigned)lane * 16u;
+  const int t0 = n >> 4, r16 = n & 15;   // fragment f reads row r16 of the wave's row block 2 f + t0
+  const unsigned sa0 = wbase + 2048u + (unsigned)(Q4K ? t0 * 64 + (16 * q + r16) * 2 : t0 * 32 + r16 * 2);
+  const unsigned za0 = wbase + 2048u + (unsigned)(Q4K ? 256 + t0 * 64 + r16 * 4 : 128 + t0 * 8 + (r16 >> 1));
+  const int zsh = 4 * (r16 & 1);
+  u32x4_t nib[2], nxt[2];
+  u32 s2[2], c2[2], sraw[2], zraw[2];
+  u32x4_t wd[2][2];                      // [step parity][fragment]: 8 fp16 weights
+  auto read_w = [&](u32x4_t(&d)[2], int so) {
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      const int gm = g0 + gi;  // the group in memory
-      wq[t] = __builtin_amdgcn_raw_buffer_load_b128(rq, lane * 16, (t * Gt + gm) * 1024, 0);
-      if (Q4K) {  // (sc, m) byte pair of the lane's sub-block; (d, dmin) of the row's super-block
-        m.sc[t] = __builtin_amdgcn_raw_buffer_load_b16(rs, 2 * lane, (t * Gt + gm) * 128, 0);
-        m.zz[t] = __builtin_amdgcn_raw_buffer_load_b32(rz, 4 * r, (t * (Gt >> 1) + (gm >> 1)) * 64, 0);
+    for (int f = 0; f < 2; ++f) {
+      d[f] = pn_lds<u32x4_t>(na0 + (unsigned)(so + 1024 * f));
+      if (Q4K) {
+        sraw[f] = pn_lds<uint16_t>(sa0 + (unsigned)(so + 128 * f));
+        zraw[f] = pn_lds<u32>(za0 + (unsigned)(so + 128 * f));
       } else {
-        m.sc[t] = __builtin_amdgcn_raw_buffer_load_b16(rs, 2 * r, (t * Gt + gm) * 32, 0);
-        m.zz[t] = __builtin_amdgcn_raw_buffer_load_b8(rz, r >> 1, (t * Gt + gm) * 8, 0);
+        sraw[f] = pn_lds<uint16_t>(sa0 + (unsigned)(so + 64 * f));
+        zraw[f] = pn_lds<unsigned char>(za0 + (unsigned)(so + 16 * f));
       }
     }
   };
-  // S = 16 s and C of deq8_f16 for the lane's row in the 4 tiles of a group, once per group
-  auto prep = [&](const PiMeta &m, u32 (&s2)[4], u32 (&c2)[4]) {
+  auto prep = [&]() {  // S = 16 s and C of deq8_f16 for the lane's row in both fragments
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
+    for (int f = 0; f < 2; ++f) {
       float s16, cz;
       if (Q4K) {
-        s16 = 16.f * __builtin_bit_cast(float, h2f_bits(m.zz[t] & 0xffffu)) * (float)(m.sc[t] & 0xffu);
-        const float dmn = __builtin_bit_cast(float, h2f_bits(m.zz[t] >> 16)) * (float)((m.sc[t] >> 8) & 0xffu);
-        cz = -s16 - dmn;
+        s16 = 16.f * __builtin_bit_cast(float, h2f_bits(zraw[f] & 0xffffu)) * (float)(sraw[f] & 0xffu);
+        cz = -s16 - __builtin_bit_cast(float, h2f_bits(zraw[f] >> 16)) * (float)((sraw[f] >> 8) & 0xffu);
       } else {
-        const float sf = __builtin_bit_cast(float, h2f_bits(m.sc[t] & 0xffffu));
+        const float sf = __builtin_bit_cast(float, h2f_bits(sraw[f]));
         s16 = 16.f * sf;
-        cz = -(16.f + (float)((m.zz[t] >> (4 * (r & 1))) & 15u)) * sf;
+        cz = -(16.f + (float)((zraw[f] >> zsh) & 15u)) * sf;
       }
       const u32 sb = f2h_bits(s16), cb = f2h_bits(cz);
-      s2[t] = sb | (sb << 16);
-      c2[t] = cb | (cb << 16);
+      s2[f] = sb | (sb << 16);
+      c2[f] = cb | (cb << 16);
     }
   };
-  auto compute2 = [&](int st, const u32x4_t(&wq)[4], const u32 (&s2)[4], const u32 (&z2)[4], int j0) {
-    const uint16_t *A_ = As + st * PI_BM * PI_LDK + (32 * g + r) * PI_LDK + 32 * qd;
+  // pair p (0..7) of a step's two fragments: 3 vector operations
+  auto deq_piece = [&](u32x4_t(&dst)[2], const u32x4_t(&src)[2], int j, int p) {
+    const int f = p >> 2, e = p & 3;
+    const u32 d = src[f][j];
+    const u32 sh = e == 0 ? d << 6 : (e == 1 ? d << 2 : (e == 2 ? d >> 2 : d >> 6));
+    const f16x2_t h = __builtin_bit_cast(f16x2_t, (sh & dqc.M) | dqc.C);
+    dst[f][e] = __builtin_bit_cast(u32, __builtin_elementwise_fma(h, __builtin_bit_cast(f16x2_t, s2[f]), __builtin_bit_cast(f16x2_t, c2[f])));
+  };
+
 #pragma unroll
-    for (int jj = 0; jj < 2; ++jj) {
-      const int j = j0 + jj;
-      f16x8_t wd[4];
+  for (int t = 0; t < R - 1; ++t)
 #pragma unroll
-      for (int t = 0; t < 4; ++t) wd[t] = deq8_f16(wq[t][j], s2[t], z2[t], dqc);
+    for (int r = 0; r < NL; ++r) request(r, t, t * SLOT);
+  PF_VMCNT((R - 2) * NL);
+  __syncthreads();
+  read_w(nib, 0);
+  prep();
 #pragma unroll
-      for (int tb = 0; tb < 2 * NBW; ++tb) {
-        const f16x8_t xa = *(const f16x8_t *)(A_ + (64 * (tb >> 1) + 16 * (tb & 1)) * PI_LDK + 8 * j);
+  for (int p = 0; p < 8; ++p) deq_piece(wd[0], nib, 0, p);
+  int so = 0, sn = SLOT, sl = (R - 1) * SLOT;   // slot offsets of slab kt, kt + 1 and kt + R - 1
+  for (int kt = 0; kt < nk; ++kt) {
+    unsigned fb[4];
 #pragma unroll
-        for (int t = 0; t < 4; ++t) acc[t][tb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa, wd[t], acc[t][tb], 0, 0, 0);
+    for (int j = 0; j < 4; ++j) fb[j] = fa0[j] + (unsigned)so;
+    auto frag = [&](int g) { return pn_lds<f16x8_t>(fb[g / NB] + (unsigned)((g % NB) * 4096)); };
+    f16x8_t fa[FD + 1];
+#pragma unroll
+    for (int g = 0; g < FD; ++g) fa[g] = frag(g);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+      const int j = g / NB, i = g % NB;
+      if (g == 2 * NB) {                // the next slab's own requests have landed: nibbles and scales into registers
+        PF_VMCNT((R - 2) * NL);
+        read_w(nxt, sn);
+        __builtin_amdgcn_sched_barrier(0);
       }
+      if (g == 3 * NB) prep();
+      auto deq = [&](int half) {        // pieces of the next step's fragments behind this product
+#pragma unroll
+        for (int p = 0; p < 8; ++p)
+          if (p * 2 * NB / 8 == 2 * i + half) deq_piece(wd[(j + 1) & 1], j < 3 ? nib : nxt, (j + 1) & 3, p);
+      };
+      acc[i][0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[g % (FD + 1)], __builtin_bit_cast(f16x8_t, wd[j & 1][0]), acc[i][0], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      if (g + FD < NG) fa[(g + FD) % (FD + 1)] = frag(g + FD);
+      deq(0);
+      __builtin_amdgcn_sched_barrier(0);
+      acc[i][1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[g % (FD + 1)], __builtin_bit_cast(f16x8_t, wd[j & 1][1]), acc[i][1], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      deq(1);
+#pragma unroll
+      for (int r = 0; r < NL; ++r)      // requests of slab kt + R - 1 in the first half of the step
+        if (r * 2 * NB / NL == g) request(r, kt + R - 1, sl);
       __builtin_amdgcn_sched_barrier(0);
     }
-  };
-  auto step = [&](int gi, const u32x4_t(&cur)[4], const PiMeta &mc, u32x4_t(&nxt)[4], PiMeta &mn) {
-    const bool more = gi + 1 < G;
-    // unconditional requests (the last group asks for itself once more), pinned in front of the products: with
-    // loads under conditions the compiler's waits for the current tiles also wait for the ones just requested
-    const int gn = more ? gi + 1 : gi;
-    gloadA(gn, 0);
-    if (NBW > 0) gloadW(nxt, mn, gn);
-    __builtin_amdgcn_sched_barrier(0);
-    u32 s2[4], c2[4];
-    if (NBW > 0) prep(mc, s2, c2);
-    if (NBW > 0) compute2(gi & 1, cur, s2, c2, 0);
-    if (more) sstore((gi + 1) & 1, 0);
-    gloadA(gn, 1);
-    __builtin_amdgcn_sched_barrier(0);
-    if (NBW > 0) compute2(gi & 1, cur, s2, c2, 2);
-    if (more) {
-      if (nb > 3) sstore((gi + 1) & 1, 1);
-      __syncthreads();
-    }
-  };
-  gloadA(0, 0);
-  if (NBW > 0) gloadW(wA, mA, 0);
-  sstore(0, 0);
-  if (nb > 3) {
-    gloadA(0, 1);
-    sstore(0, 1);
-  }
-  __syncthreads();
-  for (int gi = 0; gi < G; gi += 2) {
-    step(gi, wA, mA, wB, mB);
-    if (gi + 1 < G) step(gi + 1, wB, mB, wA, mA);
+    __syncthreads();
+    nib[0] = nxt[0]; nib[1] = nxt[1];
+    so = sn; 
+    sn = sn + SLOT == R * SLOT ? 0 : sn + SLOT;
+    sl = sl + SLOT == R * SLOT ? 0 : sl + SLOT;
   }
 }
 
-template <bool SWIGLU, bool Q4K, bool ACT16>
-__global__ __launch_bounds__(512, 1) void k_prefill_int4(const PfArgs a) {
-  extern __shared__ __align__(16) uint16_t As[];  // [2][PI_BM][PI_LDK] fp16
-  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane((tid >> 6) & 3), g = tid >> 8;
-  const int r = lane & 15, qd = lane >> 4;
+template <int NB, bool SWIGLU, bool Q4K>
+static __device__ __forceinline__ void pn_tile(const PfClass &c, const PfTile &tile, unsigned char *lds, int nt, int kt0, int nk,
+                                               int split, int tid) {
+  const int lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n = lane & 31, q = lane >> 5;
+  const int G = c.K >> 7;
+  const unsigned lds_base = (unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)lds;
+  PnSrc m;
+  m.ra = pn_rsrc(c.act);
+  m.rw = pn_rsrc((const void *)tile.w_base);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    m.a_voff[i] = 0;
+    if (i < NB) {
+      // transfer i of this wave brings rows 32 i + 8 w .. + 7, 8 lanes per row; the lane in slot s of row r fetches
+      // chunk s ^ ((r >> 1) & 7).  Byte offsets from the activation tensor's base (< 2 GiB, checked by the launcher)
+      const int rt = 32 * i + 8 * w + (lane >> 3);
+      const int row = rt < tile.rows ? rt : 0;   // rows past the group's end re-read row 0 (never stored)
+      const int grow = tile.row0 + row;
+      const int arow = c.gather ? c.gather[grow] : grow;
+      m.a_voff[i] = arow * c.act_stride * 2 + (((lane & 7) ^ ((rt >> 1) & 7)) * 16);
+    }
+  }
+  // row block t (0..3) of this wave, t = 2 f + h: fragment f's lanes 16 h .. 16 h + 15 (of 32).  w13: gate blocks
+  // (even) are fragment 0, up blocks (odd) fragment 1; w2: column halves 128 apart
+  auto rb = [&](int t) { return SWIGLU ? 16 * nt + 4 * w + (t >> 1) + 2 * (t & 1) : 16 * nt + 2 * w + 8 * (t >> 1) + (t & 1); };
+#pragma unroll
+  for (int f = 0; f < 2; ++f)
+    m.w_voff[f] = (int)c.w_off + rb(2 * f + (n >> 4)) * G * 1024 + (16 * q + (n & 15)) * 16;
+  if (Q4K) {
+    m.s_voff = (int)c.off_s + rb(lane >> 4) * G * 128 + (lane & 15) * 4;
+    m.z_voff = (int)c.off_z + rb(lane >> 4) * (G >> 1) * 64 + (lane & 15) * 4;
+    m.s_step = 0;
+  } else {
+    // lanes 0..31: 8 dwords of scales of each row block; lanes 32..39: 2 dwords of zeros of each; the rest idle copies
+    const int l = lane < 40 ? lane : 39;
+    m.s_voff = l < 32 ? (int)c.off_s + rb(l >> 3) * G * 32 + (l & 7) * 4 : (int)c.off_z + rb((l - 32) >> 1) * G * 8 + (l & 1) * 4;
+    m.s_step = l < 32 ? 32 : 8;
+    m.z_voff = 0;
+  }
+  f32x16_t acc[NB][2];
+#pragma unroll
+  for (int i = 0; i < NB; ++i)
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][h][e] = 0.f;
+  pn_mainloop<NB, Q4K>(acc, lds_base, m, kt0, nk, tid);
+  // epilogue.  acc element e of lane l: row 8*(e/4) + 4*(l/32) + e%4 of its block, column l%32
+  const int col = 32 * w + n;
+  PF_VMCNT(0);   // the transfers past the end have landed: the ring is free, and nothing is in flight at the end
+  if constexpr (SWIGLU) {
+    // the h tile (rows x 128 fp16) leaves through LDS in 16-byte stores over whole 256-byte rows
+    constexpr int HS = 2 * PF_BNH + 16;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < NB; ++i)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int row = 32 * i + 8 * (e >> 2) + 4 * q + (e & 3);
+        *(_Float16 *)(lds + row * HS + col * 2) = (_Float16)pf_silu_mul(acc[i][0][e], acc[i][1][e]);
+      }
+    __syncthreads();
+    const int chunk = tid & 15;
+    for (int row = tid >> 4; row < tile.rows; row += 16)
+      *(uint4 *)((_Float16 *)c.out + (size_t)(tile.row0 + row) * c.out_stride + nt * PF_BNH + 8 * chunk) =
+          *(const uint4 *)(lds + row * HS + chunk * 16);
+  } else {
+    float *out = (float *)c.out + (size_t)split * c.split_stride + nt * 2 * PF_BNH + col;
+#pragma unroll
+    for (int i = 0; i < NB; ++i)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int row = 32 * i + 8 * (e >> 2) + 4 * q + (e & 3);
+        if (row < tile.rows) {
+          float *o = out + (size_t)(tile.row0 + row) * c.out_stride;
+          o[0] = acc[i][0][e];
+          o[PF_BNH] = acc[i][1][e];
+        }
+      }
+  }
+}
 
+template <bool SWIGLU, bool Q4K>
+__global__ __launch_bounds__(256, 2) void k_prefill_nib(const PfArgs a) {
+  extern __shared__ __align__(16) unsigned char lds_n[];
+  const int tid = threadIdx.x;
   // block order: as in k_prefill_gemm
   int ci, pb;
   pf_block_of(a, ci, pb);
@@ -509,64 +638,14 @@ __global__ __launch_bounds__(512, 1) void k_prefill_int4(const PfArgs a) {
   else { mt = bid / c.n_ntiles; nt = bid - mt * c.n_ntiles; }
   const PfTile tile = c.tiles[mt];
   if (tile.rows <= 0) return;
-  const int K = c.K, G = K >> 7;
-  // this workgroup's window of quantisation groups (only the w2 pass is ever split: a constant 0 in the w13 pass)
-  const int Gw = SWIGLU ? G : G / ks, g0 = SWIGLU ? 0 : split * Gw;
-
-  const int ch = tid & 15, r0 = tid >> 4;
-  u32 a_off[6];  // byte offsets into the activation matrix (< 2^31: checked by the launcher)
-#pragma unroll
-  for (int i = 0; i < 6; ++i) {
-    int row = r0 + 32 * i;
-    row = row < tile.rows ? row : 0;  // rows past the group's end re-read row 0 (never stored)
-    const int grow = tile.row0 + row;
-    const int arow = c.gather ? c.gather[grow] : grow;
-    a_off[i] = ((u32)arow * (u32)c.act_stride + ch * 8) * 2;
+  // this workgroup's window of the reduction (only the w2 pass is ever split)
+  const int nk = SWIGLU ? c.K / PF_BK : c.K / PF_BK / ks, kt0 = SWIGLU ? 0 : split * nk;
+  switch ((tile.rows + 31) >> 5) {
+    case 1: pn_tile<1, SWIGLU, Q4K>(c, tile, lds_n, nt, kt0, nk, split, tid); break;
+    case 2: pn_tile<2, SWIGLU, Q4K>(c, tile, lds_n, nt, kt0, nk, split, tid); break;
+    case 3: pn_tile<3, SWIGLU, Q4K>(c, tile, lds_n, nt, kt0, nk, split, tid); break;
+    default: pn_tile<4, SWIGLU, Q4K>(c, tile, lds_n, nt, kt0, nk, split, tid); break;
   }
-  // the wave's 4 consecutive 16-row blocks: (gate, up, gate, up) of two 16-column blocks of
-  // h in the w13 pass, 64 consecutive output columns in the w2 pass
-  const int rb0 = 16 * nt + 4 * w;
-  const unsigned char *base = pf_uniform((const unsigned char *)tile.w_base);
-  const rsrc_t rq = pf_rsrc(base + c.w_off + (size_t)rb0 * G * 1024, 4u * G * 1024u);
-  const rsrc_t rs = pf_rsrc(base + c.off_s + (size_t)rb0 * G * (Q4K ? 128 : 32), 4u * G * (Q4K ? 128u : 32u));
-  const rsrc_t rz = pf_rsrc(base + c.off_z + (size_t)rb0 * G * (Q4K ? 32 : 8), 4u * G * (Q4K ? 32u : 8u));
-  const rsrc_t rx = pf_rsrc(c.act, 0x7fffffffu);
-
-  f32x4_t acc[4][6];
-#pragma unroll
-  for (int t = 0; t < 4; ++t)
-#pragma unroll
-    for (int tb = 0; tb < 6; ++tb) acc[t][tb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-
-  const int nb = (tile.rows + 31) >> 5;
-  const int nbw = (nb - g + 1) >> 1;
-  switch (nbw) {
-    case 0: pi_mainloop<0, Q4K, ACT16>(acc, As, rx, a_off, rq, rs, rz, G, g0, Gw, nb, tid); break;
-    case 1: pi_mainloop<1, Q4K, ACT16>(acc, As, rx, a_off, rq, rs, rz, G, g0, Gw, nb, tid); break;
-    case 2: pi_mainloop<2, Q4K, ACT16>(acc, As, rx, a_off, rq, rs, rz, G, g0, Gw, nb, tid); break;
-    default: pi_mainloop<3, Q4K, ACT16>(acc, As, rx, a_off, rq, rs, rz, G, g0, Gw, nb, tid); break;
-  }
-  // epilogue.  acc[t][tb] element i of lane l: weight row r of tile t, token row
-  // 32*(2*(tb/2)+g) + 16*(tb%2) + 4*qd + i of the tile
-#pragma unroll
-  for (int tb = 0; tb < 6; ++tb)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int row = 32 * (2 * (tb >> 1) + g) + 16 * (tb & 1) + 4 * qd + i;
-      if (row < tile.rows) {
-        const size_t orow = (size_t)(tile.row0 + row) * c.out_stride;
-        if (SWIGLU) {
-#pragma unroll
-          for (int b = 0; b < 2; ++b) {
-            const float gt = acc[2 * b][tb][i], up = acc[2 * b + 1][tb][i];
-            ((_Float16 *)c.out)[orow + 16 * (rb0 / 2 + b) + r] = (_Float16)pf_silu_mul(gt, up);  // h in fp16: what the w2 pass stages
-          }
-        } else {
-#pragma unroll
-          for (int t = 0; t < 4; ++t) ((float *)c.out)[(size_t)split * c.split_stride + orow + 16 * (rb0 + t) + r] = acc[t][tb][i];
-        }
-      }
-    }
 }
 
 
@@ -578,26 +657,22 @@ static int pf_slab_step(int nk) {
 }
 
 template <bool Q4K>
-static int pi_launch(bool swiglu, bool x16, const PfArgs &a, hipStream_t s) {
+static int pn_launch(bool swiglu, const PfArgs &a, hipStream_t s) {
   if (a.n_blocks_total <= 0) return MOE_OK;
   const int grid = ((a.c[0].n_blocks + 7) & ~7) + ((a.c[1].n_blocks + 7) & ~7);
-  const size_t lds = (size_t)2 * PI_BM * PI_LDK * 2;
   static bool attr_set = false;
   if (!attr_set) {
-    for (const void *f : {(const void *)k_prefill_int4<true, Q4K, false>, (const void *)k_prefill_int4<true, Q4K, true>,
-                          (const void *)k_prefill_int4<false, Q4K, true>})
-      if (int rc = moe_check_hip(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds),
-                                 "hipFuncSetAttribute(k_prefill_int4)"))
+    for (const void *f : {(const void *)k_prefill_nib<true, Q4K>, (const void *)k_prefill_nib<false, Q4K>})
+      if (int rc = moe_check_hip(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, PN_LDS),
+                                 "hipFuncSetAttribute(k_prefill_nib)"))
         return rc;
     attr_set = true;
   }
   moe_ktimer_begin(swiglu ? MOE_K_PREFILL_W13 : MOE_K_PREFILL_W2, s);
-  // the w2 pass reads the fp16 h rows of the w13 pass; the w13 pass reads bf16 x, or its fp16 copy when there is one
-  if (swiglu && x16) hipLaunchKernelGGL((k_prefill_int4<true, Q4K, true>), dim3(grid), dim3(512), lds, s, a);
-  else if (swiglu) hipLaunchKernelGGL((k_prefill_int4<true, Q4K, false>), dim3(grid), dim3(512), lds, s, a);
-  else hipLaunchKernelGGL((k_prefill_int4<false, Q4K, true>), dim3(grid), dim3(512), lds, s, a);
+  if (swiglu) hipLaunchKernelGGL((k_prefill_nib<true, Q4K>), dim3(grid), dim3(256), PN_LDS, s, a);
+  else hipLaunchKernelGGL((k_prefill_nib<false, Q4K>), dim3(grid), dim3(256), PN_LDS, s, a);
   moe_ktimer_end(swiglu ? MOE_K_PREFILL_W13 : MOE_K_PREFILL_W2, s);
-  return moe_check_launch("k_prefill_int4");
+  return moe_check_launch("k_prefill_nib");
 }
 
 static int pf_launch(bool swiglu, const PfArgs &a, hipStream_t s) {
@@ -622,16 +697,26 @@ static int pf_launch(bool swiglu, const PfArgs &a, hipStream_t s) {
 // One entry per tile of every active expert's token group (routed list: groups of more than
 // 256 rows are split evenly), and one per 256 / 128 tokens for the shared expert's two passes.  Built on the device from the dispatch result, so
 // the host never needs the counts: the launch covers the upper bound on the number of
-// blocks and entries past the real count have rows = 0.
+// blocks and entries past the real count have rows = 0.  Nibble formats: the same launch converts x to fp16 for the
+// w13 pass (8 MB read and written for 2048 x 2048, hidden behind the 4 us that the list takes).
 __global__ __launch_bounds__(1024) void k_prefill_tiles(const moe_unit *__restrict__ units, int max_units,
                                                         const unsigned long long *__restrict__ expert_ptr,
                                                         PfTile *__restrict__ tiles, int n_tiles_max,
                                                         PfTile *__restrict__ sh_tiles, int n_sh_tiles,
                                                         PfTile *__restrict__ sh_tiles2, int n_sh_tiles2,
                                                         unsigned long long shared_base, int T, int cap, int cap_s, int cap_s2,
-                                                        int *__restrict__ n_real, int *__restrict__ err) {
+                                                        int *__restrict__ n_real, int *__restrict__ err,
+                                                        const u32x4_t *__restrict__ x, u32x4_t *__restrict__ x16, int n16) {
   __shared__ int scan[1024];
   const int tid = threadIdx.x;
+  if (blockIdx.x > 0) {  // workgroups behind the first: the fp16 copy of the activations (8 values per thread)
+    const int i = ((int)blockIdx.x - 1) * 1024 + tid;
+    if (i < n16) {
+      const u32x4_t v = x[i];
+      x16[i] = u32x4_t{bf16x2_to_f16x2(v.x), bf16x2_to_f16x2(v.y), bf16x2_to_f16x2(v.z), bf16x2_to_f16x2(v.w)};
+    }
+    return;
+  }
   int total_prev = 0;
   for (int base = 0; base < max_units; base += 1024) {
     const int u = base + tid;
@@ -686,6 +771,11 @@ extern "C" int moe_prefill_tile_rows(void) { return PF_BM; }
 extern "C" int64_t moe_prefill_workspace_bytes(int T, int k, int max_units) {
   const int64_t P = (int64_t)T * k;
   return (P / 128 + max_units + 2 * ((T + 127) / 128) + 3) * (int64_t)sizeof(PfTile);  // covers every tile height in use (>= 128)
+}
+
+// where the fp16 copy of the activations stands in a workspace with room for it (phase bit 2)
+static int64_t pf_x16_offset(int T, int k, int max_units) {
+  return (moe_prefill_workspace_bytes(T, k, max_units) + 255) & ~(int64_t)255;
 }
 
 // Pieces the w2 pass leaves the shared expert's partial rows in (moe_experts_prefill_pieces).  The shared expert's
@@ -756,15 +846,29 @@ extern "C" int moe_experts_prefill_pieces(const void *x_bf16, int T, int H, int 
     return MOE_EINVAL;
   }
   const long long P = (long long)T * k;
-  const int cap = int4 ? PI_BM : PF_BM, cap_s = int4 ? PI_BM : PF_BM_SHARED, cap_s2 = PF_BM_SHARED_W2;
+  const int cap = int4 ? PN_BM : PF_BM, cap_s = int4 ? PN_BM : PF_BM_SHARED, cap_s2 = PF_BM_SHARED_W2;
+  // fp16 copy of x for the nibble formats: behind the tile list where the caller left room, else stream-ordered memory
+  void *x16 = nullptr, *x16_own = nullptr;
+  const bool convert = int4 && (phases & 1) && !((phases & 4) && (phases & 8));
+  if (int4 && (phases & 1)) {
+    if (phases & 4) x16 = (unsigned char *)tiles_ws + pf_x16_offset(T, k, max_units);
+    else if (int rc = moe_check_hip(hipMallocAsync(&x16_own, (size_t)T * H * 2, s), "hipMallocAsync(fp16 activations)")) return rc;
+    if (x16_own) x16 = x16_own;
+  }
+  struct FreeX16 {  // on every way out
+    void *p; hipStream_t s;
+    ~FreeX16() { if (p) (void)hipFreeAsync(p, s); }
+  } free_x16{x16_own, s};
+  const int n16 = convert ? (int)((long long)T * H / 8) : 0;
   const int n_r = (int)(P / cap) + max_units;
   const int n_s = shared_ptr ? (T + cap_s - 1) / cap_s : 0;
   const int n_s2 = shared_ptr ? (T + cap_s2 - 1) / cap_s2 : 0;
   int *n_real = (int *)tiles_ws;  // [0] routed tiles in use, [1] shared tiles (w13 pass), [2] shared tiles (w2 pass)
   PfTile *tiles = (PfTile *)tiles_ws + 1, *sh_tiles = tiles + n_r, *sh_tiles2 = sh_tiles + n_s;
-  hipLaunchKernelGGL(k_prefill_tiles, dim3(1), dim3(1024), 0, s, units, max_units,
+  hipLaunchKernelGGL(k_prefill_tiles, dim3(1 + (n16 + 1023) / 1024), dim3(1024), 0, s, units, max_units,
                      (const unsigned long long *)expert_ptr, tiles, n_r, sh_tiles, n_s, sh_tiles2, n_s2,
-                     (unsigned long long)(uintptr_t)shared_ptr, T, cap, cap_s, cap_s2, n_real, err);
+                     (unsigned long long)(uintptr_t)shared_ptr, T, cap, cap_s, cap_s2, n_real, err, (const u32x4_t *)x_bf16,
+                     (u32x4_t *)x16, n16);
   if (int rc = moe_check_launch("k_prefill_tiles")) return rc;
   for (int w2 = 0; w2 < 2; ++w2) {
     if (!(phases & (w2 ? 2 : 1))) continue;
@@ -781,7 +885,7 @@ extern "C" int moe_experts_prefill_pieces(const void *x_bf16, int T, int H, int 
       c.n_tiles_real = n_real + (shared ? (w2 ? 2 : 1) : 0);
       c.m_fastest = shared;
       if (!w2) {  // w13 [2I, H]: gate rows 0..I-1, up rows I..2I-1
-        c.act = (const uint16_t *)x_bf16; c.gather = shared ? nullptr : sorted_tok; c.act_stride = H;
+        c.act = (const uint16_t *)(int4 ? x16 : x_bf16); c.gather = shared ? nullptr : sorted_tok; c.act_stride = H;
         c.out = shared ? h_s : h_r; c.out_stride = Ii;
         c.K = H; c.w_off = 0; c.half_delta = Ii; c.n_cols_per_tile = PF_BNH; c.n_ntiles = Ii / PF_BNH;
       } else {    // w2 [H, I] after w13 in the expert image
@@ -803,7 +907,7 @@ extern "C" int moe_experts_prefill_pieces(const void *x_bf16, int T, int H, int 
       c.slab_step = pf_slab_step(c.K / PF_BK);
       a.n_blocks_total += c.n_blocks;
     }
-    if (int rc = q4k ? pi_launch<true>(!w2, false, a, s) : (int4 ? pi_launch<false>(!w2, false, a, s) : pf_launch(!w2, a, s))) return rc;
+    if (int rc = q4k ? pn_launch<true>(!w2, a, s) : (int4 ? pn_launch<false>(!w2, a, s) : pf_launch(!w2, a, s))) return rc;
   }
   return MOE_OK;
 }

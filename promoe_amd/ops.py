@@ -326,6 +326,12 @@ def experts_decode_q4k(x, d: Dispatch, expert_ptr: torch.Tensor, shared: torch.T
     return part_r, part_s, err, h_r, h_s
 
 
+def prefill_workspace_bytes(fmt: int, T: int, H: int, k: int, max_units: int) -> int:
+    """Workspace of experts_prefill: the tile list and, for the nibble formats, the fp16 copy of the activations."""
+    n = max(int(lib.moe_prefill_workspace_bytes(T, k, max_units)), 16)
+    return n if fmt == L.FMT_BF16 else ((n + 255) & ~255) + T * H * 2
+
+
 def experts_prefill(x, d: Dispatch, expert_ptr: torch.Tensor, shared: torch.Tensor | None,
                     H: int, I: int, I_sh: int, fmt: int = L.FMT_BF16, phases: int = 3, ws=None):
     """MFMA grouped expert product.  Returns (part_r, part_s, err, h_r, h_s, tiles).  part_s has S*T rows, S =
@@ -343,7 +349,10 @@ def experts_prefill(x, d: Dispatch, expert_ptr: torch.Tensor, shared: torch.Tens
             h_s = torch.empty(T, I_sh, dtype=torch.bfloat16, device=dev)
             part_s = torch.empty(int(lib.moe_prefill_shared_splits(fmt, T, H, I_sh)) * T, H, dtype=torch.float32, device=dev)
         err = torch.zeros(1, dtype=torch.int32, device=dev)
-        tiles = torch.empty(max(int(lib.moe_prefill_workspace_bytes(T, k, d.max_units)), 16), dtype=torch.uint8, device=dev)
+        # (nibble formats: behind the tile list, room for the fp16 copy of the activations)
+        tiles = torch.empty(prefill_workspace_bytes(fmt, T, H, k, d.max_units), dtype=torch.uint8, device=dev)
+    if fmt != L.FMT_BF16 and tiles.numel() >= prefill_workspace_bytes(fmt, T, H, k, d.max_units):
+        phases |= 4
     pieces = 1
     if part_s is not None:
         pieces = int(lib.moe_prefill_shared_splits(fmt, T, H, I_sh))

@@ -146,3 +146,31 @@ def test_prefill_wide_shared_expert_in_pieces(cuda):
     check_prefill(Q4KLayer(H=256, I=256, E=4, I_sh=16384, seed=6, shared_gate=True), 130, 2, 0, cuda)
     check_prefill(Int4Layer(H=256, I=128, E=4, I_sh=8192, seed=7), 200, 2, 1, cuda)
     check_prefill(Int4Layer(H=512, I=128, E=4, I_sh=8192, seed=8), 70, 2, 0, cuda)   # 1 x 2 tiles: 2 pieces, short last tile
+
+
+@pytest.mark.parametrize("cls,I", [(Int4Layer, 128), (Q4KLayer, 256)])
+@pytest.mark.parametrize("T", [31, 32, 33, 127, 128, 129, 257])
+def test_prefill_nibble_tile_edges(cuda, T, cls, I):
+    """Every token to one expert: row blocks of 32 and tiles of 128 rows just short, full and just over; reductions of
+    two slabs (shorter than the ring they go through) and of eight."""
+    print(f"case prefill_nibble_edges T={T} {cls.__name__}", flush=True)
+    check_prefill(cls(H=512, I=I, E=1, I_sh=I, seed=9), T, 1, 0, cuda)
+
+
+def test_prefill_nibble_without_room_for_the_converted_activations(cuda):
+    """A workspace without room for the fp16 copy of x (phase bit 2 not set): the call takes memory of its own, same bits."""
+    from promoe_amd import ops, _lib as L
+    print("case prefill_no_room", flush=True)
+    layer = Int4Layer(H=256, I=128, E=4, I_sh=128, seed=10)
+    x = bf16_dev(O.synth_acts(70, 256), cuda)
+    idx, _ = ops.topk(ops.gate_logits(x, bf16_dev(layer.wg, cuda), None), 2, 0)
+    d = ops.dispatch(idx, 4)
+    slots = [torch.from_numpy(s).to(cuda) for s in layer.slots]
+    table = torch.tensor([s.data_ptr() for s in slots], dtype=torch.int64, device=cuda)
+    shared = torch.from_numpy(layer.shared_img).to(cuda)
+    a = ops.experts_prefill(x, d, table, shared, 256, 128, 128, L.FMT_INT4_G128)
+    small = torch.empty(int(L.lib.moe_prefill_workspace_bytes(70, 2, d.max_units)), dtype=torch.uint8, device=cuda)
+    ws = tuple(torch.zeros_like(t) for t in a[:5]) + (small,)
+    b = ops.experts_prefill(x, d, table, shared, 256, 128, 128, L.FMT_INT4_G128, ws=ws)
+    torch.cuda.synchronize()
+    assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1]) and int(b[2].item()) == 0

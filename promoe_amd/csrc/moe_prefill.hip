@@ -31,8 +31,9 @@ typedef float f32x16_t __attribute__((ext_vector_type(16)));
 struct PfTile {
   unsigned long long w_base;  // expert image base (device address)
   int row0;                   // first row (sorted pair order / token order for the shared expert)
-  int rows;                   // valid rows in this tile (<= PF_BM)
+  int rows_group;             // bits 0-15 valid rows (<= PF_BM), 16-23 tiles in its group, 24-31 its place in the group
 };
+static __device__ __forceinline__ int pf_rows(const PfTile &t) { return t.rows_group & 0xffff; }
 // one GEMM problem class of a launch (routed experts / shared expert)
 struct PfClass {
   const uint16_t *act;  // bf16 activations
@@ -44,9 +45,9 @@ struct PfClass {
   long long half_delta; // weight-row offset of the second column half relative to the first
   long long off_s, off_z; // int4: byte offsets of the scale / zero sections (w_off = the nibble section)
   int act_stride, out_stride, K, n_ntiles, n_mtiles, n_cols_per_tile;
-  int m_fastest;        // block order inside the class
+  int shared;           // the shared expert's class
   int slab_step;        // storage rotation per 128-row group: smallest odd s >= 3 coprime with K/64
-  int n_blocks;         // n_mtiles * n_ntiles * ksplit
+  int n_blocks;         // n_mtiles * n_ntiles * ksplit, padded to whole rounds of runs (pf_block_of)
   int ksplit;           // int4 / q4_K w2 pass of the shared expert: workgroups per tile, each over 1/ksplit of the
                         // reduction, partial rows to out + split * split_stride (0 or 1: the whole reduction)
   long long split_stride;  // elements between the pieces of out
@@ -62,13 +63,44 @@ static __device__ __forceinline__ float pf_silu_mul(float g, float u) {
   return g * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(g * -1.44269504088896f)) * u;
 }
 
-// Which class and which block of it a physical workgroup takes: the blocks of class 0 come first, each class
-// padded to a multiple of 8 blocks, so that physical id % 8 is the XCD inside either class.  (Alternating the
-// classes in groups of 8 was measured: no gain in the w13 launch, 19 % slower in the w2 launch.)
-static __device__ __forceinline__ void pf_block_of(const PfArgs &a, int &ci, int &pb) {
-  const int pad0 = (a.c[0].n_blocks + 7) & ~7;
+// Which block of which class a physical workgroup takes; false: none.  The blocks of class 0 come first, each class
+// padded to a multiple of 8 PF_DEAL.  Workgroup i runs on XCD i % 8; runs of PF_DEAL consecutive blocks are dealt to
+// the XCDs in turn, over both classes (class 1 goes on where class 0 ended), so that the XCDs get the same number of
+// blocks of every size whatever the row counts are: the list holds the large tiles first.  (One contiguous range of the
+// list per XCD, the order before this one, left the XCDs with the popular experts' tiles busy alone: 1.4 of 2 waves per
+// SIMD on average over the w13 launch of the DeepSeek shape at 2048 tokens, 1.0 at 379.)
+// Inside the list: a group of up to PF_GROUP tiles of one expert goes through all its column tiles, tile fastest, so
+// that a run shares either a column tile's weights (many tiles) or the activation rows (one tile) in its XCD's L2.
+// Measured on one box, us a layer: DeepSeek shape 379 tokens 156 -> 148, 2048 tokens 378 -> 365, Mixtral shape 4096
+// tokens 2748 -> 2560 (eight row tiles share a column tile's weights); Qwen1.5 bf16 and q4_K prefill unchanged.
+#define PF_DEAL 8
+#define PF_GROUP 8
+static __device__ __forceinline__ bool pf_block_of(const PfArgs &a, int &ci, int &mt, int &nt, int &split) {
+  const int pad0 = a.c[0].n_blocks;
   ci = (int)blockIdx.x >= pad0;
-  pb = ci ? (int)blockIdx.x - pad0 : (int)blockIdx.x;
+  const int pb = ci ? (int)blockIdx.x - pad0 : (int)blockIdx.x;
+  const PfClass &c = a.c[ci];
+  const int ks = c.ksplit > 1 ? c.ksplit : 1;
+  const int n_tiles = *c.n_tiles_real * c.n_ntiles, n_real = n_tiles * ks;
+  int xcd = pb & 7;
+  if (ci) {
+    const int n0 = *a.c[0].n_tiles_real * a.c[0].n_ntiles * (a.c[0].ksplit > 1 ? a.c[0].ksplit : 1);
+    xcd = (xcd - (n0 + PF_DEAL - 1) / PF_DEAL) & 7;
+  }
+  const int i = pb >> 3;
+  int b = ((i / PF_DEAL) * 8 + xcd) * PF_DEAL + i % PF_DEAL;
+  if (b >= n_real) return false;
+  // a class whose reduction is split has ksplit workgroups per tile: the pieces of one tile are `n_tiles` blocks
+  // apart, so that the first piece of every tile starts before the second of any
+  split = b / n_tiles;
+  b -= split * n_tiles;
+  mt = b / c.n_ntiles;
+  const int grp = c.tiles[mt].rows_group >> 16, size = grp & 0xff;
+  mt -= (grp >> 8) & 0xff;               // the group's first tile
+  b -= mt * c.n_ntiles;
+  nt = b / size;
+  mt += b - nt * size;
+  return true;
 }
 
 // ---- bf16 experts: main loop of one wave ------------------------------------------------------------
@@ -213,24 +245,12 @@ template <bool SWIGLU>
 __global__ __launch_bounds__(256, 1) void k_prefill_gemm(const PfArgs a) {
   extern __shared__ __align__(16) uint16_t As[];  // [PF4_RING][PF_BM][PF_BK]
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  // XCD-aware order: workgroup i runs on XCD i % 8; give every XCD one contiguous range of the block list,
-  // so that blocks that share an operand (n tiles of one m tile for the routed experts, m tiles of one n
-  // tile for the shared expert) meet in one L2.  Only the tiles in use are spread over the XCDs; the launch
-  // covers an upper bound.
-  int ci, pb;
-  pf_block_of(a, ci, pb);
-  const int n_mt = *a.c[ci].n_tiles_real;
-  const int n_real = n_mt * a.c[ci].n_ntiles;
-  const int per_xcd = (n_real + 7) >> 3;
-  if ((pb >> 3) >= per_xcd) return;
-  int bid = (pb & 7) * per_xcd + (pb >> 3);
-  if (bid >= n_real) return;
+  int ci, mt, nt, split;
+  if (!pf_block_of(a, ci, mt, nt, split)) return;
   const PfClass &c = a.c[ci];
-  int mt, nt;
-  if (c.m_fastest) { nt = bid / n_mt; mt = bid - nt * n_mt; }
-  else { mt = bid / c.n_ntiles; nt = bid - mt * c.n_ntiles; }
   const PfTile tile = c.tiles[mt];
-  if (tile.rows <= 0) return;
+  const int rows = pf_rows(tile);
+  if (rows <= 0) return;
   const int K = c.K;
   const int n0 = nt * c.n_cols_per_tile;
   const uint16_t *W = (const uint16_t *)(tile.w_base + c.w_off);
@@ -241,7 +261,7 @@ __global__ __launch_bounds__(256, 1) void k_prefill_gemm(const PfArgs a) {
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
     const int rt = 32 * i + 8 * w + (lane >> 3);
-    const int row = rt < tile.rows ? rt : 0;  // rows past the group's end re-read row 0 (never stored)
+    const int row = rt < rows ? rt : 0;  // rows past the group's end re-read row 0 (never stored)
     const int grow = tile.row0 + row;
     const int arow = c.gather ? c.gather[grow] : grow;
     a_voff[i] = (arow * c.act_stride + (((lane & 7) ^ ((rt >> 1) & 7)) * 8)) * 2;
@@ -273,7 +293,7 @@ __global__ __launch_bounds__(256, 1) void k_prefill_gemm(const PfArgs a) {
 
   const int G0 = n0 / 128, G1 = G0 + (int)(c.half_delta / 128);
   const int rot0 = (int)((unsigned)(G0 * c.slab_step) % (unsigned)nk), rot1 = (int)((unsigned)(G1 * c.slab_step) % (unsigned)nk);
-  const int nb = (tile.rows + 31) >> 5;  // live row blocks (uniform for the workgroup)
+  const int nb = (rows + 31) >> 5;  // live row blocks (uniform for the workgroup)
   const unsigned lds_base = (unsigned)(uintptr_t)(__attribute__((address_space(3))) uint16_t *)As;
 #define PF_LOOPS(NTW_)                                                                                          \
   switch (nb) {                                                                                             \
@@ -286,7 +306,7 @@ __global__ __launch_bounds__(256, 1) void k_prefill_gemm(const PfArgs a) {
     case 7: pf_mainloop<7, NTW_>(acc, lds_base, ra_rsrc, a_voff, rb, b_delta1, nk, rot0, rot1, tid); break; \
     default: pf_mainloop<8, NTW_>(acc, lds_base, ra_rsrc, a_voff, rb, b_delta1, nk, rot0, rot1, tid); break; \
   }
-  if (c.m_fastest) { PF_LOOPS(false) } else { PF_LOOPS(true) }   // (m_fastest: the shared expert's class)
+  if (c.shared) { PF_LOOPS(false) } else { PF_LOOPS(true) }
 #undef PF_LOOPS
   // epilogue.  acc element e of lane l: row 8*(e/4) + 4*(l/32) + e%4, column l%32
   const int col = 32 * w + (lane & 31);
@@ -311,7 +331,7 @@ __global__ __launch_bounds__(256, 1) void k_prefill_gemm(const PfArgs a) {
       }
     __syncthreads();
     const int chunk = tid & 15;
-    for (int row = tid >> 4; row < tile.rows; row += 16) {
+    for (int row = tid >> 4; row < rows; row += 16) {
       const uint4 v = *(const uint4 *)(hs + row * HS + chunk * 16);
       *(uint4 *)((__bf16 *)c.out + (size_t)(tile.row0 + row) * c.out_stride + n0 + 8 * chunk) = v;
     }
@@ -322,7 +342,7 @@ __global__ __launch_bounds__(256, 1) void k_prefill_gemm(const PfArgs a) {
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
       const int row = 32 * i + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3);
-      if (row < tile.rows) {
+      if (row < rows) {
         const size_t orow = (size_t)(tile.row0 + row) * c.out_stride;
         if (SWIGLU) {
           ((__bf16 *)c.out)[orow + n0 + col] = (__bf16)pf_silu_mul(acc[i][0][e], acc[i][1][e]);
@@ -535,7 +555,7 @@ static __device__ __forceinline__ void pn_tile(const PfClass &c, const PfTile &t
                                                int split, int tid) {
   const int lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = lane & 31, q = lane >> 5;
-  const int G = c.K >> 7;
+  const int G = c.K >> 7, rows = pf_rows(tile);
   const unsigned lds_base = (unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)lds;
   PnSrc m;
   m.ra = pn_rsrc(c.act);
@@ -547,7 +567,7 @@ static __device__ __forceinline__ void pn_tile(const PfClass &c, const PfTile &t
       // transfer i of this wave brings rows 32 i + 8 w .. + 7, 8 lanes per row; the lane in slot s of row r fetches
       // chunk s ^ ((r >> 1) & 7).  Byte offsets from the activation tensor's base (< 2 GiB, checked by the launcher)
       const int rt = 32 * i + 8 * w + (lane >> 3);
-      const int row = rt < tile.rows ? rt : 0;   // rows past the group's end re-read row 0 (never stored)
+      const int row = rt < rows ? rt : 0;   // rows past the group's end re-read row 0 (never stored)
       const int grow = tile.row0 + row;
       const int arow = c.gather ? c.gather[grow] : grow;
       m.a_voff[i] = arow * c.act_stride * 2 + (((lane & 7) ^ ((rt >> 1) & 7)) * 16);
@@ -594,7 +614,7 @@ static __device__ __forceinline__ void pn_tile(const PfClass &c, const PfTile &t
       }
     __syncthreads();
     const int chunk = tid & 15;
-    for (int row = tid >> 4; row < tile.rows; row += 16)
+    for (int row = tid >> 4; row < rows; row += 16)
       *(uint4 *)((_Float16 *)c.out + (size_t)(tile.row0 + row) * c.out_stride + nt * PF_BNH + 8 * chunk) =
           *(const uint4 *)(lds + row * HS + chunk * 16);
   } else {
@@ -604,7 +624,7 @@ static __device__ __forceinline__ void pn_tile(const PfClass &c, const PfTile &t
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
         const int row = 32 * i + 8 * (e >> 2) + 4 * q + (e & 3);
-        if (row < tile.rows) {
+        if (row < rows) {
           float *o = out + (size_t)(tile.row0 + row) * c.out_stride;
           o[0] = acc[i][0][e];
           o[PF_BNH] = acc[i][1][e];
@@ -617,30 +637,16 @@ template <bool SWIGLU, bool Q4K>
 __global__ __launch_bounds__(256, 2) void k_prefill_nib(const PfArgs a) {
   extern __shared__ __align__(16) unsigned char lds_n[];
   const int tid = threadIdx.x;
-  // block order: as in k_prefill_gemm
-  int ci, pb;
-  pf_block_of(a, ci, pb);
+  int ci, mt, nt, split;
+  if (!pf_block_of(a, ci, mt, nt, split)) return;
   const PfClass &c = a.c[ci];
-  const int n_mt = *c.n_tiles_real;
-  // a class whose reduction is split has ksplit workgroups per tile: the pieces of one tile are `n_tiles`
-  // blocks apart, so that the first piece of every tile starts before the second of any
-  const int ks = c.ksplit > 1 ? c.ksplit : 1;
-  const int n_tiles = n_mt * c.n_ntiles;
-  const int n_real = n_tiles * ks;
-  const int per_xcd = (n_real + 7) >> 3;
-  if ((pb >> 3) >= per_xcd) return;
-  int bid = (pb & 7) * per_xcd + (pb >> 3);
-  if (bid >= n_real) return;
-  const int split = bid / n_tiles;
-  bid -= split * n_tiles;
-  int mt, nt;
-  if (c.m_fastest) { nt = bid / n_mt; mt = bid - nt * n_mt; }
-  else { mt = bid / c.n_ntiles; nt = bid - mt * c.n_ntiles; }
   const PfTile tile = c.tiles[mt];
-  if (tile.rows <= 0) return;
+  const int rows = pf_rows(tile);
+  if (rows <= 0) return;
+  const int ks = c.ksplit > 1 ? c.ksplit : 1;
   // this workgroup's window of the reduction (only the w2 pass is ever split)
   const int nk = SWIGLU ? c.K / PF_BK : c.K / PF_BK / ks, kt0 = SWIGLU ? 0 : split * nk;
-  switch ((tile.rows + 31) >> 5) {
+  switch ((rows + 31) >> 5) {
     case 1: pn_tile<1, SWIGLU, Q4K>(c, tile, lds_n, nt, kt0, nk, split, tid); break;
     case 2: pn_tile<2, SWIGLU, Q4K>(c, tile, lds_n, nt, kt0, nk, split, tid); break;
     case 3: pn_tile<3, SWIGLU, Q4K>(c, tile, lds_n, nt, kt0, nk, split, tid); break;
@@ -659,7 +665,7 @@ static int pf_slab_step(int nk) {
 template <bool Q4K>
 static int pn_launch(bool swiglu, const PfArgs &a, hipStream_t s) {
   if (a.n_blocks_total <= 0) return MOE_OK;
-  const int grid = ((a.c[0].n_blocks + 7) & ~7) + ((a.c[1].n_blocks + 7) & ~7);
+  const int grid = a.c[0].n_blocks + a.c[1].n_blocks;
   static bool attr_set = false;
   if (!attr_set) {
     for (const void *f : {(const void *)k_prefill_nib<true, Q4K>, (const void *)k_prefill_nib<false, Q4K>})
@@ -677,7 +683,7 @@ static int pn_launch(bool swiglu, const PfArgs &a, hipStream_t s) {
 
 static int pf_launch(bool swiglu, const PfArgs &a, hipStream_t s) {
   if (a.n_blocks_total <= 0) return MOE_OK;
-  const int grid = ((a.c[0].n_blocks + 7) & ~7) + ((a.c[1].n_blocks + 7) & ~7);
+  const int grid = a.c[0].n_blocks + a.c[1].n_blocks;
   const size_t lds = (size_t)PF4_RING * PF4_SLAB * 2;
   static bool attr_set = false;
   if (!attr_set) {
@@ -694,11 +700,19 @@ static int pf_launch(bool swiglu, const PfArgs &a, hipStream_t s) {
 }
 
 // ---- tile list ------------------------------------------------------------------------
-// One entry per tile of every active expert's token group (routed list: groups of more than
-// 256 rows are split evenly), and one per 256 / 128 tokens for the shared expert's two passes.  Built on the device from the dispatch result, so
-// the host never needs the counts: the launch covers the upper bound on the number of
-// blocks and entries past the real count have rows = 0.  Nibble formats: the same launch converts x to fp16 for the
-// w13 pass (8 MB read and written for 2048 x 2048, hidden behind the 4 us that the list takes).
+// One entry per tile of every active expert's token group (routed list: a group of more rows than a tile holds is
+// split evenly), and one per tile of tokens for the shared expert's two passes.  Built on the device from the
+// dispatch result, so the host never needs the counts: the launch covers the upper bound on the number of blocks and
+// entries past the real count have rows = 0.  The routed list is in order of tile height, the tallest first (four
+// classes; expert order inside a class), so that no long workgroup starts when the launch is nearly over.
+// Nibble formats: the same launch converts x to fp16 for the w13 pass (8 MB read and written for 2048 x 2048, hidden
+// behind the 4 us that the list takes).
+static __device__ __forceinline__ PfTile pf_make_tile(unsigned long long w_base, int row0, int rows, int i, int n) {
+  PfTile t;                                  // tile i of n of one expert
+  const int g0 = i / PF_GROUP * PF_GROUP;
+  t.w_base = w_base; t.row0 = row0; t.rows_group = rows | (min(PF_GROUP, n - g0) << 16) | ((i - g0) << 24);
+  return t;
+}
 __global__ __launch_bounds__(1024) void k_prefill_tiles(const moe_unit *__restrict__ units, int max_units,
                                                         const unsigned long long *__restrict__ expert_ptr,
                                                         PfTile *__restrict__ tiles, int n_tiles_max,
@@ -707,8 +721,7 @@ __global__ __launch_bounds__(1024) void k_prefill_tiles(const moe_unit *__restri
                                                         unsigned long long shared_base, int T, int cap, int cap_s, int cap_s2,
                                                         int *__restrict__ n_real, int *__restrict__ err,
                                                         const u32x4_t *__restrict__ x, u32x4_t *__restrict__ x16, int n16) {
-  __shared__ int scan[1024];
-  const int tid = threadIdx.x;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   if (blockIdx.x > 0) {  // workgroups behind the first: the fp16 copy of the activations (8 values per thread)
     const int i = ((int)blockIdx.x - 1) * 1024 + tid;
     if (i < n16) {
@@ -717,53 +730,65 @@ __global__ __launch_bounds__(1024) void k_prefill_tiles(const moe_unit *__restri
     }
     return;
   }
-  int total_prev = 0;
-  for (int base = 0; base < max_units; base += 1024) {
-    const int u = base + tid;
-    int m = 0, row0 = 0;
-    unsigned long long wb = 0;
+  __shared__ int total[4], wsum[16][4];
+  if (tid < 4) total[tid] = 0;
+  for (int i = tid; i < n_sh_tiles; i += 1024)
+    sh_tiles[i] = pf_make_tile(shared_base, i * cap_s, min(cap_s, T - i * cap_s), i, n_sh_tiles);
+  for (int i = tid; i < n_sh_tiles2; i += 1024)
+    sh_tiles2[i] = pf_make_tile(shared_base, i * cap_s2, min(cap_s2, T - i * cap_s2), i, n_sh_tiles2);
+  __syncthreads();
+  // tiles of unit u: nt of up to `per` rows (a multiple of 32); class 0 = the tallest quarter
+  int m = 0, row0 = 0, nt = 0, per = 0, cls = 0;
+  unsigned long long wb = 0;
+  auto load = [&](int u, bool report) {
+    m = 0; wb = 0; row0 = 0;
     if (u < max_units) {
       const moe_unit un = units[u];
       if (un.m > 0 && un.expert >= 0) {
         wb = expert_ptr[un.expert];
         if (wb) { m = un.m; row0 = un.row0; }
-        else moe_raise_err(err);
+        else if (report) moe_raise_err(err);
       }
     }
-    const int nt = (m + cap - 1) / cap;
-    // rows of a group are split evenly over its tiles, in multiples of 32
-    const int per = nt ? ((((m + nt - 1) / nt) + 31) & ~31) : 0;
-    scan[tid] = nt;
-    __syncthreads();
-    for (int d = 1; d < 1024; d <<= 1) {
-      const int v = tid >= d ? scan[tid - d] : 0;
-      __syncthreads();
-      scan[tid] += v;
-      __syncthreads();
+    nt = (m + cap - 1) / cap;
+    per = nt ? ((((m + nt - 1) / nt) + 31) & ~31) : 0;
+    cls = nt ? min(3, (cap - per) * 4 / cap) : 0;
+  };
+  for (int base = 0; base < max_units; base += 1024) {
+    load(base + tid, true);
+    if (nt) atomicAdd(&total[cls], nt);
+  }
+  __syncthreads();
+  int done[4] = {0, total[0], total[0] + total[1], total[0] + total[1] + total[2]};  // first free entry per class
+  const int n_all = done[3] + total[3];
+  for (int base = 0; base < max_units; base += 1024) {
+    if (max_units > 1024) load(base + tid, false);
+    // tiles of the same class in front of this unit's: inside the wave, then the waves before
+    int pos = 0;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      int v = cls == c ? nt : 0;
+      const int own = v;
+#pragma unroll
+      for (int d = 1; d < 64; d <<= 1) {
+        const int o = __shfl_up(v, d);
+        if (lane >= d) v += o;
+      }
+      if (lane == 63) wsum[wave][c] = v;
+      if (cls == c) pos = v - own;
     }
-    const int first = total_prev + scan[tid] - nt;
+    __syncthreads();
+    int first = done[cls] + pos;
+    for (int w = 0; w < 16; ++w) {
+      if (w < wave) first += wsum[w][cls];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) done[c] += wsum[w][c];
+    }
     for (int i = 0; i < nt; ++i)
-      if (first + i < n_tiles_max) {
-        PfTile t;
-        t.w_base = wb; t.row0 = row0 + i * per; t.rows = max(0, min(per, m - i * per));
-        tiles[first + i] = t;
-      }
-    total_prev += scan[1023];
+      if (first + i < n_tiles_max) tiles[first + i] = pf_make_tile(wb, row0 + i * per, max(0, min(per, m - i * per)), i, nt);
     __syncthreads();
   }
-  if (tid == 0) { n_real[0] = min(total_prev, n_tiles_max); n_real[1] = n_sh_tiles; n_real[2] = n_sh_tiles2; }
-  for (int i = total_prev + tid; i < n_tiles_max; i += 1024) {
-    PfTile t; t.w_base = 0; t.row0 = 0; t.rows = 0;
-    tiles[i] = t;
-  }
-  for (int i = tid; i < n_sh_tiles; i += 1024) {
-    PfTile t; t.w_base = shared_base; t.row0 = i * cap_s; t.rows = min(cap_s, T - i * cap_s);
-    sh_tiles[i] = t;
-  }
-  for (int i = tid; i < n_sh_tiles2; i += 1024) {
-    PfTile t; t.w_base = shared_base; t.row0 = i * cap_s2; t.rows = min(cap_s2, T - i * cap_s2);
-    sh_tiles2[i] = t;
-  }
+  if (tid == 0) { n_real[0] = min(n_all, n_tiles_max); n_real[1] = n_sh_tiles; n_real[2] = n_sh_tiles2; }
 }
 
 extern "C" int moe_prefill_tile_rows(void) { return PF_BM; }
@@ -883,7 +908,7 @@ extern "C" int moe_experts_prefill_pieces(const void *x_bf16, int T, int H, int 
       c.tiles = shared ? (w2 ? sh_tiles2 : sh_tiles) : tiles;
       c.n_mtiles = shared ? (w2 ? n_s2 : n_s) : n_r;
       c.n_tiles_real = n_real + (shared ? (w2 ? 2 : 1) : 0);
-      c.m_fastest = shared;
+      c.shared = shared;
       if (!w2) {  // w13 [2I, H]: gate rows 0..I-1, up rows I..2I-1
         c.act = (const uint16_t *)(int4 ? x16 : x_bf16); c.gather = shared ? nullptr : sorted_tok; c.act_stride = H;
         c.out = shared ? h_s : h_r; c.out_stride = Ii;
@@ -903,7 +928,7 @@ extern "C" int moe_experts_prefill_pieces(const void *x_bf16, int T, int H, int 
       }
       c.ksplit = (w2 && shared && int4) ? shared_pieces : 1;
       c.split_stride = (long long)T * H;
-      c.n_blocks = c.n_mtiles * c.n_ntiles * c.ksplit;
+      c.n_blocks = (c.n_mtiles * c.n_ntiles * c.ksplit + 8 * PF_DEAL - 1) / (8 * PF_DEAL) * (8 * PF_DEAL);  // whole rounds of runs
       c.slab_step = pf_slab_step(c.K / PF_BK);
       a.n_blocks_total += c.n_blocks;
     }

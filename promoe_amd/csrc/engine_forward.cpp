@@ -186,6 +186,7 @@ extern "C" int moe_forward_prepare(moe_engine *eng, int max_tokens) {
   size_t rows_s = T > 128 ? T : 128;
   for (int t = 1; t <= T; ++t) {
     rows_s = std::max(rows_s, (size_t)t * (size_t)moe_prefill_shared_splits(MOE_FMT_Q4K, t, H, I_sh));
+    rows_s = std::max(rows_s, (size_t)t * (size_t)moe_prefill_shared_splits(MOE_FMT_BF16, t, H, I_sh));
     if (t <= 64) rows_s = std::max(rows_s, (size_t)t * (size_t)moe_decode_shared_splits(MOE_FMT_Q4K, t, H, I_sh));
   }
   rc |= dalloc(s, &s->part_s, rows_s * H);

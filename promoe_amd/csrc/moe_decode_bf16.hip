@@ -1,0 +1,271 @@
+// bf16 experts, decode batches of up to 64 tokens (gfx950): the grouped SwiGLU expert product as a weight stream.
+//
+// What bounds it: with a few rows per expert every weight is read once and used for at most 64 tokens, so the launch
+// is as long as its bytes take (about 6 TB/s for plain reads on this chip) plus the chain kernel start -> unit ->
+// slot address -> first weights.  The tile kernels of moe_prefill.hip, which took these batches before, stage
+// activations through LDS with a barrier per slab for up to 256 rows, hold one workgroup per compute unit, and their
+// w2 pass has H / 256 workgroups per expert (40 in all for one token of the Qwen1.5 shape).
+//
+// Work split: a workgroup of four waves owns two row sets of one unit (w13: the same 16 HV rows of gate and up; w2:
+// two adjacent sets), its waves take every fourth 64-wide slab of the reduction and their sums meet in LDS once, at
+// the end.  Weights (16 HV rows x 64 k) and activation rows go global -> registers in the operand order of
+// v_mfma_f32_16x16x32_bf16, DEPTH slabs ahead; there is no barrier and no LDS in the loop.  The activation rows come
+// out of the caches (T rows, read by every workgroup of a unit): HV = 2 reads them half as often as HV = 1 and is
+// taken where its workgroups still fill the chip.
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+#include <string.h>
+
+#include "moe_common.h"
+#include "moe_kernels.h"
+#include "moe_device.h"
+
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+
+struct DbClass {
+  const uint16_t *act;   // activation rows
+  const int *gather;     // row -> activation row, or NULL
+  void *out;             // bf16 h rows (w13) or fp32 partial rows (w2)
+  long long w_off;       // byte offset of the matrix in the expert image
+  int K, act_stride, out_stride;
+  int nblk;              // workgroups per unit and window of the reduction
+  int set_delta;         // w13: 32-row blocks from gate to up (I / 32)
+  int slab_step;         // storage rotation per 128-row group (see the bf16 slot layout)
+  int ksplit;            // shared expert's w2 pass: windows of the reduction, partial rows to out + window * T * out_stride
+};
+struct DbArgs {
+  DbClass c[2];          // 0 = shared expert, 1 = routed experts
+  const moe_unit *units;
+  const unsigned long long *expert_ptr;
+  const unsigned char *shared_base;
+  int n_sh_blocks, T;
+  int *err;
+};
+
+#define DB_NO_ROW 0x7fffff00u  // length of the buffer resources and the offset that reads zeros without a memory request
+
+// One pass over up to 16 NT token rows.  wA / wB: the lane's byte offset into the two row sets' slabs, pA / pB: their
+// first slab's position (rotation), slabs kt0 .. kt0 + nk - 1 of a row of Kn slabs.
+template <bool SWIGLU, int HV, int NT, int DEPTH>
+static __device__ __forceinline__ void db_pass(const DbClass &c, float *red, const rsrc_t rw, const rsrc_t rx, const int setA,
+                                               const int setB, const int rotA, const int rotB, const int half, const int kt0,
+                                               const int nk, const int Kn, const int row_first, const int mc,
+                                               const size_t out_row0, const int out_col, const int tid) {
+  const int lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r = lane & 15, cq = lane >> 4;
+  // weights: load (h, m) of a slab = rows 16 h + r, chunk of 8 k number (j, q) = (2 m + cq / 2, cq % 2) of the block
+  const int wv = cq * 512 + half * 256 + r * 16;
+  int xv[NT];   // activations: the same chunk of token row 16 t + r
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    const int row = 16 * t + r;
+    const int gr = row_first + (row < mc ? row : mc - 1);
+    const int arow = c.gather ? c.gather[gr] : gr;
+    xv[t] = row < mc ? (int)((unsigned)arow * (unsigned)c.act_stride * 2u) + 64 * (cq & 1) + 16 * (cq >> 1) : (int)DB_NO_ROW;
+  }
+  u32x4_t wt[DEPTH][2][HV][2], xb[DEPTH][NT][2];
+  auto load = [&](const int d, const int i) {   // this wave's i-th slab: slab 4 i + w of the window
+    const int kt = 4 * i + w;
+    const bool in = kt < nk;                    // (past the end: zeros, no memory request)
+    const int kb = kt0 + (in ? kt : 0);
+    const int a = kb + rotA, b = kb + rotB;
+    const int sa = setA + (a >= Kn ? a - Kn : a) * 16384, sb = setB + (b >= Kn ? b - Kn : b) * 16384;
+    const int v = in ? wv : (int)DB_NO_ROW;
+#pragma unroll
+    for (int h = 0; h < HV; ++h)
+#pragma unroll
+      for (int m = 0; m < 2; ++m) {
+        wt[d][0][h][m] = __builtin_amdgcn_raw_buffer_load_b128(rw, v + h * 256 + m * 2048, sa, 2);
+        wt[d][1][h][m] = __builtin_amdgcn_raw_buffer_load_b128(rw, v + h * 256 + m * 2048, sb, 2);
+      }
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int m = 0; m < 2; ++m) xb[d][t][m] = __builtin_amdgcn_raw_buffer_load_b128(rx, xv[t] + 32 * m, kb * 128, 0);
+  };
+  f32x4_t acc[2][HV][NT];
+#pragma unroll
+  for (int s = 0; s < 2; ++s)
+#pragma unroll
+    for (int h = 0; h < HV; ++h)
+#pragma unroll
+      for (int t = 0; t < NT; ++t) acc[s][h][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int d = 0; d < DEPTH; ++d) load(d, d);
+  const int ni = (nk - w + 3) >> 2;
+  for (int i0 = 0; i0 < ni; i0 += DEPTH) {
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d) {
+#pragma unroll
+      for (int m = 0; m < 2; ++m)
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+          for (int h = 0; h < HV; ++h)
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+              acc[s][h][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, wt[d][s][h][m]),
+                                                                     __builtin_bit_cast(bf16x8_t, xb[d][t][m]), acc[s][h][t], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      load(d, i0 + d + DEPTH);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  // the waves' sums: red[wave][set][half][token block][element][lane]
+#pragma unroll
+  for (int s = 0; s < 2; ++s)
+#pragma unroll
+    for (int h = 0; h < HV; ++h)
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+        *(f32x4_t *)(red + ((((w * 2 + s) * HV + h) * NT + t) * 64 + lane) * 4) = acc[s][h][t];
+  __syncthreads();
+  for (int q = w; q < HV * NT; q += 4) {
+    const int h = q / NT, t = q - h * NT;
+    f32x4_t v[2];
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      v[s] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int ww = 0; ww < 4; ++ww) v[s] += *(const f32x4_t *)(red + ((((ww * 2 + s) * HV + h) * NT + t) * 64 + lane) * 4);
+    }
+    if (16 * t + r < mc) {
+      const size_t orow = (out_row0 + (size_t)(row_first + 16 * t + r)) * c.out_stride;
+      if (SWIGLU) {
+        u32 o[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const float g0 = v[0][2 * i], g1 = v[0][2 * i + 1];
+          const float h0 = g0 / (1.f + expf(-g0)) * v[1][2 * i], h1 = g1 / (1.f + expf(-g1)) * v[1][2 * i + 1];
+          o[i] = (u32)f32_to_bf16(h0) | ((u32)f32_to_bf16(h1) << 16);
+        }
+        *(uint2 *)((uint16_t *)c.out + orow + out_col + 16 * h + 4 * cq) = make_uint2(o[0], o[1]);
+      } else {
+        *(f32x4_t *)((float *)c.out + orow + out_col + 16 * h + 4 * cq) = v[0];
+        *(f32x4_t *)((float *)c.out + orow + out_col + 16 * HV + 16 * h + 4 * cq) = v[1];
+      }
+    }
+  }
+}
+
+template <bool SWIGLU, int HV>
+__global__ __launch_bounds__(256, 2) void k_decode_bf16(const DbArgs a) {
+  extern __shared__ __align__(16) float red_db[];
+  const int tid = threadIdx.x;
+  const bool sh = (int)blockIdx.x < a.n_sh_blocks;
+  const DbClass &c = a.c[sh ? 0 : 1];
+  int rr = sh ? (int)blockIdx.x : (int)blockIdx.x - a.n_sh_blocks;
+  int m, row0, win = 0;
+  const unsigned char *base;
+  if (sh) {
+    m = a.T; row0 = 0; base = a.shared_base;
+    win = rr / c.nblk; rr -= win * c.nblk;
+  } else {
+    const int u = rr / c.nblk;
+    rr -= u * c.nblk;
+    const moe_unit un = a.units[u];
+    if (un.m <= 0 || un.expert < 0) return;
+    m = un.m; row0 = un.row0;
+    base = (const unsigned char *)a.expert_ptr[un.expert];
+    if (!base) {
+      if (tid == 0) moe_raise_err(a.err);
+      return;
+    }
+  }
+  const int Kn = c.K >> 6, nk = Kn / c.ksplit, kt0 = win * nk;
+  // the two row sets: 32-row blocks (HV = 2) or halves of one (HV = 1)
+  int nbA, nbB, half = 0, out_col;
+  if (SWIGLU) {
+    nbA = HV == 2 ? rr : rr >> 1;
+    nbB = nbA + c.set_delta;
+    if (HV == 1) half = rr & 1;
+    out_col = 32 * nbA + 16 * half;
+  } else {
+    nbA = HV == 2 ? 2 * rr : rr;
+    nbB = HV == 2 ? nbA + 1 : nbA;
+    out_col = 32 * nbA;
+  }
+  const int gA = nbA >> 2, gB = nbB >> 2;
+  const int rotA = (int)((unsigned)(gA * c.slab_step) % (unsigned)Kn), rotB = (int)((unsigned)(gB * c.slab_step) % (unsigned)Kn);
+  const int setA = gA * Kn * 16384 + (nbA & 3) * 4096;
+  const int setB = gB * Kn * 16384 + (nbB & 3) * 4096 + (!SWIGLU && HV == 1 ? 256 : 0);
+  const unsigned long long wb = (unsigned long long)(base + c.w_off);
+  const rsrc_t rw = make_rsrc((const void *)(((unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(wb >> 32)) << 32) |
+                                             (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)wb)), DB_NO_ROW);
+  const rsrc_t rx = make_rsrc(c.act, DB_NO_ROW);
+  const size_t orow0 = (size_t)win * a.T;
+  const int mm = __builtin_amdgcn_readfirstlane(m), r0 = __builtin_amdgcn_readfirstlane(row0);
+#define DB_PASS(NT_, D_) db_pass<SWIGLU, HV, NT_, D_>(c, red_db, rw, rx, setA, setB, rotA, rotB, half, kt0, nk, Kn, r0, mm, orow0, out_col, tid)
+  if (mm <= 16) DB_PASS(1, HV == 2 ? 4 : 6);
+  else if (mm <= 32) DB_PASS(2, 3);
+  else DB_PASS(4, 2);
+#undef DB_PASS
+}
+
+static int db_gcd(int a, int b) { return b ? db_gcd(b, a % b) : a; }
+static int db_slab_step(int nk) {
+  int s = 3;
+  while (db_gcd(s, nk) != 1) s += 2;
+  return s;
+}
+
+template <int HV>
+static int db_launch(bool w13, const DbArgs &a, int grid, hipStream_t s) {
+  const int nt = a.T <= 16 ? 1 : (a.T <= 32 ? 2 : 4);
+  const size_t lds = (size_t)4 * 2 * HV * nt * 64 * 16;
+  moe_ktimer_begin(w13 ? MOE_K_PREFILL_W13 : MOE_K_PREFILL_W2, s);
+  if (w13) hipLaunchKernelGGL((k_decode_bf16<true, HV>), dim3(grid), dim3(256), lds, s, a);
+  else hipLaunchKernelGGL((k_decode_bf16<false, HV>), dim3(grid), dim3(256), lds, s, a);
+  moe_ktimer_end(w13 ? MOE_K_PREFILL_W13 : MOE_K_PREFILL_W2, s);
+  return moe_check_launch("k_decode_bf16");
+}
+
+// Whether a batch of T tokens goes to these kernels (m rows of a unit <= T <= 64: every unit is one pass).
+bool moe_decode_bf16_takes(int T) { return T <= 64; }
+
+// Windows of the shared expert's w2 reduction: few row sets (H / 64) over a long reduction (Qwen1.5 shape: 32 over 88
+// slabs) would outlast the routed experts' workgroups, so it is cut until there are 256 workgroups, in windows of at
+// least 16 slabs.
+int moe_decode_bf16_splits(int H, int I_sh) {
+  const int nk = I_sh / 64;
+  int s = 1;
+  while (s < 8 && (H / 64) * s < 256 && nk % (2 * s) == 0 && nk / (2 * s) >= 16) s *= 2;
+  return s;
+}
+
+int moe_decode_bf16(const void *x, int T, int H, int I, int I_sh, const moe_unit *units, int max_units, const int *sorted_tok,
+                    const uint64_t *expert_ptr, const void *shared_ptr, void *h_r, void *h_s, float *part_r, float *part_s,
+                    int pieces, int *err, int phases, hipStream_t s) {
+  DbArgs a;
+  memset(&a, 0, sizeof a);
+  a.units = units; a.expert_ptr = (const unsigned long long *)expert_ptr; a.shared_base = (const unsigned char *)shared_ptr;
+  a.T = T; a.err = err;
+  for (int w2 = 0; w2 < 2; ++w2) {
+    if (!(phases & (w2 ? 2 : 1))) continue;
+    for (int i = 0; i < 2; ++i) {
+      DbClass &c = a.c[i];
+      const int Ii = i == 0 ? I_sh : I;
+      if (!w2) {
+        c.act = (const uint16_t *)x; c.gather = i == 0 ? nullptr : sorted_tok; c.act_stride = H; c.out = i == 0 ? h_s : h_r;
+        c.out_stride = Ii; c.K = H; c.w_off = 0; c.set_delta = Ii / 32; c.ksplit = 1;
+      } else {
+        c.act = (const uint16_t *)(i == 0 ? h_s : h_r); c.gather = nullptr; c.act_stride = Ii;
+        c.out = i == 0 ? (void *)part_s : (void *)part_r; c.out_stride = H; c.K = Ii;
+        c.w_off = (long long)2 * Ii * H * 2; c.set_delta = 0; c.ksplit = i == 0 ? pieces : 1;
+      }
+      c.slab_step = c.K ? db_slab_step(c.K / 64) : 1;
+    }
+    const int sh_blk = shared_ptr ? (w2 ? H / 64 * pieces : I_sh / 32) : 0, r_blk = w2 ? H / 64 : I / 32;
+    // 16-row sets where 32-row sets would leave the chip with under four workgroups per compute unit
+    const int hv = sh_blk + max_units * r_blk < 1024 ? 1 : 2;
+    const int f = hv == 1 ? 2 : 1;
+    a.c[0].nblk = f * (shared_ptr ? sh_blk / (w2 ? pieces : 1) : 0);
+    a.c[1].nblk = f * r_blk;
+    a.n_sh_blocks = f * sh_blk;
+    const int grid = a.n_sh_blocks + max_units * a.c[1].nblk;
+    if (grid <= 0) continue;
+    if (int rc = hv == 1 ? db_launch<1>(!w2, a, grid, s) : db_launch<2>(!w2, a, grid, s)) return rc;
+  }
+  return MOE_OK;
+}

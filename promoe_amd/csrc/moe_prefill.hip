@@ -809,7 +809,9 @@ static int64_t pf_x16_offset(int T, int k, int max_units) {
 // I_sh 20480) at 512 tokens, 56 workgroups over 160 groups each: 371 us for the launch, 285 us with the reduction in 4
 // windows (8 windows: no shorter, and the combine reads twice the partial rows).  Then the reduction is cut into 2, 4
 // or 8 windows of at least 32 groups, a workgroup per tile and window, until there are 192 of them.
+// bf16 batches of decode size have a rule of their own (moe_decode_bf16_splits).
 extern "C" int moe_prefill_shared_splits(int fmt, int T, int H, int I_sh) {
+  if (fmt == MOE_FMT_BF16 && T > 0 && H > 0 && I_sh > 0 && moe_decode_bf16_takes(T)) return moe_decode_bf16_splits(H, I_sh);
   if ((fmt != MOE_FMT_INT4_G128 && fmt != MOE_FMT_Q4K) || T <= 0 || H <= 0 || I_sh <= 0) return 1;
   const int tiles = ((T + PF_BM_SHARED_W2 - 1) / PF_BM_SHARED_W2) * (H / (2 * PF_BNH));
   const int G = I_sh / 128;
@@ -838,7 +840,13 @@ extern "C" int moe_experts_prefill_pieces(const void *x_bf16, int T, int H, int 
     moe_set_error("moe_experts_prefill: shared_pieces = %d (1, 2, 4 or 8)", shared_pieces);
     return MOE_EINVAL;
   }
-  if (shared_pieces > 1 && (!shared_ptr || (fmt != MOE_FMT_INT4_G128 && fmt != MOE_FMT_Q4K) ||
+  const bool bf16_decode = fmt == MOE_FMT_BF16 && moe_decode_bf16_takes(T);
+  if (shared_pieces > 1 && bf16_decode && shared_ptr) {
+    if ((I_sh / 64) % shared_pieces != 0) {
+      moe_set_error("moe_experts_prefill: %d pieces do not divide the bf16 shared expert's I_sh / 64 (I_sh=%d)", shared_pieces, I_sh);
+      return MOE_EINVAL;
+    }
+  } else if (shared_pieces > 1 && (!shared_ptr || (fmt != MOE_FMT_INT4_G128 && fmt != MOE_FMT_Q4K) ||
                             (I_sh / 128) % (shared_pieces * 2) != 0)) {
     moe_set_error("moe_experts_prefill: %d pieces need an int4 / q4_K shared expert whose I_sh / 128 is a multiple of %d "
                   "(I_sh=%d)", shared_pieces, shared_pieces * 2, I_sh);
@@ -870,6 +878,9 @@ extern "C" int moe_experts_prefill_pieces(const void *x_bf16, int T, int H, int 
     moe_set_error("moe_experts_prefill: H %% 256 == 0 and I %% 128 == 0 required (H=%d I=%d I_sh=%d)", H, I, I_sh);
     return MOE_EINVAL;
   }
+  if (bf16_decode)
+    return moe_decode_bf16(x_bf16, T, H, I, I_sh, units, max_units, sorted_tok, expert_ptr, shared_ptr, h_r, h_s, part_r, part_s,
+                           shared_pieces, err, phases, s);
   const long long P = (long long)T * k;
   const int cap = int4 ? PN_BM : PF_BM, cap_s = int4 ? PN_BM : PF_BM_SHARED, cap_s2 = PF_BM_SHARED_W2;
   // fp16 copy of x for the nibble formats: behind the tile list where the caller left room, else stream-ordered memory

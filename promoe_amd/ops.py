@@ -360,7 +360,8 @@ def experts_prefill(x, d: Dispatch, expert_ptr: torch.Tensor, shared: torch.Tens
             part_s = torch.empty(pieces * T, H, dtype=torch.float32, device=dev)
     check(lib.moe_experts_prefill_pieces(ptr(_dev(x)), T, H, I, I_sh if shared is not None else 0, k, fmt,
                                          ptr(d.units), d.max_units, ptr(d.sorted_tok), ptr(expert_ptr),
-                                         ptr(shared), ptr(h_r), ptr(h_s), ptr(part_r), ptr(part_s), pieces, ptr(tiles),
+                                         ptr(shared), ptr(h_r), ptr(h_s), ptr(part_r), ptr(part_s),
+                                         pieces if shared is not None else 1, ptr(tiles),
                                          ptr(err), phases, cur_stream()), "moe_experts_prefill")
     return part_r, part_s, err, h_r, h_s, tiles
 

@@ -174,3 +174,23 @@ def test_prefill_nibble_without_room_for_the_converted_activations(cuda):
     b = ops.experts_prefill(x, d, table, shared, 256, 128, 128, L.FMT_INT4_G128, ws=ws)
     torch.cuda.synchronize()
     assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1]) and int(b[2].item()) == 0
+
+
+@pytest.mark.parametrize("T", [1, 15, 16, 17, 32, 33, 63, 64, 65])
+def test_bf16_decode_batch_edges(cuda, T):
+    """Every token to one expert, on the weight-stream kernel up to 64 tokens: passes of 16, 32 and 64 rows just short,
+    full and just over; a routed reduction of two slabs (fewer than the waves that share it) and a shared one of 32 in
+    two windows."""
+    from promoe_amd import _lib as L
+    print(f"case bf16_decode_edges T={T}", flush=True)
+    assert L.lib.moe_prefill_shared_splits(L.FMT_BF16, T, 256, 2048) == (2 if T <= 64 else 1)
+    check_prefill(Bf16Layer(H=256, I=128, E=1, I_sh=2048, seed=11, shared_gate=True), T, 1, 0, cuda)
+
+
+@pytest.mark.parametrize("H,I,E,I_sh", [(256, 1024, 40, 128), (2048, 128, 40, 0)])
+@pytest.mark.parametrize("T", [24, 64])
+def test_bf16_decode_batch_row_sets(cuda, T, H, I, E, I_sh):
+    """Grids of 1024 workgroups of 32-row sets and more (w13 of the first shape, w2 of the second), 16-row sets in the
+    other pass; 64 tokens over 40 experts: units of few rows and units without any."""
+    print(f"case bf16_decode_row_sets T={T} H={H}", flush=True)
+    check_prefill(Bf16Layer(H=H, I=I, E=E, I_sh=I_sh, seed=12, zipf=1.2), T, 4, 1, cuda)

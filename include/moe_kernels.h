@@ -86,6 +86,10 @@ int moe_q4k_layout_make(int H, int I, moe_int4_layout *out);
  * xor butterfly 32..1) so the result is bit-reproducible.  H % 8 == 0. */
 int moe_gate_logits(const void *x_bf16, const void *wg_bf16, const float *bias, float *logits,
                     int T, int H, int E, int ldl, void *stream);
+/* the same with the bias on the first n_bias rows only (a layer's shared-expert gate row follows the routed ones and
+ * has none) */
+int moe_gate_logits_bias_rows(const void *x, const void *wg, const float *bias, int n_bias, float *logits, int T, int H,
+                              int E, int ldl, void *stream);
 
 /* moe_gate_logits for two matrices over the same activations in ONE launch (T <= 128): wg [E, H] (+ bias) into
  * logits (row stride ldl), wg2 [E2, H] (+ bias2) into logits2 (row stride ldl2); the same bits as two calls.

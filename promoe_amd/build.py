@@ -14,7 +14,7 @@ ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libmoe_engine.so")
 
-HIP_SOURCES = ["moe_kernels.hip", "moe_prefill.hip", "moe_decode_bf16.hip"]
+HIP_SOURCES = ["moe_kernels.hip", "moe_prefill.hip", "moe_decode_bf16.hip", "moe_gate.hip"]
 CXX_SOURCES = ["moe_common.cpp", "engine_cfg.cpp", "engine_core.cpp", "engine_forward.cpp", "engine_predict.cpp", "backends.cpp"]
 
 # -packed-fp32-ops: keep hipcc from forming v_pk_*_f32 out of scalar float code.

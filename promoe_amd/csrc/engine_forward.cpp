@@ -343,15 +343,8 @@ static int route_batch(const moe_layer_desc &d, LayerState *s, const void *x, in
                                   s->sorted_tok, s->units, s->n_active, s->active_ids, max_units, host_units, host_n,
                                   host_seq, seq_val, s->gate_ws, s->gate_seq, parts, s->err_host + layer, st);
   }
-  if (!d.gate_bias) {
-    if ((rc = moe_gate_logits(x, d.gate_w, nullptr, s->logits, T, d.H, n_gate_rows, ldl, st))) return rc;
-  } else {
-    // the bias covers the routed experts only; the shared-gate row (row E) has none
-    if ((rc = moe_gate_logits(x, d.gate_w, d.gate_bias, s->logits, T, d.H, E, ldl, st))) return rc;
-    if (d.shared_gated &&
-        (rc = moe_gate_logits(x, (const uint16_t *)d.gate_w + (size_t)E * d.H, nullptr, s->logits + E, T, d.H, 1, ldl, st)))
-      return rc;
-  }
+  // the bias covers the routed experts only; the shared-gate row (row E) has none
+  if ((rc = moe_gate_logits_bias_rows(x, d.gate_w, d.gate_bias, E, s->logits, T, d.H, n_gate_rows, ldl, st))) return rc;
   return moe_topk_dispatch(s->logits, T, E, ldl, k, d.route_mode, s->idx, s->topk_w, s->counts, s->offsets,
                            s->sorted_pair, s->pos_of_pair, s->sorted_tok, s->units, s->n_active, s->active_ids,
                            max_units, host_units, host_n, host_seq, seq_val, st);
@@ -759,15 +752,8 @@ extern "C" int moe_forward(moe_engine *eng, int layer, const void *x, int T, voi
                           host_seq, st)))
       return rc;
   } else {
-    if (!d.gate_bias) {
-      if ((rc = moe_gate_logits(x, d.gate_w, nullptr, s->logits, T, d.H, n_gate_rows, ldl, st))) return rc;
-    } else {
-      // the bias covers the routed experts only; the shared-gate row (row E) has none
-      if ((rc = moe_gate_logits(x, d.gate_w, d.gate_bias, s->logits, T, d.H, E, ldl, st))) return rc;
-      if (d.shared_gated &&
-          (rc = moe_gate_logits(x, (const uint16_t *)d.gate_w + (size_t)E * d.H, nullptr, s->logits + E, T, d.H, 1, ldl, st)))
-        return rc;
-    }
+    // the bias covers the routed experts only; the shared-gate row (row E) has none
+    if ((rc = moe_gate_logits_bias_rows(x, d.gate_w, d.gate_bias, E, s->logits, T, d.H, n_gate_rows, ldl, st))) return rc;
     if ((rc = moe_topk(s->logits, T, E, ldl, k, d.route_mode, s->idx, s->topk_w, st))) return rc;
     // (the workspace is sized for max_tokens: a smaller batch needs no more of it)
     if ((rc = moe_dispatch_ws(s->idx, T, k, E, s->counts, s->offsets, s->sorted_pair, s->pos_of_pair, s->sorted_tok,

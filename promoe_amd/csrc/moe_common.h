@@ -27,3 +27,9 @@ int moe_decode_bf16_splits(int H, int I_sh);
 int moe_decode_bf16(const void *x, int T, int H, int I, int I_sh, const moe_unit *units, int max_units, const int *sorted_tok,
                     const uint64_t *expert_ptr, const void *shared_ptr, void *h_r, void *h_s, float *part_r, float *part_s,
                     int pieces, int *err, int phases, hipStream_t s);
+
+// gate logits on the matrix cores (moe_gate.hip), behind moe_gate_logits for the batches it takes; same bits.  The first
+// n_bias rows get the bias.
+bool moe_gate_tiles_take(int T, int E);
+int moe_gate_tiles(const void *x, const void *wg, const float *bias, int n_bias, float *logits, int T, int H, int E, int ldl,
+                   hipStream_t s);

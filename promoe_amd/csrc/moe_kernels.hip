@@ -87,7 +87,7 @@ static __device__ __forceinline__ float gate_row_sum(const uint16_t *__restrict_
 __global__ __launch_bounds__(256) void k_gate_logits(const uint16_t *__restrict__ x,
                                                       const uint16_t *__restrict__ wg,
                                                       const float *__restrict__ bias,
-                                                      float *__restrict__ logits, int H, int E,
+                                                      float *__restrict__ logits, int H, int E, int n_bias,
                                                       int ldl, const uint16_t *__restrict__ wg2,
                                                       const float *__restrict__ bias2,
                                                       float *__restrict__ logits2, int E2, int ldl2) {
@@ -97,107 +97,15 @@ __global__ __launch_bounds__(256) void k_gate_logits(const uint16_t *__restrict_
   const int nb1 = (E + 3) >> 2;
   if ((int)blockIdx.x >= nb1) {  // uniform per workgroup
     e = ((int)blockIdx.x - nb1) * 4 + w;
-    wg = wg2; bias = bias2; logits = logits2; E = E2; ldl = ldl2;
+    wg = wg2; bias = bias2; logits = logits2; E = E2; ldl = ldl2; n_bias = E2;
   }
   if (e >= E) return;
+  if (e >= n_bias) bias = nullptr;
   // (requested in front of the row: behind the sum it is one more trip to memory)
   const float bias_e = bias ? bias[e] : 0.f;
   asm volatile("" :: "v"(bias_e));
   const float acc = gate_row_sum(x + (size_t)t * H, wg + (size_t)e * H, H, lane);
   if (lane == 0) logits[(size_t)t * ldl + e] = bias ? acc + bias_e : acc;
-}
-
-// Large T: a workgroup takes 16 tokens (8 waves x 2) and a group of gate rows.  The rows are staged in LDS once
-// per workgroup; a wave keeps the activations of its two tokens in registers as fp32 (the lane's columns
-// 512 c + 8 lane + j) and walks the rows, so a gate row is fetched once per 16 tokens, converted once per two,
-// and the inner loop is one LDS read per eight fma's of each token.  Each (token, row) sum is formed in exactly
-// the order of k_gate_logits (lane partials over k = 512 c + 8 lane + j with one fma chain, then the xor
-// butterfly 32..1): same bits.
-#define GATE_WAVES 8
-#define GATE_TW 2                        // tokens per wave
-#define GATE_TT (GATE_WAVES * GATE_TW)  // tokens per workgroup
-template <int NCH>  // 512-column chunks of a row (H <= 512 NCH)
-__global__ __launch_bounds__(64 * GATE_WAVES) void k_gate_logits_rows(const uint16_t *__restrict__ x,
-                                                                      const uint16_t *__restrict__ wg,
-                                                                      const float *__restrict__ bias,
-                                                                      float *__restrict__ logits, int T, int H,
-                                                                      int E, int ldl, int rows_per_block) {
-  extern __shared__ uint4 gws[];  // [rows of this workgroup][H/8]
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int vpr = H >> 3;
-  const int e0 = blockIdx.y * rows_per_block;
-  const int nrow = (E - e0) < rows_per_block ? (E - e0) : rows_per_block;
-  const uint4 *wsrc = (const uint4 *)(wg + (size_t)e0 * H);
-  for (int i = tid; i < nrow * vpr; i += 64 * GATE_WAVES) gws[i] = wsrc[i];
-  const int t0 = blockIdx.x * GATE_TT + w * GATE_TW;
-  float xf[GATE_TW][NCH][8];
-#pragma unroll
-  for (int t = 0; t < GATE_TW; ++t) {
-    const int tt = (t0 + t) < T ? (t0 + t) : T - 1;  // a token past the end repeats the last one (not stored)
-#pragma unroll
-    for (int c = 0; c < NCH; ++c) {
-      const int k = c * 512 + 8 * lane;
-      const uint4 v = k < H ? *(const uint4 *)(x + (size_t)tt * H + k) : make_uint4(0, 0, 0, 0);
-      xf[t][c][0] = bf16lo(v.x); xf[t][c][1] = bf16hi(v.x); xf[t][c][2] = bf16lo(v.y); xf[t][c][3] = bf16hi(v.y);
-      xf[t][c][4] = bf16lo(v.z); xf[t][c][5] = bf16hi(v.z); xf[t][c][6] = bf16lo(v.w); xf[t][c][7] = bf16hi(v.w);
-    }
-  }
-  __syncthreads();
-  // four rows per trip (rows past the end are clamped and not stored): eight independent chains.  Their eight
-  // butterflies run as one: at the steps 32, 16 and 8 a lane keeps one half of its values and sends the other, so
-  // every sum has the operands the plain butterfly gives it (own + partner's, and a + b = b + a), with 10
-  // exchanges instead of 48.  Lane L then holds the sum of chain 4 (L>>3 & 1) + 2 (L>>4 & 1) + (L>>5 & 1).
-  constexpr int GR = 4;
-  const bool h32 = lane & 32, h16 = lane & 16, h8 = lane & 8;
-  const int mine = 4 * ((lane >> 3) & 1) + 2 * ((lane >> 4) & 1) + ((lane >> 5) & 1);  // chain = 2 * row + token
-  for (int r = 0; r < nrow; r += GR) {
-    float acc[GR * GATE_TW];
-#pragma unroll
-    for (int i = 0; i < GR * GATE_TW; ++i) acc[i] = 0.f;
-#pragma unroll
-    for (int c = 0; c < NCH; ++c) {
-      const int k = c * 512 + 8 * lane;
-      if (k < H) {
-#pragma unroll
-        for (int q = 0; q < GR; ++q) {
-          const int rq = r + q < nrow ? r + q : nrow - 1;
-          const uint4 wv = gws[rq * vpr + (k >> 3)];
-          const float wf[8] = {bf16lo(wv.x), bf16hi(wv.x), bf16lo(wv.y), bf16hi(wv.y),
-                               bf16lo(wv.z), bf16hi(wv.z), bf16lo(wv.w), bf16hi(wv.w)};
-#pragma unroll
-          for (int t = 0; t < GATE_TW; ++t) {
-            float a = acc[q * GATE_TW + t];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) a = fmaf(xf[t][c][j], wf[j], a);
-            acc[q * GATE_TW + t] = a;
-          }
-        }
-      }
-    }
-    static_assert(GR * GATE_TW == 8, "the reduction below folds eight chains");
-    float u[4], v2[2];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float keep = h32 ? acc[2 * i + 1] : acc[2 * i], send = h32 ? acc[2 * i] : acc[2 * i + 1];
-      u[i] = keep + __shfl_xor(send, 32, 64);
-    }
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const float keep = h16 ? u[2 * i + 1] : u[2 * i], send = h16 ? u[2 * i] : u[2 * i + 1];
-      v2[i] = keep + __shfl_xor(send, 16, 64);
-    }
-    float z;
-    {
-      const float keep = h8 ? v2[1] : v2[0], send = h8 ? v2[0] : v2[1];
-      z = keep + __shfl_xor(send, 8, 64);
-    }
-    z = z + __shfl_xor(z, 4, 64);
-    z = z + __shfl_xor(z, 2, 64);
-    z = z + __shfl_xor(z, 1, 64);
-    const int rq = r + (mine >> 1), tq = t0 + (mine & 1);
-    if ((lane & 7) == 0 && rq < nrow && tq < T)
-      logits[(size_t)tq * ldl + e0 + rq] = bias ? z + bias[e0 + rq] : z;
-  }
 }
 
 // ---------------------------------------------------------------------------
@@ -3048,48 +2956,21 @@ extern "C" int moe_int4_layout_make(int H, int I, moe_int4_layout *out) {
 
 extern "C" int moe_gate_logits(const void *x, const void *wg, const float *bias, float *logits,
                                int T, int H, int E, int ldl, void *stream) {
-  if (!x || !wg || !logits || T < 0 || H <= 0 || H % 8 || E <= 0 || ldl < E || T > 65535) {
+  return moe_gate_logits_bias_rows(x, wg, bias, E, logits, T, H, E, ldl, stream);
+}
+
+extern "C" int moe_gate_logits_bias_rows(const void *x, const void *wg, const float *bias, int n_bias, float *logits,
+                                         int T, int H, int E, int ldl, void *stream) {
+  if (!x || !wg || !logits || T < 0 || H <= 0 || H % 8 || E <= 0 || n_bias < 0 || n_bias > E || ldl < E || T > 65535) {
     moe_set_error("moe_gate_logits: bad argument (T=%d H=%d E=%d ldl=%d)", T, H, E, ldl);
     return MOE_EINVAL;
   }
   if (T == 0) return MOE_OK;
-  // up to 128 tokens a wave per (token, gate row) is faster than the token-tile kernel (8 us against 18 us
-  // at 128 tokens, 2048 columns, 64 rows)
-  if (T > 128 && H <= 4096) {
-    // about two workgroups per compute unit, and at most 72 KB of gate rows per workgroup so that two fit the LDS
-    static bool attr_set = false;
-    if (!attr_set) {
-      for (const void *f : {(const void *)k_gate_logits_rows<2>, (const void *)k_gate_logits_rows<4>,
-                            (const void *)k_gate_logits_rows<8>})
-        if (int rc = moe_check_hip(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 72 * 1024),
-                                   "hipFuncSetAttribute(k_gate_logits_rows)"))
-          return rc;
-      attr_set = true;
-    }
-    const int tiles = (T + GATE_TT - 1) / GATE_TT;
-    int rows_per_block = E;
-    while (rows_per_block > 1 && ((size_t)rows_per_block * H * 2 > 72 * 1024 ||
-                                  (size_t)tiles * ((E + rows_per_block - 1) / rows_per_block) < 512))
-      rows_per_block = (rows_per_block + 1) / 2;
-    const size_t lds = (size_t)rows_per_block * H * 2;
-    dim3 grid(tiles, (E + rows_per_block - 1) / rows_per_block);
-    moe_ktimer_begin(MOE_K_GATE, (hipStream_t)stream);
-    if (H <= 1024)
-      hipLaunchKernelGGL(k_gate_logits_rows<2>, grid, dim3(64 * GATE_WAVES), lds, (hipStream_t)stream, (const uint16_t *)x,
-                         (const uint16_t *)wg, bias, logits, T, H, E, ldl, rows_per_block);
-    else if (H <= 2048)
-      hipLaunchKernelGGL(k_gate_logits_rows<4>, grid, dim3(64 * GATE_WAVES), lds, (hipStream_t)stream, (const uint16_t *)x,
-                         (const uint16_t *)wg, bias, logits, T, H, E, ldl, rows_per_block);
-    else
-      hipLaunchKernelGGL(k_gate_logits_rows<8>, grid, dim3(64 * GATE_WAVES), lds, (hipStream_t)stream, (const uint16_t *)x,
-                         (const uint16_t *)wg, bias, logits, T, H, E, ldl, rows_per_block);
-    moe_ktimer_end(MOE_K_GATE, (hipStream_t)stream);
-    return moe_check_launch("k_gate_logits_rows");
-  }
+  if (moe_gate_tiles_take(T, E)) return moe_gate_tiles(x, wg, bias, n_bias, logits, T, H, E, ldl, (hipStream_t)stream);
   dim3 grid((E + 3) / 4, T);
   moe_ktimer_begin(MOE_K_GATE, (hipStream_t)stream);
   hipLaunchKernelGGL(k_gate_logits, grid, dim3(256), 0, (hipStream_t)stream, (const uint16_t *)x,
-                     (const uint16_t *)wg, bias, logits, H, E, ldl, (const uint16_t *)nullptr, (const float *)nullptr,
+                     (const uint16_t *)wg, bias, logits, H, E, n_bias, ldl, (const uint16_t *)nullptr, (const float *)nullptr,
                      (float *)nullptr, 0, 0);
   moe_ktimer_end(MOE_K_GATE, (hipStream_t)stream);
   return moe_check_launch("k_gate_logits");
@@ -3108,7 +2989,7 @@ extern "C" int moe_gate_logits_pair(const void *x, const void *wg, const float *
   dim3 grid((E + 3) / 4 + (E2 + 3) / 4, T);
   moe_ktimer_begin(MOE_K_GATE, (hipStream_t)stream);
   hipLaunchKernelGGL(k_gate_logits, grid, dim3(256), 0, (hipStream_t)stream, (const uint16_t *)x,
-                     (const uint16_t *)wg, bias, logits, H, E, ldl, (const uint16_t *)wg2, bias2, logits2, E2, ldl2);
+                     (const uint16_t *)wg, bias, logits, H, E, E, ldl, (const uint16_t *)wg2, bias2, logits2, E2, ldl2);
   moe_ktimer_end(MOE_K_GATE, (hipStream_t)stream);
   return moe_check_launch("k_gate_logits");
 }

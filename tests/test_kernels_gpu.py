@@ -46,6 +46,26 @@ def test_gate_logits_pair_bit_exact(cuda, T, H, E, E2):
     assert torch.equal(a, ops.gate_logits(x, wg)) and torch.equal(b, ops.gate_logits(x, wg2, b2))
 
 
+@pytest.mark.parametrize("T,H,E", [(313, 2048, 64), (1177, 264, 17), (328, 520, 61), (20000, 8, 1), (125, 1544, 160), (80, 4360, 250),
+                                   (5, 2048, 64)])
+def test_gate_logits_tiles(cuda, T, H, E):
+    """Batches of 20000 logits and more on the matrix cores, the last one below: bits of the ordered sums, ragged tiles
+    of tokens, rows and columns, a bias on some of the rows only, and columns behind the rows left alone."""
+    from promoe_amd import _lib as L
+    print(f"case gate_logits_tiles T={T} H={H} E={E}", flush=True)
+    x = bf16_dev(O.synth_acts(T, H, seed=2), cuda)
+    wg = bf16_dev(O.round_bf16(O.synth_weights((E, H), seed=3)), cuda)
+    n_bias, ldl = E - E // 3, E + 3
+    bias = torch.linspace(-1, 1, E, device=cuda)
+    out = torch.full((T, ldl), 7.0, device=cuda)
+    L.check(L.lib.moe_gate_logits_bias_rows(L.ptr(x), L.ptr(wg), L.ptr(bias), n_bias, L.ptr(out), T, H, E, ldl, L.cur_stream()), "gate")
+    ref = O.gate_logits_ordered(x.float().cpu().numpy(), wg.float().cpu().numpy())
+    ref[:, :n_bias] += bias.cpu().numpy()[:n_bias]
+    got = out.cpu().numpy()
+    assert np.array_equal(got[:, :E].view(np.uint32), ref.view(np.uint32))
+    assert np.all(got[:, E:] == 7.0)
+
+
 @pytest.mark.parametrize("mode", [0, 1, 2])
 @pytest.mark.parametrize("T,E,k", [(1, 64, 6), (16, 64, 6), (33, 60, 4), (5, 8, 2), (9, 64, 8), (4, 200, 8)])
 def test_topk_routing(cuda, T, E, k, mode):

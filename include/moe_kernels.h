@@ -225,6 +225,17 @@ int moe_experts_decode_int4_publish(const void *x_bf16, int T, int H, int I, int
                                     int phases, const int *n_active, moe_unit *units_host_out,
                                     int *n_active_host_out, int *seq_host_out, int seq_value, void *stream);
 
+/* Where a launch behind the routing takes the step's unit list (moe_experts_decode_q4k_publish,
+ * moe_experts_prefill_publish; the same as the host arguments of moe_experts_decode_int4_publish): the first
+ * *n_active (device) units, at most max_units, into units_host, their number into n_active_host and, once those stores
+ * have completed, seq_value into *seq_host (all pinned host memory). */
+typedef struct moe_publish {
+  const int *n_active;
+  moe_unit *units_host;
+  int *n_active_host, *seq_host;
+  int seq_value, max_units;
+} moe_publish;
+
 /* k1b + k2 + k3 for ONE token: the w13 kernel derives the routing itself from the gate logits
  * (same selection, tie rule and weights as moe_topk, same arrays as moe_dispatch, bit for bit)
  * and publishes it for the w2 pass, moe_combine and the host, so a decode step is
@@ -313,6 +324,12 @@ int moe_experts_decode_q4k(const void *x_bf16, int T, int H, int I, int I_sh, in
                            const moe_unit *units, int max_units, const int *sorted_tok,
                            const uint64_t *expert_ptr, const void *shared_ptr, void *h_r, void *h_s,
                            float *part_r, float *part_s, int *err, int phases, void *stream);
+/* The same, and one workgroup of the w13 launch sends the unit list to the host (pub, may be NULL; T >= 2). */
+int moe_experts_decode_q4k_publish(const void *x_bf16, int T, int H, int I, int I_sh, int k,
+                                   const moe_unit *units, int max_units, const int *sorted_tok,
+                                   const uint64_t *expert_ptr, const void *shared_ptr, void *h_r, void *h_s,
+                                   float *part_r, float *part_s, int *err, int phases, const moe_publish *pub,
+                                   void *stream);
 
 /* k4 (prefill): grouped SwiGLU expert product on the matrix cores for large token groups.
  * Same arguments and buffer meanings as moe_experts_decode_int4 (rows of h_r / part_r in the
@@ -350,6 +367,14 @@ int moe_experts_prefill_pieces(const void *x_bf16, int T, int H, int I, int I_sh
                                const uint64_t *expert_ptr, const void *shared_ptr, void *h_r, void *h_s,
                                float *part_r, float *part_s, int shared_pieces, void *tiles_ws, int *err,
                                int phases, void *stream);
+/* The same, and one workgroup of the tile-list launch (bf16 batches of decode size: of the w13 launch) sends the unit
+ * list to the host (pub, may be NULL; needs the w13 phase).  Two copies and an event behind the routing, the way before,
+ * stood in the stream for 9 us. */
+int moe_experts_prefill_publish(const void *x_bf16, int T, int H, int I, int I_sh, int k, int fmt,
+                                const moe_unit *units, int max_units, const int *sorted_tok,
+                                const uint64_t *expert_ptr, const void *shared_ptr, void *h_r, void *h_s,
+                                float *part_r, float *part_s, int shared_pieces, void *tiles_ws, int *err,
+                                int phases, const moe_publish *pub, void *stream);
 
 /* k5: y[t,:] = sum_j w[t,j] * part_r[pos_of_pair[t*k+j],:] + g_t * part_s[t,:], bf16 out.
  * g_t = sigmoid(shared_gate_logit[t*sg_stride]) when shared_gate_logit != NULL, else 1;

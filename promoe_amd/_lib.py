@@ -79,10 +79,12 @@ _sig("moe_predictor_precision", [vp, vp, vp])
 _sig("moe_predictor_wait_idle", [vp, C.c_int])
 _sig("moe_q4k_layout_make", [i32, i32, C.POINTER(Int4Layout)])
 _sig("moe_experts_decode_q4k", [vp, i32, i32, i32, i32, i32, vp, i32, vp, vp, vp, vp, vp, vp, vp, vp, i32, vp])
+_sig("moe_experts_decode_q4k_publish", [vp, i32, i32, i32, i32, i32, vp, i32, vp, vp, vp, vp, vp, vp, vp, vp, i32, vp, vp])
 _sig("moe_prefill_workspace_bytes", [i32, i32, i32], C.c_int64)
 _sig("moe_prefill_tile_rows", [])
 _sig("moe_experts_prefill", [vp, i32, i32, i32, i32, i32, i32, vp, i32, vp, vp, vp, vp, vp, vp, vp, vp, vp, i32, vp])
 _sig("moe_experts_prefill_pieces", [vp, i32, i32, i32, i32, i32, i32, vp, i32, vp, vp, vp, vp, vp, vp, vp, i32, vp, vp, i32, vp])
+_sig("moe_experts_prefill_publish", [vp, i32, i32, i32, i32, i32, i32, vp, i32, vp, vp, vp, vp, vp, vp, vp, i32, vp, vp, i32, vp, vp])
 _sig("moe_prefill_shared_splits", [i32, i32, i32, i32])
 _sig("moe_kernel_timing", [i32])
 _sig("moe_kernel_timing_read", [i32, C.POINTER(C.c_double), C.POINTER(i32)])

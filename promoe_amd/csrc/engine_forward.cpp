@@ -247,8 +247,15 @@ int moe_forward_harvest(moe_engine *eng, bool wait) {
       volatile int *sq = p.seq;
       if (*sq != p.seq_expected) {
         if (!wait) break;
-        // the launch that writes it is already in the compute stream
-        if (hipStreamSynchronize((hipStream_t)eng->be->compute_stream()) != hipSuccess) return MOE_EHIP;
+        // the launch that writes it is already in the compute stream; what was queued behind it stays queued (waiting
+        // for the whole stream here left the GPU without work each time the host was kPending layers ahead)
+        const auto t0 = std::chrono::steady_clock::now();
+        unsigned spins = 0;
+        while (*sq != p.seq_expected)
+          if ((++spins & 1023u) == 0 && std::chrono::steady_clock::now() - t0 > std::chrono::seconds(5)) {
+            if (hipStreamSynchronize((hipStream_t)eng->be->compute_stream()) != hipSuccess) return MOE_EHIP;
+            break;
+          }
         if (*sq != p.seq_expected) { moe_set_error("routing of layer %d never reached the host", p.layer); return MOE_EHIP; }
       }
       __atomic_thread_fence(__ATOMIC_ACQUIRE);
@@ -273,20 +280,21 @@ static bool use_prefill(const moe_layer_desc &d, int T) {
 }
 
 static int shared_pieces(const moe_layer_desc &d, int T, const LayerState *s);
-// pub / pub_seq: the pending slot whose pinned unit list the w13 launch fills (decode_publishes), or null
+// pub / pub_seq: the pending slot whose pinned unit list a launch fills (launch_publishes), or null
 static int run_units(moe_engine *eng, const moe_layer_desc &d, LayerState *s, const void *x, int T,
                      const moe_unit *units_dev, const moe_unit *units_host, int n_units, bool with_shared,
                      int layer, const uint64_t *table, hipStream_t st, LayerState::Pending *pub = nullptr,
                      int pub_seq = 0) {
+  const moe_publish out = pub ? moe_publish{s->n_active, pub->units, pub->n_active, pub->seq, pub_seq, n_units} : moe_publish{};
   if (use_prefill(d, T))
-    return moe_experts_prefill_pieces(x, T, d.H, d.I, with_shared ? d.I_sh : 0, d.top_k, d.fmt, units_dev, n_units,
-                                      s->sorted_tok, table, with_shared ? d.shared : nullptr, s->h_r, s->h_s, s->part_r,
-                                      s->part_s, with_shared ? shared_pieces(d, T, s) : 1, s->tiles_ws,
-                                      s->err_host + layer, d.fmt == MOE_FMT_BF16 ? 3 : 7, st);
+    return moe_experts_prefill_publish(x, T, d.H, d.I, with_shared ? d.I_sh : 0, d.top_k, d.fmt, units_dev, n_units,
+                                       s->sorted_tok, table, with_shared ? d.shared : nullptr, s->h_r, s->h_s, s->part_r,
+                                       s->part_s, with_shared ? shared_pieces(d, T, s) : 1, s->tiles_ws,
+                                       s->err_host + layer, d.fmt == MOE_FMT_BF16 ? 3 : 7, pub ? &out : nullptr, st);
   if (d.fmt == MOE_FMT_Q4K)
-    return moe_experts_decode_q4k(x, T, d.H, d.I, with_shared ? d.I_sh : 0, d.top_k, units_dev, n_units,
-                                  s->sorted_tok, table, with_shared ? d.shared : nullptr, s->h_r, s->h_s,
-                                  s->part_r, s->part_s, s->err_host + layer, 3, st);
+    return moe_experts_decode_q4k_publish(x, T, d.H, d.I, with_shared ? d.I_sh : 0, d.top_k, units_dev, n_units,
+                                          s->sorted_tok, table, with_shared ? d.shared : nullptr, s->h_r, s->h_s,
+                                          s->part_r, s->part_s, s->err_host + layer, 3, pub ? &out : nullptr, st);
   // the host knows the units and the slot addresses: they travel in the kernel arguments
   const uint64_t *table_host = units_host ? eng->h_table + (size_t)layer * eng->cfg.num_expert : nullptr;
   return moe_experts_decode_int4_publish(x, T, d.H, d.I, with_shared ? d.I_sh : 0, d.top_k, units_dev, n_units,
@@ -296,9 +304,10 @@ static int run_units(moe_engine *eng, const moe_layer_desc &d, LayerState *s, co
                                          pub ? pub->seq : nullptr, pub_seq, st);
 }
 
-// a decode batch whose w13 launch can send the unit list to the host itself (int4 GEMV kernels, 2 tokens and more)
-static bool decode_publishes(const moe_layer_desc &d, int T, int max_units) {
-  return d.fmt == MOE_FMT_INT4_G128 && T >= 2 && !use_prefill(d, T) && max_units > 0 && d.I > 0;
+// a batch whose expert launches can send the unit list to the host themselves: the tile kernels' list launch, the bf16
+// w13 launch, the w13 launches of the nibble formats from 2 tokens on
+static bool launch_publishes(const moe_layer_desc &d, int T, int max_units) {
+  return max_units > 0 && d.I > 0 && (T >= 2 || use_prefill(d, T));
 }
 
 // pieces the expert launch of run_units leaves the shared expert's partial rows in
@@ -738,7 +747,7 @@ extern "C" int moe_forward(moe_engine *eng, int layer, const void *x, int T, voi
     tail_seq = ++s->seq_counter;
     // the unit list reaches the host from the w13 launch where that one can carry it (its stores to pinned memory
     // hold the routing launch for about 2 us, and nothing in the w13 launch waits for them), else from here
-    w13_publishes = decode_publishes(d, T, max_units);
+    w13_publishes = launch_publishes(d, T, max_units);
     if ((rc = route_batch(d, s, x, T, E, k, n_gate_rows, ldl, max_units, layer, w13_publishes ? nullptr : pn.units,
                           w13_publishes ? nullptr : pn.n_active, w13_publishes ? nullptr : pn.seq, tail_seq, st)))
       return rc;
@@ -766,7 +775,11 @@ extern "C" int moe_forward(moe_engine *eng, int layer, const void *x, int T, voi
     if (p.busy && (rc = moe_forward_harvest(eng, true))) return rc;
     s->pend_head = (s->pend_head + 1) % LayerState::kPending;
     p.layer = layer; p.max_units = max_units; p.busy = true;
-    if (routed_by_tail) {  // the routing kernel stores the unit list in the slot's pinned memory itself
+    if (!routed_by_tail && launch_publishes(d, T, max_units)) {
+      tail_seq = ++s->seq_counter;
+      w13_publishes = true;
+    }
+    if (routed_by_tail || w13_publishes) {  // a kernel stores the unit list in the slot's pinned memory itself
       p.by_seq = true; p.seq_expected = tail_seq;
     } else {
       HIPC(hipMemcpyAsync(p.units, s->units, sizeof(moe_unit) * max_units, hipMemcpyDeviceToHost, st));
@@ -778,8 +791,10 @@ extern "C" int moe_forward(moe_engine *eng, int layer, const void *x, int T, voi
     if ((rc = moe_expert_ptr_table(eng, layer, &table))) return rc;
     if ((rc = moe_flush_table(eng, layer, st))) return rc;
     if ((rc = run_units(eng, d, s, x, T, s->units, nullptr, max_units, d.I_sh > 0, layer, table, st,
-                        w13_publishes ? &p : nullptr, tail_seq)))
+                        w13_publishes ? &p : nullptr, tail_seq))) {
+      if (w13_publishes) p.busy = false;  // (refused: nothing is on its way to the slot)
       return rc;
+    }
     const float *sg0 = d.shared_gated ? s->logits + E : nullptr;
     if ((rc = moe_combine_splits(s->part_r, d.I_sh > 0 ? s->part_s : nullptr, s->topk_w, s->pos_of_pair, sg0, ldl, y, T, d.H, k,
                                  shared_pieces(d, T, s), st)))

@@ -21,12 +21,17 @@ static __device__ __forceinline__ void moe_raise_err(int *err) {
   __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
+// what the entry points that publish a unit list ask of their descriptor
+static inline bool moe_publish_ok(const moe_publish *p, int max_units) {
+  return p->n_active && p->units_host && p->n_active_host && p->seq_host && p->max_units > 0 && p->max_units <= max_units;
+}
+
 // bf16 expert product of a decode batch (moe_decode_bf16.hip), behind moe_experts_prefill for batches it takes
 bool moe_decode_bf16_takes(int T);
 int moe_decode_bf16_splits(int H, int I_sh);
 int moe_decode_bf16(const void *x, int T, int H, int I, int I_sh, const moe_unit *units, int max_units, const int *sorted_tok,
                     const uint64_t *expert_ptr, const void *shared_ptr, void *h_r, void *h_s, float *part_r, float *part_s,
-                    int pieces, int *err, int phases, hipStream_t s);
+                    int pieces, int *err, int phases, const moe_publish *pub, hipStream_t s);
 
 // gate logits on the matrix cores (moe_gate.hip), behind moe_gate_logits for the batches it takes; same bits.  The first
 // n_bias rows get the bias.

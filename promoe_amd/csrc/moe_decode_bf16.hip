@@ -41,6 +41,7 @@ struct DbArgs {
   const unsigned char *shared_base;
   int n_sh_blocks, T;
   int *err;
+  moe_publish pub;       // w13 pass: the first workgroup takes the unit list to the host (units_host NULL: none does)
 };
 
 #define DB_NO_ROW 0x7fffff00u  // length of the buffer resources and the offset that reads zeros without a memory request
@@ -153,9 +154,12 @@ template <bool SWIGLU, int HV>
 __global__ __launch_bounds__(256, 2) void k_decode_bf16(const DbArgs a) {
   extern __shared__ __align__(16) float red_db[];
   const int tid = threadIdx.x;
-  const bool sh = (int)blockIdx.x < a.n_sh_blocks;
+  const bool pub = SWIGLU && a.pub.units_host != nullptr;
+  if (pub && blockIdx.x == 0) { publish_units(a.pub, a.units, tid, 256); return; }
+  const int bx = (int)blockIdx.x - (pub ? 1 : 0);
+  const bool sh = bx < a.n_sh_blocks;
   const DbClass &c = a.c[sh ? 0 : 1];
-  int rr = sh ? (int)blockIdx.x : (int)blockIdx.x - a.n_sh_blocks;
+  int rr = sh ? bx : bx - a.n_sh_blocks;
   int m, row0, win = 0;
   const unsigned char *base;
   if (sh) {
@@ -236,11 +240,12 @@ int moe_decode_bf16_splits(int H, int I_sh) {
 
 int moe_decode_bf16(const void *x, int T, int H, int I, int I_sh, const moe_unit *units, int max_units, const int *sorted_tok,
                     const uint64_t *expert_ptr, const void *shared_ptr, void *h_r, void *h_s, float *part_r, float *part_s,
-                    int pieces, int *err, int phases, hipStream_t s) {
+                    int pieces, int *err, int phases, const moe_publish *pub, hipStream_t s) {
   DbArgs a;
   memset(&a, 0, sizeof a);
   a.units = units; a.expert_ptr = (const unsigned long long *)expert_ptr; a.shared_base = (const unsigned char *)shared_ptr;
   a.T = T; a.err = err;
+  if (pub) a.pub = *pub;
   for (int w2 = 0; w2 < 2; ++w2) {
     if (!(phases & (w2 ? 2 : 1))) continue;
     for (int i = 0; i < 2; ++i) {
@@ -263,7 +268,7 @@ int moe_decode_bf16(const void *x, int T, int H, int I, int I_sh, const moe_unit
     a.c[0].nblk = f * (shared_ptr ? sh_blk / (w2 ? pieces : 1) : 0);
     a.c[1].nblk = f * r_blk;
     a.n_sh_blocks = f * sh_blk;
-    const int grid = a.n_sh_blocks + max_units * a.c[1].nblk;
+    const int grid = a.n_sh_blocks + max_units * a.c[1].nblk + (!w2 && pub ? 1 : 0);
     if (grid <= 0) continue;
     if (int rc = hv == 1 ? db_launch<1>(!w2, a, grid, s) : db_launch<2>(!w2, a, grid, s)) return rc;
   }

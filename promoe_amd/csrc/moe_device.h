@@ -45,6 +45,20 @@ static __device__ __forceinline__ void host_stores_done() {
 static __device__ __forceinline__ float half_bits_to_f32(uint16_t h) {
   return (float)__builtin_bit_cast(_Float16, h);
 }
+// The unit list of a step on its way to the host, by one workgroup of `threads` threads of a launch behind the routing:
+// from device memory into the pinned copy, then the sequence word the host polls.
+static __device__ __forceinline__ void publish_units(const moe_publish &p, const moe_unit *units, const int tid, const int threads) {
+  int n = *p.n_active;
+  n = n < p.max_units ? n : p.max_units;
+  for (int u = tid; u < n; u += threads) {
+    const moe_unit un = units[u];
+    host_store_unit(p.units_host, u, un.expert, un.m, un.row0);
+  }
+  if (tid == 0) host_store_i32(p.n_active_host, n);
+  host_stores_done();
+  __syncthreads();
+  if (tid == 0) __hip_atomic_store(p.seq_host, p.seq_value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 // 8 int4 weights (interleaved nibble order) x 8 bf16 activations; the weights
 // enter as the exact bf16 values 128+q (0x4300 | q), the caller removes 128*sum(x).
 // Mask and exponent pattern of dot8_q4 held in vector registers, made once per kernel: (w & M) | C is then ONE

@@ -828,17 +828,8 @@ struct GemvWork {
 // memory to the host's pinned copy while the other workgroups stream weights, then the sequence word the host
 // polls.  In the routing kernel itself these stores held the launch for 1.8 us; here nothing waits for them.
 static __device__ __forceinline__ void gemv_publish_units(const GemvArgs &a) {
-  const int tid = threadIdx.x;
-  int n = *a.p_n_active;
-  n = n < a.p_max_units ? n : a.p_max_units;
-  for (int u = tid; u < n; u += 256) {
-    const moe_unit un = a.units[u];
-    host_store_unit(a.p_host_units, u, un.expert, un.m, un.row0);
-  }
-  if (tid == 0) host_store_i32(a.p_host_n_active, n);
-  host_stores_done();
-  __syncthreads();
-  if (tid == 0) __hip_atomic_store(a.p_host_seq, a.p_seq_val, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  publish_units(moe_publish{a.p_n_active, a.p_host_units, a.p_host_n_active, a.p_host_seq, a.p_seq_val, a.p_max_units}, a.units,
+                (int)threadIdx.x, 256);
 }
 
 // Slot address of expert e: from the kernel arguments when the launch carries the table, else from the device table.
@@ -3859,6 +3850,20 @@ extern "C" int moe_experts_decode_q4k(const void *x, int T, int H, int I, int I_
                                       const uint64_t *expert_ptr, const void *shared_ptr,
                                       void *h_r, void *h_s, float *part_r, float *part_s,
                                       int *err, int phases, void *stream) {
+  return moe_experts_decode_q4k_publish(x, T, H, I, I_sh, k, units, max_units, sorted_tok, expert_ptr, shared_ptr, h_r, h_s,
+                                        part_r, part_s, err, phases, nullptr, stream);
+}
+
+extern "C" int moe_experts_decode_q4k_publish(const void *x, int T, int H, int I, int I_sh, int k,
+                                              const moe_unit *units, int max_units, const int *sorted_tok,
+                                              const uint64_t *expert_ptr, const void *shared_ptr,
+                                              void *h_r, void *h_s, float *part_r, float *part_s,
+                                              int *err, int phases, const moe_publish *pub, void *stream) {
+  if (pub && (T < 2 || !units || max_units <= 0 || !(phases & 1) || !moe_publish_ok(pub, max_units))) {
+    moe_set_error("moe_experts_decode_q4k_publish: publishing needs T >= 2, the unit list and the w13 phase (T=%d phases=%d)",
+                  T, phases);
+    return MOE_EINVAL;
+  }
   if (!x || T <= 0 || H <= 0 || H % 256 || I < 0 || I % 256 || I_sh < 0 || I_sh % 256 || !err ||
       (max_units > 0 && (!units || !sorted_tok || !expert_ptr || !h_r || !part_r || I == 0)) ||
       (shared_ptr && (!h_s || !part_s || I_sh == 0))) {
@@ -3876,6 +3881,10 @@ extern "C" int moe_experts_decode_q4k(const void *x, int T, int H, int I, int I_
   a.units = units; a.expert_ptr = (const unsigned long long *)expert_ptr;
   a.shared_base = (const unsigned char *)shared_ptr; a.T = T; a.err = err;
   a.pairs = k > 0 ? T * k : 0;
+  if (pub) {
+    a.p_host_units = pub->units_host; a.p_host_n_active = pub->n_active_host; a.p_host_seq = pub->seq_host;
+    a.p_n_active = pub->n_active; a.p_seq_val = pub->seq_value; a.p_max_units = pub->max_units;
+  }
   a.cls[0] = GemvClass{(const uint16_t *)x, nullptr, h_s, ls.off13_q, ls.off13_s, ls.off13_z,
                        H, H / 128, T == 1 ? 0 : H, I_sh, I_sh / 16, 0};
   a.cls[1] = GemvClass{(const uint16_t *)x, T == 1 ? nullptr : sorted_tok, h_r, lr.off13_q, lr.off13_s,

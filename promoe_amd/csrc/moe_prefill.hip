@@ -706,7 +706,8 @@ static int pf_launch(bool swiglu, const PfArgs &a, hipStream_t s) {
 // entries past the real count have rows = 0.  The routed list is in order of tile height, the tallest first (four
 // classes; expert order inside a class), so that no long workgroup starts when the launch is nearly over.
 // Nibble formats: the same launch converts x to fp16 for the w13 pass (8 MB read and written for 2048 x 2048, hidden
-// behind the 4 us that the list takes).
+// behind the 4 us that the list takes).  One more workgroup takes the unit list to the host: two copies and an event
+// behind the routing stood in the stream for 9 us a layer.
 static __device__ __forceinline__ PfTile pf_make_tile(unsigned long long w_base, int row0, int rows, int i, int n) {
   PfTile t;                                  // tile i of n of one expert
   const int g0 = i / PF_GROUP * PF_GROUP;
@@ -720,10 +721,13 @@ __global__ __launch_bounds__(1024) void k_prefill_tiles(const moe_unit *__restri
                                                         PfTile *__restrict__ sh_tiles2, int n_sh_tiles2,
                                                         unsigned long long shared_base, int T, int cap, int cap_s, int cap_s2,
                                                         int *__restrict__ n_real, int *__restrict__ err,
-                                                        const u32x4_t *__restrict__ x, u32x4_t *__restrict__ x16, int n16) {
+                                                        const u32x4_t *__restrict__ x, u32x4_t *__restrict__ x16, int n16,
+                                                        const moe_publish pub) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  if (blockIdx.x > 0) {  // workgroups behind the first: the fp16 copy of the activations (8 values per thread)
-    const int i = ((int)blockIdx.x - 1) * 1024 + tid;
+  const int conv0 = pub.units_host ? 2 : 1;
+  if (blockIdx.x > 0) {  // workgroups behind the first: the unit list to the host, the fp16 copy of the activations
+    if ((int)blockIdx.x < conv0) { publish_units(pub, units, tid, 1024); return; }
+    const int i = ((int)blockIdx.x - conv0) * 1024 + tid;   // (8 values per thread)
     if (i < n16) {
       const u32x4_t v = x[i];
       x16[i] = u32x4_t{bf16x2_to_f16x2(v.x), bf16x2_to_f16x2(v.y), bf16x2_to_f16x2(v.z), bf16x2_to_f16x2(v.w)};
@@ -834,7 +838,20 @@ extern "C" int moe_experts_prefill_pieces(const void *x_bf16, int T, int H, int 
                                           const uint64_t *expert_ptr, const void *shared_ptr, void *h_r, void *h_s,
                                           float *part_r, float *part_s, int shared_pieces, void *tiles_ws, int *err,
                                           int phases, void *stream) {
+  return moe_experts_prefill_publish(x_bf16, T, H, I, I_sh, k, fmt, units, max_units, sorted_tok, expert_ptr, shared_ptr, h_r,
+                                     h_s, part_r, part_s, shared_pieces, tiles_ws, err, phases, nullptr, stream);
+}
+
+extern "C" int moe_experts_prefill_publish(const void *x_bf16, int T, int H, int I, int I_sh, int k, int fmt,
+                                           const moe_unit *units, int max_units, const int *sorted_tok,
+                                           const uint64_t *expert_ptr, const void *shared_ptr, void *h_r, void *h_s,
+                                           float *part_r, float *part_s, int shared_pieces, void *tiles_ws, int *err,
+                                           int phases, const moe_publish *pub, void *stream) {
   hipStream_t s = (hipStream_t)stream;
+  if (pub && (T <= 0 || max_units <= 0 || !(phases & 1) || !moe_publish_ok(pub, max_units))) {
+    moe_set_error("moe_experts_prefill_publish: publishing needs tokens, units and the w13 phase (T=%d phases=%d)", T, phases);
+    return MOE_EINVAL;
+  }
   if (T == 0) return MOE_OK;
   if (shared_pieces != 1 && shared_pieces != 2 && shared_pieces != 4 && shared_pieces != 8) {
     moe_set_error("moe_experts_prefill: shared_pieces = %d (1, 2, 4 or 8)", shared_pieces);
@@ -880,7 +897,7 @@ extern "C" int moe_experts_prefill_pieces(const void *x_bf16, int T, int H, int 
   }
   if (bf16_decode)
     return moe_decode_bf16(x_bf16, T, H, I, I_sh, units, max_units, sorted_tok, expert_ptr, shared_ptr, h_r, h_s, part_r, part_s,
-                           shared_pieces, err, phases, s);
+                           shared_pieces, err, phases, pub, s);
   const long long P = (long long)T * k;
   const int cap = int4 ? PN_BM : PF_BM, cap_s = int4 ? PN_BM : PF_BM_SHARED, cap_s2 = PF_BM_SHARED_W2;
   // fp16 copy of x for the nibble formats: behind the tile list where the caller left room, else stream-ordered memory
@@ -901,10 +918,10 @@ extern "C" int moe_experts_prefill_pieces(const void *x_bf16, int T, int H, int 
   const int n_s2 = shared_ptr ? (T + cap_s2 - 1) / cap_s2 : 0;
   int *n_real = (int *)tiles_ws;  // [0] routed tiles in use, [1] shared tiles (w13 pass), [2] shared tiles (w2 pass)
   PfTile *tiles = (PfTile *)tiles_ws + 1, *sh_tiles = tiles + n_r, *sh_tiles2 = sh_tiles + n_s;
-  hipLaunchKernelGGL(k_prefill_tiles, dim3(1 + (n16 + 1023) / 1024), dim3(1024), 0, s, units, max_units,
+  hipLaunchKernelGGL(k_prefill_tiles, dim3(1 + (pub ? 1 : 0) + (n16 + 1023) / 1024), dim3(1024), 0, s, units, max_units,
                      (const unsigned long long *)expert_ptr, tiles, n_r, sh_tiles, n_s, sh_tiles2, n_s2,
                      (unsigned long long)(uintptr_t)shared_ptr, T, cap, cap_s, cap_s2, n_real, err, (const u32x4_t *)x_bf16,
-                     (u32x4_t *)x16, n16);
+                     (u32x4_t *)x16, n16, pub ? *pub : moe_publish{});
   if (int rc = moe_check_launch("k_prefill_tiles")) return rc;
   for (int w2 = 0; w2 < 2; ++w2) {
     if (!(phases & (w2 ? 2 : 1))) continue;

@@ -20,8 +20,10 @@ STUB(moe_decode_token_int4)
 STUB(moe_decode_token_int4_gate)
 STUB(moe_decode_token_late_expert_int4)
 STUB(moe_experts_decode_q4k)
+STUB(moe_experts_decode_q4k_publish)
 STUB(moe_experts_prefill)
 STUB(moe_experts_prefill_pieces)
+STUB(moe_experts_prefill_publish)
 STUB(moe_combine)
 STUB(moe_combine_splits)
 extern "C" int moe_decode_shared_splits(...) { return 1; }

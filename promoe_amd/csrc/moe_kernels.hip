@@ -2573,11 +2573,11 @@ static __device__ __forceinline__ void kc_pass(const GemvClass &c, unsigned char
 // activations are staged as fp16 (exact from bf16); no sums of activations are needed.  The (scale, min) pair and
 // the (d, dmin) pair of a tile travel with it, one 2-byte and one 4-byte load per lane.
 // Gt: groups per row block in memory; the pass reduces over the window of G groups that the resources start at.
-template <bool SWIGLU, int NT, int CG, int KS>
+template <bool SWIGLU, int NT, int CG, int KS, bool MASKED = false>
 static __device__ __forceinline__ void kc_pass_q4k(const GemvClass &c, unsigned char *smem, const rsrc_t rq,
                                                    const rsrc_t rs, const rsrc_t rz, const rsrc_t rx, const int Gt,
                                                    const int G, const int b, const size_t out_row0, const int row_first,
-                                                   const int mc, const DeqF16Consts &dqc) {
+                                                   const int mc, const DeqF16Consts &dqc, const unsigned tokmask = 0u) {
   constexpr int NB = 2, GW = CG / KS, WS = GW < 4 ? GW : 4, SPC = GW / WS, TBK = 16 * NT;
   constexpr int XSC = CG * 256 + 16, XV = CG * 16, NPC = TBK * XV / 256;
   static_assert(CG % KS == 0 && GW >= 1 && GW == SPC * WS && (SPC == 1 || SPC == 2) && NPC >= 1, "chunk shape");
@@ -2597,7 +2597,8 @@ static __device__ __forceinline__ void kc_pass_q4k(const GemvClass &c, unsigned 
   for (int i = 0; i < NPC; ++i) {
     const int row = (tid + 256 * i) / XV;
     const int gr = row_first + (row < mc ? row : mc - 1);
-    xoff[i] = row < mc ? (c.gather ? c.gather[gr] : gr) * c.act_stride * 2 : -1;
+    if (MASKED && tokmask != 0u) xoff[i] = row < mc ? nth_token(tokmask, row) * c.act_stride * 2 : -1;
+    else xoff[i] = row < mc ? (c.gather ? c.gather[gr] : gr) * c.act_stride * 2 : -1;
   }
   uint4 xr[NPC];
   auto load_chunk = [&](const int ch) {
@@ -2782,12 +2783,12 @@ static __device__ __forceinline__ void kc_pass_q4k(const GemvClass &c, unsigned 
 // where 16-row passes cost up to four.
 // q4_K: the shared expert's w2 class may be split (c.ksplit workgroups per group of block pairs, each over 1 / ksplit
 // of the reduction, partial rows to their own copy of the output: see k_gemv_int4).
-// ROUTE (int4 w13 pass of at most 16 tokens): the launch sums the gate rows and routes by itself, as
+// ROUTE (w13 pass of at most 16 tokens): the launch sums the gate rows and routes by itself, as
 // k_gemv_int4_mfma<.., ROUTE> does (see gemv_resolve_route_batch_n)
 template <bool SWIGLU, bool DEVUNITS, int NTMAX, int KS, bool Q4K = false, bool ROUTE = false>
 __global__ __launch_bounds__(256, 2) void k_gemv_int4_mfma_kc(const GemvArgs a) {
   constexpr int NB = 2;
-  static_assert(!ROUTE || (SWIGLU && DEVUNITS && NTMAX == 1 && !Q4K), "routing launches: int4 w13, 16-row passes");
+  static_assert(!ROUTE || (SWIGLU && DEVUNITS && NTMAX == 1), "routing launches: w13, 16-row passes");
   extern __shared__ __align__(16) unsigned char smem[];
   const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63;
@@ -2864,7 +2865,7 @@ __global__ __launch_bounds__(256, 2) void k_gemv_int4_mfma_kc(const GemvArgs a) 
       t0 += 32;
     } else {
       const int mc = left < 16 ? left : 16;
-      if constexpr (Q4K) kc_pass_q4k<SWIGLU, 1, 8, KS>(c, smem, rq, rs, rz, rx, Gt, G, b, orow0, row0 + t0, mc, dqc);
+      if constexpr (Q4K) kc_pass_q4k<SWIGLU, 1, 8, KS, ROUTE>(c, smem, rq, rs, rz, rx, Gt, G, b, orow0, row0 + t0, mc, dqc, tokmask);
       else kc_pass<SWIGLU, 1, 8, KS, ROUTE>(c, smem, rq, rs, rz, rx, b, row0 + t0, mc, q4c, tokmask);
       t0 += 16;
     }
@@ -3468,7 +3469,7 @@ static int launch_gemv_mfma_route(const GemvArgs &a_in, int units, int tb, size_
   return moe_check_launch("k_gemv_int4_mfma<route>");
 }
 
-template <int KS>
+template <int KS, bool Q4K = false>
 static int launch_gemv_mfma_kc_route(const GemvArgs &a_in, int units, hipStream_t s) {
   constexpr int PW = 4 / KS;
   GemvArgs a = a_in;
@@ -3486,14 +3487,14 @@ static int launch_gemv_mfma_kc_route(const GemvArgs &a_in, int units, hipStream_
   static bool attr_set = false;
   if (!attr_set) {
     // (the kernel also has a few hundred bytes of static LDS: dynamic + static must stay within 160 KB)
-    if (int rc = moe_check_hip(hipFuncSetAttribute((const void *)k_gemv_int4_mfma_kc<true, true, 1, KS, false, true>,
+    if (int rc = moe_check_hip(hipFuncSetAttribute((const void *)k_gemv_int4_mfma_kc<true, true, 1, KS, Q4K, true>,
                                                    hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024),
                                "hipFuncSetAttribute(k_gemv_int4_mfma_kc, routing)"))
       return rc;
     attr_set = true;
   }
   moe_ktimer_begin(MOE_K_W13, s);
-  hipLaunchKernelGGL((k_gemv_int4_mfma_kc<true, true, 1, KS, false, true>), dim3(grid), dim3(256), lds, s, a);
+  hipLaunchKernelGGL((k_gemv_int4_mfma_kc<true, true, 1, KS, Q4K, true>), dim3(grid), dim3(256), lds, s, a);
   moe_ktimer_end(MOE_K_W13, s);
   return moe_check_launch("k_gemv_int4_mfma_kc<route>");
 }
@@ -3514,6 +3515,15 @@ extern "C" int moe_decode_batch_int4_gate_fits(int T, int E, int k, int H, int I
   return 1;
 }
 
+// The same step of an int4 (q4k false) or q4_K layer
+static int decode_batch_gate(bool q4k, const void *x, int T, const void *gate_w, const float *gate_bias, int n_gate_rows,
+                             void *gate_ws, int gate_seq, float *logits, int ldl, int E, int k, int mode, int H, int I, int I_sh,
+                             const uint64_t *expert_ptr, const uint64_t *expert_ptr_host, const void *shared_ptr, int *idx, float *w,
+                             int *counts, int *offsets, int *sorted_pair, int *pos_of_pair, int *sorted_tok, moe_unit *units,
+                             int *n_active, int64_t *active_ids, int max_units, void *h_r, void *h_s, float *part_r, float *part_s,
+                             int *err, moe_unit *units_host_out, int *n_active_host_out, int *seq_host_out, int seq_value,
+                             int phases, void *stream);
+
 extern "C" int moe_decode_batch_int4_gate(const void *x, int T, const void *gate_w, const float *gate_bias,
                                           int n_gate_rows, void *gate_ws, int gate_seq, float *logits, int ldl, int E,
                                           int k, int mode, int H, int I, int I_sh, const uint64_t *expert_ptr,
@@ -3524,8 +3534,40 @@ extern "C" int moe_decode_batch_int4_gate(const void *x, int T, const void *gate
                                           float *part_r, float *part_s, int *err, moe_unit *units_host_out,
                                           int *n_active_host_out, int *seq_host_out, int seq_value, int phases,
                                           void *stream) {
+  return decode_batch_gate(false, x, T, gate_w, gate_bias, n_gate_rows, gate_ws, gate_seq, logits, ldl, E, k, mode, H, I, I_sh,
+                           expert_ptr, expert_ptr_host, shared_ptr, idx, w, counts, offsets, sorted_pair, pos_of_pair, sorted_tok,
+                           units, n_active, active_ids, max_units, h_r, h_s, part_r, part_s, err, units_host_out,
+                           n_active_host_out, seq_host_out, seq_value, phases, stream);
+}
+
+extern "C" int moe_decode_batch_q4k_gate(const void *x, int T, const void *gate_w, const float *gate_bias,
+                                         int n_gate_rows, void *gate_ws, int gate_seq, float *logits, int ldl, int E,
+                                         int k, int mode, int H, int I, int I_sh, const uint64_t *expert_ptr,
+                                         const void *shared_ptr, int *idx, float *w, int *counts, int *offsets,
+                                         int *sorted_pair, int *pos_of_pair, int *sorted_tok, moe_unit *units,
+                                         int *n_active, int64_t *active_ids, int max_units, void *h_r, void *h_s,
+                                         float *part_r, float *part_s, int *err, moe_unit *units_host_out,
+                                         int *n_active_host_out, int *seq_host_out, int seq_value, int phases,
+                                         void *stream) {
+  if (H % 256 || I % 256 || I_sh % 256) {
+    moe_set_error("moe_decode_batch_q4k_gate: q4_K experts need H and I multiples of 256 (H=%d I=%d I_sh=%d)", H, I, I_sh);
+    return MOE_EINVAL;
+  }
+  return decode_batch_gate(true, x, T, gate_w, gate_bias, n_gate_rows, gate_ws, gate_seq, logits, ldl, E, k, mode, H, I, I_sh,
+                           expert_ptr, nullptr, shared_ptr, idx, w, counts, offsets, sorted_pair, pos_of_pair, sorted_tok,
+                           units, n_active, active_ids, max_units, h_r, h_s, part_r, part_s, err, units_host_out,
+                           n_active_host_out, seq_host_out, seq_value, phases, stream);
+}
+
+static int decode_batch_gate(bool q4k, const void *x, int T, const void *gate_w, const float *gate_bias, int n_gate_rows,
+                             void *gate_ws, int gate_seq, float *logits, int ldl, int E, int k, int mode, int H, int I, int I_sh,
+                             const uint64_t *expert_ptr, const uint64_t *expert_ptr_host, const void *shared_ptr, int *idx, float *w,
+                             int *counts, int *offsets, int *sorted_pair, int *pos_of_pair, int *sorted_tok, moe_unit *units,
+                             int *n_active, int64_t *active_ids, int max_units, void *h_r, void *h_s, float *part_r, float *part_s,
+                             int *err, moe_unit *units_host_out, int *n_active_host_out, int *seq_host_out, int seq_value,
+                             int phases, void *stream) {
   if (!moe_decode_batch_int4_gate_fits(T, E, k, H, I, I_sh, n_gate_rows)) {
-    moe_set_error("moe_decode_batch_int4_gate: shape not taken (T=%d E=%d k=%d H=%d I=%d I_sh=%d rows=%d)", T, E, k, H, I,
+    moe_set_error("moe_decode_batch_gate: shape not taken (T=%d E=%d k=%d H=%d I=%d I_sh=%d rows=%d)", T, E, k, H, I,
                   I_sh, n_gate_rows);
     return MOE_EINVAL;
   }
@@ -3534,15 +3576,15 @@ extern "C" int moe_decode_batch_int4_gate(const void *x, int T, const void *gate
       !offsets || !sorted_pair || !pos_of_pair || !sorted_tok || !units || !n_active || !active_ids || max_units != mu ||
       !h_r || !part_r || !err || mode < 0 || mode > 2 || (shared_ptr && (!h_s || !part_s || I_sh == 0)) ||
       (units_host_out && (!n_active_host_out || !seq_host_out))) {
-    moe_set_error("moe_decode_batch_int4_gate: bad argument (T=%d max_units=%d, %d expected)", T, max_units, mu);
+    moe_set_error("moe_decode_batch_gate: bad argument (T=%d max_units=%d, %d expected)", T, max_units, mu);
     return MOE_EINVAL;
   }
   hipStream_t s = (hipStream_t)stream;
   if (phases & 1) {
     moe_int4_layout lr, ls;
     memset(&lr, 0, sizeof lr); memset(&ls, 0, sizeof ls);
-    if (moe_int4_layout_make(H, I, &lr)) return MOE_EINVAL;
-    if (shared_ptr && moe_int4_layout_make(H, I_sh, &ls)) return MOE_EINVAL;
+    if (q4k ? moe_q4k_layout_make(H, I, &lr) : moe_int4_layout_make(H, I, &lr)) return MOE_EINVAL;
+    if (shared_ptr && (q4k ? moe_q4k_layout_make(H, I_sh, &ls) : moe_int4_layout_make(H, I_sh, &ls))) return MOE_EINVAL;
     const bool sh = shared_ptr != nullptr;
     GemvArgs a;
     memset(&a, 0, sizeof a);
@@ -3559,12 +3601,15 @@ extern "C" int moe_decode_batch_int4_gate(const void *x, int T, const void *gate
     a.cls[0] = GemvClass{(const uint16_t *)x, nullptr, h_s, ls.off13_q, ls.off13_s, ls.off13_z, H, H / 128, H, I_sh, I_sh / 16, 0};
     a.cls[1] = GemvClass{(const uint16_t *)x, nullptr, h_r, lr.off13_q, lr.off13_s, lr.off13_z, H, H / 128, H, I, I / 16, 0};
     a.n_sh_blocks = sh ? I_sh / 16 : 0;
-    const bool whole = batch_route_whole_rows(T, H);
+    const bool whole = !q4k && batch_route_whole_rows(T, H);
     const int tg = !whole ? (T <= 8 ? 4 : 8) : (T <= 4 ? 1 : 2);   // tokens per gate workgroup: what the kernel instantiates
     a.g_parts = GATE_PARTS;
     a.g_nblk = a.g_parts * ((T + tg - 1) / tg) * ((n_gate_rows + 3) / 4);
     int rc;
-    if (!whole) {
+    if (q4k) {
+      rc = (a.n_sh_blocks + max_units * (I / 16)) / 4 >= 384 ? launch_gemv_mfma_kc_route<1, true>(a, max_units, s)
+                                                             : launch_gemv_mfma_kc_route<2, true>(a, max_units, s);
+    } else if (!whole) {
       rc = (a.n_sh_blocks + max_units * (I / 16)) / 4 >= 384 ? launch_gemv_mfma_kc_route<1>(a, max_units, s)
                                                              : launch_gemv_mfma_kc_route<2>(a, max_units, s);
     } else {
@@ -3584,7 +3629,10 @@ extern "C" int moe_decode_batch_int4_gate(const void *x, int T, const void *gate
     }
     if (rc) return rc;
   }
-  if (phases & 2)  // w2 over the unit list the first launch published
+  if ((phases & 2) && q4k)  // w2 over the unit list the first launch published
+    return moe_experts_decode_q4k(x, T, H, I, shared_ptr ? I_sh : 0, k, units, max_units, sorted_tok, expert_ptr, shared_ptr,
+                                  h_r, h_s, part_r, part_s, err, 2, stream);
+  if (phases & 2)
     return experts_decode_int4_impl(x, T, H, I, shared_ptr ? I_sh : 0, k, units, max_units, sorted_tok, expert_ptr, shared_ptr,
                                     h_r, h_s, part_r, part_s, err, nullptr, nullptr, 2, nullptr, nullptr, nullptr, nullptr, 0,
                                     expert_ptr_host, E, stream);

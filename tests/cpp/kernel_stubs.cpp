@@ -14,6 +14,7 @@ STUB(moe_route_decode)
 STUB(moe_topk_dispatch)
 STUB(moe_gate_topk_dispatch)
 STUB(moe_decode_batch_int4_gate)
+STUB(moe_decode_batch_q4k_gate)
 STUB(moe_experts_decode_int4)
 STUB(moe_experts_decode_int4_publish)
 STUB(moe_decode_token_int4)

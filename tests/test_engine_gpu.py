@@ -159,6 +159,34 @@ def test_stepwise_hooks_on_gpu_expose_resident_parameters(cuda):
 
 
 @pytest.mark.parametrize("kind", ["int4", "bf16", "q4k"])
+def test_resident_batches_account_their_hits_without_a_wait(cuda, kind):
+    """Every expert resident: the unit list of a batch comes to the host from whichever launch takes it (routing, w13, tile
+    list), more calls outstanding than there are places for them, sizes on both sides of every change of path."""
+    print(f"case engine_resident_published kind={kind}", flush=True)
+    E, k, sizes = 16, 4, (1, 2, 8, 9, 16, 17, 32, 33, 64, 65, 257, 1, 300, 2, 65, 48, 3, 512)
+    mk = {"int4": Int4Layer, "bf16": Bf16Layer, "q4k": Q4KLayer}[kind]
+    layer = mk(H=256, I=512 if kind == "q4k" else 384, E=E, I_sh=256, seed=77, zipf=1.2, shared_gate=True)
+    pm = build_engine([layer], k, cuda, max_tokens=512, cache_rate=1.0, cache_policy="lru")
+    pm.acquire_layer(0, np.arange(E, dtype=np.int64))
+    pm.release_layer(0)
+    xs = [O.synth_acts(T, 256, seed=900 + i) for i, T in enumerate(sizes)]
+    refs = [ref_forward(layer, x, k, 0) for x in xs]
+    xd = [torch.from_numpy(x).to(torch.bfloat16).to(cuda) for x in xs]
+    torch.cuda.synchronize()
+    c0 = pm.counters()
+    ys = [pm.forward(0, x) for x in xd]
+    pm.drain()
+    c1 = pm.counters()
+    torch.cuda.synchronize()
+    for T, y, ref in zip(sizes, ys, refs):
+        err = np.abs(y.float().cpu().numpy() - ref["out"]).max() / np.abs(ref["out"]).max()
+        assert err <= TOL, (T, err)
+    n_act = sum(len(np.unique(r["idx"])) for r in refs)
+    assert c1["miss"] == c0["miss"] and c1["hit"] - c0["hit"] == n_act and c1["activated"] - c0["activated"] == n_act
+    pm.close()
+
+
+@pytest.mark.parametrize("kind", ["int4", "bf16", "q4k"])
 def test_forward_prefill_sizes_through_cache(cuda, kind):
     """Token groups of prefill size take the matrix-core kernels (bf16 layers always do);
     experts are still fetched and evicted underneath, one launch per missed expert."""

@@ -194,7 +194,8 @@ extern "C" int moe_forward_prepare(moe_engine *eng, int max_tokens) {
   // the tile list and, for the nibble formats, the fp16 copy of a prefill batch's activations behind it
   rc |= dalloc(s, (unsigned char **)&s->tiles_ws,
                (((size_t)moe_prefill_workspace_bytes(T, k, s->max_units) + 255) & ~(size_t)255) + (size_t)T * H * 2);
-  s->disp_ws_bytes = moe_dispatch_workspace_bytes(T, k, E);
+  // (both dispatch forms: what max_tokens need, or 64 workgroups' counts, the most a batch of the one-launch form has)
+  s->disp_ws_bytes = std::max<int64_t>(moe_dispatch_workspace_bytes(T, k, E), E <= 256 ? 64 + 64 * (int64_t)E * 4 : 0);
   if (s->disp_ws_bytes) rc |= dalloc(s, &s->disp_ws, (size_t)s->disp_ws_bytes);
   rc |= halloc(s, &s->units_host, s->max_units);
   rc |= halloc(s, &s->units_sub_host, (size_t)s->max_units * 2);
@@ -773,11 +774,9 @@ extern "C" int moe_forward(moe_engine *eng, int layer, const void *x, int T, voi
   } else {
     // the bias covers the routed experts only; the shared-gate row (row E) has none
     if ((rc = moe_gate_logits_bias_rows(x, d.gate_w, d.gate_bias, E, s->logits, T, d.H, n_gate_rows, ldl, st))) return rc;
-    if ((rc = moe_topk(s->logits, T, E, ldl, k, d.route_mode, s->idx, s->topk_w, st))) return rc;
-    // (the workspace is sized for max_tokens: a smaller batch needs no more of it)
-    if ((rc = moe_dispatch_ws(s->idx, T, k, E, s->counts, s->offsets, s->sorted_pair, s->pos_of_pair, s->sorted_tok,
-                              s->units, s->n_active, s->active_ids, max_units, s->disp_ws, s->disp_ws_bytes,
-                              s->err_host + layer, st)))
+    if ((rc = moe_topk_dispatch_ws(s->logits, T, E, ldl, k, d.route_mode, s->idx, s->topk_w, s->counts, s->offsets,
+                                   s->sorted_pair, s->pos_of_pair, s->sorted_tok, s->units, s->n_active, s->active_ids,
+                                   max_units, s->disp_ws, s->disp_ws_bytes, s->err_host + layer, st)))
       return rc;
   }
   if (all_resident) {

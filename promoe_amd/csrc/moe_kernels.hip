@@ -309,9 +309,19 @@ __global__ __launch_bounds__(DISP_THREADS) void k_dispatch(
 // up the counts of all (the totals, hence the offsets) and of the workgroups before it (where its own pairs of an
 // expert start), and scatters.  The barrier words are zero at launch and are left zero.  A workgroup that waits
 // longer than a second raises the error word and goes on with what it has (positions stay inside the arrays).
+// TOPK: the pairs come from the logits: a workgroup first selects the experts of its own tokens (chunk / k of them, a wave per
+// token, the arithmetic of k_topk), and writes idx and wout.  Up to 64 workgroups of at least 16 tokens: both steps are chains
+// of round trips, and the top-k as a launch of its own cost 4.7 us in front of this one's 6.4.
 // ---------------------------------------------------------------------------
 #define DISPM_MAXB 64
-__global__ __launch_bounds__(DISP_THREADS) void k_dispatch_multi(
+struct DispTopk {
+  const float *logits;
+  float *w;
+  int *idx;
+  int T, ldl, mode;
+};
+template <bool TOPK>
+__global__ __launch_bounds__(DISP_THREADS) void k_dispatch_multi(const DispTopk tk,
     const int *__restrict__ idx, int P, int chunk, int k, int E, int nbits, int *__restrict__ counts,
     int *__restrict__ offsets, int *__restrict__ sorted_pair, int *__restrict__ pos_of_pair,
     int *__restrict__ sorted_tok, moe_unit *__restrict__ units, int *__restrict__ n_active,
@@ -325,7 +335,23 @@ __global__ __launch_bounds__(DISP_THREADS) void k_dispatch_multi(
   const int p0 = b * chunk;
   const int np = (P - p0) < chunk ? (P - p0) : chunk;
   const int p = p0 + tid;
-  const int e = tid < np ? idx[p] : -1;
+  int e = -1;
+  if constexpr (TOPK) {
+    int *s_idx = s_w + 16 * E;
+    const int t0 = p0 / k, nt = np / k;
+    for (int t = w; t < nt; t += 16) {
+      const float *row = tk.logits + (size_t)(t0 + t) * tk.ldl;
+      int *ir = tk.idx + (size_t)(t0 + t) * k;
+      float *wr = tk.w + (size_t)(t0 + t) * k;
+      if (E <= 64) topk_token<1, false>(row, E, k, tk.mode, lane, ir, wr, s_idx + t * k, nullptr);
+      else if (E <= 128) topk_token<2, false>(row, E, k, tk.mode, lane, ir, wr, s_idx + t * k, nullptr);
+      else topk_token<4, false>(row, E, k, tk.mode, lane, ir, wr, s_idx + t * k, nullptr);
+    }
+    __syncthreads();
+    if (tid < np) e = s_idx[tid];
+  } else {
+    if (tid < np) e = idx[p];
+  }
   for (int i = tid; i < 16 * E; i += DISP_THREADS) s_w[i] = 0;
   if (tid < 256) { s_all[tid] = 0; s_pre[tid] = 0; }
   __syncthreads();
@@ -3051,11 +3077,52 @@ extern "C" int moe_dispatch_ws(const int *idx, int T, int k, int E, int *counts,
   while ((1 << nbits) < E) ++nbits;
   const size_t lds = (size_t)16 * E * sizeof(int);
   moe_ktimer_begin(MOE_K_DISPATCH, (hipStream_t)stream);
-  hipLaunchKernelGGL(k_dispatch_multi, dim3(nb), dim3(DISP_THREADS), lds, (hipStream_t)stream, idx, P, chunk, k, E,
-                     nbits, counts, offsets, sorted_pair, pos_of_pair, sorted_tok, units, n_active,
+  hipLaunchKernelGGL(k_dispatch_multi<false>, dim3(nb), dim3(DISP_THREADS), lds, (hipStream_t)stream, DispTopk{}, idx, P,
+                     chunk, k, E, nbits, counts, offsets, sorted_pair, pos_of_pair, sorted_tok, units, n_active,
                      (long long *)active_ids, max_units, (int *)((char *)ws + 64), (unsigned *)ws, err);
   moe_ktimer_end(MOE_K_DISPATCH, (hipStream_t)stream);
   return moe_check_launch("k_dispatch_multi");
+}
+
+// Top-k and dispatch of a prefill batch in one launch: tokens per workgroup (0: not taken)
+static int topk_dispatch_tokens(int T, int k, int E) {
+  if (T <= 0 || k <= 0 || k > 32 || E <= 0 || E > 256 || k > E) return 0;
+  const int nb = (T + 15) / 16 < DISPM_MAXB ? (T + 15) / 16 : DISPM_MAXB;
+  const int tpb = (T + nb - 1) / nb;
+  return tpb * k <= DISP_THREADS ? tpb : 0;
+}
+
+extern "C" int64_t moe_topk_dispatch_workspace_bytes(int T, int k, int E) {
+  const int tpb = topk_dispatch_tokens(T, k, E);
+  return tpb ? 64 + (int64_t)((T + tpb - 1) / tpb) * E * (int64_t)sizeof(int) : 0;
+}
+
+extern "C" int moe_topk_dispatch_ws(const float *logits, int T, int E, int ldl, int k, int mode, int *idx, float *w, int *counts,
+                                    int *offsets, int *sorted_pair, int *pos_of_pair, int *sorted_tok, moe_unit *units,
+                                    int *n_active, int64_t *active_ids, int max_units, void *ws, int64_t ws_bytes,
+                                    int *err, void *stream) {
+  const int64_t need = moe_topk_dispatch_workspace_bytes(T, k, E);
+  if (need == 0 || !ws || ws_bytes < need || !err) {
+    if (int rc = moe_topk(logits, T, E, ldl, k, mode, idx, w, stream)) return rc;
+    return moe_dispatch_ws(idx, T, k, E, counts, offsets, sorted_pair, pos_of_pair, sorted_tok, units, n_active, active_ids,
+                           max_units, ws, ws_bytes, err, stream);
+  }
+  if (!logits || ldl < E || mode < 0 || mode > 2 || !idx || !w || !counts || !offsets || !sorted_pair || !pos_of_pair ||
+      !sorted_tok || !units || !n_active || !active_ids || max_units < 0 || ((uintptr_t)ws & 3)) {
+    moe_set_error("moe_topk_dispatch_ws: bad argument (T=%d k=%d E=%d)", T, k, E);
+    return MOE_EINVAL;
+  }
+  const int tpb = topk_dispatch_tokens(T, k, E), nb = (T + tpb - 1) / tpb;
+  int nbits = 0;
+  while ((1 << nbits) < E) ++nbits;
+  const size_t lds = (size_t)(16 * E + tpb * k) * sizeof(int);
+  moe_ktimer_begin(MOE_K_DISPATCH, (hipStream_t)stream);
+  hipLaunchKernelGGL(k_dispatch_multi<true>, dim3(nb), dim3(DISP_THREADS), lds, (hipStream_t)stream,
+                     DispTopk{logits, w, idx, T, ldl, mode}, (const int *)nullptr, T * k, tpb * k, k, E, nbits, counts, offsets,
+                     sorted_pair, pos_of_pair, sorted_tok, units, n_active, (long long *)active_ids, max_units,
+                     (int *)((char *)ws + 64), (unsigned *)ws, err);
+  moe_ktimer_end(MOE_K_DISPATCH, (hipStream_t)stream);
+  return moe_check_launch("k_dispatch_multi<topk>");
 }
 
 template <int TMAX, bool SW, int CH>

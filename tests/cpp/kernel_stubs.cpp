@@ -10,6 +10,7 @@ STUB(moe_gate_logits_pair)
 STUB(moe_topk)
 STUB(moe_dispatch)
 STUB(moe_dispatch_ws)
+STUB(moe_topk_dispatch_ws)
 STUB(moe_route_decode)
 STUB(moe_topk_dispatch)
 STUB(moe_gate_topk_dispatch)

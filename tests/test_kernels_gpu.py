@@ -147,6 +147,39 @@ def test_dispatch_workspace_reused(cuda):
         assert not ws[:16].any().item()
 
 
+@pytest.mark.parametrize("E,k,mode", [(8, 2, 2), (60, 4, 0), (64, 6, 1), (128, 8, 0), (256, 32, 1)])
+def test_topk_dispatch_in_one_launch_equals_the_two(cuda, E, k, mode):
+    """Sizes at which the tokens per workgroup and the number of workgroups change, ties, and NaN rows; calls that share one
+    workspace."""
+    from promoe_amd import ops
+    from promoe_amd._lib import lib, ptr, cur_stream, check
+    ws_bytes = 64 + 64 * E * 4
+    ws = torch.zeros(ws_bytes // 4, dtype=torch.int32, device=cuda)
+    gen = torch.Generator(device=cuda).manual_seed(E)
+    for T in (1, 15, 16, 17, 33, 65, 379, 1023, 1024, 1025, 2048, 4095, 1):
+        print(f"case topk_dispatch_ws T={T} E={E} k={k}", flush=True)
+        need = int(lib.moe_topk_dispatch_workspace_bytes(T, k, E))
+        tpb = -(-T // min(64, -(-T // 16)))
+        assert (need > 0) == (tpb * k <= 1024) and need <= ws_bytes
+        lg = torch.randn(T, E + 1, device=cuda, generator=gen)
+        lg[:, 1] = lg[:, 0]                      # ties
+        lg[T // 2] = lg[T // 2].round()
+        lg[T - 1, : E // 2] = float("nan")
+        idx, w = ops.topk(lg, k, mode, E)
+        ref = ops.dispatch(idx, E, single_workgroup=True)
+        d = ops.Dispatch(T, k, E, min(E, T * k), cuda)
+        idx2, w2 = torch.full_like(idx, -1), torch.zeros_like(w)
+        err = torch.zeros(1, dtype=torch.int32, device=cuda)
+        check(lib.moe_topk_dispatch_ws(ptr(lg), T, E, E + 1, k, mode, ptr(idx2), ptr(w2), ptr(d.counts), ptr(d.offsets),
+                                       ptr(d.sorted_pair), ptr(d.pos_of_pair), ptr(d.sorted_tok), ptr(d.units),
+                                       ptr(d.n_active), ptr(d.active_ids), d.max_units, ptr(ws), ws_bytes, ptr(err),
+                                       cur_stream()), "moe_topk_dispatch_ws")
+        assert int(err.item()) == 0 and not ws[:16].any().item()
+        assert torch.equal(idx, idx2) and torch.equal(w.view(torch.int32), w2.view(torch.int32))
+        for name in ("counts", "offsets", "sorted_pair", "pos_of_pair", "sorted_tok", "units", "n_active", "active_ids"):
+            assert torch.equal(getattr(d, name), getattr(ref, name)), name
+
+
 def run_layer_gpu(layer, x, k, mode, dev, resident=None, host_units=False):
     """gate -> topk -> dispatch -> int4 decode experts -> combine, all on the GPU."""
     from promoe_amd import ops

@@ -782,28 +782,27 @@ extern "C" int moe_forward(moe_engine *eng, int layer, const void *x, int T, voi
   if (all_resident) {
     LayerState::Pending &p = s->pend[s->pend_head];
     if (p.busy && (rc = moe_forward_harvest(eng, true))) return rc;
-    s->pend_head = (s->pend_head + 1) % LayerState::kPending;
-    p.layer = layer; p.max_units = max_units; p.busy = true;
+    const uint64_t *table = nullptr;
+    if ((rc = moe_expert_ptr_table(eng, layer, &table))) return rc;
+    if ((rc = moe_flush_table(eng, layer, st))) return rc;
     if (!routed_by_tail && launch_publishes(d, T, max_units)) {
       tail_seq = ++s->seq_counter;
       w13_publishes = true;
     }
-    if (routed_by_tail || w13_publishes) {  // a kernel stores the unit list in the slot's pinned memory itself
-      p.by_seq = true; p.seq_expected = tail_seq;
-    } else {
+    const bool by_seq = routed_by_tail || w13_publishes;  // a kernel stores the unit list in the slot's pinned memory itself
+    if (!by_seq) {
       HIPC(hipMemcpyAsync(p.units, s->units, sizeof(moe_unit) * max_units, hipMemcpyDeviceToHost, st));
       HIPC(hipMemcpyAsync(p.n_active, s->n_active, sizeof(int), hipMemcpyDeviceToHost, st));
       HIPC(hipEventRecord(p.ev, st));
-      p.by_seq = false;
     }
-    const uint64_t *table = nullptr;
-    if ((rc = moe_expert_ptr_table(eng, layer, &table))) return rc;
-    if ((rc = moe_flush_table(eng, layer, st))) return rc;
     if ((rc = run_units(eng, d, s, x, T, s->units, nullptr, max_units, d.I_sh > 0, layer, table, st,
-                        w13_publishes ? &p : nullptr, tail_seq))) {
-      if (w13_publishes) p.busy = false;  // (refused: nothing is on its way to the slot)
+                        w13_publishes ? &p : nullptr, tail_seq)))
       return rc;
-    }
+    // the slot is taken only now that everything that fills it is in the stream: after a failure above nobody waits for
+    // it.  (What a launch in front of the failed one still stores into it comes, in stream order, before the stores of the
+    // slot's next user, and carries another number.)
+    s->pend_head = (s->pend_head + 1) % LayerState::kPending;
+    p.layer = layer; p.max_units = max_units; p.busy = true; p.by_seq = by_seq; p.seq_expected = tail_seq;
     const float *sg0 = d.shared_gated ? s->logits + E : nullptr;
     if ((rc = moe_combine_splits(s->part_r, d.I_sh > 0 ? s->part_s : nullptr, s->topk_w, s->pos_of_pair, sg0, ldl, y, T, d.H, k,
                                  shared_pieces(d, T, s), st)))

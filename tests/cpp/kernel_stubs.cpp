@@ -1,9 +1,9 @@
 // Stand-ins for the GPU entry points of the library in the host-only sanitizer builds: the engine
-// refers to them, the host backend never calls them.
+// refers to them, the host backend never calls them.  Weak, so that a test can bring entry points of its own.
 #include <cstdint>
 #include <cstdio>
 
-#define STUB(name) extern "C" int name(...) { fprintf(stderr, "kernel entry " #name " called in the host-only build\n"); return -1; }
+#define STUB(name) extern "C" __attribute__((weak)) int name(...) { fprintf(stderr, "kernel entry " #name " called in the host-only build\n"); return -1; }
 STUB(moe_gate_logits)
 STUB(moe_gate_logits_bias_rows)
 STUB(moe_gate_logits_pair)

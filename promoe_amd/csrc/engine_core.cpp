@@ -828,9 +828,10 @@ extern "C" int moe_flush_table(moe_engine *eng, int layer, void *stream) {
   if (!eng->slots_ready) { moe_set_error("slots not initialised"); return MOE_ESTATE; }
   SpinGuard lk(eng->mu);
   if (!eng->table_dirty[layer]) return MOE_OK;
-  eng->table_dirty[layer] = 0;
   const size_t o = (size_t)layer * eng->cfg.num_expert;
-  return eng->be->flush_table(eng->d_table + o, eng->h_table + o, eng->cfg.num_expert, stream);
+  if (int rc = eng->be->flush_table(eng->d_table + o, eng->h_table + o, eng->cfg.num_expert, stream)) return rc;
+  eng->table_dirty[layer] = 0;  // (a refresh that failed is still due)
+  return MOE_OK;
 }
 
 int moe_flush_table_guarded(moe_engine *eng, int layer, void *stream, char *resident_out) {
@@ -840,8 +841,8 @@ int moe_flush_table_guarded(moe_engine *eng, int layer, void *stream, char *resi
   SpinGuard lk(eng->mu);
   const size_t o = (size_t)layer * eng->cfg.num_expert;
   if (eng->table_dirty[layer]) {
-    eng->table_dirty[layer] = 0;
     if (int rc = eng->be->flush_table(eng->d_table + o, eng->h_table + o, eng->cfg.num_expert, stream)) return rc;
+    eng->table_dirty[layer] = 0;
   }
   for (int e = 0; e < eng->cfg.num_expert; ++e) resident_out[e] = eng->h_table[o + e] != 0;
   eng->group_of(layer).guard++;

@@ -40,6 +40,7 @@ struct DbArgs {
   const unsigned long long *expert_ptr;
   const unsigned char *shared_base;
   int n_sh_blocks, T;
+  int pass_rows;         // most rows of one pass: what the launch has LDS for (16, 32 or 64)
   int *err;
   moe_publish pub;       // w13 pass: the first workgroup takes the unit list to the host (units_host NULL: none does)
 };
@@ -199,12 +200,18 @@ __global__ __launch_bounds__(256, 2) void k_decode_bf16(const DbArgs a) {
                                              (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)wb)), DB_NO_ROW);
   const rsrc_t rx = make_rsrc(c.act, DB_NO_ROW);
   const size_t orow0 = (size_t)win * a.T;
-  const int mm = __builtin_amdgcn_readfirstlane(m), r0 = __builtin_amdgcn_readfirstlane(row0);
-#define DB_PASS(NT_, D_) db_pass<SWIGLU, HV, NT_, D_>(c, red_db, rw, rx, setA, setB, rotA, rotB, half, kt0, nk, Kn, r0, mm, orow0, out_col, tid)
-  if (mm <= 16) DB_PASS(1, HV == 2 ? 4 : 6);
-  else if (mm <= 32) DB_PASS(2, 3);
-  else DB_PASS(4, 2);
+  // A unit has more rows than there are tokens where a token holds its expert more than once (a choice among fewer than
+  // k finite logits repeats one): then in further passes, each of no more rows than the LDS takes.
+  const int mm = __builtin_amdgcn_readfirstlane(m), r_0 = __builtin_amdgcn_readfirstlane(row0);
+  for (int p0 = 0; p0 < mm; p0 += a.pass_rows) {
+    const int mc = mm - p0 < a.pass_rows ? mm - p0 : a.pass_rows, r0 = r_0 + p0;
+    if (p0) __syncthreads();   // the sums of the pass before have been read
+#define DB_PASS(NT_, D_) db_pass<SWIGLU, HV, NT_, D_>(c, red_db, rw, rx, setA, setB, rotA, rotB, half, kt0, nk, Kn, r0, mc, orow0, out_col, tid)
+    if (mc <= 16) DB_PASS(1, HV == 2 ? 4 : 6);
+    else if (mc <= 32) DB_PASS(2, 3);
+    else DB_PASS(4, 2);
 #undef DB_PASS
+  }
 }
 
 static int db_gcd(int a, int b) { return b ? db_gcd(b, a % b) : a; }
@@ -216,8 +223,7 @@ static int db_slab_step(int nk) {
 
 template <int HV>
 static int db_launch(bool w13, const DbArgs &a, int grid, hipStream_t s) {
-  const int nt = a.T <= 16 ? 1 : (a.T <= 32 ? 2 : 4);
-  const size_t lds = (size_t)4 * 2 * HV * nt * 64 * 16;
+  const size_t lds = (size_t)4 * 2 * HV * (a.pass_rows / 16) * 64 * 16;
   moe_ktimer_begin(w13 ? MOE_K_PREFILL_W13 : MOE_K_PREFILL_W2, s);
   if (w13) hipLaunchKernelGGL((k_decode_bf16<true, HV>), dim3(grid), dim3(256), lds, s, a);
   else hipLaunchKernelGGL((k_decode_bf16<false, HV>), dim3(grid), dim3(256), lds, s, a);
@@ -225,7 +231,7 @@ static int db_launch(bool w13, const DbArgs &a, int grid, hipStream_t s) {
   return moe_check_launch("k_decode_bf16");
 }
 
-// Whether a batch of T tokens goes to these kernels (m rows of a unit <= T <= 64: every unit is one pass).
+// Whether a batch of T tokens goes to these kernels (a unit of up to 64 rows is one pass).
 bool moe_decode_bf16_takes(int T) { return T <= 64; }
 
 // Windows of the shared expert's w2 reduction: few row sets (H / 64) over a long reduction (Qwen1.5 shape: 32 over 88
@@ -245,6 +251,7 @@ int moe_decode_bf16(const void *x, int T, int H, int I, int I_sh, const moe_unit
   memset(&a, 0, sizeof a);
   a.units = units; a.expert_ptr = (const unsigned long long *)expert_ptr; a.shared_base = (const unsigned char *)shared_ptr;
   a.T = T; a.err = err;
+  a.pass_rows = T <= 16 ? 16 : (T <= 32 ? 32 : 64);
   if (pub) a.pub = *pub;
   for (int w2 = 0; w2 < 2; ++w2) {
     if (!(phases & (w2 ? 2 : 1))) continue;

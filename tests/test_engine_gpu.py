@@ -187,6 +187,30 @@ def test_resident_batches_account_their_hits_without_a_wait(cuda, kind):
 
 
 @pytest.mark.parametrize("kind", ["int4", "bf16", "q4k"])
+def test_gate_bias_that_leaves_fewer_experts_than_choices(cuda, kind):
+    """A gate bias of -inf for all but two experts, four choices per token: the choices past the second repeat an expert with
+    weight 0, so that from 33 tokens on an expert's unit has more rows than the batch has tokens."""
+    print(f"case engine_masked_gate kind={kind}", flush=True)
+    E, k = 8, 4
+    mk = {"int4": Int4Layer, "bf16": Bf16Layer, "q4k": Q4KLayer}[kind]
+    layer = mk(H=256, I=256, E=E, I_sh=256, seed=78)
+    layer.bias = np.full(E, -np.inf, np.float32)
+    layer.bias[[0, 5]] = 0.0
+    pm = build_engine([layer], k, cuda, max_tokens=512, cache_rate=1.0, cache_policy="lru")
+    pm.acquire_layer(0, np.arange(E, dtype=np.int64))
+    pm.release_layer(0)
+    for T in (8, 20, 32, 33, 64, 65, 300):
+        print(f"  T={T}", flush=True)
+        x = O.synth_acts(T, 256, seed=950 + T)
+        ref = ref_forward(layer, x, k, 0)["out"]
+        y = pm.forward(0, torch.from_numpy(x).to(torch.bfloat16).to(cuda))
+        torch.cuda.synchronize()
+        assert np.abs(y.float().cpu().numpy() - ref).max() <= TOL * np.abs(ref).max(), T
+    pm.drain()
+    pm.close()
+
+
+@pytest.mark.parametrize("kind", ["int4", "bf16", "q4k"])
 def test_forward_prefill_sizes_through_cache(cuda, kind):
     """Token groups of prefill size take the matrix-core kernels (bf16 layers always do);
     experts are still fetched and evicted underneath, one launch per missed expert."""

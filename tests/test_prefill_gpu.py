@@ -194,3 +194,39 @@ def test_bf16_decode_batch_row_sets(cuda, T, H, I, E, I_sh):
     other pass; 64 tokens over 40 experts: units of few rows and units without any."""
     print(f"case bf16_decode_row_sets T={T} H={H}", flush=True)
     check_prefill(Bf16Layer(H=H, I=I, E=E, I_sh=I_sh, seed=12, zipf=1.2), T, 4, 1, cuda)
+
+
+@pytest.mark.parametrize("T,k", [(1, 2), (16, 1), (16, 2), (13, 5), (16, 4), (17, 3), (32, 2), (33, 2), (40, 2), (64, 1), (64, 2), (65, 2)])
+def test_bf16_decode_batch_units_of_more_rows_than_tokens(cuda, T, k):
+    """An expert listed several times for one token: its unit has up to T k rows, more than one pass takes (16, 32 or 64 by
+    the batch) and just over, a last pass of one row among them.  Every partial row against the oracle's expert."""
+    from promoe_amd import ops, _lib as L
+    print(f"case bf16_decode_repeated_experts T={T} k={k}", flush=True)
+    H, I, E, I_sh = 256, 256, 3, 128
+    layer = Bf16Layer(H=H, I=I, E=E, I_sh=I_sh, seed=13)
+    x = O.synth_acts(T, H, seed=14)
+    idx = np.ones((T, k), np.int32)
+    if T == 33:                 # 65 rows of one expert, one of another
+        idx[0, 0] = 2
+    d = ops.dispatch(torch.from_numpy(idx).to(cuda), E)
+    slots = [torch.from_numpy(s).to(cuda) for s in layer.slots]
+    table = torch.tensor([s.data_ptr() for s in slots], dtype=torch.int64, device=cuda)
+    shared = torch.from_numpy(layer.shared_img).to(cuda)
+    part_r = torch.full((T * k, H), float("nan"), device=cuda)
+    part_s = torch.full((T, H), float("nan"), device=cuda)
+    h_r = torch.empty(T * k, I, dtype=torch.bfloat16, device=cuda)
+    h_s = torch.empty(T, I_sh, dtype=torch.bfloat16, device=cuda)
+    err = torch.zeros(1, dtype=torch.int32, device=cuda)
+    tiles = torch.empty(ops.prefill_workspace_bytes(L.FMT_BF16, T, H, k, d.max_units), dtype=torch.uint8, device=cuda)
+    ops.experts_prefill(bf16_dev(x, cuda), d, table, shared, H, I, I_sh, L.FMT_BF16, ws=(part_r, part_s, err, h_r, h_s, tiles))
+    torch.cuda.synchronize()
+    assert int(err.item()) == 0
+    pos = d.pos_of_pair.cpu().numpy()[: T * k]
+    assert np.array_equal(np.sort(pos), np.arange(T * k))
+    xt = torch.from_numpy(x)
+    ref = [O.swiglu_expert(xt, *[torch.from_numpy(w) for w in ws]).numpy() for ws in layer.experts_fp32]
+    want = np.stack([ref[idx[p // k, p % k]][p // k] for p in range(T * k)])
+    got = part_r.cpu().numpy()[pos]
+    assert np.abs(got - want).max() <= TOL * np.abs(want).max()      # (h between the passes in bf16)
+    sh = O.swiglu_expert(xt, *[torch.from_numpy(w) for w in layer.shared_fp32]).numpy()
+    assert np.abs(part_s.cpu().numpy() - sh).max() <= TOL * np.abs(sh).max()

@@ -361,12 +361,18 @@ static int route_batch(const moe_layer_desc &d, LayerState *s, const void *x, in
 }
 
 // a decode batch whose w13 launch computes the gate logits and routes by itself: int4 of 2 to 16 tokens, q4_K of 2 to 8
-// (Qwen2-57B shape, us a layer with the routing launch / routing by itself: 2 tokens 92.1 / 90.0, 3 tokens 101.6-106.5 / 100.8,
-// 4 tokens 115.7 / 112.4, 8 tokens 137.2 / 134.5, 9 tokens 141.3 / 139.9, 12 tokens 148.8 / 152.1, 16 tokens 160.2 / 163.3:
-// every workgroup of that wide shape repeats the routing, and with more tokens that costs more than the launch saved)
+// over at most 64 experts.  Every workgroup of the launch repeats the routing, and what a repetition costs grows with the
+// tokens (their selection rounds) and, past 64 experts, with the second to fourth column of logits per lane; a q4_K w13
+// launch has more workgroups than an int4 one has.  q4_K, us a layer, with the routing launch / routing by itself, at 2, 4, 8
+// tokens:
+//   3584 x 2560, 64 experts top-8    92.7 / 90.2   118.3 / 113.4   135.3 / 133.6   (12: 148.8 / 152.1, 16: 160.2 / 163.3)
+//   2048 x 1536, 64 experts top-6    42.8 / 38.4    53.9 /  50.4    69.0 /  66.7
+//   1024 x 512, 16 experts top-2     24.5 / 20.9    25.1 /  21.5    27.0 /  22.2
+//   4096 x 14336, 8 experts top-2   102.9 / 102.5  151.9 / 151.9   167.8 / 167.6
+//   2048 x 768, 128 experts top-8    33.9 / 37.3    41.7 /  46.1    58.2 /  62.0
 static bool batch_routes_in_w13(const moe_layer_desc &d, const LayerState *s, int T, int E, int k, int n_gate_rows) {
   static const bool on = [] { const char *e = getenv("MOE_BATCH_ROUTE"); return !e || atoi(e) != 0; }();
-  return on && (d.fmt == MOE_FMT_INT4_G128 || (d.fmt == MOE_FMT_Q4K && T <= 8)) && !use_prefill(d, T) &&
+  return on && (d.fmt == MOE_FMT_INT4_G128 || (d.fmt == MOE_FMT_Q4K && T <= 8 && E <= 64)) && !use_prefill(d, T) &&
          moe_decode_batch_int4_gate_fits(T, E, k, d.H, d.I, d.I_sh, n_gate_rows) &&
          moe_gate_route_ws_bytes(T, n_gate_rows) <= (int64_t)s->gate_ws_bytes;
 }

@@ -210,6 +210,27 @@ def test_gate_bias_that_leaves_fewer_experts_than_choices(cuda, kind):
     pm.close()
 
 
+@pytest.mark.parametrize("E", [64, 65, 130])
+def test_q4k_decode_batches_on_both_sides_of_the_self_routing_rule(cuda, E):
+    """2 to 8 tokens over up to 64 experts route in the w13 launch, over more in a launch of their own; 9 tokens always do."""
+    print(f"case engine_q4k_route E={E}", flush=True)
+    k = 8
+    layer = Q4KLayer(H=256, I=256, E=E, I_sh=256, seed=79, zipf=1.1, shared_gate=True)
+    pm = build_engine([layer], k, cuda, max_tokens=64, cache_rate=1.0, cache_policy="lru")
+    pm.acquire_layer(0, np.arange(E, dtype=np.int64))
+    pm.release_layer(0)
+    for T in (2, 5, 8, 9):
+        x = O.synth_acts(T, 256, seed=970 + T)
+        ref = ref_forward(layer, x, k, 0)
+        y = pm.forward(0, torch.from_numpy(x).to(torch.bfloat16).to(cuda))
+        torch.cuda.synchronize()
+        assert np.abs(y.float().cpu().numpy() - ref["out"]).max() <= TOL * np.abs(ref["out"]).max(), T
+        idx = pm.last_routing_idx(T, k)
+        assert np.array_equal(idx, ref["idx"]), T
+    pm.drain()
+    pm.close()
+
+
 @pytest.mark.parametrize("kind", ["int4", "bf16", "q4k"])
 def test_forward_prefill_sizes_through_cache(cuda, kind):
     """Token groups of prefill size take the matrix-core kernels (bf16 layers always do);

@@ -47,11 +47,11 @@ struct DbArgs {
 
 #define DB_NO_ROW 0x7fffff00u  // length of the buffer resources and the offset that reads zeros without a memory request
 
-// One pass over up to 16 NT token rows.  wA / wB: the lane's byte offset into the two row sets' slabs, pA / pB: their
-// first slab's position (rotation), slabs kt0 .. kt0 + nk - 1 of a row of Kn slabs.
+// One pass over up to 16 NT token rows.  rwA / rwB: the two row sets' rows of slabs, rotA / rotB: the position of slab 0
+// in them (rotation), slabs kt0 .. kt0 + nk - 1 of a row of Kn slabs.
 template <bool SWIGLU, int HV, int NT, int DEPTH>
-static __device__ __forceinline__ void db_pass(const DbClass &c, float *red, const rsrc_t rw, const rsrc_t rx, const int setA,
-                                               const int setB, const int rotA, const int rotB, const int half, const int kt0,
+static __device__ __forceinline__ void db_pass(const DbClass &c, float *red, const rsrc_t rwA, const rsrc_t rwB, const rsrc_t rx,
+                                               const int rotA, const int rotB, const int half, const int kt0,
                                                const int nk, const int Kn, const int row_first, const int mc,
                                                const size_t out_row0, const int out_col, const int tid) {
   const int lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -72,14 +72,14 @@ static __device__ __forceinline__ void db_pass(const DbClass &c, float *red, con
     const bool in = kt < nk;                    // (past the end: zeros, no memory request)
     const int kb = kt0 + (in ? kt : 0);
     const int a = kb + rotA, b = kb + rotB;
-    const int sa = setA + (a >= Kn ? a - Kn : a) * 16384, sb = setB + (b >= Kn ? b - Kn : b) * 16384;
+    const int sa = (a >= Kn ? a - Kn : a) * 16384, sb = (b >= Kn ? b - Kn : b) * 16384;
     const int v = in ? wv : (int)DB_NO_ROW;
 #pragma unroll
     for (int h = 0; h < HV; ++h)
 #pragma unroll
       for (int m = 0; m < 2; ++m) {
-        wt[d][0][h][m] = __builtin_amdgcn_raw_buffer_load_b128(rw, v + h * 256 + m * 2048, sa, 2);
-        wt[d][1][h][m] = __builtin_amdgcn_raw_buffer_load_b128(rw, v + h * 256 + m * 2048, sb, 2);
+        wt[d][0][h][m] = __builtin_amdgcn_raw_buffer_load_b128(rwA, v + h * 256 + m * 2048, sa, 2);
+        wt[d][1][h][m] = __builtin_amdgcn_raw_buffer_load_b128(rwB, v + h * 256 + m * 2048, sb, 2);
       }
 #pragma unroll
     for (int t = 0; t < NT; ++t)
@@ -193,11 +193,14 @@ __global__ __launch_bounds__(256, 2) void k_decode_bf16(const DbArgs a) {
   }
   const int gA = nbA >> 2, gB = nbB >> 2;
   const int rotA = (int)((unsigned)(gA * c.slab_step) % (unsigned)Kn), rotB = (int)((unsigned)(gB * c.slab_step) % (unsigned)Kn);
-  const int setA = gA * Kn * 16384 + (nbA & 3) * 4096;
-  const int setB = gB * Kn * 16384 + (nbB & 3) * 4096 + (!SWIGLU && HV == 1 ? 256 : 0);
-  const unsigned long long wb = (unsigned long long)(base + c.w_off);
-  const rsrc_t rw = make_rsrc((const void *)(((unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(wb >> 32)) << 32) |
-                                             (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)wb)), DB_NO_ROW);
+  // (64-bit bases: an expert image may have 2 GiB and more, a set's row of slabs has 256 bytes per column)
+  auto set_rsrc = [&](const int g, const int nb, const int off) {
+    const unsigned long long p = (unsigned long long)(base + c.w_off) + (unsigned long long)g * (unsigned)Kn * 16384u +
+                                 (unsigned)((nb & 3) * 4096 + off);
+    return make_rsrc((const void *)(((unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(p >> 32)) << 32) |
+                                    (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)p)), DB_NO_ROW);
+  };
+  const rsrc_t rwA = set_rsrc(gA, nbA, 0), rwB = set_rsrc(gB, nbB, !SWIGLU && HV == 1 ? 256 : 0);
   const rsrc_t rx = make_rsrc(c.act, DB_NO_ROW);
   const size_t orow0 = (size_t)win * a.T;
   // A unit has more rows than there are tokens where a token holds its expert more than once (a choice among fewer than
@@ -206,7 +209,7 @@ __global__ __launch_bounds__(256, 2) void k_decode_bf16(const DbArgs a) {
   for (int p0 = 0; p0 < mm; p0 += a.pass_rows) {
     const int mc = mm - p0 < a.pass_rows ? mm - p0 : a.pass_rows, r0 = r_0 + p0;
     if (p0) __syncthreads();   // the sums of the pass before have been read
-#define DB_PASS(NT_, D_) db_pass<SWIGLU, HV, NT_, D_>(c, red_db, rw, rx, setA, setB, rotA, rotB, half, kt0, nk, Kn, r0, mc, orow0, out_col, tid)
+#define DB_PASS(NT_, D_) db_pass<SWIGLU, HV, NT_, D_>(c, red_db, rwA, rwB, rx, rotA, rotB, half, kt0, nk, Kn, r0, mc, orow0, out_col, tid)
     if (mc <= 16) DB_PASS(1, HV == 2 ? 4 : 6);
     else if (mc <= 32) DB_PASS(2, 3);
     else DB_PASS(4, 2);

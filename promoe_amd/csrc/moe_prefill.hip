@@ -414,7 +414,9 @@ static __device__ __forceinline__ T pn_lds(unsigned addr) {
 
 // what a wave of a tile reads; offsets in bytes, voff per lane
 struct PnSrc {
-  pf_i32x4_t ra, rw;        // activation matrix; expert image
+  // activation matrix; nibbles, scales and (q4_K) super-block scales of the tile's 16 row blocks (64-bit bases: an expert
+  // image may have 2 GiB and more)
+  pf_i32x4_t ra, rw, rs, rz;
   int a_voff[4];            // row block n: the lane's row and chunk
   int w_voff[2];            // fragment f
   int s_voff, z_voff;       // scale request; q4_K: (d, dmin) request; int4: s_voff covers scales and zeros
@@ -440,9 +442,9 @@ static __device__ __forceinline__ void pn_mainloop(f32x16_t (&acc)[NB][2], const
     const int kt = kt0 + (kt_ < nk ? kt_ : nk - 1);
     if (r < NB) pn_dma16(lds_base + (unsigned)(so + (32 * r + 8 * w) * 128), m.a_voff[r], m.ra, kt * 128);
     else if (r < NB + 2) pn_dma16(wbase + (unsigned)(so + 1024 * (r - NB)), m.w_voff[r - NB], m.rw, kt * 512);
-    else if (!Q4K) pn_dma4(wbase + (unsigned)(so + 2048), m.s_voff + (kt >> 1) * m.s_step, m.rw, 0);
-    else if (r == NB + 2) pn_dma4(wbase + (unsigned)(so + 2048), m.s_voff, m.rw, kt * 64);
-    else pn_dma4(wbase + (unsigned)(so + 2048 + 256), m.z_voff, m.rw, (kt >> 2) * 64);
+    else if (!Q4K) pn_dma4(wbase + (unsigned)(so + 2048), m.s_voff + (kt >> 1) * m.s_step, m.rs, 0);
+    else if (r == NB + 2) pn_dma4(wbase + (unsigned)(so + 2048), m.s_voff, m.rs, kt * 64);
+    else pn_dma4(wbase + (unsigned)(so + 2048 + 256), m.z_voff, m.rz, (kt >> 2) * 64);
   };
   // LDS addresses in slot 0: the lane's activation chunk of product step j, its nibbles, its scale words
   unsigned fa0[4];
@@ -559,7 +561,10 @@ static __device__ __forceinline__ void pn_tile(const PfClass &c, const PfTile &t
   const unsigned lds_base = (unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)lds;
   PnSrc m;
   m.ra = pn_rsrc(c.act);
-  m.rw = pn_rsrc((const void *)tile.w_base);
+  const size_t tile0 = (size_t)16 * nt * G;   // (row block, group) pairs in front of the tile's
+  m.rw = pn_rsrc((const void *)(tile.w_base + c.w_off + tile0 * 1024));
+  m.rs = pn_rsrc((const void *)(tile.w_base + c.off_s + tile0 * (Q4K ? 128 : 32)));
+  m.rz = pn_rsrc((const void *)(tile.w_base + c.off_z + tile0 * (Q4K ? 32 : 8)));
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     m.a_voff[i] = 0;
@@ -573,20 +578,22 @@ static __device__ __forceinline__ void pn_tile(const PfClass &c, const PfTile &t
       m.a_voff[i] = arow * c.act_stride * 2 + (((lane & 7) ^ ((rt >> 1) & 7)) * 16);
     }
   }
-  // row block t (0..3) of this wave, t = 2 f + h: fragment f's lanes 16 h .. 16 h + 15 (of 32).  w13: gate blocks
+  // row block t (0..3) of this wave in the tile, t = 2 f + h: fragment f's lanes 16 h .. 16 h + 15 (of 32).  w13: gate blocks
   // (even) are fragment 0, up blocks (odd) fragment 1; w2: column halves 128 apart
-  auto rb = [&](int t) { return SWIGLU ? 16 * nt + 4 * w + (t >> 1) + 2 * (t & 1) : 16 * nt + 2 * w + 8 * (t >> 1) + (t & 1); };
+  auto rb = [&](int t) { return SWIGLU ? 4 * w + (t >> 1) + 2 * (t & 1) : 2 * w + 8 * (t >> 1) + (t & 1); };
 #pragma unroll
   for (int f = 0; f < 2; ++f)
-    m.w_voff[f] = (int)c.w_off + rb(2 * f + (n >> 4)) * G * 1024 + (16 * q + (n & 15)) * 16;
+    m.w_voff[f] = rb(2 * f + (n >> 4)) * G * 1024 + (16 * q + (n & 15)) * 16;
   if (Q4K) {
-    m.s_voff = (int)c.off_s + rb(lane >> 4) * G * 128 + (lane & 15) * 4;
-    m.z_voff = (int)c.off_z + rb(lane >> 4) * (G >> 1) * 64 + (lane & 15) * 4;
+    m.s_voff = rb(lane >> 4) * G * 128 + (lane & 15) * 4;
+    m.z_voff = rb(lane >> 4) * (G >> 1) * 64 + (lane & 15) * 4;
     m.s_step = 0;
   } else {
-    // lanes 0..31: 8 dwords of scales of each row block; lanes 32..39: 2 dwords of zeros of each; the rest idle copies
+    // lanes 0..31: 8 dwords of scales of each row block; lanes 32..39: 2 dwords of zeros of each; the rest idle copies.
+    // The zeros of the tile lie behind its scales (in the image's next section, less than 2 GiB away: the launcher)
     const int l = lane < 40 ? lane : 39;
-    m.s_voff = l < 32 ? (int)c.off_s + rb(l >> 3) * G * 32 + (l & 7) * 4 : (int)c.off_z + rb((l - 32) >> 1) * G * 8 + (l & 1) * 4;
+    const int z0 = (int)(c.off_z - c.off_s - (long long)tile0 * 24);
+    m.s_voff = l < 32 ? rb(l >> 3) * G * 32 + (l & 7) * 4 : z0 + rb((l - 32) >> 1) * G * 8 + (l & 1) * 4;
     m.s_step = l < 32 ? 32 : 8;
     m.z_voff = 0;
   }
@@ -895,6 +902,13 @@ extern "C" int moe_experts_prefill_publish(const void *x_bf16, int T, int H, int
     moe_set_error("moe_experts_prefill: H %% 256 == 0 and I %% 128 == 0 required (H=%d I=%d I_sh=%d)", H, I, I_sh);
     return MOE_EINVAL;
   }
+  {  // offsets inside a 128-row group of a bf16 matrix (256 bytes per column) and inside 16 row blocks of nibbles (128)
+    const int most = int4 ? 1 << 24 : 1 << 23;
+    if (H >= most || I >= most || (shared_ptr && I_sh >= most)) {
+      moe_set_error("moe_experts_prefill: rows of %d columns and more are not supported (H=%d I=%d I_sh=%d)", most, H, I, I_sh);
+      return MOE_EINVAL;
+    }
+  }
   if (bf16_decode)
     return moe_decode_bf16(x_bf16, T, H, I, I_sh, units, max_units, sorted_tok, expert_ptr, shared_ptr, h_r, h_s, part_r, part_s,
                            shared_pieces, err, phases, pub, s);
@@ -953,6 +967,10 @@ extern "C" int moe_experts_prefill_publish(const void *x_bf16, int T, int H, int
         c.w_off = w2 ? lay.off2_q : lay.off13_q;
         c.off_s = w2 ? lay.off2_s : lay.off13_s;
         c.off_z = w2 ? lay.off2_z : lay.off13_z;
+        if (!q4k && c.off_z - c.off_s >= (1ll << 31) - (1ll << 24)) {  // (pn_tile: the zeros are addressed from the scales)
+          moe_set_error("moe_experts_prefill: the scales of an expert of %d x %d take 2 GiB or more", H, Ii);
+          return MOE_EINVAL;
+        }
       }
       c.ksplit = (w2 && shared && int4) ? shared_pieces : 1;
       c.split_stride = (long long)T * H;

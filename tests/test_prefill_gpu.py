@@ -230,3 +230,60 @@ def test_bf16_decode_batch_units_of_more_rows_than_tokens(cuda, T, k):
     assert np.abs(got - want).max() <= TOL * np.abs(want).max()      # (h between the passes in bf16)
     sh = O.swiglu_expert(xt, *[torch.from_numpy(w) for w in layer.shared_fp32]).numpy()
     assert np.abs(part_s.cpu().numpy() - sh).max() <= TOL * np.abs(sh).max()
+
+
+def _last_columns_image(kind, H, I, dev):
+    """Image of an H x I expert whose weights are zero but for the last columns of the intermediate dimension (bf16, int4: 128,
+    q4_K: 256), made from a small expert of just these: the image, and the small expert's fp32 weights."""
+    from promoe_amd import layout as LY
+    small_I = 256 if kind == "q4k" else 128
+    cls = {"bf16": Bf16Layer, "int4": Int4Layer, "q4k": Q4KLayer}[kind]
+    layer = cls(H=H, I=small_I, E=1, seed=15)
+    src = torch.from_numpy(layer.slots[0]).to(dev)
+    if kind == "bf16":
+        big = torch.zeros(LY.bf16_expert_bytes(H, I), dtype=torch.uint8, device=dev)
+        nk, group = H // 64, H // 64 * 16384                       # w13: 128-row groups of nk slabs, rotated by group
+        for m in range(2):                                         # gate, up: the last group of each half
+            t = src[m * group:(m + 1) * group].view(nk, 16384).roll(-((m * LY.slab_step(nk)) % nk), 0)
+            g = (m + 1) * I // 128 - 1
+            big[g * group:(g + 1) * group] = t.roll((g * LY.slab_step(nk)) % nk, 0).reshape(-1)
+        nk = I // 64
+        s2, b2 = src[2 * group:].view(H // 128, 2, 16384), big[2 * I * H * 2:].view(H // 128, nk, 16384)
+        for g in range(H // 128):
+            for j in range(2):
+                b2[g, (nk - 2 + j + g * LY.slab_step(nk)) % nk] = s2[g, (j + g * LY.slab_step(2)) % 2]
+        return big, layer.experts_fp32[0]
+    mk = LY.int4_layout if kind == "int4" else LY.q4k_layout
+    ls, lb = mk(H, small_I), mk(H, I)
+    big = torch.zeros(lb["total_bytes"], dtype=torch.uint8, device=dev)
+    for sec, per in (("q", 1024), ("s", 32 if kind == "int4" else 128), ("z", 8 if kind == "int4" else 32)):  # bytes per tile
+        n13 = 2 * small_I // 16 * (H // 128) * per
+        end = lb["off13_" + sec] + 2 * I // 16 * (H // 128) * per
+        big[end - n13:end] = src[ls["off13_" + sec]:ls["off13_" + sec] + n13]
+        gs, gb = small_I // 128 * per, I // 128 * per
+        rows = H // 16
+        big[lb["off2_" + sec]:lb["off2_" + sec] + rows * gb].view(rows, gb)[:, gb - gs:] = \
+            src[ls["off2_" + sec]:ls["off2_" + sec] + rows * gs].view(rows, gs)
+    return big, layer.experts_fp32[0]
+
+
+@pytest.mark.parametrize("kind,H,I", [("bf16", 256, 2097408), ("int4", 1024, 1400064), ("q4k", 1024, 1400064), ("int4", 256, 1408),
+                                      ("q4k", 256, 1536), ("bf16", 256, 1408)])
+def test_expert_images_of_two_gib_and_more(cuda, kind, H, I):
+    """Offsets inside an expert image past 31 bits (and the same construction on a small expert): only the weights at the far
+    end of each matrix are not zero."""
+    from promoe_amd import ops, _lib as L
+    print(f"case prefill_large_image {kind} H={H} I={I}", flush=True)
+    img, ws = _last_columns_image(kind, H, I, cuda)
+    assert I < 10000 or img.numel() >= 1 << 31
+    T = 3
+    x = O.synth_acts(T, H, seed=16)
+    d = ops.dispatch(torch.zeros(T, 1, dtype=torch.int32, device=cuda), 1)
+    table = torch.tensor([img.data_ptr()], dtype=torch.int64, device=cuda)
+    fmt = {"bf16": L.FMT_BF16, "int4": L.FMT_INT4_G128, "q4k": L.FMT_Q4K}[kind]
+    part_r, _, err, *_ = ops.experts_prefill(bf16_dev(x, cuda), d, table, None, H, I, 0, fmt)
+    torch.cuda.synchronize()
+    assert int(err.item()) == 0
+    ref = O.swiglu_expert(torch.from_numpy(x), *[torch.from_numpy(np.asarray(w)) for w in ws]).numpy()
+    got = part_r.cpu().numpy()
+    assert np.abs(got - ref).max() <= TOL * np.abs(ref).max()

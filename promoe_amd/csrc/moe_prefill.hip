@@ -47,7 +47,7 @@ struct PfClass {
   int act_stride, out_stride, K, n_ntiles, n_mtiles, n_cols_per_tile;
   int shared;           // the shared expert's class
   int slab_step;        // storage rotation per 128-row group: smallest odd s >= 3 coprime with K/64
-  int n_blocks;         // n_mtiles * n_ntiles * ksplit, padded to whole rounds of runs (pf_block_of)
+  int n_blocks;         // n_mtiles * n_ntiles * ksplit, padded (pf_padded)
   int ksplit;           // int4 / q4_K w2 pass of the shared expert: workgroups per tile, each over 1/ksplit of the
                         // reduction, partial rows to out + split * split_stride (0 or 1: the whole reduction)
   long long split_stride;  // elements between the pieces of out
@@ -64,17 +64,25 @@ static __device__ __forceinline__ float pf_silu_mul(float g, float u) {
 }
 
 // Which block of which class a physical workgroup takes; false: none.  The blocks of class 0 come first, each class
-// padded to a multiple of 8 PF_DEAL.  Workgroup i runs on XCD i % 8; runs of PF_DEAL consecutive blocks are dealt to
-// the XCDs in turn, over both classes (class 1 goes on where class 0 ended), so that the XCDs get the same number of
+// padded (pf_padded).  Workgroup i runs on XCD i % 8; runs of PF_DEAL consecutive blocks are dealt to
+// the XCDs in turn, so that the XCDs get the same number of
 // blocks of every size whatever the row counts are: the list holds the large tiles first.  (One contiguous range of the
 // list per XCD, the order before this one, left the XCDs with the popular experts' tiles busy alone: 1.4 of 2 waves per
 // SIMD on average over the w13 launch of the DeepSeek shape at 2048 tokens, 1.0 at 379.)
 // Inside the list: a group of up to PF_GROUP tiles of one expert goes through all its column tiles, tile fastest, so
 // that a run shares either a column tile's weights (many tiles) or the activation rows (one tile) in its XCD's L2.
-// Measured on one box, us a layer: DeepSeek shape 379 tokens 156 -> 148, 2048 tokens 378 -> 365, Mixtral shape 4096
-// tokens 2748 -> 2560 (eight row tiles share a column tile's weights); Qwen1.5 bf16 and q4_K prefill unchanged.
+// EVEN (bf16 kernel: one workgroup per compute unit, so that a run too many is a quarter of a round of its XCD): the blocks
+// of a class past its last whole round of 8 runs are spread evenly.  Otherwise class 1 goes on at the XCD where class 0
+// ended, and the last round is runs as well: what the nibble kernel's short launches are faster with.
+// Measured, us, contiguous ranges / runs / even, w13 and w2 launch:
+//   bf16, Qwen1.5 shape    65 tokens 115.5 / 116.2 / 116.7 and 77.6 / 88.3 / 77.8, 379 tokens 135.6 / 136.5 / 136.5 and
+//                          91.1 / 93.4 / 91.6, 1999 tokens 228 / 224 / 224 and 132 / 131 / 135
+//   bf16, Mixtral shape    1024 tokens 489 / 423 / 424 and 287 / 289 / 287, 2048 tokens 909 / 738 / 737 and 519 / 470 / 467
+//   int4, DeepSeek shape   (runs / even) 65 tokens 34.3 / 34.5 and 31.7 / 33.1, 200 tokens 44.9 / 46.5 and 36.4 / 37.6, 2048
+//                          tokens 194 / 193 and 109 / 110
 #define PF_DEAL 8
 #define PF_GROUP 8
+template <bool EVEN>
 static __device__ __forceinline__ bool pf_block_of(const PfArgs &a, int &ci, int &mt, int &nt, int &split) {
   const int pad0 = a.c[0].n_blocks;
   ci = (int)blockIdx.x >= pad0;
@@ -83,12 +91,17 @@ static __device__ __forceinline__ bool pf_block_of(const PfArgs &a, int &ci, int
   const int ks = c.ksplit > 1 ? c.ksplit : 1;
   const int n_tiles = *c.n_tiles_real * c.n_ntiles, n_real = n_tiles * ks;
   int xcd = pb & 7;
-  if (ci) {
+  if (!EVEN && ci) {
     const int n0 = *a.c[0].n_tiles_real * a.c[0].n_ntiles * (a.c[0].ksplit > 1 ? a.c[0].ksplit : 1);
     xcd = (xcd - (n0 + PF_DEAL - 1) / PF_DEAL) & 7;
   }
-  const int i = pb >> 3;
-  int b = ((i / PF_DEAL) * 8 + xcd) * PF_DEAL + i % PF_DEAL;
+  const int i = pb >> 3, first = i / PF_DEAL * (8 * PF_DEAL), j = i % PF_DEAL;  // first: the round's first block
+  int b = first + xcd * PF_DEAL + j;
+  if (EVEN && n_real - first < 8 * PF_DEAL) {
+    const int each = (n_real - first + 7) >> 3;
+    if (j >= each) return false;
+    b = first + xcd * each + j;
+  }
   if (b >= n_real) return false;
   // a class whose reduction is split has ksplit workgroups per tile: the pieces of one tile are `n_tiles` blocks
   // apart, so that the first piece of every tile starts before the second of any
@@ -246,7 +259,7 @@ __global__ __launch_bounds__(256, 1) void k_prefill_gemm(const PfArgs a) {
   extern __shared__ __align__(16) uint16_t As[];  // [PF4_RING][PF_BM][PF_BK]
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   int ci, mt, nt, split;
-  if (!pf_block_of(a, ci, mt, nt, split)) return;
+  if (!pf_block_of<true>(a, ci, mt, nt, split)) return;
   const PfClass &c = a.c[ci];
   const PfTile tile = c.tiles[mt];
   const int rows = pf_rows(tile);
@@ -645,7 +658,7 @@ __global__ __launch_bounds__(256, 2) void k_prefill_nib(const PfArgs a) {
   extern __shared__ __align__(16) unsigned char lds_n[];
   const int tid = threadIdx.x;
   int ci, mt, nt, split;
-  if (!pf_block_of(a, ci, mt, nt, split)) return;
+  if (!pf_block_of<false>(a, ci, mt, nt, split)) return;
   const PfClass &c = a.c[ci];
   const PfTile tile = c.tiles[mt];
   const int rows = pf_rows(tile);
@@ -667,6 +680,14 @@ static int pf_slab_step(int nk) {
   int s = 3;
   while (pf_gcd(s, nk) != 1) s += 2;
   return s;
+}
+
+// Workgroups of a class of `blocks` blocks: whole rounds of 8 runs, or, where less than a round is spread evenly (EVEN), an
+// even share per XCD (56 idle workgroups between the shared expert's 8 w2 blocks and the routed ones of a 65-token batch of
+// the Qwen1.5 shape made that launch 85 us instead of 78)
+static int pf_padded(bool even, int blocks) {
+  const int q = even && blocks < 8 * PF_DEAL ? 8 : 8 * PF_DEAL;
+  return (blocks + q - 1) / q * q;
 }
 
 template <bool Q4K>
@@ -974,7 +995,7 @@ extern "C" int moe_experts_prefill_publish(const void *x_bf16, int T, int H, int
       }
       c.ksplit = (w2 && shared && int4) ? shared_pieces : 1;
       c.split_stride = (long long)T * H;
-      c.n_blocks = (c.n_mtiles * c.n_ntiles * c.ksplit + 8 * PF_DEAL - 1) / (8 * PF_DEAL) * (8 * PF_DEAL);  // whole rounds of runs
+      c.n_blocks = pf_padded(!int4, c.n_mtiles * c.n_ntiles * c.ksplit);
       c.slab_step = pf_slab_step(c.K / PF_BK);
       a.n_blocks_total += c.n_blocks;
     }

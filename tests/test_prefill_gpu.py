@@ -287,3 +287,35 @@ def test_expert_images_of_two_gib_and_more(cuda, kind, H, I):
     ref = O.swiglu_expert(torch.from_numpy(x), *[torch.from_numpy(np.asarray(w)) for w in ws]).numpy()
     got = part_r.cpu().numpy()
     assert np.abs(got - ref).max() <= TOL * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("cls", [Int4Layer, Bf16Layer])
+@pytest.mark.parametrize("T", [1023, 1024, 1025, 2100])
+def test_prefill_tile_list_of_many_units(cuda, T, cls):
+    """Unit lists just short of, as long as and longer than one scan of the tile list takes: every token a unit of its own, and
+    the rows of every third a unit of 40 or 130 rows; the same partial rows as from one unit of all tokens."""
+    from promoe_amd import ops, _lib as L
+    print(f"case prefill_many_units T={T} {cls.__name__}", flush=True)
+    layer = cls(H=256, I=128, E=1, seed=18)
+    fmt = L.FMT_BF16 if cls is Bf16Layer else L.FMT_INT4_G128
+    slot = torch.from_numpy(layer.slots[0]).to(cuda)
+    table = torch.tensor([slot.data_ptr()], dtype=torch.int64, device=cuda)
+    sizes = [(1, 1, 40, 1, 1, 130)[u % 6] for u in range(T)]
+    P = sum(sizes)
+    x = bf16_dev(O.synth_acts(P, 256, seed=19), cuda)
+    d = ops.dispatch(torch.zeros(P, 1, dtype=torch.int32, device=cuda), 1)
+    ref = ops.experts_prefill(x, d, table, None, 256, 128, 0, fmt)
+    many = ops.Dispatch(P, 1, 1, T, cuda)
+    many.sorted_tok = d.sorted_tok
+    rows0 = np.concatenate([[0], np.cumsum(sizes)[:-1]])
+    u = np.stack([np.zeros(T), sizes, rows0, np.zeros(T)], axis=1).astype(np.int32)
+    u[T // 2] = (-1, 0, 0, 0)                     # an unused entry in the middle
+    many.units = torch.from_numpy(u).to(cuda)
+    got = ops.experts_prefill(x, many, table, None, 256, 128, 0, fmt,
+                              ws=(torch.full_like(ref[0], float("nan")), None, ref[2], ref[3], None,
+                                  torch.zeros(ops.prefill_workspace_bytes(fmt, P, 256, 1, T), dtype=torch.uint8, device=cuda)))
+    torch.cuda.synchronize()
+    assert int(got[2].item()) == 0
+    live = torch.ones(P, dtype=torch.bool, device=cuda)
+    live[rows0[T // 2]: rows0[T // 2] + sizes[T // 2]] = False
+    assert torch.equal(got[0][live], ref[0][live]) and bool(torch.isnan(got[0][~live]).all())

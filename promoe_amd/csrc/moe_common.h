@@ -35,6 +35,6 @@ int moe_decode_bf16(const void *x, int T, int H, int I, int I_sh, const moe_unit
 
 // gate logits on the matrix cores (moe_gate.hip), behind moe_gate_logits for the batches it takes; same bits.  The first
 // n_bias rows get the bias.
-bool moe_gate_tiles_take(int T, int E);
+bool moe_gate_tiles_take(int T, int H, int E);
 int moe_gate_tiles(const void *x, const void *wg, const float *bias, int n_bias, float *logits, int T, int H, int E, int ldl,
                    hipStream_t s);

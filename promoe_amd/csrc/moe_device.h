@@ -176,3 +176,70 @@ static __device__ __forceinline__ u32 f2h_bits(float f) {  // fp32 -> fp16 bits 
   return (u32)__builtin_bit_cast(uint16_t, (_Float16)f);
 }
 
+// The sum of one (token, gate row) pair by one wave, in a fixed order (bit-reproducible): lane partials over
+// k = 512 c + 8 lane + j with one fma chain, then the xor butterfly 32..1.  Every lane returns the sum.
+// All loads of the row go out back to back, without a condition around any of them (a lane past the end of the row
+// reads column 0 and drops the result): with a condition per 512-column chunk the compiler put a full wait for
+// memory between the chunks, and a 2048-wide row took four round trips to memory instead of one.
+template <int NCH>
+static __device__ __forceinline__ float gate_row_partial(const uint16_t *__restrict__ xr, const uint16_t *__restrict__ wr,
+                                                         const int H, const int lane) {
+  uint4 xq[NCH], wq[NCH];
+#pragma unroll
+  for (int c = 0; c < NCH; ++c) {
+    const int k = c * 512 + 8 * lane;
+    const int kk = k < H ? k : 0;
+    xq[c] = *(const uint4 *)(xr + kk);
+    wq[c] = *(const uint4 *)(wr + kk);
+  }
+  float acc = 0.f;
+#pragma unroll
+  for (int c = 0; c < NCH; ++c) {
+    float t = acc;
+    t = fmaf(bf16lo(xq[c].x), bf16lo(wq[c].x), t);
+    t = fmaf(bf16hi(xq[c].x), bf16hi(wq[c].x), t);
+    t = fmaf(bf16lo(xq[c].y), bf16lo(wq[c].y), t);
+    t = fmaf(bf16hi(xq[c].y), bf16hi(wq[c].y), t);
+    t = fmaf(bf16lo(xq[c].z), bf16lo(wq[c].z), t);
+    t = fmaf(bf16hi(xq[c].z), bf16hi(wq[c].z), t);
+    t = fmaf(bf16lo(xq[c].w), bf16lo(wq[c].w), t);
+    t = fmaf(bf16hi(xq[c].w), bf16hi(wq[c].w), t);
+    acc = (c * 512 + 8 * lane < H) ? t : acc;
+  }
+  return acc;
+}
+
+static __device__ __forceinline__ float gate_row_sum(const uint16_t *__restrict__ xr, const uint16_t *__restrict__ wr,
+                                                     const int H, const int lane) {
+  float acc = 0.f;
+  const int nch = (H + 511) >> 9;  // wave-uniform
+  switch (nch) {
+    case 1: acc = gate_row_partial<1>(xr, wr, H, lane); break;
+    case 2: acc = gate_row_partial<2>(xr, wr, H, lane); break;
+    case 3: acc = gate_row_partial<3>(xr, wr, H, lane); break;
+    case 4: acc = gate_row_partial<4>(xr, wr, H, lane); break;
+    case 5: acc = gate_row_partial<5>(xr, wr, H, lane); break;
+    case 6: acc = gate_row_partial<6>(xr, wr, H, lane); break;
+    case 7: acc = gate_row_partial<7>(xr, wr, H, lane); break;
+    case 8: acc = gate_row_partial<8>(xr, wr, H, lane); break;
+    default:
+      for (int c = 0; c < H; c += 512) {
+        const int k = c + 8 * lane;
+        if (k < H) {
+          const uint4 xv = *(const uint4 *)(xr + k);
+          const uint4 wv = *(const uint4 *)(wr + k);
+          acc = fmaf(bf16lo(xv.x), bf16lo(wv.x), acc);
+          acc = fmaf(bf16hi(xv.x), bf16hi(wv.x), acc);
+          acc = fmaf(bf16lo(xv.y), bf16lo(wv.y), acc);
+          acc = fmaf(bf16hi(xv.y), bf16hi(wv.y), acc);
+          acc = fmaf(bf16lo(xv.z), bf16lo(wv.z), acc);
+          acc = fmaf(bf16hi(xv.z), bf16hi(wv.z), acc);
+          acc = fmaf(bf16lo(xv.w), bf16lo(wv.w), acc);
+          acc = fmaf(bf16hi(xv.w), bf16hi(wv.w), acc);
+        }
+      }
+  }
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) acc = acc + __shfl_xor(acc, m, 64);
+  return acc;
+}

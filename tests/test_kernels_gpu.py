@@ -66,6 +66,28 @@ def test_gate_logits_tiles(cuda, T, H, E):
     assert np.all(got[:, E:] == 7.0)
 
 
+@pytest.mark.parametrize("T,H,E", [(500, 512, 66), (700, 1024, 19), (777, 1032, 34), (401, 4360, 50), (1300, 504, 17), (1001, 1024, 33),
+                                   (320, 2056, 65), (216, 776, 60), (217, 776, 60), (334, 1032, 60)])
+def test_gate_logits_tiles_rows_behind_the_last_tile(cuda, T, H, E):
+    """One, two and more rows behind the last whole tile of 16, in every form of the kernel (rows of up to 512, 1024 and more
+    columns), with a bias on all rows, and on none of the last; the last batch below and the first above the line."""
+    from promoe_amd import _lib as L
+    print(f"case gate_logits_rest T={T} H={H} E={E}", flush=True)
+    x = bf16_dev(O.synth_acts(T, H, seed=4), cuda)
+    wg = bf16_dev(O.round_bf16(O.synth_weights((E, H), seed=5)), cuda)
+    bias = torch.linspace(-1, 1, E, device=cuda)
+    ref0 = O.gate_logits_ordered(x.float().cpu().numpy(), wg.float().cpu().numpy())
+    for n_bias in (E, E - 1, E // 16 * 16):
+        out = torch.full((T, E + 1), 7.0, device=cuda)
+        L.check(L.lib.moe_gate_logits_bias_rows(L.ptr(x), L.ptr(wg), L.ptr(bias), n_bias, L.ptr(out), T, H, E, E + 1, L.cur_stream()),
+                "gate")
+        ref = ref0.copy()
+        ref[:, :n_bias] += bias.cpu().numpy()[:n_bias]
+        got = out.cpu().numpy()
+        assert np.array_equal(got[:, :E].view(np.uint32), ref.view(np.uint32)), n_bias
+        assert np.all(got[:, E:] == 7.0)
+
+
 @pytest.mark.parametrize("mode", [0, 1, 2])
 @pytest.mark.parametrize("T,E,k", [(1, 64, 6), (16, 64, 6), (33, 60, 4), (5, 8, 2), (9, 64, 8), (4, 200, 8)])
 def test_topk_routing(cuda, T, E, k, mode):

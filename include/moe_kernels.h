@@ -361,7 +361,7 @@ int moe_experts_decode_q4k_publish(const void *x_bf16, int T, int H, int I, int 
  *               needs no copy of the dispatch counts.
  *   phases    : bit 0 = w13 + SwiGLU, bit 1 = w2; bit 2 (nibble formats) = tiles_ws has room for the fp16 copy of
  *               x behind the list, T*H*2 bytes at the next multiple of 256 (without it the call takes and returns
- *               stream-ordered memory for the copy); bit 3, with bit 2 = that room already holds the copy of this x.
+ *               stream-ordered memory for the copy).
  * Between the two passes h_r / h_s hold bf16 for MOE_FMT_BF16 and fp16 for the nibble formats (whose matrix-core
  * operands are fp16: the w2 pass then stages them without a conversion); both passes of a batch go through this entry.
  * H % 256 == 0, I % 128 == 0, I_sh % 128 == 0.  The reference leaves this product to the

@@ -952,8 +952,8 @@ extern "C" int moe_experts_prefill_publish(const void *x_bf16, int T, int H, int
   const int cap = int4 ? PN_BM : PF_BM, cap_s = int4 ? PN_BM : PF_BM_SHARED, cap_s2 = PF_BM_SHARED_W2;
   // fp16 copy of x for the nibble formats: behind the tile list where the caller left room, else stream-ordered memory
   void *x16 = nullptr, *x16_own = nullptr;
-  const bool convert = int4 && (phases & 1) && !((phases & 4) && (phases & 8));
-  if (int4 && (phases & 1)) {
+  const bool convert = int4 && (phases & 1);
+  if (convert) {
     if (phases & 4) x16 = (unsigned char *)tiles_ws + pf_x16_offset(T, k, max_units);
     else if (int rc = moe_check_hip(hipMallocAsync(&x16_own, (size_t)T * H * 2, s), "hipMallocAsync(fp16 activations)")) return rc;
     if (x16_own) x16 = x16_own;

@@ -176,6 +176,24 @@ def test_prefill_nibble_without_room_for_the_converted_activations(cuda):
     assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1]) and int(b[2].item()) == 0
 
 
+def test_prefill_converts_the_activations_of_every_call(cuda):
+    """Two calls that share a workspace with room for the fp16 copy: the second is over its own x, whatever bits above the
+    documented ones its phases have."""
+    from promoe_amd import ops, _lib as L
+    print("case prefill_converts_each_call", flush=True)
+    layer = Int4Layer(H=256, I=128, E=2, I_sh=128, seed=20)
+    xs = [bf16_dev(O.synth_acts(70, 256, seed=70 + i), cuda) for i in range(2)]
+    d = ops.dispatch(torch.zeros(70, 1, dtype=torch.int32, device=cuda), 2)
+    slots = [torch.from_numpy(s).to(cuda) for s in layer.slots]
+    table = torch.tensor([s.data_ptr() for s in slots], dtype=torch.int64, device=cuda)
+    shared = torch.from_numpy(layer.shared_img).to(cuda)
+    ref = ops.experts_prefill(xs[1], d, table, shared, 256, 128, 128, L.FMT_INT4_G128)
+    ws = ops.experts_prefill(xs[0], d, table, shared, 256, 128, 128, L.FMT_INT4_G128)
+    got = ops.experts_prefill(xs[1], d, table, shared, 256, 128, 128, L.FMT_INT4_G128, phases=3 | 8, ws=ws)
+    torch.cuda.synchronize()
+    assert torch.equal(got[0], ref[0]) and torch.equal(got[1], ref[1]) and int(got[2].item()) == 0
+
+
 @pytest.mark.parametrize("T", [1, 15, 16, 17, 32, 33, 63, 64, 65])
 def test_bf16_decode_batch_edges(cuda, T):
     """Every token to one expert, on the weight-stream kernel up to 64 tokens: passes of 16, 32 and 64 rows just short,

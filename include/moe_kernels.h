@@ -374,12 +374,14 @@ int moe_experts_prefill(const void *x_bf16, int T, int H, int I, int I_sh, int k
                         float *part_r, float *part_s, void *tiles_ws, int *err, int phases,
                         void *stream);
 
-/* The same with the shared expert's partial rows of the w2 pass in shared_pieces pieces (1, 2, 4 or 8; nibble
- * formats only): part_s holds shared_pieces * T rows, piece s at part_s + s*T*H, each the product over one window
- * of the I_sh columns; moe_combine_splits adds them.  moe_prefill_shared_splits(fmt, T, H, I_sh) = the number of
- * pieces worth taking: more than 1 where the shared expert's workgroups of that pass (ceil(T/128) * H/256, each over
- * the whole reduction) are few and the reduction is long, so that they would outlast the rest of the launch
- * (Qwen2-57B shape at 512 tokens: 4).  No reference counterpart (see moe_decode_shared_splits). */
+/* The same with the shared expert's partial rows of the w2 pass in shared_pieces pieces (1, 2, 4 or 8): part_s holds
+ * shared_pieces * T rows, piece s at part_s + s*T*H, each the product over one window of the I_sh columns;
+ * moe_combine_splits adds them.  The pieces must divide I_sh / 64 (bf16 batches of at most 64 tokens) or I_sh / 256 (nibble
+ * formats); other bf16 batches take 1.  moe_prefill_shared_splits(fmt, T, H, I_sh) = the number of pieces worth taking, and
+ * what part_s has to hold if that number is passed: more than 1 where the shared expert's workgroups of that pass are few
+ * and the reduction is long, so that they would outlast the rest of the launch: nibble formats by their ceil(T/128) * H/256
+ * tiles (Qwen2-57B shape at 512 tokens: 4), bf16 batches of at most 64 tokens by their H/64 row sets (Qwen1.5 shape: 4 up to
+ * 64 tokens, 1 above).  No reference counterpart (see moe_decode_shared_splits). */
 int moe_prefill_shared_splits(int fmt, int T, int H, int I_sh);
 int moe_experts_prefill_pieces(const void *x_bf16, int T, int H, int I, int I_sh, int k, int fmt,
                                const moe_unit *units, int max_units, const int *sorted_tok,

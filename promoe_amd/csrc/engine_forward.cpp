@@ -248,8 +248,9 @@ int moe_forward_harvest(moe_engine *eng, bool wait) {
       volatile int *sq = p.seq;
       if (*sq != p.seq_expected) {
         if (!wait) break;
-        // the launch that writes it is already in the compute stream; what was queued behind it stays queued (waiting
-        // for the whole stream here left the GPU without work each time the host was kPending layers ahead)
+        // the launch that writes it is already in the compute stream.  A waiting harvest empties every slot, so of the
+        // kPending layers queued only what stands behind the newest layer's publishing launch is still ahead of the GPU
+        // when the host goes on (waiting for the whole stream left it without work)
         const auto t0 = std::chrono::steady_clock::now();
         unsigned spins = 0;
         while (*sq != p.seq_expected)

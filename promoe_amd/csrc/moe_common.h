@@ -26,6 +26,15 @@ static inline bool moe_publish_ok(const moe_publish *p, int max_units) {
   return p->n_active && p->units_host && p->n_active_host && p->seq_host && p->max_units > 0 && p->max_units <= max_units;
 }
 
+// Storage rotation of a bf16 matrix per 128-row group of nk slabs: smallest odd s >= 3 coprime with nk (the slot layout)
+static inline int moe_bf16_slab_step(int nk) {
+  for (int s = 3;; s += 2) {
+    int a = s, b = nk;
+    while (b) { const int r = a % b; a = b; b = r; }
+    if (a == 1) return s;
+  }
+}
+
 // bf16 expert product of a decode batch (moe_decode_bf16.hip), behind moe_experts_prefill for batches it takes
 bool moe_decode_bf16_takes(int T);
 int moe_decode_bf16_splits(int H, int I_sh);

@@ -217,13 +217,6 @@ __global__ __launch_bounds__(256, 2) void k_decode_bf16(const DbArgs a) {
   }
 }
 
-static int db_gcd(int a, int b) { return b ? db_gcd(b, a % b) : a; }
-static int db_slab_step(int nk) {
-  int s = 3;
-  while (db_gcd(s, nk) != 1) s += 2;
-  return s;
-}
-
 template <int HV>
 static int db_launch(bool w13, const DbArgs &a, int grid, hipStream_t s) {
   const size_t lds = (size_t)4 * 2 * HV * (a.pass_rows / 16) * 64 * 16;
@@ -269,7 +262,7 @@ int moe_decode_bf16(const void *x, int T, int H, int I, int I_sh, const moe_unit
         c.out = i == 0 ? (void *)part_s : (void *)part_r; c.out_stride = H; c.K = Ii;
         c.w_off = (long long)2 * Ii * H * 2; c.set_delta = 0; c.ksplit = i == 0 ? pieces : 1;
       }
-      c.slab_step = c.K ? db_slab_step(c.K / 64) : 1;
+      c.slab_step = c.K ? moe_bf16_slab_step(c.K / 64) : 1;
     }
     const int sh_blk = shared_ptr ? (w2 ? H / 64 * pieces : I_sh / 32) : 0, r_blk = w2 ? H / 64 : I / 32;
     // 16-row sets where 32-row sets would leave the chip with under four workgroups per compute unit

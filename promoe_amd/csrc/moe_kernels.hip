@@ -242,7 +242,7 @@ __global__ __launch_bounds__(DISP_THREADS) void k_dispatch(
 // expert start), and scatters.  The barrier words are zero at launch and are left zero.  A workgroup that waits
 // longer than a second raises the error word and goes on with what it has (positions stay inside the arrays).
 // TOPK: the pairs come from the logits: a workgroup first selects the experts of its own tokens (chunk / k of them, a wave per
-// token, the arithmetic of k_topk), and writes idx and wout.  Up to 64 workgroups of at least 16 tokens: both steps are chains
+// token, the arithmetic of k_topk), and writes idx and wout.  One workgroup per 16 tokens begun, up to 64, with even shares of the tokens: both steps are chains
 // of round trips, and the top-k as a launch of its own cost 4.7 us in front of this one's 6.4.
 // ---------------------------------------------------------------------------
 #define DISPM_MAXB 64
@@ -250,7 +250,7 @@ struct DispTopk {
   const float *logits;
   float *w;
   int *idx;
-  int T, ldl, mode;
+  int ldl, mode;
 };
 template <bool TOPK>
 __global__ __launch_bounds__(DISP_THREADS) void k_dispatch_multi(const DispTopk tk,
@@ -3050,7 +3050,7 @@ extern "C" int moe_topk_dispatch_ws(const float *logits, int T, int E, int ldl, 
   const size_t lds = (size_t)(16 * E + tpb * k) * sizeof(int);
   moe_ktimer_begin(MOE_K_DISPATCH, (hipStream_t)stream);
   hipLaunchKernelGGL(k_dispatch_multi<true>, dim3(nb), dim3(DISP_THREADS), lds, (hipStream_t)stream,
-                     DispTopk{logits, w, idx, T, ldl, mode}, (const int *)nullptr, T * k, tpb * k, k, E, nbits, counts, offsets,
+                     DispTopk{logits, w, idx, ldl, mode}, (const int *)nullptr, T * k, tpb * k, k, E, nbits, counts, offsets,
                      sorted_pair, pos_of_pair, sorted_tok, units, n_active, (long long *)active_ids, max_units,
                      (int *)((char *)ws + 64), (unsigned *)ws, err);
   moe_ktimer_end(MOE_K_DISPATCH, (hipStream_t)stream);

@@ -8,7 +8,9 @@
 // columns: for w13 the two column halves are the SAME columns of gate and up (SwiGLU fused in the epilogue),
 // for w2 they are adjacent column blocks.  K advances 64 at a time; the activation slab goes global -> LDS
 // directly (a ring of four slabs), the weight fragments go global -> registers in operand order and feed
-// v_mfma_f32_32x32x16_bf16.  int4 / q4_K experts: 8 waves, fragments dequantised in registers (below).
+// v_mfma_f32_32x32x16_bf16.  int4 / q4_K experts: four waves on a tile of up to 128 rows, two workgroups per compute unit,
+// activations, nibbles and scales through one LDS ring, fragments dequantised in registers between the products (below).
+// bf16 batches of up to 64 tokens go to moe_decode_bf16.hip.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include <string.h>
@@ -36,9 +38,9 @@ struct PfTile {
 static __device__ __forceinline__ int pf_rows(const PfTile &t) { return t.rows_group & 0xffff; }
 // one GEMM problem class of a launch (routed experts / shared expert)
 struct PfClass {
-  const uint16_t *act;  // bf16 activations
+  const uint16_t *act;  // activations: bf16, or fp16 for the nibble formats (the copy of x, then the h rows)
   const int *gather;    // row -> activation row, or NULL
-  void *out;            // bf16 h (SWIGLU) or fp32 partial rows
+  void *out;            // h rows in the format of the activations (SWIGLU) or fp32 partial rows
   const PfTile *tiles;
   const int *n_tiles_real;  // device: tiles actually in use (<= n_mtiles, the launch's upper bound)
   long long w_off;      // byte offset of the matrix inside the expert image
@@ -356,13 +358,9 @@ __global__ __launch_bounds__(256, 1) void k_prefill_gemm(const PfArgs a) {
     for (int e = 0; e < 16; ++e) {
       const int row = 32 * i + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3);
       if (row < rows) {
-        const size_t orow = (size_t)(tile.row0 + row) * c.out_stride;
-        if (SWIGLU) {
-          ((__bf16 *)c.out)[orow + n0 + col] = (__bf16)pf_silu_mul(acc[i][0][e], acc[i][1][e]);
-        } else {
-          ((float *)c.out)[orow + n0 + col] = acc[i][0][e];
-          ((float *)c.out)[orow + n0 + PF_BNH + col] = acc[i][1][e];
-        }
+        float *o = (float *)c.out + (size_t)(tile.row0 + row) * c.out_stride + n0 + col;
+        o[0] = acc[i][0][e];
+        o[PF_BNH] = acc[i][1][e];
       }
     }
 }
@@ -674,13 +672,6 @@ __global__ __launch_bounds__(256, 2) void k_prefill_nib(const PfArgs a) {
   }
 }
 
-
-static int pf_gcd(int a, int b) { return b ? pf_gcd(b, a % b) : a; }
-static int pf_slab_step(int nk) {
-  int s = 3;
-  while (pf_gcd(s, nk) != 1) s += 2;
-  return s;
-}
 
 // Workgroups of a class of `blocks` blocks: whole rounds of 8 runs, or, where less than a round is spread evenly (EVEN), an
 // even share per XCD (56 idle workgroups between the shared expert's 8 w2 blocks and the routed ones of a 65-token batch of
@@ -1011,7 +1002,7 @@ extern "C" int moe_experts_prefill_publish(const void *x_bf16, int T, int H, int
       c.ksplit = (w2 && shared && int4) ? shared_pieces : 1;
       c.split_stride = (long long)T * H;
       c.n_blocks = pf_padded(!int4, c.n_mtiles * c.n_ntiles * c.ksplit);
-      c.slab_step = pf_slab_step(c.K / PF_BK);
+      c.slab_step = moe_bf16_slab_step(c.K / PF_BK);
       a.n_blocks_total += c.n_blocks;
     }
     if (int rc = q4k ? pn_launch<true>(!w2, a, s) : (int4 ? pn_launch<false>(!w2, a, s) : pf_launch(!w2, a, s))) return rc;

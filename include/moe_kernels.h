@@ -132,8 +132,9 @@ int moe_dispatch_ws(const int *idx, int T, int k, int E, int *counts, int *offse
                     int *pos_of_pair, int *sorted_tok, moe_unit *units, int *n_active,
                     int64_t *active_ids, int max_units, void *ws, int64_t ws_bytes, int *err, void *stream);
 
-/* k1b + k2 of a prefill batch in one launch: moe_topk followed by moe_dispatch_ws, bit for bit (and exactly those two
- * where moe_topk_dispatch_workspace_bytes is 0 or ws is smaller).  ws, err: as for moe_dispatch_ws. */
+/* k1b + k2 of a batch: moe_topk followed by moe_dispatch_ws, bit for bit; in one launch for small batches, where that is
+ * faster (E <= 64, T <= 512, T*k <= 2048, and a ws of moe_topk_dispatch_workspace_bytes), else exactly those two.
+ * ws, err: as for moe_dispatch_ws. */
 int64_t moe_topk_dispatch_workspace_bytes(int T, int k, int E);
 int moe_topk_dispatch_ws(const float *logits, int T, int E, int ldl, int k, int mode, int *idx, float *w, int *counts,
                          int *offsets, int *sorted_pair, int *pos_of_pair, int *sorted_tok, moe_unit *units,

@@ -12,6 +12,10 @@
 // v_mfma_f32_16x16x32_bf16, DEPTH slabs ahead; there is no barrier and no LDS in the loop.  The activation rows come
 // out of the caches (T rows, read by every workgroup of a unit): HV = 2 reads them half as often as HV = 1 and is
 // taken where its workgroups still fill the chip.
+//
+// Measured (us, both launches, tile kernels / these): Qwen1.5 shape 1 token 73.2 / 31.5, 4 tokens 82.9 / 62.5, 16 tokens
+// 155 / 131, 64 tokens 199 / 181; Mixtral shape 1 token 231 / 119, 8 tokens 420 / 355, 64 tokens 480 / 443 (up to 6.4 TB/s);
+// 8 experts of 2048 x 4096 that all see every token: 16 tokens 103 / 79, 48 tokens 109 / 99, 64 tokens 111 / 111: there the line.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include <string.h>

@@ -242,8 +242,9 @@ __global__ __launch_bounds__(DISP_THREADS) void k_dispatch(
 // expert start), and scatters.  The barrier words are zero at launch and are left zero.  A workgroup that waits
 // longer than a second raises the error word and goes on with what it has (positions stay inside the arrays).
 // TOPK: the pairs come from the logits: a workgroup first selects the experts of its own tokens (chunk / k of them, a wave per
-// token, the arithmetic of k_topk), and writes idx and wout.  One workgroup per 16 tokens begun, up to 64, with even shares of the tokens: both steps are chains
-// of round trips, and the top-k as a launch of its own cost 4.7 us in front of this one's 6.4.
+// token, the arithmetic of k_topk), and writes idx and wout.  One workgroup per 16 tokens begun, up to 64, with even shares of
+// the tokens: both steps are chains of round trips, and for small batches the top-k as a launch of its own costs more than
+// the chains grow (topk_dispatch_pays).
 // ---------------------------------------------------------------------------
 #define DISPM_MAXB 64
 struct DispTopk {
@@ -3023,6 +3024,12 @@ static int topk_dispatch_tokens(int T, int k, int E) {
   const int tpb = (T + nb - 1) / nb;
   return tpb * k <= DISP_THREADS ? tpb : 0;
 }
+// Where the one launch is faster than the two.  It saves a launch (about 5 us with its trip to memory) and pays with the
+// tokens' selection chains on at most 64 workgroups, which grow with tokens, choices and columns of logits per lane, where
+// k_topk has a wave per token on the whole chip.  us, two launches / one: 64 experts top-6, 33 tokens 9.6 / 8.6, 256 tokens
+// 11.2 / 10.0, 379 tokens 10.6 / 10.6, 1024 tokens 11.4 / 13.4, 4096 tokens 12.8 / 21.0; 8 experts top-2, 64 tokens 9.2 / 7.1, 512
+// tokens 9.2 / 9.1, 4096 tokens 11.0 / 16.4; 256 experts top-8, 33 tokens 10.1 / 11.0, 4096 tokens 19.2 / 37.4.
+static bool topk_dispatch_pays(int T, int k, int E) { return E <= 64 && T <= 512 && T * k <= 2048; }
 
 extern "C" int64_t moe_topk_dispatch_workspace_bytes(int T, int k, int E) {
   const int tpb = topk_dispatch_tokens(T, k, E);
@@ -3034,7 +3041,7 @@ extern "C" int moe_topk_dispatch_ws(const float *logits, int T, int E, int ldl, 
                                     int *n_active, int64_t *active_ids, int max_units, void *ws, int64_t ws_bytes,
                                     int *err, void *stream) {
   const int64_t need = moe_topk_dispatch_workspace_bytes(T, k, E);
-  if (need == 0 || !ws || ws_bytes < need || !err) {
+  if (need == 0 || !ws || ws_bytes < need || !err || !topk_dispatch_pays(T, k, E)) {
     if (int rc = moe_topk(logits, T, E, ldl, k, mode, idx, w, stream)) return rc;
     return moe_dispatch_ws(idx, T, k, E, counts, offsets, sorted_pair, pos_of_pair, sorted_tok, units, n_active, active_ids,
                            max_units, ws, ws_bytes, err, stream);

@@ -387,9 +387,13 @@ __global__ __launch_bounds__(256, 1) void k_prefill_gemm(const PfArgs a) {
 // Measured (one box, w13 / w2 launch; in brackets the kernel before: eight waves, the weights of a tile dequantised
 // by two of them each, activations converted and nibbles loaded through registers one group ahead): DeepSeek shape
 // 2048 tokens 215 / 121 us (305 / 167), 379 tokens 76 / 49 (115 / 65), Mixtral shape 4096 tokens 1733 / 991 (2132 /
-// 1038), Qwen2-57B shape q4_K 512 tokens 408 / 219 (577 / 303).  What bounds it: on the large shapes the power limit
-// (matrix cores busy 78 % of the cycles of the Mixtral w13 launch, at 1.4 GHz); tiles of 256 rows with one workgroup
-// per compute unit halve the dequantisation per product and lose 8 to 15 % on all but that shape (+1 %).
+// 1038), Qwen2-57B shape q4_K 512 tokens 408 / 219 (577 / 303); with the block order of pf_block_of 194 / 109, 62 / 43,
+// 1622 / 893 and 320 / 187.
+// What bounds it: on the Mixtral shape the power limit (matrix cores busy 78 % and 69 % of the cycles of the two launches,
+// which run at 1.46 and 1.51 GHz); on the others partly (DeepSeek shape, 2048 tokens: 59 % and 50 % at 1.70 and 1.81 GHz;
+// Qwen2-57B shape, 512 tokens: 61 % and 49 % at 1.65 and 1.78 GHz), with 0.8 to 0.9 vector cycles of dequantisation per
+// matrix cycle.  Tiles of 256 rows with one workgroup per compute unit halve the dequantisation per product and lose 8 to
+// 15 % on all but the Mixtral shape (+1 %).
 typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
 
 #define PN_BM 128                         // most rows of one tile: 4 blocks of 32 (128 accumulator registers)

@@ -276,9 +276,7 @@ __global__ __launch_bounds__(DISP_THREADS) void k_dispatch_multi(const DispTopk 
       const float *row = tk.logits + (size_t)(t0 + t) * tk.ldl;
       int *ir = tk.idx + (size_t)(t0 + t) * k;
       float *wr = tk.w + (size_t)(t0 + t) * k;
-      if (E <= 64) topk_token<1, false>(row, E, k, tk.mode, lane, ir, wr, s_idx + t * k, nullptr);
-      else if (E <= 128) topk_token<2, false>(row, E, k, tk.mode, lane, ir, wr, s_idx + t * k, nullptr);
-      else topk_token<4, false>(row, E, k, tk.mode, lane, ir, wr, s_idx + t * k, nullptr);
+      topk_token<1, false>(row, E, k, tk.mode, lane, ir, wr, s_idx + t * k, nullptr);   // (E <= 64)
     }
     __syncthreads();
     if (tid < np) e = s_idx[tid];

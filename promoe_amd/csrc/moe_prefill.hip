@@ -66,11 +66,10 @@ static __device__ __forceinline__ float pf_silu_mul(float g, float u) {
 }
 
 // Which block of which class a physical workgroup takes; false: none.  The blocks of class 0 come first, each class
-// padded (pf_padded).  Workgroup i runs on XCD i % 8; runs of PF_DEAL consecutive blocks are dealt to
-// the XCDs in turn, so that the XCDs get the same number of
-// blocks of every size whatever the row counts are: the list holds the large tiles first.  (One contiguous range of the
-// list per XCD, the order before this one, left the XCDs with the popular experts' tiles busy alone: 1.4 of 2 waves per
-// SIMD on average over the w13 launch of the DeepSeek shape at 2048 tokens, 1.0 at 379.)
+// padded (pf_padded).  Workgroup i runs on XCD i % 8; runs of PF_DEAL consecutive blocks are dealt to the XCDs in turn, so
+// that the XCDs get the same number of blocks of every size whatever the row counts are: the list holds the large tiles
+// first.  (One contiguous range of the list per XCD, the order before this one, left the XCDs with the popular experts'
+// tiles busy alone: 1.4 of 2 waves per SIMD on average over the w13 launch of the DeepSeek shape at 2048 tokens, 1.0 at 379.)
 // Inside the list: a group of up to PF_GROUP tiles of one expert goes through all its column tiles, tile fastest, so
 // that a run shares either a column tile's weights (many tiles) or the activation rows (one tile) in its XCD's L2.
 // EVEN (bf16 kernel: one workgroup per compute unit, so that a run too many is a quarter of a round of its XCD): the blocks

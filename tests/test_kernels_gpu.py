@@ -49,7 +49,7 @@ def test_gate_logits_pair_bit_exact(cuda, T, H, E, E2):
 @pytest.mark.parametrize("T,H,E", [(313, 2048, 64), (1177, 264, 17), (328, 520, 61), (20000, 8, 1), (125, 1544, 160), (80, 4360, 250),
                                    (5, 2048, 64)])
 def test_gate_logits_tiles(cuda, T, H, E):
-    """Batches of 20000 logits and more on the matrix cores, the last one below: bits of the ordered sums, ragged tiles
+    """Batches on the matrix cores (from 20000 logits on), the last one below: bits of the ordered sums, ragged tiles
     of tokens, rows and columns, a bias on some of the rows only, and columns behind the rows left alone."""
     from promoe_amd import _lib as L
     print(f"case gate_logits_tiles T={T} H={H} E={E}", flush=True)
@@ -172,7 +172,7 @@ def test_dispatch_workspace_reused(cuda):
 @pytest.mark.parametrize("E,k,mode", [(8, 2, 2), (60, 4, 0), (64, 6, 1), (128, 8, 0), (256, 32, 1)])
 def test_topk_dispatch_in_one_launch_equals_the_two(cuda, E, k, mode):
     """Sizes at which the tokens per workgroup and the number of workgroups change, ties, and NaN rows; calls that share one
-    workspace."""
+    workspace.  (One launch up to 64 experts, 512 tokens and 2048 pairs; past these sizes the entry makes the two itself.)"""
     from promoe_amd import ops
     from promoe_amd._lib import lib, ptr, cur_stream, check
     ws_bytes = 64 + 64 * E * 4

@@ -152,7 +152,7 @@ def test_prefill_wide_shared_expert_in_pieces(cuda):
 @pytest.mark.parametrize("T", [31, 32, 33, 127, 128, 129, 257])
 def test_prefill_nibble_tile_edges(cuda, T, cls, I):
     """Every token to one expert: row blocks of 32 and tiles of 128 rows just short, full and just over; reductions of
-    two slabs (shorter than the ring they go through) and of eight."""
+    two slabs (q4_K: four; shorter than the ring they go through) and of eight."""
     print(f"case prefill_nibble_edges T={T} {cls.__name__}", flush=True)
     check_prefill(cls(H=512, I=I, E=1, I_sh=I, seed=9), T, 1, 0, cuda)
 

@@ -39,3 +39,16 @@ def test_headers_compile_as_c():
         r = subprocess.run(["gcc", "-std=c99", "-Wall", "-Werror", "-I", os.path.join(ROOT, "include"), "-c", c,
                             "-o", os.path.join(d, "t.o")], capture_output=True, text=True)
         assert r.returncode == 0, r.stderr
+
+
+def test_expert_rows_past_the_kernels_addressing_are_refused_on_the_host():
+    """Rows of 2^24 columns (bf16: 2^23) of an expert: an error before anything is launched (no GPU needed)."""
+    import torch  # noqa: F401
+    from promoe_amd import _lib as L
+    p = 4096                                     # never read
+    for fmt, most in ((L.FMT_INT4_G128, 1 << 24), (L.FMT_Q4K, 1 << 24), (L.FMT_BF16, 1 << 23)):
+        for T in (1, 65):
+            if T * most * 2 >= 1 << 31:          # refused for the activations' size already
+                continue
+            rc = L.lib.moe_experts_prefill(p, T, 256, most, 0, 1, fmt, p, 1, p, p, None, p, None, p, None, p, p, 3, None)
+            assert rc != 0 and b"columns and more" in L.lib.moe_last_error(), (fmt, T)

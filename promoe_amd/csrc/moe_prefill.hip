@@ -8,7 +8,7 @@
 // columns: for w13 the two column halves are the SAME columns of gate and up (SwiGLU fused in the epilogue),
 // for w2 they are adjacent column blocks.  K advances 64 at a time; the activation slab goes global -> LDS
 // directly (a ring of four slabs), the weight fragments go global -> registers in operand order and feed
-// v_mfma_f32_32x32x16_bf16.  int4 / q4_K experts: four waves on a tile of up to 128 rows, two workgroups per compute unit,
+// v_mfma_f32_32x32x16_bf16.  q4_K experts: four waves on a tile of up to 128 rows, two workgroups per compute unit,
 // activations, nibbles and scales through one LDS ring, fragments dequantised in registers between the products (below).
 // bf16 batches of up to 64 tokens go to moe_decode_bf16.hip.
 #include <hip/hip_runtime.h>
@@ -53,6 +53,7 @@ struct PfClass {
   int ksplit;           // int4 / q4_K w2 pass of the shared expert: workgroups per tile, each over 1/ksplit of the
                         // reduction, partial rows to out + split * split_stride (0 or 1: the whole reduction)
   long long split_stride;  // elements between the pieces of out
+  int act_rows, out_rows;  // int4: rows of the activation matrix and of h (w13), whose groups lie one after the other
 };
 struct PfArgs {
   PfClass c[2];
@@ -364,7 +365,7 @@ __global__ __launch_bounds__(256, 1) void k_prefill_gemm(const PfArgs a) {
     }
 }
 
-// ---- int4-g128 and q4_K experts ---------------------------------------------------------
+// ---- q4_K experts -----------------------------------------------------------------------------
 // A workgroup of four waves (one per SIMD, two workgroups per compute unit) computes a tile of up to 128 rows x
 // (128 + 128) columns; wave w owns 32 columns of both halves (for w13 the same columns of gate and up, for w2
 // adjacent column blocks) and ALL row blocks of the tile, so every weight is dequantised once per tile.  K advances
@@ -397,8 +398,8 @@ typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
 
 #define PN_BM 128                         // most rows of one tile: 4 blocks of 32 (128 accumulator registers)
 #define PN_LDS 81920                      // half of a compute unit's LDS
-template <bool Q4K> struct PnSlab {       // one ring slot: activations, then per wave 2 KiB of nibbles and the scales
-  static constexpr int SB = Q4K ? 512 : 256;                 // scale bytes of one wave
+struct PnSlab {                           // one ring slot: activations, then per wave 2 KiB of nibbles and the scales
+  static constexpr int SB = 512;                             // scale bytes of one wave
   static constexpr int bytes(int nb) { return nb * 4096 + 4 * (2048 + SB); }
   static constexpr int ring(int nb) { return PN_LDS / bytes(nb) < 8 ? PN_LDS / bytes(nb) : 8; }
 };
@@ -428,22 +429,20 @@ static __device__ __forceinline__ T pn_lds(unsigned addr) {
 
 // what a wave of a tile reads; offsets in bytes, voff per lane
 struct PnSrc {
-  // activation matrix; nibbles, scales and (q4_K) super-block scales of the tile's 16 row blocks (64-bit bases: an expert
+  // activation matrix; nibbles, scales and super-block scales of the tile's 16 row blocks (64-bit bases: an expert
   // image may have 2 GiB and more)
   pf_i32x4_t ra, rw, rs, rz;
   int a_voff[4];            // row block n: the lane's row and chunk
   int w_voff[2];            // fragment f
-  int s_voff, z_voff;       // scale request; q4_K: (d, dmin) request; int4: s_voff covers scales and zeros
-  int s_step;               // int4: what s_voff advances by per quantisation group (scales and zeros differ)
+  int s_voff, z_voff;       // scale request; (d, dmin) request
 };
 
 // acc[i][f]: row block i, fragment (column half) f; slabs kt0 .. kt0 + nk - 1 (64 k each), nk >= 2 and even
-template <int NB, bool Q4K>
+template <int NB>
 static __device__ __forceinline__ void pn_mainloop(f32x16_t (&acc)[NB][2], const unsigned lds_base, const PnSrc &m, const int kt0,
                                                    const int nk, const int tid) {
-  constexpr int SB = PnSlab<Q4K>::SB, SLOT = PnSlab<Q4K>::bytes(NB), R = PnSlab<Q4K>::ring(NB);
-  constexpr int NS_ = Q4K ? 2 : 1;         // scale requests of a slab
-  constexpr int NL = NB + 2 + NS_;         // requests of a slab
+  constexpr int SB = PnSlab::SB, SLOT = PnSlab::bytes(NB), R = PnSlab::ring(NB);
+  constexpr int NL = NB + 4;               // requests of a slab
   static_assert(R >= 3 && (R - 2) * NL < 63, "ring depth");
   constexpr int NG = 4 * NB;               // product groups of a slab (two products each)
   constexpr int FD = NG < 4 ? NG : 4;      // activation fragments read ahead
@@ -456,7 +455,6 @@ static __device__ __forceinline__ void pn_mainloop(f32x16_t (&acc)[NB][2], const
     const int kt = kt0 + (kt_ < nk ? kt_ : nk - 1);
     if (r < NB) pn_dma16(lds_base + (unsigned)(so + (32 * r + 8 * w) * 128), m.a_voff[r], m.ra, kt * 128);
     else if (r < NB + 2) pn_dma16(wbase + (unsigned)(so + 1024 * (r - NB)), m.w_voff[r - NB], m.rw, kt * 512);
-    else if (!Q4K) pn_dma4(wbase + (unsigned)(so + 2048), m.s_voff + (kt >> 1) * m.s_step, m.rs, 0);
     else if (r == NB + 2) pn_dma4(wbase + (unsigned)(so + 2048), m.s_voff, m.rs, kt * 64);
     else pn_dma4(wbase + (unsigned)(so + 2048 + 256), m.z_voff, m.rz, (kt >> 2) * 64);
   };
@@ -466,9 +464,8 @@ static __device__ __forceinline__ void pn_mainloop(f32x16_t (&acc)[NB][2], const
   for (int j = 0; j < 4; ++j) fa0[j] = lds_base + (unsigned)(n * 128 + (((4 * q + j) ^ ((n >> 1) & 7)) * 16));
   const unsigned na0 = wbase + (unsigned)lane * 16u;
   const int t0 = n >> 4, r16 = n & 15;   // fragment f reads row r16 of the wave's row block 2 f + t0
-  const unsigned sa0 = wbase + 2048u + (unsigned)(Q4K ? t0 * 64 + (16 * q + r16) * 2 : t0 * 32 + r16 * 2);
-  const unsigned za0 = wbase + 2048u + (unsigned)(Q4K ? 256 + t0 * 64 + r16 * 4 : 128 + t0 * 8 + (r16 >> 1));
-  const int zsh = 4 * (r16 & 1);
+  const unsigned sa0 = wbase + 2048u + (unsigned)(t0 * 64 + (16 * q + r16) * 2);
+  const unsigned za0 = wbase + 2048u + (unsigned)(256 + t0 * 64 + r16 * 4);
   u32x4_t nib[2], nxt[2];
   u32 s2[2], c2[2], sraw[2], zraw[2];
   u32x4_t wd[2][2];                      // [step parity][fragment]: 8 fp16 weights
@@ -476,27 +473,15 @@ static __device__ __forceinline__ void pn_mainloop(f32x16_t (&acc)[NB][2], const
 #pragma unroll
     for (int f = 0; f < 2; ++f) {
       d[f] = pn_lds<u32x4_t>(na0 + (unsigned)(so + 1024 * f));
-      if (Q4K) {
-        sraw[f] = pn_lds<uint16_t>(sa0 + (unsigned)(so + 128 * f));
-        zraw[f] = pn_lds<u32>(za0 + (unsigned)(so + 128 * f));
-      } else {
-        sraw[f] = pn_lds<uint16_t>(sa0 + (unsigned)(so + 64 * f));
-        zraw[f] = pn_lds<unsigned char>(za0 + (unsigned)(so + 16 * f));
-      }
+      sraw[f] = pn_lds<uint16_t>(sa0 + (unsigned)(so + 128 * f));
+      zraw[f] = pn_lds<u32>(za0 + (unsigned)(so + 128 * f));
     }
   };
   auto prep = [&]() {  // S = 16 s and C of deq8_f16 for the lane's row in both fragments
 #pragma unroll
     for (int f = 0; f < 2; ++f) {
-      float s16, cz;
-      if (Q4K) {
-        s16 = 16.f * __builtin_bit_cast(float, h2f_bits(zraw[f] & 0xffffu)) * (float)(sraw[f] & 0xffu);
-        cz = -s16 - __builtin_bit_cast(float, h2f_bits(zraw[f] >> 16)) * (float)((sraw[f] >> 8) & 0xffu);
-      } else {
-        const float sf = __builtin_bit_cast(float, h2f_bits(sraw[f]));
-        s16 = 16.f * sf;
-        cz = -(16.f + (float)((zraw[f] >> zsh) & 15u)) * sf;
-      }
+      const float s16 = 16.f * __builtin_bit_cast(float, h2f_bits(zraw[f] & 0xffffu)) * (float)(sraw[f] & 0xffu);
+      const float cz = -s16 - __builtin_bit_cast(float, h2f_bits(zraw[f] >> 16)) * (float)((sraw[f] >> 8) & 0xffu);
       const u32 sb = f2h_bits(s16), cb = f2h_bits(cz);
       s2[f] = sb | (sb << 16);
       c2[f] = cb | (cb << 16);
@@ -566,7 +551,7 @@ static __device__ __forceinline__ void pn_mainloop(f32x16_t (&acc)[NB][2], const
   }
 }
 
-template <int NB, bool SWIGLU, bool Q4K>
+template <int NB, bool SWIGLU>
 static __device__ __forceinline__ void pn_tile(const PfClass &c, const PfTile &tile, unsigned char *lds, int nt, int kt0, int nk,
                                                int split, int tid) {
   const int lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -577,8 +562,8 @@ static __device__ __forceinline__ void pn_tile(const PfClass &c, const PfTile &t
   m.ra = pn_rsrc(c.act);
   const size_t tile0 = (size_t)16 * nt * G;   // (row block, group) pairs in front of the tile's
   m.rw = pn_rsrc((const void *)(tile.w_base + c.w_off + tile0 * 1024));
-  m.rs = pn_rsrc((const void *)(tile.w_base + c.off_s + tile0 * (Q4K ? 128 : 32)));
-  m.rz = pn_rsrc((const void *)(tile.w_base + c.off_z + tile0 * (Q4K ? 32 : 8)));
+  m.rs = pn_rsrc((const void *)(tile.w_base + c.off_s + tile0 * 128));
+  m.rz = pn_rsrc((const void *)(tile.w_base + c.off_z + tile0 * 32));
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     m.a_voff[i] = 0;
@@ -598,19 +583,8 @@ static __device__ __forceinline__ void pn_tile(const PfClass &c, const PfTile &t
 #pragma unroll
   for (int f = 0; f < 2; ++f)
     m.w_voff[f] = rb(2 * f + (n >> 4)) * G * 1024 + (16 * q + (n & 15)) * 16;
-  if (Q4K) {
-    m.s_voff = rb(lane >> 4) * G * 128 + (lane & 15) * 4;
-    m.z_voff = rb(lane >> 4) * (G >> 1) * 64 + (lane & 15) * 4;
-    m.s_step = 0;
-  } else {
-    // lanes 0..31: 8 dwords of scales of each row block; lanes 32..39: 2 dwords of zeros of each; the rest idle copies.
-    // The zeros of the tile lie behind its scales (in the image's next section, less than 2 GiB away: the launcher)
-    const int l = lane < 40 ? lane : 39;
-    const int z0 = (int)(c.off_z - c.off_s - (long long)tile0 * 24);
-    m.s_voff = l < 32 ? rb(l >> 3) * G * 32 + (l & 7) * 4 : z0 + rb((l - 32) >> 1) * G * 8 + (l & 1) * 4;
-    m.s_step = l < 32 ? 32 : 8;
-    m.z_voff = 0;
-  }
+  m.s_voff = rb(lane >> 4) * G * 128 + (lane & 15) * 4;
+  m.z_voff = rb(lane >> 4) * (G >> 1) * 64 + (lane & 15) * 4;
   f32x16_t acc[NB][2];
 #pragma unroll
   for (int i = 0; i < NB; ++i)
@@ -618,7 +592,7 @@ static __device__ __forceinline__ void pn_tile(const PfClass &c, const PfTile &t
     for (int h = 0; h < 2; ++h)
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][h][e] = 0.f;
-  pn_mainloop<NB, Q4K>(acc, lds_base, m, kt0, nk, tid);
+  pn_mainloop<NB>(acc, lds_base, m, kt0, nk, tid);
   // epilogue.  acc element e of lane l: row 8*(e/4) + 4*(l/32) + e%4 of its block, column l%32
   const int col = 32 * w + n;
   PF_VMCNT(0);   // the transfers past the end have landed: the ring is free, and nothing is in flight at the end
@@ -654,7 +628,7 @@ static __device__ __forceinline__ void pn_tile(const PfClass &c, const PfTile &t
   }
 }
 
-template <bool SWIGLU, bool Q4K>
+template <bool SWIGLU>
 __global__ __launch_bounds__(256, 2) void k_prefill_nib(const PfArgs a) {
   extern __shared__ __align__(16) unsigned char lds_n[];
   const int tid = threadIdx.x;
@@ -668,13 +642,14 @@ __global__ __launch_bounds__(256, 2) void k_prefill_nib(const PfArgs a) {
   // this workgroup's window of the reduction (only the w2 pass is ever split)
   const int nk = SWIGLU ? c.K / PF_BK : c.K / PF_BK / ks, kt0 = SWIGLU ? 0 : split * nk;
   switch ((rows + 31) >> 5) {
-    case 1: pn_tile<1, SWIGLU, Q4K>(c, tile, lds_n, nt, kt0, nk, split, tid); break;
-    case 2: pn_tile<2, SWIGLU, Q4K>(c, tile, lds_n, nt, kt0, nk, split, tid); break;
-    case 3: pn_tile<3, SWIGLU, Q4K>(c, tile, lds_n, nt, kt0, nk, split, tid); break;
-    default: pn_tile<4, SWIGLU, Q4K>(c, tile, lds_n, nt, kt0, nk, split, tid); break;
+    case 1: pn_tile<1, SWIGLU>(c, tile, lds_n, nt, kt0, nk, split, tid); break;
+    case 2: pn_tile<2, SWIGLU>(c, tile, lds_n, nt, kt0, nk, split, tid); break;
+    case 3: pn_tile<3, SWIGLU>(c, tile, lds_n, nt, kt0, nk, split, tid); break;
+    default: pn_tile<4, SWIGLU>(c, tile, lds_n, nt, kt0, nk, split, tid); break;
   }
 }
 
+#include "moe_prefill_int4.h"
 
 // Workgroups of a class of `blocks` blocks: whole rounds of 8 runs, or, where less than a round is spread evenly (EVEN), an
 // even share per XCD (56 idle workgroups between the shared expert's 8 w2 blocks and the routed ones of a 65-token batch of
@@ -684,23 +659,25 @@ static int pf_padded(bool even, int blocks) {
   return (blocks + q - 1) / q * q;
 }
 
-template <bool Q4K>
-static int pn_launch(bool swiglu, const PfArgs &a, hipStream_t s) {
+static int pn_launch(bool swiglu, bool q4k, const PfArgs &a, hipStream_t s) {
   if (a.n_blocks_total <= 0) return MOE_OK;
   const int grid = a.c[0].n_blocks + a.c[1].n_blocks;
   static bool attr_set = false;
   if (!attr_set) {
-    for (const void *f : {(const void *)k_prefill_nib<true, Q4K>, (const void *)k_prefill_nib<false, Q4K>})
+    for (const void *f : {(const void *)k_prefill_nib<true>, (const void *)k_prefill_nib<false>,
+                          (const void *)k_prefill_int4<true>, (const void *)k_prefill_int4<false>})
       if (int rc = moe_check_hip(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, PN_LDS),
-                                 "hipFuncSetAttribute(k_prefill_nib)"))
+                                 "hipFuncSetAttribute(k_prefill_nib, k_prefill_int4)"))
         return rc;
     attr_set = true;
   }
   moe_ktimer_begin(swiglu ? MOE_K_PREFILL_W13 : MOE_K_PREFILL_W2, s);
-  if (swiglu) hipLaunchKernelGGL((k_prefill_nib<true, Q4K>), dim3(grid), dim3(256), PN_LDS, s, a);
-  else hipLaunchKernelGGL((k_prefill_nib<false, Q4K>), dim3(grid), dim3(256), PN_LDS, s, a);
+  if (q4k && swiglu) hipLaunchKernelGGL(k_prefill_nib<true>, dim3(grid), dim3(256), PN_LDS, s, a);
+  else if (q4k) hipLaunchKernelGGL(k_prefill_nib<false>, dim3(grid), dim3(256), PN_LDS, s, a);
+  else if (swiglu) hipLaunchKernelGGL(k_prefill_int4<true>, dim3(grid), dim3(256), PN_LDS, s, a);
+  else hipLaunchKernelGGL(k_prefill_int4<false>, dim3(grid), dim3(256), PN_LDS, s, a);
   moe_ktimer_end(swiglu ? MOE_K_PREFILL_W13 : MOE_K_PREFILL_W2, s);
-  return moe_check_launch("k_prefill_nib");
+  return moe_check_launch(q4k ? "k_prefill_nib" : "k_prefill_int4");
 }
 
 static int pf_launch(bool swiglu, const PfArgs &a, hipStream_t s) {
@@ -727,7 +704,7 @@ static int pf_launch(bool swiglu, const PfArgs &a, hipStream_t s) {
 // dispatch result, so the host never needs the counts: the launch covers the upper bound on the number of blocks, and
 // blocks past the real count find nothing to do.  The routed list is in order of tile height, the tallest first (four
 // classes; expert order inside a class), so that no long workgroup starts when the launch is nearly over.
-// Nibble formats: the same launch converts x to fp16 for the w13 pass (8 MB read and written for 2048 x 2048, hidden
+// Nibble formats: the same launch converts x for the w13 pass (q4_K to fp16, int4 to records) (8 MB read and written for 2048 x 2048, hidden
 // behind the 4 us that the list takes).  One more workgroup takes the unit list to the host: two copies and an event
 // behind the routing stood in the stream for 9 us a layer.
 static __device__ __forceinline__ PfTile pf_make_tile(unsigned long long w_base, int row0, int rows, int i, int n) {
@@ -743,14 +720,15 @@ __global__ __launch_bounds__(1024) void k_prefill_tiles(const moe_unit *__restri
                                                         PfTile *__restrict__ sh_tiles2, int n_sh_tiles2,
                                                         unsigned long long shared_base, int T, int cap, int cap_s, int cap_s2,
                                                         int *__restrict__ n_real, int *__restrict__ err,
-                                                        const u32x4_t *__restrict__ x, u32x4_t *__restrict__ x16, int n16,
+                                                        const u32x4_t *__restrict__ x, u32x4_t *__restrict__ x16, int n16, int K6,
                                                         const moe_publish pub) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int conv0 = pub.units_host ? 2 : 1;
-  if (blockIdx.x > 0) {  // workgroups behind the first: the unit list to the host, the fp16 copy of the activations
+  if (blockIdx.x > 0) {  // workgroups behind the first: the unit list to the host, the copy of the activations
     if ((int)blockIdx.x < conv0) { publish_units(pub, units, tid, 1024); return; }
-    const int i = ((int)blockIdx.x - conv0) * 1024 + tid;   // (8 values per thread)
-    if (i < n16) {
+    const int i = ((int)blockIdx.x - conv0) * 1024 + tid;
+    if (K6) p6_convert_x(x, (unsigned char *)x16, K6, T, i);   // 32 values per thread
+    else if (i < n16) {                                          // 8
       const u32x4_t v = x[i];
       x16[i] = u32x4_t{bf16x2_to_f16x2(v.x), bf16x2_to_f16x2(v.y), bf16x2_to_f16x2(v.z), bf16x2_to_f16x2(v.w)};
     }
@@ -836,10 +814,10 @@ extern "C" int moe_prefill_tile_rows(void) { return PF_BM; }
 
 extern "C" int64_t moe_prefill_workspace_bytes(int T, int k, int max_units) {
   const int64_t P = (int64_t)T * k;
-  return (P / 128 + max_units + 2 * ((T + 127) / 128) + 3) * (int64_t)sizeof(PfTile);  // covers every tile height in use (>= 128)
+  return (P / 64 + max_units + 2 * ((T + 63) / 64) + 3) * (int64_t)sizeof(PfTile);  // covers every tile height in use (>= 64)
 }
 
-// where the fp16 copy of the activations stands in a workspace with room for it (phase bit 2)
+// where the copy of the activations stands in a workspace with room for it (phase bit 2)
 static int64_t pf_x16_offset(int T, int k, int max_units) {
   return (moe_prefill_workspace_bytes(T, k, max_units) + 255) & ~(int64_t)255;
 }
@@ -916,7 +894,7 @@ extern "C" int moe_experts_prefill_publish(const void *x_bf16, int T, int H, int
     return MOE_EINVAL;
   }
   const bool q4k = fmt == MOE_FMT_Q4K;
-  const bool int4 = fmt == MOE_FMT_INT4_G128 || q4k;  // nibble tiles + fp16 operands
+  const bool int4 = fmt == MOE_FMT_INT4_G128 || q4k;  // nibble tiles
   if (q4k && (H % 256 || I % 256 || (shared_ptr && I_sh % 256))) {
     moe_set_error("moe_experts_prefill: q4_K experts need H, I multiples of 256 (H=%d I=%d I_sh=%d)", H, I, I_sh);
     return MOE_EINVAL;
@@ -943,8 +921,17 @@ extern "C" int moe_experts_prefill_publish(const void *x_bf16, int T, int H, int
     return moe_decode_bf16(x_bf16, T, H, I, I_sh, units, max_units, sorted_tok, expert_ptr, shared_ptr, h_r, h_s, part_r, part_s,
                            shared_pieces, err, phases, pub, s);
   const long long P = (long long)T * k;
-  const int cap = int4 ? PN_BM : PF_BM, cap_s = int4 ? PN_BM : PF_BM_SHARED, cap_s2 = PF_BM_SHARED_W2;
-  // fp16 copy of x for the nibble formats: behind the tile list where the caller left room, else stream-ordered memory
+  // int4: tiles of up to 64 instead of 128 rows where the experts' groups are short (most tiles then are no taller anyway, and the
+  // popular experts' are spread over more workgroups) or where 128 rows leave compute units idle.  Tile list and both launches,
+  // us, 128 / 64 rows: DeepSeek shape 300 tokens (28 rows per expert) 91 / 84, 379 (36) 104 / 96, 500 (47) 117 / 113, 700 (66)
+  // 129 / 128, 1000 (94) 166 / 182; Mixtral shape 65 (16) 183 / 183, 200 (50) 251 / 253, 300 (75) 305 / 336; 16 experts of
+  // 1024 x 512 top-2, 64 workgroups: 256 tokens 37 / 28.
+  const int n_units = max_units < P ? max_units : (int)P;
+  const bool short_tiles = fmt == MOE_FMT_INT4_G128 && P <= 1 << 20 &&   // (k_prefill_tiles counts tiles in 16 bits)
+                           (P <= 52ll * n_units || (P / PN_BM + n_units) * (I / PF_BNH) + (shared_ptr ? (T / PN_BM + 1ll) * (I_sh / PF_BNH) : 0) <= 512);
+  const int cap = short_tiles ? 64 : int4 ? PN_BM : PF_BM, cap_s = short_tiles ? 64 : int4 ? PN_BM : PF_BM_SHARED;
+  const int cap_s2 = short_tiles ? 64 : PF_BM_SHARED_W2;
+  // copy of x for the nibble formats (q4_K fp16, int4 records): behind the tile list where the caller left room, else stream-ordered memory
   void *x16 = nullptr, *x16_own = nullptr;
   const bool convert = int4 && (phases & 1);
   if (convert) {
@@ -956,7 +943,7 @@ extern "C" int moe_experts_prefill_publish(const void *x_bf16, int T, int H, int
     void *p; hipStream_t s;
     ~FreeX16() { if (p) (void)hipFreeAsync(p, s); }
   } free_x16{x16_own, s};
-  const int n16 = convert ? (int)((long long)T * H / 8) : 0;
+  const int n16 = convert ? (int)((long long)T * H / (q4k ? 8 : 32)) : 0;   // threads of the conversion
   const int n_r = (int)(P / cap) + max_units;
   const int n_s = shared_ptr ? (T + cap_s - 1) / cap_s : 0;
   const int n_s2 = shared_ptr ? (T + cap_s2 - 1) / cap_s2 : 0;
@@ -965,7 +952,7 @@ extern "C" int moe_experts_prefill_publish(const void *x_bf16, int T, int H, int
   hipLaunchKernelGGL(k_prefill_tiles, dim3(1 + (pub ? 1 : 0) + (n16 + 1023) / 1024), dim3(1024), 0, s, units, max_units,
                      (const unsigned long long *)expert_ptr, tiles, n_r, sh_tiles, n_s, sh_tiles2, n_s2,
                      (unsigned long long)(uintptr_t)shared_ptr, T, cap, cap_s, cap_s2, n_real, err, (const u32x4_t *)x_bf16,
-                     (u32x4_t *)x16, n16, pub ? *pub : moe_publish{});
+                     (u32x4_t *)x16, n16, q4k ? 0 : H, pub ? *pub : moe_publish{});
   if (int rc = moe_check_launch("k_prefill_tiles")) return rc;
   for (int w2 = 0; w2 < 2; ++w2) {
     if (!(phases & (w2 ? 2 : 1))) continue;
@@ -1003,12 +990,14 @@ extern "C" int moe_experts_prefill_publish(const void *x_bf16, int T, int H, int
         }
       }
       c.ksplit = (w2 && shared && int4) ? shared_pieces : 1;
+      c.act_rows = w2 && !shared ? (int)P : T;
+      c.out_rows = shared ? T : (int)P;
       c.split_stride = (long long)T * H;
       c.n_blocks = pf_padded(!int4, c.n_mtiles * c.n_ntiles * c.ksplit);
       c.slab_step = moe_bf16_slab_step(c.K / PF_BK);
       a.n_blocks_total += c.n_blocks;
     }
-    if (int rc = q4k ? pn_launch<true>(!w2, a, s) : (int4 ? pn_launch<false>(!w2, a, s) : pf_launch(!w2, a, s))) return rc;
+    if (int rc = int4 ? pn_launch(!w2, q4k, a, s) : pf_launch(!w2, a, s)) return rc;
   }
   return MOE_OK;
 }

@@ -2834,6 +2834,10 @@ __global__ __launch_bounds__(256, 2) void k_gemv_int4_mfma_kc(const GemvArgs a) 
 // ---------------------------------------------------------------------------
 // k5 combine
 // ---------------------------------------------------------------------------
+// Bound by the partial rows' bytes (6 TB/s at 2048 tokens).  KK: rows requested together, the smallest of 2, 4, 6, 8 that
+// takes a token's k: with eight for every k the requests past k repeat the last row, and Mixtral's 4096 tokens of two took 35 us, 30.5
+// with two (4 of 4: 15.0 -> 14.5 at 1999 tokens of 2048 columns, 6 of 6: 5.6 -> 5.35 at 379).
+template <int KK>
 __global__ __launch_bounds__(256) void k_combine(const float *__restrict__ part_r,
                                                   const float *__restrict__ part_s,
                                                   const float *__restrict__ topk_w,
@@ -2845,22 +2849,22 @@ __global__ __launch_bounds__(256) void k_combine(const float *__restrict__ part_
   const int n = (blockIdx.x * 256 + threadIdx.x) * 4;
   if (n >= H) return;
   float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-  // eight partial rows at a time: positions and weights first, then the rows, then the
-  // fma chain in pair order (two round trips per eight rows instead of two per row)
-  for (int j0 = 0; j0 < k; j0 += 8) {
-    float wj[8];
-    int pos[8];
-    float4 v[8];
+  // KK partial rows at a time: positions and weights first, then the rows, then the
+  // fma chain in pair order (two round trips per KK rows instead of two per row)
+  for (int j0 = 0; j0 < k; j0 += KK) {
+    float wj[KK];
+    int pos[KK];
+    float4 v[KK];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
+    for (int j = 0; j < KK; ++j) {
       const int jj = j0 + j < k ? j0 + j : k - 1;
       wj[j] = topk_w[(size_t)t * k + jj];
       pos[j] = pos_of_pair[(size_t)t * k + jj];
     }
 #pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] = *(const float4 *)(part_r + (size_t)pos[j] * H + n);
+    for (int j = 0; j < KK; ++j) v[j] = *(const float4 *)(part_r + (size_t)pos[j] * H + n);
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
+    for (int j = 0; j < KK; ++j)
       if (j0 + j < k) {
         acc.x = fmaf(wj[j], v[j].x, acc.x); acc.y = fmaf(wj[j], v[j].y, acc.y);
         acc.z = fmaf(wj[j], v[j].z, acc.z); acc.w = fmaf(wj[j], v[j].w, acc.w);
@@ -4071,8 +4075,13 @@ extern "C" int moe_combine_splits(const float *part_r, const float *part_s, cons
   if (T == 0) return MOE_OK;
   dim3 grid((H / 4 + 255) / 256, T);
   moe_ktimer_begin(MOE_K_COMBINE, (hipStream_t)stream);
-  hipLaunchKernelGGL(k_combine, grid, dim3(256), 0, (hipStream_t)stream, part_r, part_s, topk_w,
-                     pos_of_pair, sg_logit, sg_stride, (uint16_t *)y, H, k, n_shared_splits);
+#define COMB_LAUNCH(KK_) hipLaunchKernelGGL(k_combine<KK_>, grid, dim3(256), 0, (hipStream_t)stream, part_r, part_s, topk_w, \
+                                            pos_of_pair, sg_logit, sg_stride, (uint16_t *)y, H, k, n_shared_splits)
+  if (k <= 2) COMB_LAUNCH(2);
+  else if (k <= 4) COMB_LAUNCH(4);
+  else if (k <= 6) COMB_LAUNCH(6);
+  else COMB_LAUNCH(8);
+#undef COMB_LAUNCH
   moe_ktimer_end(MOE_K_COMBINE, (hipStream_t)stream);
   return moe_check_launch("k_combine");
 }

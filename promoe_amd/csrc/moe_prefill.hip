@@ -713,18 +713,17 @@ static __device__ __forceinline__ PfTile pf_make_tile(unsigned long long w_base,
   t.w_base = w_base; t.row0 = row0; t.rows_group = rows | (min(PF_GROUP, n - g0) << 16) | ((i - g0) << 24);
   return t;
 }
+struct PfList { PfTile *tiles, *sh_tiles; int n_tiles_max, n_sh_tiles, cap, cap_s; };   // cap: rows per tile
+struct PfLists { PfList l[2]; };
 __global__ __launch_bounds__(1024) void k_prefill_tiles(const moe_unit *__restrict__ units, int max_units,
-                                                        const unsigned long long *__restrict__ expert_ptr,
-                                                        PfTile *__restrict__ tiles, int n_tiles_max,
-                                                        PfTile *__restrict__ sh_tiles, int n_sh_tiles,
-                                                        PfTile *__restrict__ sh_tiles2, int n_sh_tiles2,
-                                                        unsigned long long shared_base, int T, int cap, int cap_s, int cap_s2,
+                                                        const unsigned long long *__restrict__ expert_ptr, const PfLists lists,
+                                                        unsigned long long shared_base, int T,
                                                         int *__restrict__ n_real, int *__restrict__ err,
                                                         const u32x4_t *__restrict__ x, u32x4_t *__restrict__ x16, int n16, int K6,
                                                         const moe_publish pub) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int conv0 = pub.units_host ? 2 : 1;
-  if (blockIdx.x > 0) {  // workgroups behind the first: the unit list to the host, the copy of the activations
+  const int conv0 = pub.units_host ? 3 : 2;
+  if (blockIdx.x > 1) {  // workgroups behind the first two: the unit list to the host, the copy of the activations
     if ((int)blockIdx.x < conv0) { publish_units(pub, units, tid, 1024); return; }
     const int i = ((int)blockIdx.x - conv0) * 1024 + tid;
     if (K6) p6_convert_x(x, (unsigned char *)x16, K6, T, i);   // 32 values per thread
@@ -736,11 +735,12 @@ __global__ __launch_bounds__(1024) void k_prefill_tiles(const moe_unit *__restri
   }
   __shared__ int total[4];
   __shared__ unsigned long long wsum[16];
+  const PfList &l = lists.l[blockIdx.x];   // the w13 pass's list, the w2 pass's
+  PfTile *const tiles = l.tiles;
+  const int cap = l.cap, n_tiles_max = l.n_tiles_max;
   if (tid < 4) total[tid] = 0;
-  for (int i = tid; i < n_sh_tiles; i += 1024)
-    sh_tiles[i] = pf_make_tile(shared_base, i * cap_s, min(cap_s, T - i * cap_s), i, n_sh_tiles);
-  for (int i = tid; i < n_sh_tiles2; i += 1024)
-    sh_tiles2[i] = pf_make_tile(shared_base, i * cap_s2, min(cap_s2, T - i * cap_s2), i, n_sh_tiles2);
+  for (int i = tid; i < l.n_sh_tiles; i += 1024)
+    l.sh_tiles[i] = pf_make_tile(shared_base, i * l.cap_s, min(l.cap_s, T - i * l.cap_s), i, l.n_sh_tiles);
   __syncthreads();
   // tiles of unit u: nt of up to `per` rows (a multiple of 32); class 0 = the tallest quarter
   int m = 0, row0 = 0, nt = 0, per = 0, cls = 0;
@@ -752,7 +752,7 @@ __global__ __launch_bounds__(1024) void k_prefill_tiles(const moe_unit *__restri
       if (un.m > 0 && un.expert >= 0) {
         wb = expert_ptr[un.expert];
         if (wb) { m = un.m; row0 = un.row0; }
-        else if (report) moe_raise_err(err);
+        else if (report && blockIdx.x == 0) moe_raise_err(err);
       }
     }
     nt = (m + cap - 1) / cap;
@@ -807,14 +807,14 @@ __global__ __launch_bounds__(1024) void k_prefill_tiles(const moe_unit *__restri
       __syncthreads();
     }
   }
-  if (tid == 0) { n_real[0] = min(n_all, n_tiles_max); n_real[1] = n_sh_tiles; n_real[2] = n_sh_tiles2; }
+  if (tid == 0) { n_real[2 * blockIdx.x] = min(n_all, n_tiles_max); n_real[2 * blockIdx.x + 1] = l.n_sh_tiles; }
 }
 
 extern "C" int moe_prefill_tile_rows(void) { return PF_BM; }
 
 extern "C" int64_t moe_prefill_workspace_bytes(int T, int k, int max_units) {
   const int64_t P = (int64_t)T * k;
-  return (P / 64 + max_units + 2 * ((T + 63) / 64) + 3) * (int64_t)sizeof(PfTile);  // covers every tile height in use (>= 64)
+  return 2 * (P / 64 + max_units + (T + 63) / 64 + 2) * (int64_t)sizeof(PfTile);  // two lists; covers every tile height in use (>= 64)
 }
 
 // where the copy of the activations stands in a workspace with room for it (phase bit 2)
@@ -921,16 +921,21 @@ extern "C" int moe_experts_prefill_publish(const void *x_bf16, int T, int H, int
     return moe_decode_bf16(x_bf16, T, H, I, I_sh, units, max_units, sorted_tok, expert_ptr, shared_ptr, h_r, h_s, part_r, part_s,
                            shared_pieces, err, phases, pub, s);
   const long long P = (long long)T * k;
-  // int4: tiles of up to 64 instead of 128 rows where the experts' groups are short (most tiles then are no taller anyway, and the
-  // popular experts' are spread over more workgroups) or where 128 rows leave compute units idle.  Tile list and both launches,
-  // us, 128 / 64 rows: DeepSeek shape 300 tokens (28 rows per expert) 91 / 84, 379 (36) 104 / 96, 500 (47) 117 / 113, 700 (66)
-  // 129 / 128, 1000 (94) 166 / 182; Mixtral shape 65 (16) 183 / 183, 200 (50) 251 / 253, 300 (75) 305 / 336; 16 experts of
-  // 1024 x 512 top-2, 64 workgroups: 256 tokens 37 / 28.
+  // int4: tiles of up to 64 instead of 128 rows in a launch whose workgroups then still are on the chip all at once (two per compute
+  // unit; half a tile per unit is what splitting its rows evenly leaves), and in the w2 pass, whose reduction is short, also up
+  // to 72 rows per unit.  us, 128 / 64 rows:
+  //   w13  DeepSeek shape 100 tokens 39.4 / 31.7 (495 workgroups of 64 rows), 150 tokens 42.8 / 46.3 (572), 379 tokens 56 / 60; Mixtral
+  //        shape 200 tokens 139 / 139, 300 tokens 175 / 212; 16 experts of 1024 x 512, 256 tokens 25.1 / 19.3, 4096 tokens 43 / 47
+  //   w2   DeepSeek shape 150 tokens 44 / 34, 379 tokens 47 / 37, 700 tokens (66 rows per expert) 52 / 46, 1000 tokens (94) 59 / 63;
+  //        Mixtral shape 300 tokens 140 / 130, 800 tokens 199 / 185 (464 workgroups), 1024 tokens 227 / 289 (576)
   const int n_units = max_units < P ? max_units : (int)P;
-  const bool short_tiles = fmt == MOE_FMT_INT4_G128 && P <= 1 << 20 &&   // (k_prefill_tiles counts tiles in 16 bits)
-                           (P <= 52ll * n_units || (P / PN_BM + n_units) * (I / PF_BNH) + (shared_ptr ? (T / PN_BM + 1ll) * (I_sh / PF_BNH) : 0) <= 512);
-  const int cap = short_tiles ? 64 : int4 ? PN_BM : PF_BM, cap_s = short_tiles ? 64 : int4 ? PN_BM : PF_BM_SHARED;
-  const int cap_s2 = short_tiles ? 64 : PF_BM_SHARED_W2;
+  auto short_tiles = [&](bool w2) {
+    if (fmt != MOE_FMT_INT4_G128 || P > 1 << 20) return false;   // (k_prefill_tiles counts tiles in 16 bits)
+    const long long cols = w2 ? H / (2 * PF_BNH) : I / PF_BNH, cols_s = shared_ptr ? (w2 ? H / (2 * PF_BNH) : I_sh / PF_BNH) : 0;
+    return (P / 64 + n_units / 2) * cols + (T + 63) / 64 * cols_s <= 512 || (w2 && P <= 72ll * n_units);
+  };
+  const int cap[2] = {short_tiles(false) ? 64 : int4 ? PN_BM : PF_BM, short_tiles(true) ? 64 : int4 ? PN_BM : PF_BM};
+  const int cap_s[2] = {short_tiles(false) ? 64 : int4 ? PN_BM : PF_BM_SHARED, short_tiles(true) ? 64 : PF_BM_SHARED_W2};
   // copy of x for the nibble formats (q4_K fp16, int4 records): behind the tile list where the caller left room, else stream-ordered memory
   void *x16 = nullptr, *x16_own = nullptr;
   const bool convert = int4 && (phases & 1);
@@ -944,15 +949,20 @@ extern "C" int moe_experts_prefill_publish(const void *x_bf16, int T, int H, int
     ~FreeX16() { if (p) (void)hipFreeAsync(p, s); }
   } free_x16{x16_own, s};
   const int n16 = convert ? (int)((long long)T * H / (q4k ? 8 : 32)) : 0;   // threads of the conversion
-  const int n_r = (int)(P / cap) + max_units;
-  const int n_s = shared_ptr ? (T + cap_s - 1) / cap_s : 0;
-  const int n_s2 = shared_ptr ? (T + cap_s2 - 1) / cap_s2 : 0;
-  int *n_real = (int *)tiles_ws;  // [0] routed tiles in use, [1] shared tiles (w13 pass), [2] shared tiles (w2 pass)
-  PfTile *tiles = (PfTile *)tiles_ws + 1, *sh_tiles = tiles + n_r, *sh_tiles2 = sh_tiles + n_s;
-  hipLaunchKernelGGL(k_prefill_tiles, dim3(1 + (pub ? 1 : 0) + (n16 + 1023) / 1024), dim3(1024), 0, s, units, max_units,
-                     (const unsigned long long *)expert_ptr, tiles, n_r, sh_tiles, n_s, sh_tiles2, n_s2,
-                     (unsigned long long)(uintptr_t)shared_ptr, T, cap, cap_s, cap_s2, n_real, err, (const u32x4_t *)x_bf16,
-                     (u32x4_t *)x16, n16, q4k ? 0 : H, pub ? *pub : moe_publish{});
+  int *n_real = (int *)tiles_ws;  // tiles in use: w13 routed, shared, w2 routed, shared
+  PfLists lists;
+  PfTile *next = (PfTile *)tiles_ws + 1;
+  for (int w2 = 0; w2 < 2; ++w2) {
+    PfList &l = lists.l[w2];
+    l.cap = cap[w2]; l.cap_s = cap_s[w2];
+    l.n_tiles_max = (int)(P / l.cap) + max_units;
+    l.n_sh_tiles = shared_ptr ? (T + l.cap_s - 1) / l.cap_s : 0;
+    l.tiles = next; l.sh_tiles = next + l.n_tiles_max;
+    next = l.sh_tiles + l.n_sh_tiles;
+  }
+  hipLaunchKernelGGL(k_prefill_tiles, dim3(2 + (pub ? 1 : 0) + (n16 + 1023) / 1024), dim3(1024), 0, s, units, max_units,
+                     (const unsigned long long *)expert_ptr, lists, (unsigned long long)(uintptr_t)shared_ptr, T, n_real, err,
+                     (const u32x4_t *)x_bf16, (u32x4_t *)x16, n16, q4k ? 0 : H, pub ? *pub : moe_publish{});
   if (int rc = moe_check_launch("k_prefill_tiles")) return rc;
   for (int w2 = 0; w2 < 2; ++w2) {
     if (!(phases & (w2 ? 2 : 1))) continue;
@@ -964,9 +974,10 @@ extern "C" int moe_experts_prefill_publish(const void *x_bf16, int T, int H, int
       if (shared && !shared_ptr) continue;
       PfClass &c = a.c[n++];
       const int Ii = shared ? I_sh : I;
-      c.tiles = shared ? (w2 ? sh_tiles2 : sh_tiles) : tiles;
-      c.n_mtiles = shared ? (w2 ? n_s2 : n_s) : n_r;
-      c.n_tiles_real = n_real + (shared ? (w2 ? 2 : 1) : 0);
+      const PfList &l = lists.l[w2];
+      c.tiles = shared ? l.sh_tiles : l.tiles;
+      c.n_mtiles = shared ? l.n_sh_tiles : l.n_tiles_max;
+      c.n_tiles_real = n_real + 2 * w2 + shared;
       c.shared = shared;
       if (!w2) {  // w13 [2I, H]: gate rows 0..I-1, up rows I..2I-1
         c.act = (const uint16_t *)(int4 ? x16 : x_bf16); c.gather = shared ? nullptr : sorted_tok; c.act_stride = H;

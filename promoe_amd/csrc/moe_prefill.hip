@@ -719,13 +719,14 @@ __global__ __launch_bounds__(1024) void k_prefill_tiles(const moe_unit *__restri
                                                         const unsigned long long *__restrict__ expert_ptr, const PfLists lists,
                                                         unsigned long long shared_base, int T,
                                                         int *__restrict__ n_real, int *__restrict__ err,
-                                                        const u32x4_t *__restrict__ x, u32x4_t *__restrict__ x16, int n16, int K6,
+                                                        const u32x4_t *__restrict__ x, u32x4_t *__restrict__ x16, int n16, int conv_threads, int K6,
                                                         const moe_publish pub) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int conv0 = pub.units_host ? 3 : 2;
   if (blockIdx.x > 1) {  // workgroups behind the first two: the unit list to the host, the copy of the activations
     if ((int)blockIdx.x < conv0) { publish_units(pub, units, tid, 1024); return; }
-    const int i = ((int)blockIdx.x - conv0) * 1024 + tid;
+    if (tid >= conv_threads) return;
+    const int i = ((int)blockIdx.x - conv0) * conv_threads + tid;
     if (K6) p6_convert_x(x, (unsigned char *)x16, K6, T, i);   // 32 values per thread
     else if (i < n16) {                                          // 8
       const u32x4_t v = x[i];
@@ -960,9 +961,10 @@ extern "C" int moe_experts_prefill_publish(const void *x_bf16, int T, int H, int
     l.tiles = next; l.sh_tiles = next + l.n_tiles_max;
     next = l.sh_tiles + l.n_sh_tiles;
   }
-  hipLaunchKernelGGL(k_prefill_tiles, dim3(2 + (pub ? 1 : 0) + (n16 + 1023) / 1024), dim3(1024), 0, s, units, max_units,
+  const int conv_threads = n16 > 256 * 512 ? 1024 : n16 > 256 * 256 ? 512 : 256;   // (up to a workgroup per compute unit)
+  hipLaunchKernelGGL(k_prefill_tiles, dim3(2 + (pub ? 1 : 0) + (n16 + conv_threads - 1) / conv_threads), dim3(1024), 0, s, units, max_units,
                      (const unsigned long long *)expert_ptr, lists, (unsigned long long)(uintptr_t)shared_ptr, T, n_real, err,
-                     (const u32x4_t *)x_bf16, (u32x4_t *)x16, n16, q4k ? 0 : H, pub ? *pub : moe_publish{});
+                     (const u32x4_t *)x_bf16, (u32x4_t *)x16, n16, conv_threads, q4k ? 0 : H, pub ? *pub : moe_publish{});
   if (int rc = moe_check_launch("k_prefill_tiles")) return rc;
   for (int w2 = 0; w2 < 2; ++w2) {
     if (!(phases & (w2 ? 2 : 1))) continue;

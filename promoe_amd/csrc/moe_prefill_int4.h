@@ -238,83 +238,112 @@ static __device__ __forceinline__ void p6_tile(const PfClass &c, const PfTile &t
     if (t < 4) p6_dma16(lds0 + (unsigned)(M::W0 + slot * M::W + w * 4096 + t * 1024), w_voff, rw, (rb(t) * G + g) * 1024, ~0ull);
     else p6_dma4(lds0 + (unsigned)(M::S0 + slot * M::S + w * 256), s_voff, rs, g * 32, P6_LANES<32>);
   };
-#pragma unroll
-  for (int g = 0; g < M::RW; ++g)
-#pragma unroll
-    for (int t = 0; t < M::NW; ++t) req_w(t, g, g);
   int a_voff[M::Q];                           // unit u = row u / U, piece u % U
 #pragma unroll
   for (int q = 0; q < M::Q; ++q) {
     const int u = M::PER_WAVE * w + 64 * q + lane, r = u / M::U;
     a_voff[q] = act_row(r) + (u - r * M::U) * 16;
   }
+  // zero points (below): CH groups' sums a time, request rq of this wave = 64 (quad, row) pairs
+  constexpr int CH = NB >= 3 ? 16 : 8, CQ = CH / 4, XR = (CQ * NB + 7) / 8;
+  int x_voff[XR];
+#pragma unroll
+  for (int rq = 0; rq < XR; ++rq) x_voff[rq] = act_row((64 * (4 * rq + w) + lane) % (32 * NB)) + P6_SUMS;
+  // (the rows' loads are waited for here: behind a request in assembly their wait would be for that one too)
+#pragma unroll
+  for (int q = 0; q < M::Q; ++q) __asm__ volatile("" : "+v"(a_voff[q]));
+#pragma unroll
+  for (int rq = 0; rq < XR; ++rq) __asm__ volatile("" : "+v"(x_voff[rq]));
   // request q of a group's activations
   auto req_a = [&](int q, int g_, int slot) {
     const int g = g0 + (g_ < ng ? g_ : ng - 1);
     p6_dma16(lds0 + (unsigned)(slot * M::A + (M::PER_WAVE * w + 64 * q) * 16), a_voff[q], ra, g * g_step,
              q + 1 < M::Q ? ~0ull : P6_LANES<M::LAST>);
   };
+  // a chunk of the zero points' operands, into the slot of the activations' ring that is filled last
+  constexpr int X0 = (M::RA - 1) * M::A, ZS = X0 + CQ * 32 * NB * 16, ZZ = ZS + 4 * 4 * CH * 32;
+  static_assert(ZZ + 4 * 4 * CH * 8 <= X0 + M::A, "the slot holds a chunk");
+  const int z0 = (int)(c.off_z - c.off_s - (long long)tile0 * 24);   // from the tile's scales to its zeros (launcher: below 2 GiB)
+  const int q_last = (g0 + ng - 1) >> 2;
+  auto req_zero = [&](int q0) {
 #pragma unroll
-  for (int g = 0; g < M::RA - 1; ++g)
+    for (int rq = 0; rq < XR; ++rq) {     // 64 rows' sums of four groups
+      const int req = 4 * rq + w;
+      if (req < CQ * NB / 2) {
+        const int q = (64 * req + lane) / (32 * NB);
+        p6_dma16(lds0 + (unsigned)(X0 + 1024 * req), x_voff[rq] + 4 * min(q0 + q, q_last) * g_step, ra, 0, ~0ull);
+      }
+    }
+#pragma unroll
+    for (int rq = 0; rq < CH / 8; ++rq) {  // scales: 2 CH pieces of 16 bytes per row block; zeros: 2 CH dwords
+      const int u = 64 * rq + lane, t = u / (2 * CH), v = u - t * 2 * CH;
+      const int b = rb(t) * G + min(4 * q0 + (v >> 1), G - 1);
+      p6_dma16(lds0 + (unsigned)(ZS + w * 4 * CH * 32 + 1024 * rq), b * 32 + (v & 1) * 16, rs, 0, ~0ull);
+      p6_dma4(lds0 + (unsigned)(ZZ + w * 4 * CH * 8 + 256 * rq), z0 + b * 8 + (v & 1) * 4, rs, 0, ~0ull);
+    }
+  };
+  // what the zero points and group 0 need, then the groups behind it
+  req_zero(g0 >> 2);
+#pragma unroll
+  for (int q = 0; q < M::NA; ++q) req_a(q, 0, 0);
+#pragma unroll
+  for (int t = 0; t < M::NW; ++t) req_w(t, 0, 0);
+#pragma unroll
+  for (int g = 1; g < M::RA - 1; ++g)
 #pragma unroll
     for (int q = 0; q < M::NA; ++q) req_a(q, g, g);
+#pragma unroll
+  for (int g = 1; g < M::RW; ++g)
+#pragma unroll
+    for (int t = 0; t < M::NW; ++t) req_w(t, g, g);
   f32x16_t acc[NB][2];
   // zero points: acc = - sum_g (s z) X as products of the two bf16 pieces of either, four groups an instruction (lane
-  // half h: groups 4 p + 2 h, + 1)
+  // half h: groups 4 p + 2 h, + 1).  Sums, scales and zeros of CH groups come together, through LDS, in front of group 0, which
+  // is on its way meanwhile.  (Loaded by every wave into registers, the sums four times and behind the first groups' requests, this
+  // took 17 of 178 us of the w13 launch of the DeepSeek shape at 2048 tokens and 12 of 99 of the w2 launch: now 173 and 93.5;
+  // Mixtral shape 4096 tokens 1395 / 690 -> 1349 / 667, 379 tokens 51.5 / 35.5 -> 49.4 / 34.1.)
+#pragma unroll
+  for (int i = 0; i < NB; ++i)
+#pragma unroll
+    for (int f = 0; f < 2; ++f)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][f][e] = 0.f;
   {
+    const unsigned xr = lds0 + (unsigned)(X0 + n * 16 + 8 * h);
+    const unsigned sr = lds0 + (unsigned)(ZS + (w * 4 + (n >> 4)) * CH * 32 + 64 * h + r16 * 2);
+    const unsigned zr = lds0 + (unsigned)(ZZ + (w * 4 + (n >> 4)) * CH * 8 + 16 * h + (r16 >> 1));
+    const int zsh = 4 * (r16 & 1);
+    for (int q0 = g0 >> 2; q0 <= q_last; q0 += CQ) {
+      if (q0 > g0 >> 2) {
+        __syncthreads();     // the chunk before has been read
+        req_zero(q0);
+        PF_VMCNT(0);
+      } else PF_VMCNT((M::RA - 1) * M::NA + M::RW * M::NW);   // all but the groups' requests behind it
+      __syncthreads();
 #pragma unroll
-    for (int i = 0; i < NB; ++i)
-#pragma unroll
-      for (int f = 0; f < 2; ++f)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) acc[i][f][e] = 0.f;
-    const unsigned char *xs[NB];
-#pragma unroll
-    for (int i = 0; i < NB; ++i) xs[i] = (const unsigned char *)c.act + act_row(32 * i + n) + P6_SUMS;
-    const unsigned char *ps[2], *pz[2];
-#pragma unroll
-    for (int f = 0; f < 2; ++f) {
-      const size_t b = (size_t)16 * nt * G + (size_t)rb(2 * f + (n >> 4)) * G;
-      ps[f] = (const unsigned char *)tile.w_base + c.off_s + b * 32 + r16 * 2;
-      pz[f] = (const unsigned char *)tile.w_base + c.off_z + b * 8 + (r16 >> 1);
-    }
-    for (int p0 = 0; p0 < ng; p0 += 16) {     // 16 groups' loads go out together
-      p6_u32x2_t xv[4][NB];
-      uint16_t sr[4][2][2];
-      unsigned char zr[4][2][2];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int p = min(p0 + 4 * q, (ng - 1) & ~3);
-        const int gp = min(g0 + p + 2 * h, (g0 + ng - 1) & ~1);   // (g0 is even)
-#pragma unroll
-        for (int i = 0; i < NB; ++i) xv[q][i] = *(const p6_u32x2_t *)(xs[i] + (size_t)(gp & ~3) * g_step + 8 * ((gp >> 1) & 1));
+      for (int q = 0; q < CQ; ++q) {
+        if (q0 + q > q_last) break;
+        u32x4_t xa[NB], wb[2];
+        bool on[2];
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-          const int g = g0 + min(p + 2 * h + j, ng - 1);
+          const int g = 4 * (q0 + q) + 2 * h + j;
+          on[j] = g >= g0 && g < g0 + ng;    // (groups past the end have no sum)
 #pragma unroll
           for (int f = 0; f < 2; ++f) {
-            sr[q][j][f] = *(const uint16_t *)(ps[f] + (size_t)g * 32);
-            zr[q][j][f] = pz[f][(size_t)g * 8];
+            const float sc = half_bits_to_f32(pn_lds<uint16_t>(sr + (unsigned)(2 * f * CH * 32 + 128 * q + 32 * j)));
+            const u32 z = (pn_lds<unsigned char>(zr + (unsigned)(2 * f * CH * 8 + 32 * q + 8 * j)) >> zsh) & 15u;
+            const float v = on[j] ? -sc * (float)z : 0.f;   // 15 significant bits: its upper half and what that leaves are bf16
+            const u32 v1 = __float_as_uint(v), v2 = __float_as_uint(v - __uint_as_float(v1 & 0xffff0000u));
+            wb[f][2 * j] = __builtin_amdgcn_perm(v1, v1, 0x03020302u);
+            wb[f][2 * j + 1] = __builtin_amdgcn_perm(v2, v2, 0x03020302u);
           }
         }
-      }
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        if (p0 + 4 * q >= ng) break;
-        u32x4_t xa[NB], wb[2];
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          const bool on = p0 + 4 * q + 2 * h + j < ng;   // (groups past the end have no sum)
-#pragma unroll
-          for (int i = 0; i < NB; ++i) xa[i][2 * j] = xa[i][2 * j + 1] = on ? xv[q][i][j] : 0u;
-#pragma unroll
-          for (int f = 0; f < 2; ++f) {
-            const float z = (float)((zr[q][j][f] >> (4 * (r16 & 1))) & 15);
-            const float v = on ? -half_bits_to_f32(sr[q][j][f]) * z : 0.f;      // 15 significant bits: two bf16 hold it exactly
-            const u32 v1 = f32_to_bf16(v), v2 = f32_to_bf16(v - __uint_as_float(v1 << 16));
-            wb[f][2 * j] = v1 | (v1 << 16);
-            wb[f][2 * j + 1] = v2 | (v2 << 16);
-          }
+        for (int i = 0; i < NB; ++i) {
+          const p6_u32x2_t xv = pn_lds<p6_u32x2_t>(xr + (unsigned)((q * 32 * NB + 32 * i) * 16));
+          const u32 x0 = on[0] ? xv.x : 0u, x1 = on[1] ? xv.y : 0u;
+          xa[i] = u32x4_t{x0, x0, x1, x1};
         }
 #pragma unroll
         for (int i = 0; i < NB; ++i)
@@ -325,7 +354,7 @@ static __device__ __forceinline__ void p6_tile(const PfClass &c, const PfTile &t
       }
     }
   }
-  PF_VMCNT(0);   // (the loads above came behind the requests: those have landed)
+  PF_VMCNT((M::RA - 2) * M::NA + (M::RW - 1) * M::NW);   // group 0 is there (the loop's first barrier follows)
   // LDS addresses: the lane's pieces of a slab's row, its block scales, its nibbles and scales
   const unsigned fa = lds0 + (unsigned)(n * M::ROW + 16 * h), fb = lds0 + (unsigned)(n * M::ROW + (W13 ? 96 : 64) + 8 * h);
   const unsigned fs = lds0 + (unsigned)(n * M::ROW + R::SCALES + 2 * h);

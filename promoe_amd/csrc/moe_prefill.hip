@@ -80,8 +80,8 @@ static __device__ __forceinline__ float pf_silu_mul(float g, float u) {
 //   bf16, Qwen1.5 shape    65 tokens 115.5 / 116.2 / 116.7 and 77.6 / 88.3 / 77.8, 379 tokens 135.6 / 136.5 / 136.5 and
 //                          91.1 / 93.4 / 91.6, 1999 tokens 228 / 224 / 224 and 132 / 131 / 135
 //   bf16, Mixtral shape    1024 tokens 489 / 423 / 424 and 287 / 289 / 287, 2048 tokens 909 / 738 / 737 and 519 / 470 / 467
-//   int4, DeepSeek shape   (runs / even) 65 tokens 34.3 / 34.5 and 31.7 / 33.1, 200 tokens 44.9 / 46.5 and 36.4 / 37.6, 2048
-//                          tokens 194 / 193 and 109 / 110
+//   int4, DeepSeek shape   (runs / even; a kernel before the present one) 65 tokens 34.3 / 34.5 and 31.7 / 33.1, 200 tokens
+//                          44.9 / 46.5 and 36.4 / 37.6, 2048 tokens 194 / 193 and 109 / 110
 #define PF_DEAL 8
 #define PF_GROUP 8
 template <bool EVEN>
@@ -384,16 +384,15 @@ __global__ __launch_bounds__(256, 1) void k_prefill_gemm(const PfArgs a) {
 //     products of step j, in pieces of one pair (order pinned by sched_barrier);
 //   * two workgroups per compute unit cover each other's barriers, prologues and epilogues.
 // h rows leave the w13 pass as fp16, so that the w2 pass brings them into LDS as they are.
-// Measured (one box, w13 / w2 launch; in brackets the kernel before: eight waves, the weights of a tile dequantised
-// by two of them each, activations converted and nibbles loaded through registers one group ahead): DeepSeek shape
-// 2048 tokens 215 / 121 us (305 / 167), 379 tokens 76 / 49 (115 / 65), Mixtral shape 4096 tokens 1733 / 991 (2132 /
-// 1038), Qwen2-57B shape q4_K 512 tokens 408 / 219 (577 / 303); with the block order of pf_block_of 194 / 109, 62 / 43,
-// 1622 / 893 and 320 / 187.
-// What bounds it: on the Mixtral shape the power limit (matrix cores busy 78 % and 69 % of the cycles of the two launches,
-// which run at 1.46 and 1.51 GHz); on the others partly (DeepSeek shape, 2048 tokens: 59 % and 50 % at 1.70 and 1.81 GHz;
-// Qwen2-57B shape, 512 tokens: 61 % and 49 % at 1.65 and 1.78 GHz), with 0.8 to 0.9 vector cycles of dequantisation per
-// matrix cycle.  Tiles of 256 rows with one workgroup per compute unit halve the dequantisation per product and lose 8 to
-// 15 % on all but the Mixtral shape (+1 %).
+// Measured (w13 / w2 launch; in brackets the kernel before: eight waves, the weights of a tile dequantised by two of them
+// each, activations converted and nibbles loaded through registers one group ahead): Qwen2-57B shape, 512 tokens 408 / 219
+// us (577 / 303); with the block order of pf_block_of 320 / 187.
+// What bounds it: partly the power limit (Qwen2-57B shape, 512 tokens: matrix cores busy 61 % and 49 % of the cycles of the two
+// launches, at 1.65 and 1.78 GHz), with 0.8 to 0.9 vector cycles of dequantisation per matrix cycle.  Its tiles stay at 128
+// rows: with 64 the Qwen2-57B shape takes 635 instead of 553 us a layer at 512 tokens and 226 instead of 220 at 65; with 256
+// and one workgroup per compute unit it takes 8 to 15 % more.
+// int4 experts have a kernel of their own (moe_prefill_int4.h): a q4_K sub-block has a scale and a minimum of its own per 32
+// weights, four times the folds and zero-point products per output.
 typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
 
 #define PN_BM 128                         // most rows of one tile: 4 blocks of 32 (128 accumulator registers)
@@ -942,7 +941,7 @@ extern "C" int moe_experts_prefill_publish(const void *x_bf16, int T, int H, int
   const bool convert = int4 && (phases & 1);
   if (convert) {
     if (phases & 4) x16 = (unsigned char *)tiles_ws + pf_x16_offset(T, k, max_units);
-    else if (int rc = moe_check_hip(hipMallocAsync(&x16_own, (size_t)T * H * 2, s), "hipMallocAsync(fp16 activations)")) return rc;
+    else if (int rc = moe_check_hip(hipMallocAsync(&x16_own, (size_t)T * H * 2, s), "hipMallocAsync(activations' copy)")) return rc;
     if (x16_own) x16 = x16_own;
   }
   struct FreeX16 {  // on every way out
@@ -997,7 +996,7 @@ extern "C" int moe_experts_prefill_publish(const void *x_bf16, int T, int H, int
         c.w_off = w2 ? lay.off2_q : lay.off13_q;
         c.off_s = w2 ? lay.off2_s : lay.off13_s;
         c.off_z = w2 ? lay.off2_z : lay.off13_z;
-        if (!q4k && c.off_z - c.off_s >= (1ll << 31) - (1ll << 24)) {  // (pn_tile: the zeros are addressed from the scales)
+        if (!q4k && c.off_z - c.off_s >= (1ll << 31) - (1ll << 24)) {  // (p6_tile: the zeros are addressed from the scales)
           moe_set_error("moe_experts_prefill: the scales of an expert of %d x %d take 2 GiB or more", H, Ii);
           return MOE_EINVAL;
         }

@@ -15,11 +15,12 @@
 // Error against 64 bits (2-norm of the partial rows): 2048 x 1408 1.04e-3, 4096 x 4096 1.06e-3, where dequantising to fp16
 // had 3.17e-3 and 3.18e-3 (the rounding of -(16 + z) s, common to the 128 weights of a group's row).
 // Measured against that kernel (four waves, dequantisation between the products; w13 / w2 launch under the profiler, us):
-// Mixtral shape 4096 tokens 1437 / 710 (1658 / 891), DeepSeek shape 2048 tokens 182 / 102 (200 / 114), 379 tokens 52 / 42
+// Mixtral shape 4096 tokens 1349 / 667 (1658 / 891), DeepSeek shape 2048 tokens 173 / 93 (200 / 114), 379 tokens 49 / 34
 // (64 / 45).
-// What bounds it: without the requests in the loop the same launches take 1142 / 562 and 148 / 81, without the folds 1331 / 686
-// and 172 / 99: the Mixtral launches run at 1.74 GHz (power), the others at 2.0 to 2.2 with the matrix cores 41 and 23 % busy, two
-// waves per SIMD that wait a sixth of the time for a group to arrive.
+// What bounds it (a build whose launches took 1437 / 710 and 182 / 102; Mixtral shape, then DeepSeek shape): without the requests in
+// the loop 1142 / 562 and 148 / 81, without the folds 1331 / 686 and 172 / 99.  The Mixtral launches run at 1.74 GHz (power), the
+// others at 2.0 to 2.2 with the matrix cores 41 and 23 % busy, two waves per SIMD that wait a sixth of the time for a group to
+// arrive; the split of the h rows is 13 % of a DeepSeek w13 launch.
 #pragma once
 
 typedef int p6_i32x8_t __attribute__((ext_vector_type(8)));

@@ -100,7 +100,7 @@ def launches_timed(torch, launch_n, n, replay_once=False):
 
 PROFILE_DIR = os.path.join(os.path.dirname(os.path.abspath(__file__)), "profiles")
 DECODE_SOURCES = ["promoe_amd/csrc/" + f for f in ("moe_kernels.hip", "moe_decode_bf16.hip", "moe_device.h", "moe_common.h")]
-PREFILL_SOURCES = ["promoe_amd/csrc/" + f for f in ("moe_prefill.hip", "moe_prefill_int4.h", "moe_gate.hip", "moe_decode_bf16.hip", "moe_device.h",
+PREFILL_SOURCES = ["promoe_amd/csrc/" + f for f in ("moe_prefill.hip", "moe_gate.hip", "moe_decode_bf16.hip", "moe_device.h",
                                                     "moe_common.h")]
 
 
@@ -226,7 +226,7 @@ def prefill_leg(torch, name, T, H, E, I, k, I_sh, fmt, gated, mode, steps=20):
             "expert_flops": flops, "weight_bytes": wbytes,
             "layer_TFLOPs": (flops + 2.0 * T * wg.shape[0] * H) / t_layer / 1e12,
             "roofline": {"bound": "mfma", "kernel": "%s (w13 + SwiGLU, routed + shared in one launch)" %
-                         ("k_prefill_gemm<true>" if fmt == L.FMT_BF16 else "k_prefill_nib<true>" if fmt == L.FMT_Q4K else "k_prefill_int4<true>"),
+                         ("k_prefill_gemm<true>" if fmt == L.FMT_BF16 else "k_prefill_nib<true,%s>" % ("true" if fmt == L.FMT_Q4K else "false")),
                          "achieved": ach, "peak": MFMA_PEAK_TFLOPS, "unit": "TFLOP/s", "frac": ach / MFMA_PEAK_TFLOPS,
                          # HBM bytes per launch from the committed FETCH_SIZE / WRITE_SIZE counter summary (null for a
                          # leg without counters, or when the kernel sources changed since they were taken)
@@ -347,7 +347,7 @@ def decode_leg(torch, name, fmt, T, H, E, I, k, I_sh, gated, mode, layers, zipf,
             "algorithmic_bytes_per_step": step_bytes, "layer_GBps": step_bytes / t_layer / 1e9,
             "roofline": {"bound": "hbm", "kernel": ("k_gemv_int4_mfma%s<route> (gate rows + routing + w13 + SwiGLU in one launch)"
                                                     % ("" if T <= 8 and H <= 2048 else "_kc")) if batch_path else
-                                                   ("%s<true> (w13 + SwiGLU)" % ("k_prefill_nib" if q4k else "k_prefill_int4") if tiles else
+                                                   ("k_prefill_nib<true,%s> (w13 + SwiGLU)" % ("true" if q4k else "false") if tiles else
                                                     "k_gemv_int4%s (w13 + SwiGLU)" % (("_mfma_kc<q4_K>" if T > 1 else "<q4_K>") if q4k else ("_mfma_kc" if (T > 16 or H > 2048) and T > 1 else ("_mfma" if T > 1 else "")))),
                          "achieved": ach, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": ach / HBM_PEAK_GBS, "traffic": None,
                          "algorithmic_bytes_per_launch": w13_bytes, "avg_launch_us": t_w13 * 1e6,

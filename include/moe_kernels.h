@@ -355,18 +355,16 @@ int moe_experts_decode_q4k_publish(const void *x_bf16, int T, int H, int I, int 
  * Same arguments and buffer meanings as moe_experts_decode_int4 (rows of h_r / part_r in the
  * sorted pair order; expert_ptr[e] == 0 for an active expert sets *err |= 1 and skips it).
  *   fmt       : MOE_FMT_BF16 (expert image = blocked w13 [2I,H] then blocked w2 [H,I]; bf16 MFMA),
- *               MOE_FMT_Q4K (nibble tiles dequantised in registers to fp16 operands, activations converted to
- *               fp16 once per call; tiles of up to 128 rows) or MOE_FMT_INT4_G128 (nibbles as exact 6-bit operands of
- *               the scaled matrix instructions, scales and zeros in fp32, activations split once per call into two
- *               numbers of 4 and 3 (x) or 4 and 4 (h) significant bits with one scale per 32; tiles of up to 64 or 128 rows)
+ *               MOE_FMT_INT4_G128 or MOE_FMT_Q4K (nibble tiles dequantised in registers to fp16
+ *               operands, activations converted to fp16 once per call; tiles of 128 rows)
  *   tiles_ws  : device workspace of moe_prefill_workspace_bytes(T, k, max_units) bytes; the
  *               list of row tiles per expert is built there by a kernel, so the host
  *               needs no copy of the dispatch counts.
- *   phases    : bit 0 = w13 + SwiGLU, bit 1 = w2; bit 2 (nibble formats) = tiles_ws has room for the copy of
+ *   phases    : bit 0 = w13 + SwiGLU, bit 1 = w2; bit 2 (nibble formats) = tiles_ws has room for the fp16 copy of
  *               x behind the list, T*H*2 bytes at the next multiple of 256 (without it the call takes and returns
  *               stream-ordered memory for the copy).
- * Between the two passes h_r / h_s hold bf16 for MOE_FMT_BF16, fp16 for MOE_FMT_Q4K and the w2 pass's split operands
- * for MOE_FMT_INT4_G128 (same room); both passes of a batch go through this entry.
+ * Between the two passes h_r / h_s hold bf16 for MOE_FMT_BF16 and fp16 for the nibble formats (whose matrix-core
+ * operands are fp16: the w2 pass then stages them without a conversion); both passes of a batch go through this entry.
  * H % 256 == 0, I % 128 == 0, I_sh % 128 == 0.  The reference leaves this product to the
  * framework's own expert modules (SimulateMoeLayer.forward, transformers-deepseek-moe.py:36-49). */
 int64_t moe_prefill_workspace_bytes(int T, int k, int max_units);

@@ -134,7 +134,7 @@ static __device__ __forceinline__ u32 bload1(rsrc_t r, int voff, int soff) {
 }
 
 // ---------------------------------------------------------------------------
-// fp16 operands for the matrix cores from nibble formats (the q4_K tile kernel, q4_K decode)
+// fp16 operands for the matrix cores from nibble formats (int4-g128 and q4_K tile kernels, q4_K decode)
 // ---------------------------------------------------------------------------
 typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
 static __device__ __forceinline__ u32 bf16x2_to_f16x2(u32 d) {
@@ -144,10 +144,11 @@ static __device__ __forceinline__ u32 bf16x2_to_f16x2(u32 d) {
 }
 // Dequantisation of 8 nibbles of a dword into 8 fp16 weights with ONE packed fma per pair: a nibble is masked into
 // mantissa bits 6..9 of an fp16 with the exponent of 1.0, which makes the exact value h = 1 + q/16; with S = 16 s and
-// C = -(16 s + m), both prepared once per sub-block and row, h S + C = q s - m.  The product is exact inside the fma; C
-// carries the one extra rounding (2^-11 of at most 31 s, i.e. 0.015 of a quantisation step, a bias common to the
-// weights of a sub-block's row).  The form before this one (h = 1024 + q) was exact up to the final rounding and cost
-// three packed operations per pair, in kernels that are bound by these operations.
+// C = -(16 + zero) s (int4) or C = -(16 s + m) (q4_K), both prepared once per group and row, h S + C = (q - zero) s
+// or q s - m.  The product is exact inside the fma; C carries the one extra rounding (2^-11 of at most 31 s, i.e.
+// 0.015 of a quantisation step, a bias common to the 128 weights of a group row).  The form before this one
+// ((h - (1024 + zero)) s with h = 1024 + q) was exact up to the final rounding and cost a packed subtract and
+// a packed multiply per pair (three operations for q4_K), in kernels that are bound by these operations.
 // Mask and exponent pattern are held in vector registers, made once per kernel: (x & M) | C is then ONE
 // v_and_or_b32 (a VOP3 instruction takes no literal and one scalar operand on this target).
 struct DeqF16Consts { u32 M, C; };

@@ -8,7 +8,7 @@
 // columns: for w13 the two column halves are the SAME columns of gate and up (SwiGLU fused in the epilogue),
 // for w2 they are adjacent column blocks.  K advances 64 at a time; the activation slab goes global -> LDS
 // directly (a ring of four slabs), the weight fragments go global -> registers in operand order and feed
-// v_mfma_f32_32x32x16_bf16.  q4_K experts: four waves on a tile of up to 128 rows, two workgroups per compute unit,
+// v_mfma_f32_32x32x16_bf16.  int4 / q4_K experts: four waves on a tile of up to 128 rows, two workgroups per compute unit,
 // activations, nibbles and scales through one LDS ring, fragments dequantised in registers between the products (below).
 // bf16 batches of up to 64 tokens go to moe_decode_bf16.hip.
 #include <hip/hip_runtime.h>
@@ -53,7 +53,6 @@ struct PfClass {
   int ksplit;           // int4 / q4_K w2 pass of the shared expert: workgroups per tile, each over 1/ksplit of the
                         // reduction, partial rows to out + split * split_stride (0 or 1: the whole reduction)
   long long split_stride;  // elements between the pieces of out
-  int act_rows, out_rows;  // int4: rows of the activation matrix and of h (w13), whose groups lie one after the other
 };
 struct PfArgs {
   PfClass c[2];
@@ -80,8 +79,8 @@ static __device__ __forceinline__ float pf_silu_mul(float g, float u) {
 //   bf16, Qwen1.5 shape    65 tokens 115.5 / 116.2 / 116.7 and 77.6 / 88.3 / 77.8, 379 tokens 135.6 / 136.5 / 136.5 and
 //                          91.1 / 93.4 / 91.6, 1999 tokens 228 / 224 / 224 and 132 / 131 / 135
 //   bf16, Mixtral shape    1024 tokens 489 / 423 / 424 and 287 / 289 / 287, 2048 tokens 909 / 738 / 737 and 519 / 470 / 467
-//   int4, DeepSeek shape   (runs / even; a kernel before the present one) 65 tokens 34.3 / 34.5 and 31.7 / 33.1, 200 tokens
-//                          44.9 / 46.5 and 36.4 / 37.6, 2048 tokens 194 / 193 and 109 / 110
+//   int4, DeepSeek shape   (runs / even) 65 tokens 34.3 / 34.5 and 31.7 / 33.1, 200 tokens 44.9 / 46.5 and 36.4 / 37.6, 2048
+//                          tokens 194 / 193 and 109 / 110
 #define PF_DEAL 8
 #define PF_GROUP 8
 template <bool EVEN>
@@ -365,7 +364,7 @@ __global__ __launch_bounds__(256, 1) void k_prefill_gemm(const PfArgs a) {
     }
 }
 
-// ---- q4_K experts -----------------------------------------------------------------------------
+// ---- int4-g128 and q4_K experts ---------------------------------------------------------
 // A workgroup of four waves (one per SIMD, two workgroups per compute unit) computes a tile of up to 128 rows x
 // (128 + 128) columns; wave w owns 32 columns of both halves (for w13 the same columns of gate and up, for w2
 // adjacent column blocks) and ALL row blocks of the tile, so every weight is dequantised once per tile.  K advances
@@ -384,21 +383,22 @@ __global__ __launch_bounds__(256, 1) void k_prefill_gemm(const PfArgs a) {
 //     products of step j, in pieces of one pair (order pinned by sched_barrier);
 //   * two workgroups per compute unit cover each other's barriers, prologues and epilogues.
 // h rows leave the w13 pass as fp16, so that the w2 pass brings them into LDS as they are.
-// Measured (w13 / w2 launch; in brackets the kernel before: eight waves, the weights of a tile dequantised by two of them
-// each, activations converted and nibbles loaded through registers one group ahead): Qwen2-57B shape, 512 tokens 408 / 219
-// us (577 / 303); with the block order of pf_block_of 320 / 187.
-// What bounds it: partly the power limit (Qwen2-57B shape, 512 tokens: matrix cores busy 61 % and 49 % of the cycles of the two
-// launches, at 1.65 and 1.78 GHz), with 0.8 to 0.9 vector cycles of dequantisation per matrix cycle.  Its tiles stay at 128
-// rows: with 64 the Qwen2-57B shape takes 635 instead of 553 us a layer at 512 tokens and 226 instead of 220 at 65; with 256
-// and one workgroup per compute unit it takes 8 to 15 % more.
-// int4 experts have a kernel of their own (moe_prefill_int4.h): a q4_K sub-block has a scale and a minimum of its own per 32
-// weights, four times the folds and zero-point products per output.
+// Measured (one box, w13 / w2 launch; in brackets the kernel before: eight waves, the weights of a tile dequantised
+// by two of them each, activations converted and nibbles loaded through registers one group ahead): DeepSeek shape
+// 2048 tokens 215 / 121 us (305 / 167), 379 tokens 76 / 49 (115 / 65), Mixtral shape 4096 tokens 1733 / 991 (2132 /
+// 1038), Qwen2-57B shape q4_K 512 tokens 408 / 219 (577 / 303); with the block order of pf_block_of 194 / 109, 62 / 43,
+// 1622 / 893 and 320 / 187.
+// What bounds it: on the Mixtral shape the power limit (matrix cores busy 78 % and 69 % of the cycles of the two launches,
+// which run at 1.46 and 1.51 GHz); on the others partly (DeepSeek shape, 2048 tokens: 59 % and 50 % at 1.70 and 1.81 GHz;
+// Qwen2-57B shape, 512 tokens: 61 % and 49 % at 1.65 and 1.78 GHz), with 0.8 to 0.9 vector cycles of dequantisation per
+// matrix cycle.  Tiles of 256 rows with one workgroup per compute unit halve the dequantisation per product and lose 8 to
+// 15 % on all but the Mixtral shape (+1 %).
 typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
 
 #define PN_BM 128                         // most rows of one tile: 4 blocks of 32 (128 accumulator registers)
 #define PN_LDS 81920                      // half of a compute unit's LDS
-struct PnSlab {                           // one ring slot: activations, then per wave 2 KiB of nibbles and the scales
-  static constexpr int SB = 512;                             // scale bytes of one wave
+template <bool Q4K> struct PnSlab {       // one ring slot: activations, then per wave 2 KiB of nibbles and the scales
+  static constexpr int SB = Q4K ? 512 : 256;                 // scale bytes of one wave
   static constexpr int bytes(int nb) { return nb * 4096 + 4 * (2048 + SB); }
   static constexpr int ring(int nb) { return PN_LDS / bytes(nb) < 8 ? PN_LDS / bytes(nb) : 8; }
 };
@@ -428,20 +428,22 @@ static __device__ __forceinline__ T pn_lds(unsigned addr) {
 
 // what a wave of a tile reads; offsets in bytes, voff per lane
 struct PnSrc {
-  // activation matrix; nibbles, scales and super-block scales of the tile's 16 row blocks (64-bit bases: an expert
+  // activation matrix; nibbles, scales and (q4_K) super-block scales of the tile's 16 row blocks (64-bit bases: an expert
   // image may have 2 GiB and more)
   pf_i32x4_t ra, rw, rs, rz;
   int a_voff[4];            // row block n: the lane's row and chunk
   int w_voff[2];            // fragment f
-  int s_voff, z_voff;       // scale request; (d, dmin) request
+  int s_voff, z_voff;       // scale request; q4_K: (d, dmin) request; int4: s_voff covers scales and zeros
+  int s_step;               // int4: what s_voff advances by per quantisation group (scales and zeros differ)
 };
 
 // acc[i][f]: row block i, fragment (column half) f; slabs kt0 .. kt0 + nk - 1 (64 k each), nk >= 2 and even
-template <int NB>
+template <int NB, bool Q4K>
 static __device__ __forceinline__ void pn_mainloop(f32x16_t (&acc)[NB][2], const unsigned lds_base, const PnSrc &m, const int kt0,
                                                    const int nk, const int tid) {
-  constexpr int SB = PnSlab::SB, SLOT = PnSlab::bytes(NB), R = PnSlab::ring(NB);
-  constexpr int NL = NB + 4;               // requests of a slab
+  constexpr int SB = PnSlab<Q4K>::SB, SLOT = PnSlab<Q4K>::bytes(NB), R = PnSlab<Q4K>::ring(NB);
+  constexpr int NS_ = Q4K ? 2 : 1;         // scale requests of a slab
+  constexpr int NL = NB + 2 + NS_;         // requests of a slab
   static_assert(R >= 3 && (R - 2) * NL < 63, "ring depth");
   constexpr int NG = 4 * NB;               // product groups of a slab (two products each)
   constexpr int FD = NG < 4 ? NG : 4;      // activation fragments read ahead
@@ -454,6 +456,7 @@ static __device__ __forceinline__ void pn_mainloop(f32x16_t (&acc)[NB][2], const
     const int kt = kt0 + (kt_ < nk ? kt_ : nk - 1);
     if (r < NB) pn_dma16(lds_base + (unsigned)(so + (32 * r + 8 * w) * 128), m.a_voff[r], m.ra, kt * 128);
     else if (r < NB + 2) pn_dma16(wbase + (unsigned)(so + 1024 * (r - NB)), m.w_voff[r - NB], m.rw, kt * 512);
+    else if (!Q4K) pn_dma4(wbase + (unsigned)(so + 2048), m.s_voff + (kt >> 1) * m.s_step, m.rs, 0);
     else if (r == NB + 2) pn_dma4(wbase + (unsigned)(so + 2048), m.s_voff, m.rs, kt * 64);
     else pn_dma4(wbase + (unsigned)(so + 2048 + 256), m.z_voff, m.rz, (kt >> 2) * 64);
   };
@@ -463,8 +466,9 @@ static __device__ __forceinline__ void pn_mainloop(f32x16_t (&acc)[NB][2], const
   for (int j = 0; j < 4; ++j) fa0[j] = lds_base + (unsigned)(n * 128 + (((4 * q + j) ^ ((n >> 1) & 7)) * 16));
   const unsigned na0 = wbase + (unsigned)lane * 16u;
   const int t0 = n >> 4, r16 = n & 15;   // fragment f reads row r16 of the wave's row block 2 f + t0
-  const unsigned sa0 = wbase + 2048u + (unsigned)(t0 * 64 + (16 * q + r16) * 2);
-  const unsigned za0 = wbase + 2048u + (unsigned)(256 + t0 * 64 + r16 * 4);
+  const unsigned sa0 = wbase + 2048u + (unsigned)(Q4K ? t0 * 64 + (16 * q + r16) * 2 : t0 * 32 + r16 * 2);
+  const unsigned za0 = wbase + 2048u + (unsigned)(Q4K ? 256 + t0 * 64 + r16 * 4 : 128 + t0 * 8 + (r16 >> 1));
+  const int zsh = 4 * (r16 & 1);
   u32x4_t nib[2], nxt[2];
   u32 s2[2], c2[2], sraw[2], zraw[2];
   u32x4_t wd[2][2];                      // [step parity][fragment]: 8 fp16 weights
@@ -472,15 +476,27 @@ static __device__ __forceinline__ void pn_mainloop(f32x16_t (&acc)[NB][2], const
 #pragma unroll
     for (int f = 0; f < 2; ++f) {
       d[f] = pn_lds<u32x4_t>(na0 + (unsigned)(so + 1024 * f));
-      sraw[f] = pn_lds<uint16_t>(sa0 + (unsigned)(so + 128 * f));
-      zraw[f] = pn_lds<u32>(za0 + (unsigned)(so + 128 * f));
+      if (Q4K) {
+        sraw[f] = pn_lds<uint16_t>(sa0 + (unsigned)(so + 128 * f));
+        zraw[f] = pn_lds<u32>(za0 + (unsigned)(so + 128 * f));
+      } else {
+        sraw[f] = pn_lds<uint16_t>(sa0 + (unsigned)(so + 64 * f));
+        zraw[f] = pn_lds<unsigned char>(za0 + (unsigned)(so + 16 * f));
+      }
     }
   };
   auto prep = [&]() {  // S = 16 s and C of deq8_f16 for the lane's row in both fragments
 #pragma unroll
     for (int f = 0; f < 2; ++f) {
-      const float s16 = 16.f * __builtin_bit_cast(float, h2f_bits(zraw[f] & 0xffffu)) * (float)(sraw[f] & 0xffu);
-      const float cz = -s16 - __builtin_bit_cast(float, h2f_bits(zraw[f] >> 16)) * (float)((sraw[f] >> 8) & 0xffu);
+      float s16, cz;
+      if (Q4K) {
+        s16 = 16.f * __builtin_bit_cast(float, h2f_bits(zraw[f] & 0xffffu)) * (float)(sraw[f] & 0xffu);
+        cz = -s16 - __builtin_bit_cast(float, h2f_bits(zraw[f] >> 16)) * (float)((sraw[f] >> 8) & 0xffu);
+      } else {
+        const float sf = __builtin_bit_cast(float, h2f_bits(sraw[f]));
+        s16 = 16.f * sf;
+        cz = -(16.f + (float)((zraw[f] >> zsh) & 15u)) * sf;
+      }
       const u32 sb = f2h_bits(s16), cb = f2h_bits(cz);
       s2[f] = sb | (sb << 16);
       c2[f] = cb | (cb << 16);
@@ -550,7 +566,7 @@ static __device__ __forceinline__ void pn_mainloop(f32x16_t (&acc)[NB][2], const
   }
 }
 
-template <int NB, bool SWIGLU>
+template <int NB, bool SWIGLU, bool Q4K>
 static __device__ __forceinline__ void pn_tile(const PfClass &c, const PfTile &tile, unsigned char *lds, int nt, int kt0, int nk,
                                                int split, int tid) {
   const int lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -561,8 +577,8 @@ static __device__ __forceinline__ void pn_tile(const PfClass &c, const PfTile &t
   m.ra = pn_rsrc(c.act);
   const size_t tile0 = (size_t)16 * nt * G;   // (row block, group) pairs in front of the tile's
   m.rw = pn_rsrc((const void *)(tile.w_base + c.w_off + tile0 * 1024));
-  m.rs = pn_rsrc((const void *)(tile.w_base + c.off_s + tile0 * 128));
-  m.rz = pn_rsrc((const void *)(tile.w_base + c.off_z + tile0 * 32));
+  m.rs = pn_rsrc((const void *)(tile.w_base + c.off_s + tile0 * (Q4K ? 128 : 32)));
+  m.rz = pn_rsrc((const void *)(tile.w_base + c.off_z + tile0 * (Q4K ? 32 : 8)));
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     m.a_voff[i] = 0;
@@ -582,8 +598,19 @@ static __device__ __forceinline__ void pn_tile(const PfClass &c, const PfTile &t
 #pragma unroll
   for (int f = 0; f < 2; ++f)
     m.w_voff[f] = rb(2 * f + (n >> 4)) * G * 1024 + (16 * q + (n & 15)) * 16;
-  m.s_voff = rb(lane >> 4) * G * 128 + (lane & 15) * 4;
-  m.z_voff = rb(lane >> 4) * (G >> 1) * 64 + (lane & 15) * 4;
+  if (Q4K) {
+    m.s_voff = rb(lane >> 4) * G * 128 + (lane & 15) * 4;
+    m.z_voff = rb(lane >> 4) * (G >> 1) * 64 + (lane & 15) * 4;
+    m.s_step = 0;
+  } else {
+    // lanes 0..31: 8 dwords of scales of each row block; lanes 32..39: 2 dwords of zeros of each; the rest idle copies.
+    // The zeros of the tile lie behind its scales (in the image's next section, less than 2 GiB away: the launcher)
+    const int l = lane < 40 ? lane : 39;
+    const int z0 = (int)(c.off_z - c.off_s - (long long)tile0 * 24);
+    m.s_voff = l < 32 ? rb(l >> 3) * G * 32 + (l & 7) * 4 : z0 + rb((l - 32) >> 1) * G * 8 + (l & 1) * 4;
+    m.s_step = l < 32 ? 32 : 8;
+    m.z_voff = 0;
+  }
   f32x16_t acc[NB][2];
 #pragma unroll
   for (int i = 0; i < NB; ++i)
@@ -591,7 +618,7 @@ static __device__ __forceinline__ void pn_tile(const PfClass &c, const PfTile &t
     for (int h = 0; h < 2; ++h)
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][h][e] = 0.f;
-  pn_mainloop<NB>(acc, lds_base, m, kt0, nk, tid);
+  pn_mainloop<NB, Q4K>(acc, lds_base, m, kt0, nk, tid);
   // epilogue.  acc element e of lane l: row 8*(e/4) + 4*(l/32) + e%4 of its block, column l%32
   const int col = 32 * w + n;
   PF_VMCNT(0);   // the transfers past the end have landed: the ring is free, and nothing is in flight at the end
@@ -627,7 +654,7 @@ static __device__ __forceinline__ void pn_tile(const PfClass &c, const PfTile &t
   }
 }
 
-template <bool SWIGLU>
+template <bool SWIGLU, bool Q4K>
 __global__ __launch_bounds__(256, 2) void k_prefill_nib(const PfArgs a) {
   extern __shared__ __align__(16) unsigned char lds_n[];
   const int tid = threadIdx.x;
@@ -641,14 +668,13 @@ __global__ __launch_bounds__(256, 2) void k_prefill_nib(const PfArgs a) {
   // this workgroup's window of the reduction (only the w2 pass is ever split)
   const int nk = SWIGLU ? c.K / PF_BK : c.K / PF_BK / ks, kt0 = SWIGLU ? 0 : split * nk;
   switch ((rows + 31) >> 5) {
-    case 1: pn_tile<1, SWIGLU>(c, tile, lds_n, nt, kt0, nk, split, tid); break;
-    case 2: pn_tile<2, SWIGLU>(c, tile, lds_n, nt, kt0, nk, split, tid); break;
-    case 3: pn_tile<3, SWIGLU>(c, tile, lds_n, nt, kt0, nk, split, tid); break;
-    default: pn_tile<4, SWIGLU>(c, tile, lds_n, nt, kt0, nk, split, tid); break;
+    case 1: pn_tile<1, SWIGLU, Q4K>(c, tile, lds_n, nt, kt0, nk, split, tid); break;
+    case 2: pn_tile<2, SWIGLU, Q4K>(c, tile, lds_n, nt, kt0, nk, split, tid); break;
+    case 3: pn_tile<3, SWIGLU, Q4K>(c, tile, lds_n, nt, kt0, nk, split, tid); break;
+    default: pn_tile<4, SWIGLU, Q4K>(c, tile, lds_n, nt, kt0, nk, split, tid); break;
   }
 }
 
-#include "moe_prefill_int4.h"
 
 // Workgroups of a class of `blocks` blocks: whole rounds of 8 runs, or, where less than a round is spread evenly (EVEN), an
 // even share per XCD (56 idle workgroups between the shared expert's 8 w2 blocks and the routed ones of a 65-token batch of
@@ -658,25 +684,23 @@ static int pf_padded(bool even, int blocks) {
   return (blocks + q - 1) / q * q;
 }
 
-static int pn_launch(bool swiglu, bool q4k, const PfArgs &a, hipStream_t s) {
+template <bool Q4K>
+static int pn_launch(bool swiglu, const PfArgs &a, hipStream_t s) {
   if (a.n_blocks_total <= 0) return MOE_OK;
   const int grid = a.c[0].n_blocks + a.c[1].n_blocks;
   static bool attr_set = false;
   if (!attr_set) {
-    for (const void *f : {(const void *)k_prefill_nib<true>, (const void *)k_prefill_nib<false>,
-                          (const void *)k_prefill_int4<true>, (const void *)k_prefill_int4<false>})
+    for (const void *f : {(const void *)k_prefill_nib<true, Q4K>, (const void *)k_prefill_nib<false, Q4K>})
       if (int rc = moe_check_hip(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, PN_LDS),
-                                 "hipFuncSetAttribute(k_prefill_nib, k_prefill_int4)"))
+                                 "hipFuncSetAttribute(k_prefill_nib)"))
         return rc;
     attr_set = true;
   }
   moe_ktimer_begin(swiglu ? MOE_K_PREFILL_W13 : MOE_K_PREFILL_W2, s);
-  if (q4k && swiglu) hipLaunchKernelGGL(k_prefill_nib<true>, dim3(grid), dim3(256), PN_LDS, s, a);
-  else if (q4k) hipLaunchKernelGGL(k_prefill_nib<false>, dim3(grid), dim3(256), PN_LDS, s, a);
-  else if (swiglu) hipLaunchKernelGGL(k_prefill_int4<true>, dim3(grid), dim3(256), PN_LDS, s, a);
-  else hipLaunchKernelGGL(k_prefill_int4<false>, dim3(grid), dim3(256), PN_LDS, s, a);
+  if (swiglu) hipLaunchKernelGGL((k_prefill_nib<true, Q4K>), dim3(grid), dim3(256), PN_LDS, s, a);
+  else hipLaunchKernelGGL((k_prefill_nib<false, Q4K>), dim3(grid), dim3(256), PN_LDS, s, a);
   moe_ktimer_end(swiglu ? MOE_K_PREFILL_W13 : MOE_K_PREFILL_W2, s);
-  return moe_check_launch(q4k ? "k_prefill_nib" : "k_prefill_int4");
+  return moe_check_launch("k_prefill_nib");
 }
 
 static int pf_launch(bool swiglu, const PfArgs &a, hipStream_t s) {
@@ -703,7 +727,7 @@ static int pf_launch(bool swiglu, const PfArgs &a, hipStream_t s) {
 // dispatch result, so the host never needs the counts: the launch covers the upper bound on the number of blocks, and
 // blocks past the real count find nothing to do.  The routed list is in order of tile height, the tallest first (four
 // classes; expert order inside a class), so that no long workgroup starts when the launch is nearly over.
-// Nibble formats: the same launch converts x for the w13 pass (q4_K to fp16, int4 to records) (8 MB read and written for 2048 x 2048, hidden
+// Nibble formats: the same launch converts x to fp16 for the w13 pass (8 MB read and written for 2048 x 2048, hidden
 // behind the 4 us that the list takes).  One more workgroup takes the unit list to the host: two copies and an event
 // behind the routing stood in the stream for 9 us a layer.
 static __device__ __forceinline__ PfTile pf_make_tile(unsigned long long w_base, int row0, int rows, int i, int n) {
@@ -712,22 +736,21 @@ static __device__ __forceinline__ PfTile pf_make_tile(unsigned long long w_base,
   t.w_base = w_base; t.row0 = row0; t.rows_group = rows | (min(PF_GROUP, n - g0) << 16) | ((i - g0) << 24);
   return t;
 }
-struct PfList { PfTile *tiles, *sh_tiles; int n_tiles_max, n_sh_tiles, cap, cap_s; };   // cap: rows per tile
-struct PfLists { PfList l[2]; };
 __global__ __launch_bounds__(1024) void k_prefill_tiles(const moe_unit *__restrict__ units, int max_units,
-                                                        const unsigned long long *__restrict__ expert_ptr, const PfLists lists,
-                                                        unsigned long long shared_base, int T,
+                                                        const unsigned long long *__restrict__ expert_ptr,
+                                                        PfTile *__restrict__ tiles, int n_tiles_max,
+                                                        PfTile *__restrict__ sh_tiles, int n_sh_tiles,
+                                                        PfTile *__restrict__ sh_tiles2, int n_sh_tiles2,
+                                                        unsigned long long shared_base, int T, int cap, int cap_s, int cap_s2,
                                                         int *__restrict__ n_real, int *__restrict__ err,
-                                                        const u32x4_t *__restrict__ x, u32x4_t *__restrict__ x16, int n16, int conv_threads, int K6,
+                                                        const u32x4_t *__restrict__ x, u32x4_t *__restrict__ x16, int n16,
                                                         const moe_publish pub) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int conv0 = pub.units_host ? 3 : 2;
-  if (blockIdx.x > 1) {  // workgroups behind the first two: the unit list to the host, the copy of the activations
+  const int conv0 = pub.units_host ? 2 : 1;
+  if (blockIdx.x > 0) {  // workgroups behind the first: the unit list to the host, the fp16 copy of the activations
     if ((int)blockIdx.x < conv0) { publish_units(pub, units, tid, 1024); return; }
-    if (tid >= conv_threads) return;
-    const int i = ((int)blockIdx.x - conv0) * conv_threads + tid;
-    if (K6) p6_convert_x(x, (unsigned char *)x16, K6, T, i);   // 32 values per thread
-    else if (i < n16) {                                          // 8
+    const int i = ((int)blockIdx.x - conv0) * 1024 + tid;   // (8 values per thread)
+    if (i < n16) {
       const u32x4_t v = x[i];
       x16[i] = u32x4_t{bf16x2_to_f16x2(v.x), bf16x2_to_f16x2(v.y), bf16x2_to_f16x2(v.z), bf16x2_to_f16x2(v.w)};
     }
@@ -735,12 +758,11 @@ __global__ __launch_bounds__(1024) void k_prefill_tiles(const moe_unit *__restri
   }
   __shared__ int total[4];
   __shared__ unsigned long long wsum[16];
-  const PfList &l = lists.l[blockIdx.x];   // the w13 pass's list, the w2 pass's
-  PfTile *const tiles = l.tiles;
-  const int cap = l.cap, n_tiles_max = l.n_tiles_max;
   if (tid < 4) total[tid] = 0;
-  for (int i = tid; i < l.n_sh_tiles; i += 1024)
-    l.sh_tiles[i] = pf_make_tile(shared_base, i * l.cap_s, min(l.cap_s, T - i * l.cap_s), i, l.n_sh_tiles);
+  for (int i = tid; i < n_sh_tiles; i += 1024)
+    sh_tiles[i] = pf_make_tile(shared_base, i * cap_s, min(cap_s, T - i * cap_s), i, n_sh_tiles);
+  for (int i = tid; i < n_sh_tiles2; i += 1024)
+    sh_tiles2[i] = pf_make_tile(shared_base, i * cap_s2, min(cap_s2, T - i * cap_s2), i, n_sh_tiles2);
   __syncthreads();
   // tiles of unit u: nt of up to `per` rows (a multiple of 32); class 0 = the tallest quarter
   int m = 0, row0 = 0, nt = 0, per = 0, cls = 0;
@@ -752,7 +774,7 @@ __global__ __launch_bounds__(1024) void k_prefill_tiles(const moe_unit *__restri
       if (un.m > 0 && un.expert >= 0) {
         wb = expert_ptr[un.expert];
         if (wb) { m = un.m; row0 = un.row0; }
-        else if (report && blockIdx.x == 0) moe_raise_err(err);
+        else if (report) moe_raise_err(err);
       }
     }
     nt = (m + cap - 1) / cap;
@@ -807,17 +829,17 @@ __global__ __launch_bounds__(1024) void k_prefill_tiles(const moe_unit *__restri
       __syncthreads();
     }
   }
-  if (tid == 0) { n_real[2 * blockIdx.x] = min(n_all, n_tiles_max); n_real[2 * blockIdx.x + 1] = l.n_sh_tiles; }
+  if (tid == 0) { n_real[0] = min(n_all, n_tiles_max); n_real[1] = n_sh_tiles; n_real[2] = n_sh_tiles2; }
 }
 
 extern "C" int moe_prefill_tile_rows(void) { return PF_BM; }
 
 extern "C" int64_t moe_prefill_workspace_bytes(int T, int k, int max_units) {
   const int64_t P = (int64_t)T * k;
-  return 2 * (P / 64 + max_units + (T + 63) / 64 + 2) * (int64_t)sizeof(PfTile);  // two lists; covers every tile height in use (>= 64)
+  return (P / 128 + max_units + 2 * ((T + 127) / 128) + 3) * (int64_t)sizeof(PfTile);  // covers every tile height in use (>= 128)
 }
 
-// where the copy of the activations stands in a workspace with room for it (phase bit 2)
+// where the fp16 copy of the activations stands in a workspace with room for it (phase bit 2)
 static int64_t pf_x16_offset(int T, int k, int max_units) {
   return (moe_prefill_workspace_bytes(T, k, max_units) + 255) & ~(int64_t)255;
 }
@@ -894,7 +916,7 @@ extern "C" int moe_experts_prefill_publish(const void *x_bf16, int T, int H, int
     return MOE_EINVAL;
   }
   const bool q4k = fmt == MOE_FMT_Q4K;
-  const bool int4 = fmt == MOE_FMT_INT4_G128 || q4k;  // nibble tiles
+  const bool int4 = fmt == MOE_FMT_INT4_G128 || q4k;  // nibble tiles + fp16 operands
   if (q4k && (H % 256 || I % 256 || (shared_ptr && I_sh % 256))) {
     moe_set_error("moe_experts_prefill: q4_K experts need H, I multiples of 256 (H=%d I=%d I_sh=%d)", H, I, I_sh);
     return MOE_EINVAL;
@@ -921,49 +943,29 @@ extern "C" int moe_experts_prefill_publish(const void *x_bf16, int T, int H, int
     return moe_decode_bf16(x_bf16, T, H, I, I_sh, units, max_units, sorted_tok, expert_ptr, shared_ptr, h_r, h_s, part_r, part_s,
                            shared_pieces, err, phases, pub, s);
   const long long P = (long long)T * k;
-  // int4: tiles of up to 64 instead of 128 rows in a launch whose workgroups then still are on the chip all at once (two per compute
-  // unit; half a tile per unit is what splitting its rows evenly leaves), and in the w2 pass, whose reduction is short, also up
-  // to 72 rows per unit.  us, 128 / 64 rows:
-  //   w13  DeepSeek shape 100 tokens 39.4 / 31.7 (495 workgroups of 64 rows), 150 tokens 42.8 / 46.3 (572), 379 tokens 56 / 60; Mixtral
-  //        shape 200 tokens 139 / 139, 300 tokens 175 / 212; 16 experts of 1024 x 512, 256 tokens 25.1 / 19.3, 4096 tokens 43 / 47
-  //   w2   DeepSeek shape 150 tokens 44 / 34, 379 tokens 47 / 37, 700 tokens (66 rows per expert) 52 / 46, 1000 tokens (94) 59 / 63;
-  //        Mixtral shape 300 tokens 140 / 130, 800 tokens 199 / 185 (464 workgroups), 1024 tokens 227 / 289 (576)
-  const int n_units = max_units < P ? max_units : (int)P;
-  auto short_tiles = [&](bool w2) {
-    if (fmt != MOE_FMT_INT4_G128 || P > 1 << 20) return false;   // (k_prefill_tiles counts tiles in 16 bits)
-    const long long cols = w2 ? H / (2 * PF_BNH) : I / PF_BNH, cols_s = shared_ptr ? (w2 ? H / (2 * PF_BNH) : I_sh / PF_BNH) : 0;
-    return (P / 64 + n_units / 2) * cols + (T + 63) / 64 * cols_s <= 512 || (w2 && P <= 72ll * n_units);
-  };
-  const int cap[2] = {short_tiles(false) ? 64 : int4 ? PN_BM : PF_BM, short_tiles(true) ? 64 : int4 ? PN_BM : PF_BM};
-  const int cap_s[2] = {short_tiles(false) ? 64 : int4 ? PN_BM : PF_BM_SHARED, short_tiles(true) ? 64 : PF_BM_SHARED_W2};
-  // copy of x for the nibble formats (q4_K fp16, int4 records): behind the tile list where the caller left room, else stream-ordered memory
+  const int cap = int4 ? PN_BM : PF_BM, cap_s = int4 ? PN_BM : PF_BM_SHARED, cap_s2 = PF_BM_SHARED_W2;
+  // fp16 copy of x for the nibble formats: behind the tile list where the caller left room, else stream-ordered memory
   void *x16 = nullptr, *x16_own = nullptr;
   const bool convert = int4 && (phases & 1);
   if (convert) {
     if (phases & 4) x16 = (unsigned char *)tiles_ws + pf_x16_offset(T, k, max_units);
-    else if (int rc = moe_check_hip(hipMallocAsync(&x16_own, (size_t)T * H * 2, s), "hipMallocAsync(activations' copy)")) return rc;
+    else if (int rc = moe_check_hip(hipMallocAsync(&x16_own, (size_t)T * H * 2, s), "hipMallocAsync(fp16 activations)")) return rc;
     if (x16_own) x16 = x16_own;
   }
   struct FreeX16 {  // on every way out
     void *p; hipStream_t s;
     ~FreeX16() { if (p) (void)hipFreeAsync(p, s); }
   } free_x16{x16_own, s};
-  const int n16 = convert ? (int)((long long)T * H / (q4k ? 8 : 32)) : 0;   // threads of the conversion
-  int *n_real = (int *)tiles_ws;  // tiles in use: w13 routed, shared, w2 routed, shared
-  PfLists lists;
-  PfTile *next = (PfTile *)tiles_ws + 1;
-  for (int w2 = 0; w2 < 2; ++w2) {
-    PfList &l = lists.l[w2];
-    l.cap = cap[w2]; l.cap_s = cap_s[w2];
-    l.n_tiles_max = (int)(P / l.cap) + max_units;
-    l.n_sh_tiles = shared_ptr ? (T + l.cap_s - 1) / l.cap_s : 0;
-    l.tiles = next; l.sh_tiles = next + l.n_tiles_max;
-    next = l.sh_tiles + l.n_sh_tiles;
-  }
-  const int conv_threads = n16 > 256 * 512 ? 1024 : n16 > 256 * 256 ? 512 : 256;   // (up to a workgroup per compute unit)
-  hipLaunchKernelGGL(k_prefill_tiles, dim3(2 + (pub ? 1 : 0) + (n16 + conv_threads - 1) / conv_threads), dim3(1024), 0, s, units, max_units,
-                     (const unsigned long long *)expert_ptr, lists, (unsigned long long)(uintptr_t)shared_ptr, T, n_real, err,
-                     (const u32x4_t *)x_bf16, (u32x4_t *)x16, n16, conv_threads, q4k ? 0 : H, pub ? *pub : moe_publish{});
+  const int n16 = convert ? (int)((long long)T * H / 8) : 0;
+  const int n_r = (int)(P / cap) + max_units;
+  const int n_s = shared_ptr ? (T + cap_s - 1) / cap_s : 0;
+  const int n_s2 = shared_ptr ? (T + cap_s2 - 1) / cap_s2 : 0;
+  int *n_real = (int *)tiles_ws;  // [0] routed tiles in use, [1] shared tiles (w13 pass), [2] shared tiles (w2 pass)
+  PfTile *tiles = (PfTile *)tiles_ws + 1, *sh_tiles = tiles + n_r, *sh_tiles2 = sh_tiles + n_s;
+  hipLaunchKernelGGL(k_prefill_tiles, dim3(1 + (pub ? 1 : 0) + (n16 + 1023) / 1024), dim3(1024), 0, s, units, max_units,
+                     (const unsigned long long *)expert_ptr, tiles, n_r, sh_tiles, n_s, sh_tiles2, n_s2,
+                     (unsigned long long)(uintptr_t)shared_ptr, T, cap, cap_s, cap_s2, n_real, err, (const u32x4_t *)x_bf16,
+                     (u32x4_t *)x16, n16, pub ? *pub : moe_publish{});
   if (int rc = moe_check_launch("k_prefill_tiles")) return rc;
   for (int w2 = 0; w2 < 2; ++w2) {
     if (!(phases & (w2 ? 2 : 1))) continue;
@@ -975,10 +977,9 @@ extern "C" int moe_experts_prefill_publish(const void *x_bf16, int T, int H, int
       if (shared && !shared_ptr) continue;
       PfClass &c = a.c[n++];
       const int Ii = shared ? I_sh : I;
-      const PfList &l = lists.l[w2];
-      c.tiles = shared ? l.sh_tiles : l.tiles;
-      c.n_mtiles = shared ? l.n_sh_tiles : l.n_tiles_max;
-      c.n_tiles_real = n_real + 2 * w2 + shared;
+      c.tiles = shared ? (w2 ? sh_tiles2 : sh_tiles) : tiles;
+      c.n_mtiles = shared ? (w2 ? n_s2 : n_s) : n_r;
+      c.n_tiles_real = n_real + (shared ? (w2 ? 2 : 1) : 0);
       c.shared = shared;
       if (!w2) {  // w13 [2I, H]: gate rows 0..I-1, up rows I..2I-1
         c.act = (const uint16_t *)(int4 ? x16 : x_bf16); c.gather = shared ? nullptr : sorted_tok; c.act_stride = H;
@@ -996,20 +997,18 @@ extern "C" int moe_experts_prefill_publish(const void *x_bf16, int T, int H, int
         c.w_off = w2 ? lay.off2_q : lay.off13_q;
         c.off_s = w2 ? lay.off2_s : lay.off13_s;
         c.off_z = w2 ? lay.off2_z : lay.off13_z;
-        if (!q4k && c.off_z - c.off_s >= (1ll << 31) - (1ll << 24)) {  // (p6_tile: the zeros are addressed from the scales)
+        if (!q4k && c.off_z - c.off_s >= (1ll << 31) - (1ll << 24)) {  // (pn_tile: the zeros are addressed from the scales)
           moe_set_error("moe_experts_prefill: the scales of an expert of %d x %d take 2 GiB or more", H, Ii);
           return MOE_EINVAL;
         }
       }
       c.ksplit = (w2 && shared && int4) ? shared_pieces : 1;
-      c.act_rows = w2 && !shared ? (int)P : T;
-      c.out_rows = shared ? T : (int)P;
       c.split_stride = (long long)T * H;
       c.n_blocks = pf_padded(!int4, c.n_mtiles * c.n_ntiles * c.ksplit);
       c.slab_step = moe_bf16_slab_step(c.K / PF_BK);
       a.n_blocks_total += c.n_blocks;
     }
-    if (int rc = int4 ? pn_launch(!w2, q4k, a, s) : pf_launch(!w2, a, s)) return rc;
+    if (int rc = q4k ? pn_launch<true>(!w2, a, s) : (int4 ? pn_launch<false>(!w2, a, s) : pf_launch(!w2, a, s))) return rc;
   }
   return MOE_OK;
 }

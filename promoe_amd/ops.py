@@ -327,7 +327,7 @@ def experts_decode_q4k(x, d: Dispatch, expert_ptr: torch.Tensor, shared: torch.T
 
 
 def prefill_workspace_bytes(fmt: int, T: int, H: int, k: int, max_units: int) -> int:
-    """Workspace of experts_prefill: the tile list and, for the nibble formats, the converted copy of the activations."""
+    """Workspace of experts_prefill: the tile list and, for the nibble formats, the fp16 copy of the activations."""
     n = max(int(lib.moe_prefill_workspace_bytes(T, k, max_units)), 16)
     return n if fmt == L.FMT_BF16 else ((n + 255) & ~255) + T * H * 2
 
@@ -349,7 +349,7 @@ def experts_prefill(x, d: Dispatch, expert_ptr: torch.Tensor, shared: torch.Tens
             h_s = torch.empty(T, I_sh, dtype=torch.bfloat16, device=dev)
             part_s = torch.empty(int(lib.moe_prefill_shared_splits(fmt, T, H, I_sh)) * T, H, dtype=torch.float32, device=dev)
         err = torch.zeros(1, dtype=torch.int32, device=dev)
-        # (nibble formats: behind the tile list, room for the converted copy of the activations)
+        # (nibble formats: behind the tile list, room for the fp16 copy of the activations)
         tiles = torch.empty(prefill_workspace_bytes(fmt, T, H, k, d.max_units), dtype=torch.uint8, device=dev)
     if fmt != L.FMT_BF16 and tiles.numel() >= prefill_workspace_bytes(fmt, T, H, k, d.max_units):
         phases |= 4

@@ -356,7 +356,8 @@ int moe_experts_decode_q4k_publish(const void *x_bf16, int T, int H, int I, int 
  * sorted pair order; expert_ptr[e] == 0 for an active expert sets *err |= 1 and skips it).
  *   fmt       : MOE_FMT_BF16 (expert image = blocked w13 [2I,H] then blocked w2 [H,I]; bf16 MFMA),
  *               MOE_FMT_INT4_G128 or MOE_FMT_Q4K (nibble tiles dequantised in registers to fp16
- *               operands, activations converted to fp16 once per call; tiles of 128 rows)
+ *               operands, activations converted to fp16 once per call (x and h are infinite past 65504);
+ *               tiles of up to 128 rows)
  *   tiles_ws  : device workspace of moe_prefill_workspace_bytes(T, k, max_units) bytes; the
  *               list of row tiles per expert is built there by a kernel, so the host
  *               needs no copy of the dispatch counts.

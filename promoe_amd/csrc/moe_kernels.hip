@@ -2834,9 +2834,10 @@ __global__ __launch_bounds__(256, 2) void k_gemv_int4_mfma_kc(const GemvArgs a) 
 // ---------------------------------------------------------------------------
 // k5 combine
 // ---------------------------------------------------------------------------
-// Bound by the partial rows' bytes (6 TB/s at 2048 tokens).  KK: rows requested together, the smallest of 2, 4, 6, 8 that
-// takes a token's k: with eight for every k the requests past k repeat the last row, and Mixtral's 4096 tokens of two took 35 us, 30.5
-// with two (4 of 4: 15.0 -> 14.5 at 1999 tokens of 2048 columns, 6 of 6: 5.6 -> 5.35 at 379).
+// Bound by the partial rows' bytes (2048 tokens of six and a shared row, 2048 columns: 126 MB in 20.4 us, 6.2 TB/s).  KK: rows
+// requested together, the smallest of 2, 4, 6, 8 that takes a token's k: with eight for every k the requests past k repeat the last row.
+// Eight / KK, mean of a launch under the profiler: 4096 tokens of two, 4096 columns, 34.4 / 30.5 us; 1999 of four, 2048 columns, 15.3 / 15.1;
+// 379 of six 5.9 / 5.55; 2048 of six 20.4 / 20.4.
 template <int KK>
 __global__ __launch_bounds__(256) void k_combine(const float *__restrict__ part_r,
                                                   const float *__restrict__ part_s,

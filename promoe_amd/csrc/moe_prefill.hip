@@ -383,16 +383,21 @@ __global__ __launch_bounds__(256, 1) void k_prefill_gemm(const PfArgs a) {
 //     products of step j, in pieces of one pair (order pinned by sched_barrier);
 //   * two workgroups per compute unit cover each other's barriers, prologues and epilogues.
 // h rows leave the w13 pass as fp16, so that the w2 pass brings them into LDS as they are.
-// Measured (one box, w13 / w2 launch; in brackets the kernel before: eight waves, the weights of a tile dequantised
-// by two of them each, activations converted and nibbles loaded through registers one group ahead): DeepSeek shape
-// 2048 tokens 215 / 121 us (305 / 167), 379 tokens 76 / 49 (115 / 65), Mixtral shape 4096 tokens 1733 / 991 (2132 /
-// 1038), Qwen2-57B shape q4_K 512 tokens 408 / 219 (577 / 303); with the block order of pf_block_of 194 / 109, 62 / 43,
-// 1622 / 893 and 320 / 187.
+// Measured (mean of a launch under the profiler, w13 / w2, whole layers one after the other; outside it 5 to 8 % less): DeepSeek
+// shape 2048 tokens 221 / 124 us, 379 tokens 65 / 46, Mixtral shape 4096 tokens 1672 / 907, Qwen2-57B shape q4_K 512 tokens 399 /
+// 222.  The kernel before (eight waves, the weights of a tile dequantised by two of them each, activations converted and
+// nibbles loaded through registers one group ahead; its blocks dealt in contiguous ranges) against this one with the same
+// ranges: 305 / 167 and 215 / 121, 115 / 65 and 76 / 49, 2132 / 1038 and 1733 / 991, 577 / 303 and 408 / 219.
 // What bounds it: on the Mixtral shape the power limit (matrix cores busy 78 % and 69 % of the cycles of the two launches,
 // which run at 1.46 and 1.51 GHz); on the others partly (DeepSeek shape, 2048 tokens: 59 % and 50 % at 1.70 and 1.81 GHz;
 // Qwen2-57B shape, 512 tokens: 61 % and 49 % at 1.65 and 1.78 GHz), with 0.8 to 0.9 vector cycles of dequantisation per
 // matrix cycle.  Tiles of 256 rows with one workgroup per compute unit halve the dequantisation per product and lose 8 to
-// 15 % on all but the Mixtral shape (+1 %).
+// 15 % on all but the Mixtral shape (+1 %).  q4_K tiles of 64 rows: the Qwen2-57B shape takes 635 instead of 553 us a layer at 512
+// tokens and 226 instead of 220 at 65.
+// int4 on the scaled 6- and 8-bit matrix formats (a nibble is an fp6 number as it is; x and h split into two pieces) takes 0.83 to
+// 0.88 of a layer's time, but holds fewer bits of x and h than fp16: with weights that fp16 holds exactly the partial rows are off by
+// 1.0e-3 in norm against 64 bits, 2.0e-4 here, and single elements of h by up to 2^-8 of themselves, 2^-11 here.  More pieces do
+// not help: three 6-bit pieces of h are 18 bits a value where the rows have 16, two 8-bit pieces of x take the fp16 products' time.
 typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
 
 #define PN_BM 128                         // most rows of one tile: 4 blocks of 32 (128 accumulator registers)

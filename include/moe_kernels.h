@@ -399,6 +399,16 @@ int moe_experts_prefill_publish(const void *x_bf16, int T, int H, int I, int I_s
                                 float *part_r, float *part_s, int shared_pieces, void *tiles_ws, int *err,
                                 int phases, const moe_publish *pub, void *stream);
 
+/* The same with the routed experts' partial rows of the w2 pass in routed_pieces pieces as well (1 to 8, nibble formats): part_r
+ * holds routed_pieces * T * k rows, piece s at part_r + s*T*k*H, each the product over one window of the I columns (whole
+ * 64-column slabs, at least two); moe_combine_windows adds them.  moe_prefill_routed_windows = the number of pieces worth taking. */
+int moe_prefill_routed_windows(int fmt, int T, int k, int E, int H, int I);
+int moe_experts_prefill_windows(const void *x_bf16, int T, int H, int I, int I_sh, int k, int fmt,
+                                const moe_unit *units, int max_units, const int *sorted_tok,
+                                const uint64_t *expert_ptr, const void *shared_ptr, void *h_r, void *h_s,
+                                float *part_r, float *part_s, int shared_pieces, int routed_pieces, void *tiles_ws,
+                                int *err, int phases, const moe_publish *pub, void *stream);
+
 /* k5: y[t,:] = sum_j w[t,j] * part_r[pos_of_pair[t*k+j],:] + g_t * part_s[t,:], bf16 out.
  * g_t = sigmoid(shared_gate_logit[t*sg_stride]) when shared_gate_logit != NULL, else 1;
  * part_s may be NULL (no shared expert). */
@@ -410,6 +420,12 @@ int moe_combine(const float *part_r, const float *part_s, const float *topk_w,
 int moe_combine_splits(const float *part_r, const float *part_s, const float *topk_w,
                        const int *pos_of_pair, const float *shared_gate_logit, int sg_stride, void *y_bf16,
                        int T, int H, int k, int n_shared_splits, void *stream);
+
+/* the same with the routed experts' partial rows in n_routed_splits pieces (piece s at part_r + s*T*k*H), added in piece
+ * order before the routing weight is applied */
+int moe_combine_windows(const float *part_r, const float *part_s, const float *topk_w,
+                        const int *pos_of_pair, const float *shared_gate_logit, int sg_stride, void *y_bf16,
+                        int T, int H, int k, int n_routed_splits, int n_shared_splits, void *stream);
 
 /* Per-kernel timing with HIP events recorded on the launch stream around every kernel
  * the launchers below start (no reference counterpart; used by the benchmark to report

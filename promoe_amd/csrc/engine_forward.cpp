@@ -12,11 +12,17 @@
 
 #include "engine_internal.h"
 
+// (weak: host-only builds of the engine, over stand-ins for the kernels, may lack them; called where a plan says so only)
+extern "C" {
+extern __attribute__((weak)) decltype(moe_experts_prefill_windows) moe_experts_prefill_windows;
+extern __attribute__((weak)) decltype(moe_combine_windows) moe_combine_windows;
+}
+
 struct LayerState {
   int max_tokens = 0, max_k = 0, max_units = 0;
   int E = 0, H = 0, I = 0, I_sh = 0;
   float *logits = nullptr, *topk_w = nullptr, *part_r = nullptr, *part_s = nullptr;
-  size_t part_s_elems = 0;  // floats behind part_s
+  size_t part_r_elems = 0, part_s_elems = 0;  // floats behind part_r and part_s
   int *idx = nullptr, *counts = nullptr, *offsets = nullptr, *sorted_pair = nullptr, *pos_of_pair = nullptr,
       *sorted_tok = nullptr, *n_active = nullptr;
   unsigned char *unit_ws = nullptr;  // resolved units of the one-token path (16 bytes each)
@@ -179,7 +185,14 @@ extern "C" int moe_forward_prepare(moe_engine *eng, int max_tokens) {
   rc |= dalloc(s, &s->active_ids, s->max_units);
   rc |= dalloc(s, (uint16_t **)&s->h_r, P * I);
   rc |= dalloc(s, (uint16_t **)&s->h_s, (size_t)T * I_sh);
-  rc |= dalloc(s, &s->part_r, P * H);
+  // a prefill batch of a nibble format over few wide experts may leave the routed experts' partial rows in pieces (pieces x
+  // pairs rows, largest over the batch sizes the workspace admits)
+  size_t rows_r = P;
+  for (auto &d : eng->layer_desc)
+    for (int t = 65; d.gate_w && t <= T; ++t)
+      rows_r = std::max(rows_r, (size_t)t * d.top_k * (size_t)moe_prefill_routed_windows(d.fmt, t, d.top_k, E, d.H, d.I));
+  s->part_r_elems = rows_r * H;
+  rc |= dalloc(s, &s->part_r, s->part_r_elems);
   // q4_K decode batches (at most 64 tokens) may leave the shared expert's partial rows in up to 8 pieces, and so
   // may a prefill batch of a nibble format whose shared expert is wide (pieces x tokens rows, largest over the
   // batch sizes the workspace admits)
@@ -282,17 +295,25 @@ static bool use_prefill(const moe_layer_desc &d, int T) {
 }
 
 static int shared_pieces(const moe_layer_desc &d, int T, const LayerState *s);
+static int routed_pieces(const moe_layer_desc &d, int T, const LayerState *s);
 // pub / pub_seq: the pending slot whose pinned unit list a launch fills (launch_publishes), or null
 static int run_units(moe_engine *eng, const moe_layer_desc &d, LayerState *s, const void *x, int T,
                      const moe_unit *units_dev, const moe_unit *units_host, int n_units, bool with_shared,
                      int layer, const uint64_t *table, hipStream_t st, LayerState::Pending *pub = nullptr,
                      int pub_seq = 0) {
   const moe_publish out = pub ? moe_publish{s->n_active, pub->units, pub->n_active, pub->seq, pub_seq, n_units} : moe_publish{};
-  if (use_prefill(d, T))
-    return moe_experts_prefill_publish(x, T, d.H, d.I, with_shared ? d.I_sh : 0, d.top_k, d.fmt, units_dev, n_units,
-                                       s->sorted_tok, table, with_shared ? d.shared : nullptr, s->h_r, s->h_s, s->part_r,
-                                       s->part_s, with_shared ? shared_pieces(d, T, s) : 1, s->tiles_ws,
-                                       s->err_host + layer, d.fmt == MOE_FMT_BF16 ? 3 : 7, pub ? &out : nullptr, st);
+  if (use_prefill(d, T)) {
+    const int rp = routed_pieces(d, T, s), sp = with_shared ? shared_pieces(d, T, s) : 1, phases = d.fmt == MOE_FMT_BF16 ? 3 : 7;
+    const int I_sh = with_shared ? d.I_sh : 0;
+    const void *shared = with_shared ? d.shared : nullptr;
+    if (rp > 1)
+      return moe_experts_prefill_windows(x, T, d.H, d.I, I_sh, d.top_k, d.fmt, units_dev, n_units, s->sorted_tok, table, shared,
+                                         s->h_r, s->h_s, s->part_r, s->part_s, sp, rp, s->tiles_ws, s->err_host + layer, phases,
+                                         pub ? &out : nullptr, st);
+    return moe_experts_prefill_publish(x, T, d.H, d.I, I_sh, d.top_k, d.fmt, units_dev, n_units, s->sorted_tok, table, shared,
+                                       s->h_r, s->h_s, s->part_r, s->part_s, sp, s->tiles_ws, s->err_host + layer, phases,
+                                       pub ? &out : nullptr, st);
+  }
   if (d.fmt == MOE_FMT_Q4K)
     return moe_experts_decode_q4k_publish(x, T, d.H, d.I, with_shared ? d.I_sh : 0, d.top_k, units_dev, n_units,
                                           s->sorted_tok, table, with_shared ? d.shared : nullptr, s->h_r, s->h_s,
@@ -321,6 +342,21 @@ static int shared_pieces(const moe_layer_desc &d, int T, const LayerState *s) {
     return (size_t)sp * T * d.H <= s->part_s_elems ? sp : 1;
   }
   return d.fmt == MOE_FMT_Q4K ? moe_decode_shared_splits(MOE_FMT_Q4K, T, d.H, d.I_sh) : 1;
+}
+
+// and the routed experts' partial rows
+static int routed_pieces(const moe_layer_desc &d, int T, const LayerState *s) {
+  if (!use_prefill(d, T)) return 1;
+  const int rp = moe_prefill_routed_windows(d.fmt, T, d.top_k, s->E, d.H, d.I);
+  return (size_t)rp * T * d.top_k * d.H <= s->part_r_elems ? rp : 1;
+}
+
+// the combine behind run_units
+static int combine_pieces(const moe_layer_desc &d, const LayerState *s, const float *sg, int ldl, void *y, int T, hipStream_t st) {
+  const float *part_s = d.I_sh > 0 ? s->part_s : nullptr;
+  const int rp = routed_pieces(d, T, s), sp = shared_pieces(d, T, s);
+  if (rp > 1) return moe_combine_windows(s->part_r, part_s, s->topk_w, s->pos_of_pair, sg, ldl, y, T, d.H, d.top_k, rp, sp, st);
+  return moe_combine_splits(s->part_r, part_s, s->topk_w, s->pos_of_pair, sg, ldl, y, T, d.H, d.top_k, sp, st);
 }
 
 // what the one-token w2 + combine kernel asks of a layer (its waves stage what they need themselves, so the
@@ -811,9 +847,7 @@ extern "C" int moe_forward(moe_engine *eng, int layer, const void *x, int T, voi
     s->pend_head = (s->pend_head + 1) % LayerState::kPending;
     p.layer = layer; p.max_units = max_units; p.busy = true; p.by_seq = by_seq; p.seq_expected = tail_seq;
     const float *sg0 = d.shared_gated ? s->logits + E : nullptr;
-    if ((rc = moe_combine_splits(s->part_r, d.I_sh > 0 ? s->part_s : nullptr, s->topk_w, s->pos_of_pair, sg0, ldl, y, T, d.H, k,
-                                 shared_pieces(d, T, s), st)))
-      return rc;
+    if ((rc = combine_pieces(d, s, sg0, ldl, y, T, st))) return rc;
     if (layer + 1 == eng->cfg.num_layer && (rc = moe_report_layer_logits(eng, layer + 1, y, 1, T, d.H))) return rc;
     return moe_layer_done(eng, layer);
   }
@@ -890,9 +924,7 @@ extern "C" int moe_forward(moe_engine *eng, int layer, const void *x, int T, voi
     if ((rc = moe_expert_launched(eng, layer, (int)id))) return rc;
   }
   const float *sg = d.shared_gated ? s->logits + E : nullptr;
-  if ((rc = moe_combine_splits(s->part_r, d.I_sh > 0 ? s->part_s : nullptr, s->topk_w, s->pos_of_pair, sg, ldl, y, T, d.H, k,
-                               shared_pieces(d, T, s), st)))
-    return rc;
+  if ((rc = combine_pieces(d, s, sg, ldl, y, T, st))) return rc;
   // MoeLayerHook.post_forward (utils/hooks.py:220-223)
   if (layer + 1 == eng->cfg.num_layer && (rc = moe_report_layer_logits(eng, layer + 1, y, 1, T, d.H))) return rc;
   return moe_layer_done(eng, layer);

@@ -85,3 +85,20 @@ extern "C" int moe_kernel_timing_read(int kernel_id, double *total_ms, int *call
   *calls = n;
   return MOE_OK;
 }
+
+// Pieces the w2 pass leaves the routed experts' partial rows in (moe_experts_prefill_windows).  A few wide experts have few
+// tiles of a long reduction (Mixtral shape, 256 tokens: 128 workgroups over 224 slabs, half the chip idle for 190 us; 2048
+// tokens: 592 workgroups for 512 places, 80 of them in a second round of 290 us).  Windows of at least 32 slabs, until the
+// launch has about three workgroups per compute unit (an expert has at least one tile, and one more per 128 rows); the rows
+// of more pieces cost the launch and the combine more than the last round has left.  us a layer, 1 / 2 / 4 / 8 pieces, Mixtral
+// shape: 128 tokens 272 / 230 / 224 / 230, 379 tokens 382 / 333 / 328 / 343, 512 470 / 453 / 446 / 456, 1024 777 / 744 / 744 / 778,
+// 2048 1454 / 1427 / 1431 / 1504, 4096 2589 / 2569 / 2627 / 2778.  Short reductions lose: DeepSeek shape (22 slabs) 128 tokens 91.1 /
+// 93.8, 2048 367 / 392; Qwen2-57B shape (40 slabs) 128 tokens 312 / 312 / 322, 512 610 / 620 / 663.
+extern "C" int moe_prefill_routed_windows(int fmt, int T, int k, int E, int H, int I) {
+  if ((fmt != MOE_FMT_INT4_G128 && fmt != MOE_FMT_Q4K) || T <= 0 || k <= 0 || E <= 0 || H <= 0 || I <= 0) return 1;
+  const long long P = (long long)T * k, wgs = ((P < E ? P : E) + P / 128) * (H / 256);
+  const int nk = I / 64;
+  int s = 1;
+  while (s < 4 && wgs * s < 768 && nk % (s * 2) == 0 && nk / (s * 2) >= 32) s *= 2;
+  return s;
+}

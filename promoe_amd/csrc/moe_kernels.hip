@@ -2845,7 +2845,7 @@ __global__ __launch_bounds__(256) void k_combine(const float *__restrict__ part_
                                                   const int *__restrict__ pos_of_pair,
                                                   const float *__restrict__ sg_logit,
                                                   int sg_stride, uint16_t *__restrict__ y, int H,
-                                                  int k, int n_sh_splits) {
+                                                  int k, int n_r_splits, int n_sh_splits) {
   const int t = blockIdx.y;
   const int n = (blockIdx.x * 256 + threadIdx.x) * 4;
   if (n >= H) return;
@@ -2864,6 +2864,15 @@ __global__ __launch_bounds__(256) void k_combine(const float *__restrict__ part_
     }
 #pragma unroll
     for (int j = 0; j < KK; ++j) v[j] = *(const float4 *)(part_r + (size_t)pos[j] * H + n);
+    // routed experts whose reduction was split over workgroups: their pieces, added in split order
+    for (int sp = 1; sp < n_r_splits; ++sp) {
+      const float *ps = part_r + (size_t)sp * gridDim.y * k * H + n;
+      float4 u[KK];
+#pragma unroll
+      for (int j = 0; j < KK; ++j) u[j] = *(const float4 *)(ps + (size_t)pos[j] * H);
+#pragma unroll
+      for (int j = 0; j < KK; ++j) { v[j].x += u[j].x; v[j].y += u[j].y; v[j].z += u[j].z; v[j].w += u[j].w; }
+    }
 #pragma unroll
     for (int j = 0; j < KK; ++j)
       if (j0 + j < k) {
@@ -4068,16 +4077,22 @@ extern "C" int moe_gate_topk_dispatch(const void *x, const void *wg, const float
 extern "C" int moe_combine_splits(const float *part_r, const float *part_s, const float *topk_w,
                                   const int *pos_of_pair, const float *sg_logit, int sg_stride, void *y,
                                   int T, int H, int k, int n_shared_splits, void *stream) {
+  return moe_combine_windows(part_r, part_s, topk_w, pos_of_pair, sg_logit, sg_stride, y, T, H, k, 1, n_shared_splits, stream);
+}
+
+extern "C" int moe_combine_windows(const float *part_r, const float *part_s, const float *topk_w,
+                                   const int *pos_of_pair, const float *sg_logit, int sg_stride, void *y,
+                                   int T, int H, int k, int n_routed_splits, int n_shared_splits, void *stream) {
   if (!y || T < 0 || H <= 0 || H % 4 || k < 0 || (k > 0 && (!part_r || !topk_w || !pos_of_pair)) ||
-      T > 65535 || n_shared_splits < 1 || n_shared_splits > 8) {
-    moe_set_error("moe_combine: bad argument (T=%d H=%d k=%d splits=%d)", T, H, k, n_shared_splits);
+      T > 65535 || n_routed_splits < 1 || n_routed_splits > 8 || n_shared_splits < 1 || n_shared_splits > 8) {
+    moe_set_error("moe_combine: bad argument (T=%d H=%d k=%d splits=%d, %d)", T, H, k, n_routed_splits, n_shared_splits);
     return MOE_EINVAL;
   }
   if (T == 0) return MOE_OK;
   dim3 grid((H / 4 + 255) / 256, T);
   moe_ktimer_begin(MOE_K_COMBINE, (hipStream_t)stream);
 #define COMB_LAUNCH(KK_) hipLaunchKernelGGL(k_combine<KK_>, grid, dim3(256), 0, (hipStream_t)stream, part_r, part_s, topk_w, \
-                                            pos_of_pair, sg_logit, sg_stride, (uint16_t *)y, H, k, n_shared_splits)
+                                            pos_of_pair, sg_logit, sg_stride, (uint16_t *)y, H, k, n_routed_splits, n_shared_splits)
   if (k <= 2) COMB_LAUNCH(2);
   else if (k <= 4) COMB_LAUNCH(4);
   else if (k <= 6) COMB_LAUNCH(6);

@@ -50,8 +50,8 @@ struct PfClass {
   int shared;           // the shared expert's class
   int slab_step;        // storage rotation per 128-row group: smallest odd s >= 3 coprime with K/64
   int n_blocks;         // n_mtiles * n_ntiles * ksplit, padded (pf_padded)
-  int ksplit;           // int4 / q4_K w2 pass of the shared expert: workgroups per tile, each over 1/ksplit of the
-                        // reduction, partial rows to out + split * split_stride (0 or 1: the whole reduction)
+  int ksplit;           // int4 / q4_K w2 pass: workgroups per tile, each over 1/ksplit of the reduction, partial rows
+                        // to out + split * split_stride (0 or 1: the whole reduction)
   long long split_stride;  // elements between the pieces of out
 };
 struct PfArgs {
@@ -442,7 +442,7 @@ struct PnSrc {
   int s_step;               // int4: what s_voff advances by per quantisation group (scales and zeros differ)
 };
 
-// acc[i][f]: row block i, fragment (column half) f; slabs kt0 .. kt0 + nk - 1 (64 k each), nk >= 2 and even
+// acc[i][f]: row block i, fragment (column half) f; slabs kt0 .. kt0 + nk - 1 (64 k each), nk >= 2
 template <int NB, bool Q4K>
 static __device__ __forceinline__ void pn_mainloop(f32x16_t (&acc)[NB][2], const unsigned lds_base, const PnSrc &m, const int kt0,
                                                    const int nk, const int tid) {
@@ -884,11 +884,37 @@ extern "C" int moe_experts_prefill_pieces(const void *x_bf16, int T, int H, int 
                                      h_s, part_r, part_s, shared_pieces, tiles_ws, err, phases, nullptr, stream);
 }
 
+static int experts_prefill(bool windows, const void *x_bf16, int T, int H, int I, int I_sh, int k, int fmt,
+                           const moe_unit *units, int max_units, const int *sorted_tok,
+                           const uint64_t *expert_ptr, const void *shared_ptr, void *h_r, void *h_s,
+                           float *part_r, float *part_s, int shared_pieces, int routed_pieces,
+                           void *tiles_ws, int *err, int phases, const moe_publish *pub, void *stream);
+
 extern "C" int moe_experts_prefill_publish(const void *x_bf16, int T, int H, int I, int I_sh, int k, int fmt,
                                            const moe_unit *units, int max_units, const int *sorted_tok,
                                            const uint64_t *expert_ptr, const void *shared_ptr, void *h_r, void *h_s,
                                            float *part_r, float *part_s, int shared_pieces, void *tiles_ws, int *err,
                                            int phases, const moe_publish *pub, void *stream) {
+  return experts_prefill(false, x_bf16, T, H, I, I_sh, k, fmt, units, max_units, sorted_tok, expert_ptr, shared_ptr, h_r, h_s,
+                         part_r, part_s, shared_pieces, 1, tiles_ws, err, phases, pub, stream);
+}
+
+extern "C" int moe_experts_prefill_windows(const void *x_bf16, int T, int H, int I, int I_sh, int k, int fmt,
+                                           const moe_unit *units, int max_units, const int *sorted_tok,
+                                           const uint64_t *expert_ptr, const void *shared_ptr, void *h_r, void *h_s,
+                                           float *part_r, float *part_s, int shared_pieces, int routed_pieces,
+                                           void *tiles_ws, int *err, int phases, const moe_publish *pub, void *stream) {
+  return experts_prefill(true, x_bf16, T, H, I, I_sh, k, fmt, units, max_units, sorted_tok, expert_ptr, shared_ptr, h_r, h_s,
+                         part_r, part_s, shared_pieces, routed_pieces, tiles_ws, err, phases, pub, stream);
+}
+
+// windows: moe_experts_prefill_windows, whose pieces are windows of whole slabs; the older entries take the shared expert's
+// in pairs of quantisation groups and leave the routed experts' rows whole
+static int experts_prefill(bool windows, const void *x_bf16, int T, int H, int I, int I_sh, int k, int fmt,
+                           const moe_unit *units, int max_units, const int *sorted_tok,
+                           const uint64_t *expert_ptr, const void *shared_ptr, void *h_r, void *h_s,
+                           float *part_r, float *part_s, int shared_pieces, int routed_pieces,
+                           void *tiles_ws, int *err, int phases, const moe_publish *pub, void *stream) {
   hipStream_t s = (hipStream_t)stream;
   if (pub && (T <= 0 || max_units <= 0 || !(phases & 1) || !moe_publish_ok(pub, max_units))) {
     moe_set_error("moe_experts_prefill_publish: publishing needs tokens, units and the w13 phase (T=%d phases=%d)", T, phases);
@@ -906,14 +932,20 @@ extern "C" int moe_experts_prefill_publish(const void *x_bf16, int T, int H, int
       return MOE_EINVAL;
     }
   } else if (shared_pieces > 1 && (!shared_ptr || (fmt != MOE_FMT_INT4_G128 && fmt != MOE_FMT_Q4K) ||
-                            (I_sh / 128) % (shared_pieces * 2) != 0)) {
-    moe_set_error("moe_experts_prefill: %d pieces need an int4 / q4_K shared expert whose I_sh / 128 is a multiple of %d "
-                  "(I_sh=%d)", shared_pieces, shared_pieces * 2, I_sh);
+                                   (windows ? (I_sh / 64) % shared_pieces || I_sh / 64 / shared_pieces < 2
+                                            : (I_sh / 128) % (shared_pieces * 2) != 0))) {
+    moe_set_error("moe_experts_prefill: %d pieces need an int4 / q4_K shared expert whose I_sh / %d is a multiple of %d "
+                  "(I_sh=%d)", shared_pieces, windows ? 64 : 128, windows ? shared_pieces : shared_pieces * 2, I_sh);
     return MOE_EINVAL;
   }
   if (!x_bf16 || T < 0 || k <= 0 || max_units < 0 || !units || !sorted_tok || !expert_ptr || !tiles_ws || !err ||
       !h_r || !part_r || (shared_ptr && (!h_s || !part_s || I_sh <= 0))) {
     moe_set_error("moe_experts_prefill: NULL or negative argument");
+    return MOE_EINVAL;
+  }
+  if (routed_pieces < 1 || routed_pieces > 8 || (routed_pieces > 1 && (fmt == MOE_FMT_BF16 || I % 64 || (I / 64) % routed_pieces ||
+                                                                       I / 64 / routed_pieces < 2))) {
+    moe_set_error("moe_experts_prefill: %d windows of a reduction over %d columns of the routed experts (format %d)", routed_pieces, I, fmt);
     return MOE_EINVAL;
   }
   if (fmt != MOE_FMT_BF16 && fmt != MOE_FMT_INT4_G128 && fmt != MOE_FMT_Q4K) {
@@ -1007,8 +1039,8 @@ extern "C" int moe_experts_prefill_publish(const void *x_bf16, int T, int H, int
           return MOE_EINVAL;
         }
       }
-      c.ksplit = (w2 && shared && int4) ? shared_pieces : 1;
-      c.split_stride = (long long)T * H;
+      c.ksplit = (w2 && int4) ? (shared ? shared_pieces : routed_pieces) : 1;
+      c.split_stride = (shared ? (long long)T : P) * H;
       c.n_blocks = pf_padded(!int4, c.n_mtiles * c.n_ntiles * c.ksplit);
       c.slab_step = moe_bf16_slab_step(c.K / PF_BK);
       a.n_blocks_total += c.n_blocks;

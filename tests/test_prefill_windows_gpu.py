@@ -1,0 +1,100 @@
+"""The w2 pass of the nibble tile kernels with the reduction cut into windows, and the combine that adds the pieces."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import moe_oracle as O
+from tests.synth import Int4Layer, Q4KLayer
+
+pytestmark = pytest.mark.gpu
+
+
+def _passes(layer, fmt, T, k, dev, routed, shared):
+    """Partial rows of one batch, pieces apart: [routed, T k, H], [shared, T, H]."""
+    from promoe_amd import ops, _lib as L
+    H, I, I_sh, E = layer.H, layer.I, layer.I_sh, layer.E
+    x = torch.from_numpy(O.synth_acts(T, H, seed=3)).to(torch.bfloat16).to(dev)
+    idx = torch.from_numpy(np.stack([np.random.default_rng(t).permutation(E)[:k] for t in range(T)]).astype(np.int32)).to(dev)
+    d = ops.dispatch(idx, E)
+    slots = [torch.from_numpy(s).to(dev) for s in layer.slots]
+    table = torch.tensor([s.data_ptr() for s in slots], dtype=torch.int64, device=dev)
+    sh = torch.from_numpy(layer.shared_img).to(dev)
+    part_r = torch.full((routed, T * k, H), float("nan"), device=dev)
+    part_s = torch.full((shared, T, H), float("nan"), device=dev)
+    h_r = torch.empty(T * k, I, dtype=torch.float16, device=dev)
+    h_s = torch.empty(T, I_sh, dtype=torch.float16, device=dev)
+    err = torch.zeros(1, dtype=torch.int32, device=dev)
+    ws = torch.empty(ops.prefill_workspace_bytes(fmt, T, H, k, d.max_units), dtype=torch.uint8, device=dev)
+    p = L.ptr
+    L.check(L.lib.moe_experts_prefill_windows(p(x), T, H, I, I_sh, k, fmt, p(d.units), d.max_units, p(d.sorted_tok), p(table),
+                                              p(sh), p(h_r), p(h_s), p(part_r), p(part_s), shared, routed, p(ws), p(err), 3 | 4,
+                                              None, L.cur_stream()), "moe_experts_prefill_windows")
+    torch.cuda.synchronize()
+    assert int(err.item()) == 0
+    return part_r, part_s, d
+
+
+@pytest.mark.parametrize("cls,I,I_sh,T,routed,shared", [
+    (Int4Layer, 384, 640, 70, 3, 2),      # windows of two and five slabs: shorter than the ring, inside a quantisation group
+    (Int4Layer, 1408, 256, 129, 2, 1),     # eleven slabs; second tiles of few rows
+    (Int4Layer, 2048, 2816, 97, 8, 2),    # the most windows; the shared expert in two windows of eleven groups
+    (Q4KLayer, 768, 512, 65, 3, 1),       # windows of four slabs: whole super-blocks
+    (Q4KLayer, 512, 512, 200, 4, 2),      # windows of two slabs: half a super-block
+])
+def test_pieces_add_up_to_the_whole_rows(cuda, cls, I, I_sh, T, routed, shared):
+    from promoe_amd import _lib as L
+    print(f"case windows {cls.__name__} I={I} I_sh={I_sh} T={T} routed={routed} shared={shared}", flush=True)
+    H, k = 512, 2
+    layer = cls(H=H, I=I, E=5, I_sh=I_sh, seed=21)
+    fmt = L.FMT_Q4K if cls is Q4KLayer else L.FMT_INT4_G128
+    r1, s1, _ = _passes(layer, fmt, T, k, cuda, 1, 1)
+    rn, sn, d = _passes(layer, fmt, T, k, cuda, routed, shared)
+    # the same products, added in another order: fp32 sums of up to 2816 terms differ by some units of 2^-24 of their norm
+    for one, many in ((r1, rn), (s1, sn)):
+        assert torch.isfinite(many).all()
+        diff = (many.double().sum(0) - one[0].double()).norm() / one[0].double().norm()
+        assert diff <= 1e-5, float(diff)
+    # the combine: pieces in order, then weight and sum, as separate fp32 operations would give it
+    w = torch.rand(T, k, device=cuda)
+    y = torch.empty(T, H, dtype=torch.bfloat16, device=cuda)
+    p = L.ptr
+    L.check(L.lib.moe_combine_windows(p(rn), p(sn), p(w), p(d.pos_of_pair), None, 0, p(y), T, H, k, routed, shared,
+                                      L.cur_stream()), "moe_combine_windows")
+    rows = rn.double().sum(0)[d.pos_of_pair[: T * k].long()].view(T, k, H)
+    want = (rows * w.double()[:, :, None]).sum(1) + sn.double().sum(0)
+    # bf16 out: half a unit in the last place, and fp32 sums of a few terms
+    bound = 2.0 ** -8 * want.abs() + 1e-5 * ((rows.abs() * w.double()[:, :, None]).sum(1) + sn.double().abs().sum(0))
+    assert ((y.double() - want).abs() <= bound).all()
+
+
+def test_windows_that_do_not_divide_the_reduction_are_refused(cuda):
+    from promoe_amd import _lib as L
+    p = 4096                                     # never read
+    for fmt, I, routed in ((L.FMT_INT4_G128, 384, 4), (L.FMT_INT4_G128, 128, 2), (L.FMT_BF16, 512, 2), (L.FMT_INT4_G128, 1024, 9),
+                           (L.FMT_INT4_G128, 1024, 0)):
+        rc = L.lib.moe_experts_prefill_windows(p, 70, 256, I, 0, 2, fmt, p, 4, p, p, None, p, None, p, None, 1, routed, p, p, 3,
+                                               None, None)
+        assert rc != 0 and b"windows" in L.lib.moe_last_error(), (fmt, I, routed)
+
+
+@pytest.mark.parametrize("cache_rate", [1.0, 0.5])
+def test_layer_of_few_wide_experts(cuda, cache_rate):
+    """A layer whose routed reduction the engine cuts into windows, every expert resident and half of them."""
+    from promoe_amd import _lib as L
+    from tests.test_engine_gpu import build_engine, ref_forward
+    print(f"case wide experts cache_rate={cache_rate}", flush=True)
+    H, I, E, k = 256, 4096, 4, 2
+    assert L.lib.moe_prefill_routed_windows(L.FMT_INT4_G128, 70, k, E, H, I) == 2
+    assert L.lib.moe_prefill_routed_windows(L.FMT_INT4_G128, 256, 2, 8, 4096, 14336) == 4   # Mixtral shape
+    assert L.lib.moe_prefill_routed_windows(L.FMT_INT4_G128, 4096, 2, 8, 4096, 14336) == 1
+    assert L.lib.moe_prefill_routed_windows(L.FMT_INT4_G128, 128, 6, 64, 2048, 1408) == 1   # DeepSeek shape: 22 slabs
+    layer = Int4Layer(H=H, I=I, E=E, I_sh=256, seed=5)
+    pm = build_engine([layer], k, cuda, max_tokens=70, cache_rate=cache_rate, cache_policy="lru")
+    for T in (70, 65, 40, 70):
+        x = O.synth_acts(T, H, seed=T)
+        y = pm.forward(0, torch.from_numpy(x).to(torch.bfloat16).to(cuda))
+        torch.cuda.synchronize()
+        ref = ref_forward(layer, x, k, 0)
+        err = float(np.abs(y.float().cpu().numpy() - ref["out"]).max() / np.abs(ref["out"]).max())
+        assert err <= 2e-2, (T, err)
+    pm.close()

@@ -200,6 +200,7 @@ extern "C" int moe_forward_prepare(moe_engine *eng, int max_tokens) {
   for (int t = 1; t <= T; ++t) {
     rows_s = std::max(rows_s, (size_t)t * (size_t)moe_prefill_shared_splits(MOE_FMT_Q4K, t, H, I_sh));
     rows_s = std::max(rows_s, (size_t)t * (size_t)moe_prefill_shared_splits(MOE_FMT_BF16, t, H, I_sh));
+    rows_s = std::max(rows_s, (size_t)t * (size_t)moe_prefill_shared_windows(MOE_FMT_INT4_G128, t, H, I_sh));
     if (t <= 64) rows_s = std::max(rows_s, (size_t)t * (size_t)moe_decode_shared_splits(MOE_FMT_Q4K, t, H, I_sh));
   }
   rc |= dalloc(s, &s->part_s, rows_s * H);
@@ -306,7 +307,7 @@ static int run_units(moe_engine *eng, const moe_layer_desc &d, LayerState *s, co
     const int rp = routed_pieces(d, T, s), sp = with_shared ? shared_pieces(d, T, s) : 1, phases = d.fmt == MOE_FMT_BF16 ? 3 : 7;
     const int I_sh = with_shared ? d.I_sh : 0;
     const void *shared = with_shared ? d.shared : nullptr;
-    if (rp > 1)
+    if (d.fmt != MOE_FMT_BF16 && (rp > 1 || sp > 1))
       return moe_experts_prefill_windows(x, T, d.H, d.I, I_sh, d.top_k, d.fmt, units_dev, n_units, s->sorted_tok, table, shared,
                                          s->h_r, s->h_s, s->part_r, s->part_s, sp, rp, s->tiles_ws, s->err_host + layer, phases,
                                          pub ? &out : nullptr, st);
@@ -338,7 +339,7 @@ static int shared_pieces(const moe_layer_desc &d, int T, const LayerState *s) {
   if (d.I_sh <= 0) return 1;
   if (use_prefill(d, T)) {
     // (what the workspace was sized for; a layer narrower than the widest one could ask for more pieces than fit)
-    const int sp = moe_prefill_shared_splits(d.fmt, T, d.H, d.I_sh);
+    const int sp = moe_prefill_shared_windows(d.fmt, T, d.H, d.I_sh);
     return (size_t)sp * T * d.H <= s->part_s_elems ? sp : 1;
   }
   return d.fmt == MOE_FMT_Q4K ? moe_decode_shared_splits(MOE_FMT_Q4K, T, d.H, d.I_sh) : 1;

@@ -102,3 +102,16 @@ extern "C" int moe_prefill_routed_windows(int fmt, int T, int k, int E, int H, i
   while (s < 4 && wgs * s < 768 && nk % (s * 2) == 0 && nk / (s * 2) >= 32) s *= 2;
   return s;
 }
+
+// Pieces for the shared expert's partial rows of moe_experts_prefill_windows: those of moe_prefill_shared_splits, and two for an
+// int4 shared expert of 32 slabs and more in a launch of few of its tiles.  There its workgroups, each over a reduction twice as
+// long as the routed experts', are the last to end (DeepSeek shape, 128 tokens: 8 workgroups of 44 slabs, 36 us, beside 280 of
+// 22 slabs).  us a layer, one piece / two, DeepSeek shape: 65 tokens 85.9 / 73.4, 128 104.2 / 91.2, 200 115.7 / 103.0, 379 145.3 /
+// 133.3, 512 156.3 / 152.8; past 32 tiles the shared expert's workgroups start a full round and the pieces only cost the
+// combine: 1024 tokens 229.9 / 232.4, 2048 367.2 / 374.1.
+extern "C" int moe_prefill_shared_windows(int fmt, int T, int H, int I_sh) {
+  const int s = moe_prefill_shared_splits(fmt, T, H, I_sh);
+  if (s > 1 || fmt != MOE_FMT_INT4_G128 || T <= 0 || H <= 0 || I_sh <= 0) return s;
+  const int tiles = (T + 127) / 128 * (H / 256), nk = I_sh / 64;
+  return tiles <= 32 && nk % 2 == 0 && nk >= 32 ? 2 : 1;
+}

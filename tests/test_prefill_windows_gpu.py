@@ -98,3 +98,28 @@ def test_layer_of_few_wide_experts(cuda, cache_rate):
         err = float(np.abs(y.float().cpu().numpy() - ref["out"]).max() / np.abs(ref["out"]).max())
         assert err <= 2e-2, (T, err)
     pm.close()
+
+
+@pytest.mark.parametrize("cache_rate", [1.0, 0.5])
+def test_layer_with_a_shared_expert_in_two_windows(cuda, cache_rate):
+    """An int4 shared expert whose reduction is twice the routed experts' and too short for moe_prefill_shared_splits."""
+    from promoe_amd import _lib as L
+    from tests.test_engine_gpu import build_engine, ref_forward
+    print(f"case shared windows cache_rate={cache_rate}", flush=True)
+    H, I_sh, k = 256, 2176, 2
+    lib, i4 = L.lib, L.FMT_INT4_G128
+    assert lib.moe_prefill_shared_splits(i4, 130, H, I_sh) == 1 and lib.moe_prefill_shared_windows(i4, 130, H, I_sh) == 2
+    assert lib.moe_prefill_shared_windows(i4, 512, 2048, 2816) == 2      # DeepSeek shape: 32 tiles
+    assert lib.moe_prefill_shared_windows(i4, 513, 2048, 2816) == 1
+    assert lib.moe_prefill_shared_windows(i4, 130, H, 1920) == 1         # 30 slabs
+    assert lib.moe_prefill_shared_windows(i4, 200, 256, 8192) == 2 and lib.moe_prefill_shared_windows(L.FMT_Q4K, 512, 3584, 20480) == 4
+    layer = Int4Layer(H=H, I=1024, E=4, I_sh=I_sh, seed=6)
+    pm = build_engine([layer], k, cuda, max_tokens=130, cache_rate=cache_rate, cache_policy="lru")
+    for T in (130, 65, 128):
+        x = O.synth_acts(T, H, seed=T)
+        y = pm.forward(0, torch.from_numpy(x).to(torch.bfloat16).to(cuda))
+        torch.cuda.synchronize()
+        ref = ref_forward(layer, x, k, 0)
+        err = float(np.abs(y.float().cpu().numpy() - ref["out"]).max() / np.abs(ref["out"]).max())
+        assert err <= 2e-2, (T, err)
+    pm.close()

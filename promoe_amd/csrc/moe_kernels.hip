@@ -623,8 +623,8 @@ struct GemvArgs {
   int g_rows, g_nbias, g_nblk, g_seq;
   int unit_slots;               // chunked-K launches of more than 16 tokens: slots of `units` when at most 64, else 0
   int pairs;                    // T k of the step (0: unknown)
-  int row_split;                // w2 launches of more than 32 tokens: a unit of more than 32 rows has two workgroups
-                                // per group of block pairs, rows 0..31 and 32.., and so has the shared expert
+  int row_split;                // 0, or 16 / 32: a unit of more rows than that has two workgroups per group of block pairs,
+                                // rows 0 .. row_split - 1 and the others, and so has the shared expert
   // w13 launches of a decode batch that sum the gate rows and route by themselves (k_gemv_int4_mfma<.., ROUTE>):
   // 8-byte words per copy of the hand-over area, row stride of the logits in memory
   int g_copy_words, g_ldl;
@@ -780,6 +780,7 @@ struct GemvWork {
   const unsigned char *base;
   int m, row0, b;
   int half;  // row_split: which half of the unit's rows
+  bool shared;  // the shared expert
 };
 // The publishing workgroup of a w13 launch (the last one of its grid): the unit list of the step goes from device
 // memory to the host's pinned copy while the other workgroups stream weights, then the sequence word the host
@@ -833,6 +834,7 @@ static __device__ __forceinline__ GemvWork gemv_resolve(const GemvArgs &a, const
   const int u = sh ? 0 : rr / c.nblk;
   wk.b = rr - u * c.nblk;
   wk.half = 0;
+  wk.shared = sh;
   if (BY_ROWS && sh && a.row_split) {  // the shared expert's workgroups come twice, one set per half of the rows
     wk.half = bx >= (n_sh >> 1) ? 1 : 0;
     wk.b = bx - (wk.half ? (n_sh >> 1) : 0);
@@ -848,15 +850,15 @@ static __device__ __forceinline__ GemvWork gemv_resolve(const GemvArgs &a, const
       } else if (BY_ROWS && a.unit_slots > 0) {
         const rsrc_t ru = make_rsrc(a.units, (u32)a.unit_slots * 16u);
         const u32x4_t ul = __builtin_amdgcn_raw_buffer_load_b128(ru, lane * 16, 0, 0);  // past the list: zeros
-        const int ml = (int)ul.y;
-        const unsigned long long c3 = __ballot(ml > 32), c2 = __ballot(ml > 16 && ml <= 32),
+        const int ml = (int)ul.y, most = a.row_split ? a.row_split : 32;
+        const unsigned long long c3 = __ballot(ml > most), c2 = __ballot(ml > 16 && ml <= most),
                                  c1 = __ballot(ml > 0 && ml <= 16), c0 = ~(c3 | c2 | c1);
         const unsigned long long below = (1ull << lane) - 1ull;
         const int n3 = __popcll(c3), n2 = __popcll(c2), n1 = __popcll(c1);
-        const int rank = ml > 32 ? __popcll(c3 & below)
+        const int rank = ml > most ? __popcll(c3 & below)
                          : ml > 16 ? n3 + __popcll(c2 & below)
                          : ml > 0 ? n3 + n2 + __popcll(c1 & below) : n3 + n2 + n1 + __popcll(c0 & below);
-        // row_split: the n3 units of more than 32 rows take two positions each (rows 0..31, rows 32..)
+        // row_split: the n3 units of more rows than that take two positions each (rows 0 .. row_split - 1, the others)
         int ur = u;
         if (a.row_split) {
           if (u < 2 * n3) { wk.half = u & 1; ur = u >> 1; }
@@ -2740,9 +2742,11 @@ static __device__ __forceinline__ void kc_pass_q4k(const GemvClass &c, unsigned 
 // where 16-row passes cost up to four.
 // q4_K: the shared expert's w2 class may be split (c.ksplit workgroups per group of block pairs, each over 1 / ksplit
 // of the reduction, partial rows to their own copy of the output: see k_gemv_int4).
+// KSS: waves per block pair of the shared expert's class, where that is more than the routed experts' KS.
+// BY_ROWS: the units are ranked by their rows (gemv_resolve), and split where a.row_split says so.
 // ROUTE (w13 pass of at most 16 tokens): the launch sums the gate rows and routes by itself, as
 // k_gemv_int4_mfma<.., ROUTE> does (see gemv_resolve_route_batch_n)
-template <bool SWIGLU, bool DEVUNITS, int NTMAX, int KS, bool Q4K = false, bool ROUTE = false>
+template <bool SWIGLU, bool DEVUNITS, int NTMAX, int KS, bool Q4K = false, bool ROUTE = false, int KSS = KS, bool BY_ROWS = (NTMAX > 1)>
 __global__ __launch_bounds__(256, 2) void k_gemv_int4_mfma_kc(const GemvArgs a) {
   constexpr int NB = 2;
   static_assert(!ROUTE || (SWIGLU && DEVUNITS && NTMAX == 1), "routing launches: w13, 16-row passes");
@@ -2775,7 +2779,7 @@ __global__ __launch_bounds__(256, 2) void k_gemv_int4_mfma_kc(const GemvArgs a) 
       wk = gemv_resolve_route_batch<4>(a, lane, w, bx - a.n_sh_blocks, tokmask);
     }
   } else {
-    wk = gemv_resolve<DEVUNITS, (NTMAX > 1)>(a, bx, lane);
+    wk = gemv_resolve<DEVUNITS, BY_ROWS>(a, bx, lane);
   }
   const GemvClass &c = wk.c;
   const int m = wk.m, row0 = wk.row0;
@@ -2791,42 +2795,52 @@ __global__ __launch_bounds__(256, 2) void k_gemv_int4_mfma_kc(const GemvArgs a) 
   const int nsp = (Q4K && c.ksplit > 1) ? c.ksplit : 1;
   const int split = nsp > 1 ? wk.b % nsp : 0;
   const int G = Gt / nsp, g0 = split * G;   // this workgroup's window of the reduction
-  const int b = (nsp > 1 ? wk.b / nsp : wk.b) * (4 / KS) + w / KS;  // the wave's block pair
-  const int rbA = 2 * b;
-  constexpr int SCB = Q4K ? 128 : 32, ZZB = Q4K ? 32 : 8;  // bytes of section s / z per tile
-  const rsrc_t rq = make_rsrc(base + c.off_q + ((size_t)rbA * Gt + g0) * 1024, (u32)(Gt + G) * 1024u);
-  const rsrc_t rs = make_rsrc(base + c.off_s + ((size_t)rbA * Gt + g0) * SCB, (u32)(Gt + G) * SCB);
-  const rsrc_t rz = make_rsrc(base + c.off_z + ((size_t)rbA * Gt + g0) * ZZB, (u32)(Gt + G) * ZZB);
-  const rsrc_t rx = make_rsrc((const unsigned char *)c.act + (size_t)g0 * 256, KC_NO_ROW);
-  const Q4Consts q4c = q4_consts();
-  const DeqF16Consts dqc = deq_f16_consts();
-  const size_t orow0 = (size_t)split * a.T;
+  auto rows_of = [&](auto ks_) {
+    constexpr int K_S = decltype(ks_)::value;
+    const int b = (nsp > 1 ? wk.b / nsp : wk.b) * (4 / K_S) + w / K_S;  // the wave's block pair
+    const int rbA = 2 * b;
+    constexpr int SCB = Q4K ? 128 : 32, ZZB = Q4K ? 32 : 8;  // bytes of section s / z per tile
+    const rsrc_t rq = make_rsrc(base + c.off_q + ((size_t)rbA * Gt + g0) * 1024, (u32)(Gt + G) * 1024u);
+    const rsrc_t rs = make_rsrc(base + c.off_s + ((size_t)rbA * Gt + g0) * SCB, (u32)(Gt + G) * SCB);
+    const rsrc_t rz = make_rsrc(base + c.off_z + ((size_t)rbA * Gt + g0) * ZZB, (u32)(Gt + G) * ZZB);
+    const rsrc_t rx = make_rsrc((const unsigned char *)c.act + (size_t)g0 * 256, KC_NO_ROW);
+    const Q4Consts q4c = q4_consts();
+    const DeqF16Consts dqc = deq_f16_consts();
+    const size_t orow0 = (size_t)split * a.T;
 
-  // rows of this workgroup: all of the unit's, or one half of a unit of more than 32 rows (row_split)
-  int r_lo = 0, r_hi = m;
-  if (NTMAX > 1 && a.row_split) {
-    if (m > 32) { r_lo = wk.half ? 32 : 0; r_hi = wk.half ? m : 32; }
-    else if (wk.half) return;
-  }
-  for (int t0 = r_lo; t0 < r_hi;) {
-    const int left = r_hi - t0;
-    if (NTMAX >= 4 && left > 32) {
-      const int mc = left < 64 ? left : 64;
-      if constexpr (Q4K) kc_pass_q4k<SWIGLU, 4, 2, KS>(c, smem, rq, rs, rz, rx, Gt, G, b, orow0, row0 + t0, mc, dqc);
-      else kc_pass<SWIGLU, 4, 2, KS>(c, smem, rq, rs, rz, rx, b, row0 + t0, mc, q4c);
-      t0 += 64;
-    } else if (NTMAX >= 2 && left > 16) {
-      const int mc = left < 32 ? left : 32;
-      if constexpr (Q4K) kc_pass_q4k<SWIGLU, 2, 4, KS>(c, smem, rq, rs, rz, rx, Gt, G, b, orow0, row0 + t0, mc, dqc);
-      else kc_pass<SWIGLU, 2, 4, KS>(c, smem, rq, rs, rz, rx, b, row0 + t0, mc, q4c);
-      t0 += 32;
-    } else {
-      const int mc = left < 16 ? left : 16;
-      if constexpr (Q4K) kc_pass_q4k<SWIGLU, 1, 8, KS, ROUTE>(c, smem, rq, rs, rz, rx, Gt, G, b, orow0, row0 + t0, mc, dqc, tokmask);
-      else kc_pass<SWIGLU, 1, 8, KS, ROUTE>(c, smem, rq, rs, rz, rx, b, row0 + t0, mc, q4c, tokmask);
-      t0 += 16;
+    // rows of this workgroup: all of the unit's, or one half of a unit of more than row_split rows
+    int r_lo = 0, r_hi = m;
+    if (BY_ROWS && a.row_split && (DEVUNITS || wk.shared)) {   // (units by value: the halves are units of their own)
+      const int most = a.row_split;
+      if (m > most) { r_lo = wk.half ? most : 0; r_hi = wk.half ? m : most; }
+      else if (wk.half) return;
     }
-    if (t0 < r_hi) __syncthreads();  // the next pass restages chunk buffer 0
+    for (int t0 = r_lo; t0 < r_hi;) {
+      const int left = r_hi - t0;
+      if (NTMAX >= 4 && left > 32) {
+        const int mc = left < 64 ? left : 64;
+        if constexpr (Q4K) kc_pass_q4k<SWIGLU, 4, 2, K_S>(c, smem, rq, rs, rz, rx, Gt, G, b, orow0, row0 + t0, mc, dqc);
+        else kc_pass<SWIGLU, 4, 2, K_S>(c, smem, rq, rs, rz, rx, b, row0 + t0, mc, q4c);
+        t0 += 64;
+      } else if (NTMAX >= 2 && left > 16) {
+        const int mc = left < 32 ? left : 32;
+        if constexpr (Q4K) kc_pass_q4k<SWIGLU, 2, 4, K_S>(c, smem, rq, rs, rz, rx, Gt, G, b, orow0, row0 + t0, mc, dqc);
+        else kc_pass<SWIGLU, 2, 4, K_S>(c, smem, rq, rs, rz, rx, b, row0 + t0, mc, q4c);
+        t0 += 32;
+      } else {
+        const int mc = left < 16 ? left : 16;
+        if constexpr (Q4K) kc_pass_q4k<SWIGLU, 1, 8, K_S, ROUTE>(c, smem, rq, rs, rz, rx, Gt, G, b, orow0, row0 + t0, mc, dqc, tokmask);
+        else kc_pass<SWIGLU, 1, 8, K_S, ROUTE>(c, smem, rq, rs, rz, rx, b, row0 + t0, mc, q4c, tokmask);
+        t0 += 16;
+      }
+      if (t0 < r_hi) __syncthreads();  // the next pass restages chunk buffer 0
+    }
+  };
+  if constexpr (KSS != KS) {
+    if (wk.shared) rows_of(std::integral_constant<int, KSS>());
+    else rows_of(std::integral_constant<int, KS>());
+  } else {
+    rows_of(std::integral_constant<int, KS>());
   }
   KC_STAMP(4);
 }
@@ -3219,9 +3233,10 @@ static size_t gemv_mfma_kc_lds(int nt, int cg) {
 
 // chunked-K form: a workgroup takes 4 / KS block pairs of a unit (both classes' pair counts are
 // multiples of four: I and H are multiples of 128)
-template <bool SW, int NTMAX, int KS, bool Q4K = false>
+template <bool SW, int NTMAX, int KS, bool Q4K = false, int KSS = KS, int RS = (!SW && NTMAX >= 4 ? 32 : 0)>
 static int launch_gemv_mfma_kc_ks(const GemvArgs &a_in, int grid_in, hipStream_t s) {
-  constexpr int PW = 4 / KS;
+  constexpr int PW = 4 / KS, PWS = 4 / KSS;
+  constexpr bool BY_ROWS = NTMAX > 1 || RS > 0;
   GemvArgs a = a_in;
   const int units = a.cls[1].nblk > 0 ? (grid_in - a.n_sh_blocks) / a.cls[1].nblk : 0;
   // q4_K, shared expert's w2 class: nblk counts ksplit workgroups per block pair
@@ -3234,36 +3249,35 @@ static int launch_gemv_mfma_kc_ks(const GemvArgs &a_in, int grid_in, hipStream_t
     moe_set_error("k_gemv_int4_mfma_kc<q4_K>: a reduction window must hold whole 256-wide super-blocks");
     return MOE_EINVAL;
   }
-  if (a.n_sh_blocks > 0) { a.cls[0].nblk /= PW; a.n_sh_blocks /= PW; }
+  if (a.n_sh_blocks > 0) { a.cls[0].nblk /= PWS; a.n_sh_blocks /= PWS; }
   a.cls[1].nblk /= PW;
-  a.unit_slots = (NTMAX > 1 && a.units && units <= 64) ? units : 0;
-  // w2 pass above 32 tokens: its launch ends with the workgroups of the units that have the most rows (the shared
-  // expert's above all: every token's row against the longest reduction), and the chip has room beside them, so
-  // those units get a second workgroup per group of block pairs for the rows from 32 on.  At most pairs / 33 units
-  // can have more than 32 rows.  The weights of such a unit are streamed twice (few units, from the caches the
-  // second time).
+  a.unit_slots = (BY_ROWS && a.units && units <= 64) ? units : 0;
+  // RS: a launch ends with the workgroups of the units that have the most rows (the shared expert's above all: every
+  // token's row, in the w2 pass against the longest reduction), and the chip has room beside them, so those units get a
+  // second workgroup per group of block pairs for the rows from RS on.  At most pairs / (RS + 1) units can have more than
+  // RS rows.  The weights of such a unit are streamed twice (few units, from the caches the second time).
   int units_grid = units;
-  if (!SW && NTMAX >= 4 && a.unit_slots > 0 && a.pairs > 0 && !a.kunits_dev) {
-    a.row_split = 1;
-    const int extra = a.pairs / 33 < units ? a.pairs / 33 : units;
+  if (RS > 0 && a.unit_slots > 0 && a.pairs > 0 && !a.kunits_dev) {
+    a.row_split = RS;
+    const int extra = a.pairs / (RS + 1) < units ? a.pairs / (RS + 1) : units;
     units_grid = units + extra;
     a.n_sh_blocks *= 2;
-  } else if (!SW && NTMAX >= 4 && !a.units && !a.kunits_dev && units > 0 && units <= GEMV_MAX_KUNITS) {
+  } else if (RS > 0 && !a.units && !a.kunits_dev && units > 0 && units <= GEMV_MAX_KUNITS) {
     // the same split for units that travel by value: the halves become entries of their own, most rows first
     int heavy = 0;
-    for (int u = 0; u < units; ++u) heavy += a.ku[u].m > 32;
+    for (int u = 0; u < units; ++u) heavy += a.ku[u].m > RS;
     if (units + heavy <= GEMV_MAX_KUNITS) {
       KUnit out[GEMV_MAX_KUNITS];
       int n = 0;
       for (int u = 0; u < units; ++u)
-        if (a.ku[u].m > 32) {
-          out[n++] = KUnit{a.ku[u].base, 32, a.ku[u].row0};
-          out[n++] = KUnit{a.ku[u].base, a.ku[u].m - 32, a.ku[u].row0 + 32};
+        if (a.ku[u].m > RS) {
+          out[n++] = KUnit{a.ku[u].base, RS, a.ku[u].row0};
+          out[n++] = KUnit{a.ku[u].base, a.ku[u].m - RS, a.ku[u].row0 + RS};
         }
       for (int u = 0; u < units; ++u)
-        if (a.ku[u].m <= 32) out[n++] = a.ku[u];
+        if (a.ku[u].m <= RS) out[n++] = a.ku[u];
       for (int u = 0; u < n; ++u) a.ku[u] = out[u];
-      a.row_split = 1;
+      a.row_split = RS;
       units_grid = n;
       a.n_sh_blocks *= 2;
     }
@@ -3274,10 +3288,10 @@ static int launch_gemv_mfma_kc_ks(const GemvArgs &a_in, int grid_in, hipStream_t
   if (NTMAX >= 4 && gemv_mfma_kc_lds(4, 2) > lds) lds = gemv_mfma_kc_lds(4, 2);
   static bool attr_set = false;
   if (!attr_set) {
-    hipError_t e = hipFuncSetAttribute((const void *)k_gemv_int4_mfma_kc<SW, true, NTMAX, KS, Q4K>,
+    hipError_t e = hipFuncSetAttribute((const void *)k_gemv_int4_mfma_kc<SW, true, NTMAX, KS, Q4K, false, KSS, BY_ROWS>,
                                        hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
     if (e == hipSuccess)
-      e = hipFuncSetAttribute((const void *)k_gemv_int4_mfma_kc<SW, false, NTMAX, KS, Q4K>,
+      e = hipFuncSetAttribute((const void *)k_gemv_int4_mfma_kc<SW, false, NTMAX, KS, Q4K, false, KSS, BY_ROWS>,
                               hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
     if (e != hipSuccess) {
       moe_set_error("hipFuncSetAttribute(max dynamic LDS): %s", hipGetErrorString(e));
@@ -3286,8 +3300,8 @@ static int launch_gemv_mfma_kc_ks(const GemvArgs &a_in, int grid_in, hipStream_t
     attr_set = true;
   }
   moe_ktimer_begin(SW ? MOE_K_W13 : MOE_K_W2, s);
-  if (a.units) hipLaunchKernelGGL((k_gemv_int4_mfma_kc<SW, true, NTMAX, KS, Q4K>), dim3(grid), dim3(256), lds, s, a);
-  else hipLaunchKernelGGL((k_gemv_int4_mfma_kc<SW, false, NTMAX, KS, Q4K>), dim3(grid), dim3(256), lds, s, a);
+  if (a.units) hipLaunchKernelGGL((k_gemv_int4_mfma_kc<SW, true, NTMAX, KS, Q4K, false, KSS, BY_ROWS>), dim3(grid), dim3(256), lds, s, a);
+  else hipLaunchKernelGGL((k_gemv_int4_mfma_kc<SW, false, NTMAX, KS, Q4K, false, KSS, BY_ROWS>), dim3(grid), dim3(256), lds, s, a);
   moe_ktimer_end(SW ? MOE_K_W13 : MOE_K_W2, s);
   return moe_check_launch("k_gemv_int4_mfma_kc");
 }
@@ -3300,6 +3314,39 @@ template <bool SW, int NTMAX, bool Q4K = false>
 static int launch_gemv_mfma_kc(const GemvArgs &a, int grid, hipStream_t s) {
   if (grid / 4 >= 384) return launch_gemv_mfma_kc_ks<SW, NTMAX, 1, Q4K>(a, grid, s);
   return launch_gemv_mfma_kc_ks<SW, NTMAX, 2, Q4K>(a, grid, s);
+}
+
+// int4: the same choice of KS, and the split of the rows and of the shared expert's reduction by the batch.
+// Up to 16 tokens the shared expert's workgroups of the w2 pass give two waves to a block pair where its reduction is the
+// longer one (KSS = 2): they are the last to end (DeepSeek shape, 22 groups beside 11).  From 17 to 32 tokens that pass splits
+// units at 16 rows, from 33 to 48 both passes at 32 (BY_ROWS; a unit list of more than 64 slots is not ranked, its units take
+// passes of up to 32 and 64 rows as before).  us a layer, DeepSeek shape, before / now: 9 tokens 42.3 / 40.5, 12 44.0 / 42.0,
+// 16 45.6 / 44.4, 17 61.2 / 53.5, 24 64.6 / 56.9, 32 67.9 / 63.3, 33 74.2 / 69.8, 48 75.1 / 70.9; Mixtral shape (no shared expert,
+// units of equal size) within 1 %.  Past 48 tokens the splits gain nothing (64: 77.5 / 77.8 to 78.6).  Other splits: w13 at 16 rows
+// for 17 to 32 tokens 54.2 -> 56.5, 63.3 -> 64.6; w2 at 16 rows with KSS = 2 53.4, 55.7 and 66.0 at 17, 24 and 32 tokens.
+template <bool SW>
+static int launch_gemv_int4_kc(const GemvArgs &a, int grid, int T, hipStream_t s) {
+  const bool one = grid / 4 >= 384;
+  const bool long_shared = a.n_sh_blocks > 0 && a.cls[0].G > a.cls[1].G;
+  const int units = a.cls[1].nblk > 0 ? (grid - a.n_sh_blocks) / a.cls[1].nblk : 0;
+  if (T <= 16) {
+    if constexpr (!SW) {
+      if (one && long_shared) return launch_gemv_mfma_kc_ks<SW, 1, 1, false, 2>(a, grid, s);
+    }
+    return launch_gemv_mfma_kc<SW, 1>(a, grid, s);
+  }
+  if (T > 48) return launch_gemv_mfma_kc<SW, 4>(a, grid, s);
+  if (units > 64) return T > 32 ? launch_gemv_mfma_kc<SW, 4>(a, grid, s) : launch_gemv_mfma_kc<SW, 2>(a, grid, s);
+  if (T <= 32) {
+    if constexpr (!SW) {
+      if (one) return launch_gemv_mfma_kc_ks<SW, 1, 1, false, 1, 16>(a, grid, s);
+    }
+    return launch_gemv_mfma_kc<SW, 2>(a, grid, s);
+  }
+  if constexpr (!SW) {
+    if (one && long_shared) return launch_gemv_mfma_kc_ks<SW, 2, 1, false, 2, 32>(a, grid, s);
+  }
+  return one ? launch_gemv_mfma_kc_ks<SW, 2, 1, false, 1, 32>(a, grid, s) : launch_gemv_mfma_kc_ks<SW, 2, 2, false, 2, 32>(a, grid, s);
 }
 
 template <bool SW>
@@ -3319,9 +3366,7 @@ static int launch_gemv_t(const GemvArgs &a, int grid, int T, int Kmax, int G_rou
     // above 48 tokens - at 40 and 48 they tie on the first shape and lose 128 to 85 us on the second -,
     // the w13 pass only under skewed routing)
     if (T >= 16 || !whole_rows_fit) {
-      if (T > 32) return launch_gemv_mfma_kc<SW, 4>(a, grid, s);
-      if (T > 16) return launch_gemv_mfma_kc<SW, 2>(a, grid, s);
-      return launch_gemv_mfma_kc<SW, 1>(a, grid, s);
+      return launch_gemv_int4_kc<SW>(a, grid, T, s);
     }
     int tb = 1;
     while (tb < T && tb < 16) tb <<= 1;

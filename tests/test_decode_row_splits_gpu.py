@@ -1,0 +1,47 @@
+"""int4 decode batches on the chunked-K kernel: units split at 16 and 32 rows, and a shared expert whose block pairs have more
+waves than the routed experts'."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import moe_oracle as O
+from tests.synth import Int4Layer
+from tests.test_kernels_gpu import check_layer
+
+pytestmark = pytest.mark.gpu
+
+
+# launches of at least 1536 block pairs in the w2 pass (the first; the shared expert's reduction is the longer one) and in the
+# w13 pass (the second); Zipf routing: units of 1 to all rows
+@pytest.mark.parametrize("H,I,I_sh", [(2048, 128, 256), (256, 1024, 256)])
+@pytest.mark.parametrize("T", [12, 16, 17, 32, 33, 48, 49, 64])
+def test_batches_at_the_edges_of_the_splits(cuda, T, H, I, I_sh):
+    print(f"case decode_row_splits T={T} H={H}", flush=True)
+    check_layer(Int4Layer(H=H, I=I, E=24, I_sh=I_sh, seed=31, zipf=1.2), T, 4, 0, cuda)
+
+
+@pytest.mark.parametrize("T", [20, 40])
+def test_units_of_more_than_twice_the_split(cuda, T):
+    """An expert listed twice for every token: its second half is longer than the split, units from the device list and by value."""
+    from promoe_amd import ops
+    print(f"case decode_row_splits repeated T={T}", flush=True)
+    H, I, E = 2048, 128, 24
+    layer = Int4Layer(H=H, I=I, E=E, I_sh=0, seed=32)
+    x = O.synth_acts(T, H, seed=5)
+    xd = torch.from_numpy(x).to(torch.bfloat16).to(cuda)
+    idx = np.ones((T, 2), np.int32)
+    d = ops.dispatch(torch.from_numpy(idx).to(cuda), E)
+    slots = [torch.from_numpy(s).to(cuda) for s in layer.slots]
+    table = torch.tensor([s.data_ptr() for s in slots], dtype=torch.int64, device=cuda)
+    wg, wu, wd = layer.experts_fp32[1]
+    g, u = x @ wg.T, x @ wu.T
+    want = (g / (1.0 + np.exp(-g)) * u) @ wd.T                    # every row of a token
+    tok = d.sorted_tok.cpu().numpy()[: 2 * T]
+    for host_units in (False, True):
+        part_r, _, err, _, _ = ops.experts_decode_int4(xd, d, table, None, H, I, 0, host_units=host_units)
+        torch.cuda.synchronize()
+        assert int(err.item()) == 0
+        got = part_r.cpu().numpy()
+        assert np.isfinite(got).all()
+        # h in bf16 between the passes: 2^-9 of each of 128 terms
+        assert np.abs(got - want[tok]).max() <= 2e-2 * np.abs(want).max(), host_units

@@ -214,6 +214,18 @@ int moe_decode_batch_q4k_gate(const void *x_bf16, int T, const void *gate_w_bf16
                               float *part_r, float *part_s, int *err, moe_unit *units_host_out,
                               int *n_active_host_out, int *seq_host_out, int seq_value, int phases, void *stream);
 
+/* The w13 pass of the same for bf16 layers, 1 to 16 tokens (other limits: moe_decode_batch_int4_gate_fits with at least 2 for T;
+ * H % 256 == 0): gate rows, routing, w13 and SwiGLU in one launch.  The w2 pass is moe_experts_prefill_pieces with phase bit 1
+ * over the published units.  No reference counterpart. */
+int moe_decode_batch_bf16_gate(const void *x_bf16, int T, const void *gate_w_bf16, const float *gate_bias,
+                               int n_gate_rows, void *gate_ws, int gate_seq, float *logits, int ldl, int E,
+                               int k, int mode, int H, int I, int I_sh, const uint64_t *expert_ptr,
+                               const void *shared_ptr, int *idx, float *w, int *counts, int *offsets,
+                               int *sorted_pair, int *pos_of_pair, int *sorted_tok, moe_unit *units,
+                               int *n_active, int64_t *active_ids, int max_units, void *h_r, void *h_s, int *err,
+                               moe_unit *units_host_out, int *n_active_host_out, int *seq_host_out, int seq_value,
+                               void *stream);
+
 /* k3 (decode): int4 grouped SwiGLU expert product through the slot table.
  *   expert_ptr[e] : device address of expert e's slot (0 = not resident -> *err |= 1)
  *   shared_ptr    : resident shared expert (intermediate I_sh) or NULL

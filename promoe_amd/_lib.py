@@ -67,6 +67,8 @@ _sig("moe_decode_batch_int4_gate", [vp, i32, vp, vp, i32, vp, i32, vp, i32, i32,
      [i32] + [vp] * 8 + [i32, i32, vp])
 _sig("moe_decode_batch_q4k_gate", [vp, i32, vp, vp, i32, vp, i32, vp, i32, i32, i32, i32, i32, i32, i32] + [vp] * 12 +
      [i32] + [vp] * 8 + [i32, i32, vp])
+_sig("moe_decode_batch_bf16_gate", [vp, i32, vp, vp, i32, vp, i32, vp, i32, i32, i32, i32, i32, i32, i32] + [vp] * 12 + [i32] +
+     [vp] * 6 + [i32, vp])
 _sig("moe_noalloc_scratch_bytes", [], i64)
 _sig("moe_decode_token_int4_noalloc", [vp, vp, i32, i32, i32, i32, i32, i32, vp, vp, vp, vp, vp, vp])
 _sig("moe_decode_token_int4", [vp, vp, i32, i32, i32, i32, i32, i32, vp, vp, vp] + [vp] * 15 + [vp, vp, vp, i32, i32, vp, vp, vp])

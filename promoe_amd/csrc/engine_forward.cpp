@@ -16,6 +16,7 @@
 extern "C" {
 extern __attribute__((weak)) decltype(moe_experts_prefill_windows) moe_experts_prefill_windows;
 extern __attribute__((weak)) decltype(moe_combine_windows) moe_combine_windows;
+extern __attribute__((weak)) decltype(moe_decode_batch_bf16_gate) moe_decode_batch_bf16_gate;
 }
 
 struct LayerState {
@@ -399,7 +400,7 @@ static int route_batch(const moe_layer_desc &d, LayerState *s, const void *x, in
 }
 
 // a decode batch whose w13 launch computes the gate logits and routes by itself: int4 of 2 to 16 tokens, q4_K of 2 to 8
-// over at most 64 experts.  Every workgroup of the launch repeats the routing, and what a repetition costs grows with the
+// over at most 64 experts, bf16 below.  Every workgroup of the launch repeats the routing, and what a repetition costs grows with the
 // tokens (their selection rounds) and, past 64 experts, with the second to fourth column of logits per lane; a q4_K w13
 // launch has more workgroups than an int4 one has.  q4_K, us a layer, with the routing launch / routing by itself, at 2, 4, 8
 // tokens:
@@ -408,11 +409,21 @@ static int route_batch(const moe_layer_desc &d, LayerState *s, const void *x, in
 //   1024 x 512, 16 experts top-2     24.5 / 20.9    25.1 /  21.5    27.0 /  22.2
 //   4096 x 14336, 8 experts top-2   102.9 / 102.5  151.9 / 151.9   167.8 / 167.6
 //   2048 x 768, 128 experts top-8    33.9 / 37.3    41.7 /  46.1    58.2 /  62.0
+// bf16 (1 to 16 tokens): the shared expert's workgroups stream while the others route; without one only up to 8 tokens, and
+// up to 4 past 64 experts.  us a layer at 1, 4, 8, 12, 16 tokens, launches apart / in one:
+//   2048 x 1408, 60 experts top-4, shared 5632   40.7 / 34.9   68.1 / 62.8   103.1 / 98.4   130.8 / 126.5   131.0 / 126.7
+//   2048 x 1408, 64 experts top-6, shared 2816   43.2 / 38.1   56.2 / 50.3    61.9 / 56.5    82.0 / 82.1     90.6 / 86.3
+//   1024 x 512, 16 experts top-2                 21.5 / 16.6   20.8 / 17.8    27.6 / 23.8
+//   4096 x 14336, 8 experts top-2               123.5 / 118.1 329.4 / 330.2  389.5 / 388.6  390.7 / 397.1   436.8 / 441.4
+//   2048 x 768, 128 experts top-8                34.7 / 30.7   70.7 / 68.6    94.8 / 95.1   111.9 / 116.6   143.0 / 147.9
 static bool batch_routes_in_w13(const moe_layer_desc &d, const LayerState *s, int T, int E, int k, int n_gate_rows) {
   static const bool on = [] { const char *e = getenv("MOE_BATCH_ROUTE"); return !e || atoi(e) != 0; }();
-  return on && (d.fmt == MOE_FMT_INT4_G128 || (d.fmt == MOE_FMT_Q4K && T <= 8 && E <= 64)) && !use_prefill(d, T) &&
-         moe_decode_batch_int4_gate_fits(T, E, k, d.H, d.I, d.I_sh, n_gate_rows) &&
-         moe_gate_route_ws_bytes(T, n_gate_rows) <= (int64_t)s->gate_ws_bytes;
+  if (!on || moe_gate_route_ws_bytes(T, n_gate_rows) > (int64_t)s->gate_ws_bytes) return false;
+  if (d.fmt == MOE_FMT_BF16)
+    return T <= 16 && (T <= 4 || (E <= 64 && (T <= 8 || d.I_sh > 0))) &&
+           moe_decode_batch_int4_gate_fits(T < 2 ? 2 : T, E, k, d.H, d.I, d.I_sh, n_gate_rows);
+  return (d.fmt == MOE_FMT_INT4_G128 || (d.fmt == MOE_FMT_Q4K && T <= 8 && E <= 64)) && !use_prefill(d, T) &&
+         moe_decode_batch_int4_gate_fits(T, E, k, d.H, d.I, d.I_sh, n_gate_rows);
 }
 
 extern "C" int moe_forward(moe_engine *eng, int layer, const void *x, int T, void *y) {
@@ -661,7 +672,7 @@ extern "C" int moe_forward(moe_engine *eng, int layer, const void *x, int T, voi
   bool routed_by_tail = false, w13_publishes = false;
   int tail_seq = 0, host_seq = 0;  // host_seq != 0: the unit list comes to units_host with this value in *opt_seq
   if (all_resident && batch_routes_in_w13(d, s, T, E, k, n_gate_rows)) {
-    // 2 to 16 tokens, nothing for the host to decide: the w13 launch sums the gate rows, routes by itself and hands
+    // 2 to 16 tokens (bf16: from 1), nothing for the host to decide: the w13 launch sums the gate rows, routes by itself and hands
     // the unit list to the host through the pending slot's pinned memory; then w2 and the combine (three launches)
     LayerState::Pending &p = s->pend[s->pend_head];
     if (p.busy && (rc = moe_forward_harvest(eng, true))) return rc;
@@ -671,7 +682,18 @@ extern "C" int moe_forward(moe_engine *eng, int layer, const void *x, int T, voi
     if ((rc = moe_expert_ptr_table(eng, layer, &table))) return rc;
     if ((rc = moe_flush_table(eng, layer, st))) return rc;
     s->gate_seq = s->gate_seq < 0x7fffffff ? s->gate_seq + 1 : 1;
-    if (d.fmt == MOE_FMT_Q4K)
+    const void *shared = d.I_sh > 0 ? d.shared : nullptr;
+    if (d.fmt == MOE_FMT_BF16) {
+      rc = moe_decode_batch_bf16_gate(x, T, d.gate_w, d.gate_bias, n_gate_rows, s->gate_ws, s->gate_seq, s->logits, ldl, E,
+                                      k, d.route_mode, d.H, d.I, d.I_sh, table, shared, s->idx, s->topk_w, s->counts,
+                                      s->offsets, s->sorted_pair, s->pos_of_pair, s->sorted_tok, s->units, s->n_active,
+                                      s->active_ids, max_units, s->h_r, s->h_s, s->err_host + layer, p.units, p.n_active,
+                                      p.seq, seq, st);
+      if (!rc)
+        rc = moe_experts_prefill_publish(x, T, d.H, d.I, d.I_sh, k, d.fmt, s->units, max_units, s->sorted_tok, table, shared,
+                                         s->h_r, s->h_s, s->part_r, s->part_s, shared_pieces(d, T, s), s->tiles_ws,
+                                         s->err_host + layer, 2, nullptr, st);
+    } else if (d.fmt == MOE_FMT_Q4K)
       rc = moe_decode_batch_q4k_gate(x, T, d.gate_w, d.gate_bias, n_gate_rows, s->gate_ws, s->gate_seq, s->logits, ldl, E,
                                      k, d.route_mode, d.H, d.I, d.I_sh, table, d.I_sh > 0 ? d.shared : nullptr, s->idx,
                                      s->topk_w, s->counts, s->offsets, s->sorted_pair, s->pos_of_pair, s->sorted_tok,

@@ -10,6 +10,7 @@
 #include "moe_kernels.h"
 #include "moe_common.h"
 #include "moe_device.h"
+#include "moe_decode_bf16.h"
 
 // ---------------------------------------------------------------------------
 // k1a gate logits: one wave per (token, expert row)
@@ -2846,6 +2847,45 @@ __global__ __launch_bounds__(256, 2) void k_gemv_int4_mfma_kc(const GemvArgs a) 
 }
 
 // ---------------------------------------------------------------------------
+// bf16 decode batches whose w13 launch sums the gate rows and routes by itself, as k_gemv_int4_mfma<.., ROUTE> does (see
+// gemv_resolve_route_batch_n): gate workgroups, the publishing workgroup, the shared expert's, then one set per unit slot.
+// The products are those of k_decode_bf16 (work split and bits).  What it is for: gate logits and routing were two launches of
+// 2.8 and 4.4 us in front of a w13 launch of 20 to 21 us (Qwen1.5 shape, one token); in one launch the shared expert's half of
+// the bytes streams while the others route, and the launch takes 19 to 21 us in all: layer 40.7 -> 34.9 us.
+// ---------------------------------------------------------------------------
+struct DbRouteArgs {
+  GemvArgs g;      // routing; cls[1]: activations, K and workgroups per unit slot
+  DbClass c[2];    // 0 = shared expert, 1 = routed experts
+};
+template <int HV, int TPW>
+__global__ __launch_bounds__(256, 2) void k_decode_bf16_route(const DbRouteArgs ra) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  const GemvArgs &a = ra.g;
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int bx = (int)blockIdx.x;
+  if (bx < a.g_nblk) { gate_rows_batch_tg<TPW == 4 ? 8 : TPW>(a, lane, w, bx); return; }
+  bx -= a.g_nblk;
+  if (bx == 0) { route_publish_batch(a, smem); return; }
+  bx -= 1;
+  const bool sh = bx < a.n_sh_blocks;
+  unsigned tokmask = 0u;
+  GemvWork wk;
+  if (sh) { wk.b = bx; wk.m = a.T; wk.row0 = 0; wk.base = a.shared_base; }
+  else wk = gemv_resolve_route_batch<TPW>(a, lane, w, bx - a.n_sh_blocks, tokmask);
+  if (wk.m <= 0) return;
+  if (wk.base == nullptr) {
+    if (tid == 0) moe_raise_err(a.err);
+    return;
+  }
+  const DbClass &c = ra.c[sh ? 0 : 1];
+  const int Kn = c.K >> 6, mc = __builtin_amdgcn_readfirstlane(wk.m), row0 = __builtin_amdgcn_readfirstlane(wk.row0);
+  const DbSets ws = db_sets<true, HV>(c, wk.base, wk.b);
+  auto row_of = [&](const int row) { return sh ? row : nth_token(tokmask, row); };
+  db_pass<true, HV, 1, (HV == 2 ? 4 : 6)>(c, (float *)smem, ws.rwA, ws.rwB, make_rsrc(c.act, DB_NO_ROW), ws.rotA, ws.rotB, ws.half, 0,
+                                          Kn, Kn, row0, mc, 0, ws.out_col, tid, row_of);
+}
+
+// ---------------------------------------------------------------------------
 // k5 combine
 // ---------------------------------------------------------------------------
 // Bound by the partial rows' bytes (2048 tokens of six and a shared row, 2048 columns: 126 MB in 20.4 us, 6.2 TB/s).  KK: rows
@@ -3700,6 +3740,76 @@ static int decode_batch_gate(bool q4k, const void *x, int T, const void *gate_w,
                                     h_r, h_s, part_r, part_s, err, nullptr, nullptr, 2, nullptr, nullptr, nullptr, nullptr, 0,
                                     expert_ptr_host, E, stream);
   return MOE_OK;
+}
+
+template <int HV, int TPW>
+static int launch_decode_bf16_route(const DbRouteArgs &ra, int grid, hipStream_t s) {
+  size_t lds = (size_t)4 * 2 * HV * 64 * 16;
+  if (lds < RB_PUBLISH_LDS) lds = RB_PUBLISH_LDS;
+  moe_ktimer_begin(MOE_K_PREFILL_W13, s);
+  hipLaunchKernelGGL((k_decode_bf16_route<HV, TPW>), dim3(grid), dim3(256), lds, s, ra);
+  moe_ktimer_end(MOE_K_PREFILL_W13, s);
+  return moe_check_launch("k_decode_bf16_route");
+}
+
+extern "C" int moe_decode_batch_bf16_gate(const void *x, int T, const void *gate_w, const float *gate_bias,
+                                          int n_gate_rows, void *gate_ws, int gate_seq, float *logits, int ldl, int E,
+                                          int k, int mode, int H, int I, int I_sh, const uint64_t *expert_ptr,
+                                          const void *shared_ptr, int *idx, float *w, int *counts, int *offsets,
+                                          int *sorted_pair, int *pos_of_pair, int *sorted_tok, moe_unit *units,
+                                          int *n_active, int64_t *active_ids, int max_units, void *h_r, void *h_s, int *err,
+                                          moe_unit *units_host_out, int *n_active_host_out, int *seq_host_out, int seq_value,
+                                          void *stream) {
+  if (T < 1 || !moe_decode_batch_int4_gate_fits(T < 2 ? 2 : T, E, k, H, I, I_sh, n_gate_rows) || H % 256) {
+    moe_set_error("moe_decode_batch_bf16_gate: shape not taken (T=%d E=%d k=%d H=%d I=%d I_sh=%d rows=%d)", T, E, k, H, I, I_sh,
+                  n_gate_rows);
+    return MOE_EINVAL;
+  }
+  const int mu = E < T * k ? E : T * k;
+  if (!x || !gate_w || !gate_ws || gate_seq == 0 || !logits || ldl < n_gate_rows || !expert_ptr || !idx || !w || !counts ||
+      !offsets || !sorted_pair || !pos_of_pair || !sorted_tok || !units || !n_active || !active_ids || max_units != mu ||
+      !h_r || !err || mode < 0 || mode > 2 || (shared_ptr && (!h_s || I_sh == 0)) ||
+      (units_host_out && (!n_active_host_out || !seq_host_out))) {
+    moe_set_error("moe_decode_batch_bf16_gate: bad argument (T=%d max_units=%d, %d expected)", T, max_units, mu);
+    return MOE_EINVAL;
+  }
+  hipStream_t s = (hipStream_t)stream;
+  const bool sh = shared_ptr != nullptr;
+  DbRouteArgs ra;
+  memset(&ra, 0, sizeof ra);
+  GemvArgs &a = ra.g;
+  gemv_set_table(a, expert_ptr, nullptr, E);
+  a.shared_base = (const unsigned char *)shared_ptr; a.T = T; a.err = err; a.pairs = T * k;
+  a.r_E = E; a.r_k = k; a.r_mode = mode; a.r_idx = idx; a.r_w = w; a.r_counts = counts; a.r_offsets = offsets;
+  a.r_sorted_pair = sorted_pair; a.r_pos_of_pair = pos_of_pair; a.r_sorted_tok = sorted_tok; a.r_units = units;
+  a.r_n_active = n_active; a.r_active_ids = (long long *)active_ids;
+  a.r_host_units = units_host_out; a.p_host_n_active = units_host_out ? n_active_host_out : nullptr;
+  a.r_host_seq = units_host_out ? seq_host_out : nullptr; a.r_host_seq_val = seq_value; a.p_max_units = max_units;
+  a.g_w = (const uint16_t *)gate_w; a.g_bias = gate_bias; a.g_stamp = (unsigned long long *)gate_ws;
+  a.g_logits_out = logits; a.g_ldl = ldl; a.g_rows = n_gate_rows; a.g_nbias = gate_bias ? E : 0; a.g_seq = gate_seq;
+  a.g_copy_words = T * n_gate_rows > GATE_COPY_WORDS ? T * n_gate_rows : GATE_COPY_WORDS;
+  // 16-row sets where 32-row sets would leave the chip with under four workgroups per compute unit (k_decode_bf16's rule)
+  const int sh_blk = sh ? I_sh / 32 : 0, r_blk = I / 32;
+  const int hv = sh_blk + max_units * r_blk < 1024 ? 1 : 2, f = hv == 1 ? 2 : 1;
+  for (int i = 0; i < 2; ++i) {
+    DbClass &c = ra.c[i];
+    const int Ii = i == 0 ? I_sh : I;
+    c.act = (const uint16_t *)x; c.act_stride = H; c.out = i == 0 ? h_s : h_r; c.out_stride = Ii; c.K = H; c.set_delta = Ii / 32;
+    c.ksplit = 1; c.nblk = f * (i == 0 ? sh_blk : r_blk); c.slab_step = moe_bf16_slab_step(H / 64);
+  }
+  a.cls[0] = GemvClass{(const uint16_t *)x, nullptr, h_s, 0, 0, 0, H, H / 128, H, I_sh, f * sh_blk, 0};
+  a.cls[1] = GemvClass{(const uint16_t *)x, nullptr, h_r, 0, 0, 0, H, H / 128, H, I, f * r_blk, 0};
+  a.n_sh_blocks = f * sh_blk;
+  const int tg = T <= 4 ? 1 : (T <= 8 ? 2 : 8);   // tokens per gate workgroup: what the kernel instantiates
+  a.g_parts = GATE_PARTS;
+  a.g_nblk = a.g_parts * ((T + tg - 1) / tg) * ((n_gate_rows + 3) / 4);
+  a.g_cache_from = 256 * 2 + a.g_nblk;  // two workgroups per compute unit at a time
+  const int grid = a.g_nblk + 1 + a.n_sh_blocks + max_units * a.cls[1].nblk;
+  if (hv == 1)
+    return T <= 4 ? launch_decode_bf16_route<1, 1>(ra, grid, s)
+                  : (T <= 8 ? launch_decode_bf16_route<1, 2>(ra, grid, s) : launch_decode_bf16_route<1, 4>(ra, grid, s));
+  return T <= 4 ? launch_decode_bf16_route<2, 1>(ra, grid, s)
+                : (T <= 8 ? launch_decode_bf16_route<2, 2>(ra, grid, s) : launch_decode_bf16_route<2, 4>(ra, grid, s));
 }
 
 extern "C" int moe_decode_token_late_expert_int4(const void *x, int H, int I, uint64_t slot_addr, int pos, void *h_r,

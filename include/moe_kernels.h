@@ -214,7 +214,7 @@ int moe_decode_batch_q4k_gate(const void *x_bf16, int T, const void *gate_w_bf16
                               float *part_r, float *part_s, int *err, moe_unit *units_host_out,
                               int *n_active_host_out, int *seq_host_out, int seq_value, int phases, void *stream);
 
-/* The w13 pass of the same for bf16 layers, 1 to 16 tokens (other limits: moe_decode_batch_int4_gate_fits with at least 2 for T;
+/* The w13 pass of the same for bf16 layers, 1 to 32 tokens (T k <= 512; other limits: moe_decode_batch_int4_gate_fits with 2 for T;
  * H % 256 == 0): gate rows, routing, w13 and SwiGLU in one launch.  The w2 pass is moe_experts_prefill_pieces with phase bit 1
  * over the published units.  No reference counterpart. */
 int moe_decode_batch_bf16_gate(const void *x_bf16, int T, const void *gate_w_bf16, const float *gate_bias,

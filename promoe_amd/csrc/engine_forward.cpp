@@ -409,10 +409,10 @@ static int route_batch(const moe_layer_desc &d, LayerState *s, const void *x, in
 //   1024 x 512, 16 experts top-2     24.5 / 20.9    25.1 /  21.5    27.0 /  22.2
 //   4096 x 14336, 8 experts top-2   102.9 / 102.5  151.9 / 151.9   167.8 / 167.6
 //   2048 x 768, 128 experts top-8    33.9 / 37.3    41.7 /  46.1    58.2 /  62.0
-// bf16 (1 to 16 tokens): the shared expert's workgroups stream while the others route; without one only up to 8 tokens, and
-// up to 4 past 64 experts.  us a layer at 1, 4, 8, 12, 16 tokens, launches apart / in one:
-//   2048 x 1408, 60 experts top-4, shared 5632   40.7 / 34.9   68.1 / 62.8   103.1 / 98.4   130.8 / 126.5   131.0 / 126.7
-//   2048 x 1408, 64 experts top-6, shared 2816   43.2 / 38.1   56.2 / 50.3    61.9 / 56.5    82.0 / 82.1     90.6 / 86.3
+// bf16 (1 to 32 tokens): the shared expert's workgroups stream while the others route; without one only up to 8 tokens, and
+// up to 4 past 64 experts.  us a layer at 1, 4, 8, 12, 16 tokens (24, 32 behind them), launches apart / in one:
+//   2048 x 1408, 60 experts top-4, shared 5632   40.7 / 34.9   68.1 / 62.8   103.1 / 98.4   130.8 / 126.5   131.0 / 126.7   149.0 / 145.5   175.5 / 173.0
+//   2048 x 1408, 64 experts top-6, shared 2816   43.2 / 38.1   56.2 / 50.3    61.9 / 56.5    82.0 / 82.1     90.6 / 86.3     98.4 / 97.9   107.6 / 107.0
 //   1024 x 512, 16 experts top-2                 21.5 / 16.6   20.8 / 17.8    27.6 / 23.8
 //   4096 x 14336, 8 experts top-2               123.5 / 118.1 329.4 / 330.2  389.5 / 388.6  390.7 / 397.1   436.8 / 441.4
 //   2048 x 768, 128 experts top-8                34.7 / 30.7   70.7 / 68.6    94.8 / 95.1   111.9 / 116.6   143.0 / 147.9
@@ -420,8 +420,8 @@ static bool batch_routes_in_w13(const moe_layer_desc &d, const LayerState *s, in
   static const bool on = [] { const char *e = getenv("MOE_BATCH_ROUTE"); return !e || atoi(e) != 0; }();
   if (!on || moe_gate_route_ws_bytes(T, n_gate_rows) > (int64_t)s->gate_ws_bytes) return false;
   if (d.fmt == MOE_FMT_BF16)
-    return T <= 16 && (T <= 4 || (E <= 64 && (T <= 8 || d.I_sh > 0))) &&
-           moe_decode_batch_int4_gate_fits(T < 2 ? 2 : T, E, k, d.H, d.I, d.I_sh, n_gate_rows);
+    return T <= 32 && T * k <= 512 && (T <= 4 || (E <= 64 && (T <= 8 || d.I_sh > 0))) &&
+           moe_decode_batch_int4_gate_fits(2, E, k, d.H, d.I, d.I_sh, n_gate_rows);
   return (d.fmt == MOE_FMT_INT4_G128 || (d.fmt == MOE_FMT_Q4K && T <= 8 && E <= 64)) && !use_prefill(d, T) &&
          moe_decode_batch_int4_gate_fits(T, E, k, d.H, d.I, d.I_sh, n_gate_rows);
 }
@@ -672,7 +672,7 @@ extern "C" int moe_forward(moe_engine *eng, int layer, const void *x, int T, voi
   bool routed_by_tail = false, w13_publishes = false;
   int tail_seq = 0, host_seq = 0;  // host_seq != 0: the unit list comes to units_host with this value in *opt_seq
   if (all_resident && batch_routes_in_w13(d, s, T, E, k, n_gate_rows)) {
-    // 2 to 16 tokens (bf16: from 1), nothing for the host to decide: the w13 launch sums the gate rows, routes by itself and hands
+    // 2 to 16 tokens (bf16: 1 to 32), nothing for the host to decide: the w13 launch sums the gate rows, routes by itself and hands
     // the unit list to the host through the pending slot's pinned memory; then w2 and the combine (three launches)
     LayerState::Pending &p = s->pend[s->pend_head];
     if (p.busy && (rc = moe_forward_harvest(eng, true))) return rc;

@@ -1120,7 +1120,7 @@ static __device__ __forceinline__ GemvWork gemv_resolve_route(const GemvArgs &a,
 // at most once, so a unit's rows are its tokens in token order).  Every workgroup works from the same words with
 // the same rounds, so all of them and the publisher agree.
 // ---------------------------------------------------------------------------
-#define RB_MAXT 16
+#define RB_MAXT 32   // (the nibble kernels: 16)
 #define RB_MAX_UNITS 256   // unit slots of such a launch: min(E, T k) <= 256
 // gate rows of a batch: a workgroup takes four gate rows (a wave per row) and TG = ceil(T / 4) tokens; the row is
 // read once and every token's sum is the fma chain of gate_row_partial over the same chunks, then the same
@@ -1213,7 +1213,7 @@ static __device__ __forceinline__ void gate_rows_batch_tg(const GemvArgs &a, con
 }
 
 // LDS the publishing workgroup of such a launch takes from the launch's dynamic area
-#define RB_PUBLISH_LDS (2048 + 2048 + 1040 + 48 + RB_MAXT * GROUTE_MAX_ROWS * 4)
+#define RB_PUBLISH_LDS(T_) (2048 + 2048 + 1040 + 48 + (T_) * GROUTE_MAX_ROWS * 4)
 static __device__ __forceinline__ void route_publish_batch(const GemvArgs &a, unsigned char *smem) {
   int *s_idx = (int *)smem;                                            // [ROUTE_MAXP]
   unsigned long long *s_mask = (unsigned long long *)(smem + 2048);    // [RB_MAXT .. ROUTE_MAXT][4]
@@ -1405,7 +1405,7 @@ static __device__ __forceinline__ GemvWork gemv_resolve_route_batch_n(const Gemv
     const unsigned long long actm = __ballot(cnt[r] > 0);
     const unsigned long long b0 = __ballot((cnt[r] & 1) != 0), b1 = __ballot((cnt[r] & 2) != 0),
                              b2 = __ballot((cnt[r] & 4) != 0), b3 = __ballot((cnt[r] & 8) != 0),
-                             b4 = __ballot((cnt[r] & 16) != 0);
+                             b4 = __ballot((cnt[r] & 16) != 0), b5 = __ballot((cnt[r] & 32) != 0);
     const int na = __popcll(actm);
     if (!found && u < cum_act + na) {
       unsigned long long mm = actm;
@@ -1413,7 +1413,7 @@ static __device__ __forceinline__ GemvWork gemv_resolve_route_batch_n(const Gemv
       const int src = __builtin_amdgcn_readfirstlane((int)__builtin_ctzll(mm));  // expert 64 r + src
       const unsigned long long sb = (1ull << src) - 1ull;
       row0 = cum_rows + __popcll(b0 & sb) + 2 * __popcll(b1 & sb) + 4 * __popcll(b2 & sb) + 8 * __popcll(b3 & sb) +
-             16 * __popcll(b4 & sb);
+             16 * __popcll(b4 & sb) + 32 * __popcll(b5 & sb);
       m = __builtin_amdgcn_readlane(cnt[r], src);
       tm = (unsigned)__builtin_amdgcn_readlane((int)mk[r], src);
       lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)ptrs[r], src);
@@ -1424,7 +1424,7 @@ static __device__ __forceinline__ GemvWork gemv_resolve_route_batch_n(const Gemv
       const unsigned long long lb = (1ull << lane) - 1ull;
       const int ui = cum_act + __popcll(actm & lb);
       const int rw = cum_rows + __popcll(b0 & lb) + 2 * __popcll(b1 & lb) + 4 * __popcll(b2 & lb) + 8 * __popcll(b3 & lb) +
-                     16 * __popcll(b4 & lb);
+                     16 * __popcll(b4 & lb) + 32 * __popcll(b5 & lb);
       if (ui < RB_MAX_UNITS) {
         const u32 seq = (u32)a.g_seq;
         __builtin_amdgcn_raw_buffer_store_b64(u32x2_t{(u32)ptrs[r], seq}, rrec, (ui * 4 + 0) * 8, 0, 1 /* sc0 */);
@@ -1434,7 +1434,7 @@ static __device__ __forceinline__ GemvWork gemv_resolve_route_batch_n(const Gemv
       }
     }
     cum_act += na;
-    cum_rows += __popcll(b0) + 2 * __popcll(b1) + 4 * __popcll(b2) + 8 * __popcll(b3) + 16 * __popcll(b4);
+    cum_rows += __popcll(b0) + 2 * __popcll(b1) + 4 * __popcll(b2) + 8 * __popcll(b3) + 16 * __popcll(b4) + 32 * __popcll(b5);
   }
   if (w == 0 && !gate_timeout_any) {  // the slots past the last unit: records of no rows
     const int nslots = a.p_max_units < RB_MAX_UNITS ? a.p_max_units : RB_MAX_UNITS;
@@ -1448,7 +1448,7 @@ static __device__ __forceinline__ GemvWork gemv_resolve_route_batch_n(const Gemv
   return wk;
 }
 
-// TPW: the launch's tokens per wave (1: up to 4 tokens, 2: up to 8, 4: up to 16); E up to 64 pays for one column
+// TPW: the launch's tokens per wave (1: up to 4 tokens, 2: up to 8, 4: up to 16, 8: up to 32); E up to 64 pays for one column
 template <int TPW>
 static __device__ __forceinline__ GemvWork gemv_resolve_route_batch(const GemvArgs &a, int lane, int w, int rr, unsigned &tokmask) {
   if (a.r_E <= 64) return gemv_resolve_route_batch_n<1, TPW>(a, lane, w, rr, tokmask);
@@ -1456,9 +1456,10 @@ static __device__ __forceinline__ GemvWork gemv_resolve_route_batch(const GemvAr
 }
 
 // the i-th token (i-th set bit) of a unit's token mask
+template <int MAXT = 16>
 static __device__ __forceinline__ int nth_token(unsigned mask, const int i) {
 #pragma unroll
-  for (int q = 0; q < RB_MAXT - 1; ++q)
+  for (int q = 0; q < MAXT - 1; ++q)
     if (q < i) mask &= mask - 1u;
   return mask ? __builtin_ctz(mask) : 0;
 }
@@ -2863,7 +2864,7 @@ __global__ __launch_bounds__(256, 2) void k_decode_bf16_route(const DbRouteArgs 
   const GemvArgs &a = ra.g;
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   int bx = (int)blockIdx.x;
-  if (bx < a.g_nblk) { gate_rows_batch_tg<TPW == 4 ? 8 : TPW>(a, lane, w, bx); return; }
+  if (bx < a.g_nblk) { gate_rows_batch_tg<(TPW >= 4 ? 8 : TPW)>(a, lane, w, bx); return; }
   bx -= a.g_nblk;
   if (bx == 0) { route_publish_batch(a, smem); return; }
   bx -= 1;
@@ -2880,9 +2881,13 @@ __global__ __launch_bounds__(256, 2) void k_decode_bf16_route(const DbRouteArgs 
   const DbClass &c = ra.c[sh ? 0 : 1];
   const int Kn = c.K >> 6, mc = __builtin_amdgcn_readfirstlane(wk.m), row0 = __builtin_amdgcn_readfirstlane(wk.row0);
   const DbSets ws = db_sets<true, HV>(c, wk.base, wk.b);
-  auto row_of = [&](const int row) { return sh ? row : nth_token(tokmask, row); };
-  db_pass<true, HV, 1, (HV == 2 ? 4 : 6)>(c, (float *)smem, ws.rwA, ws.rwB, make_rsrc(c.act, DB_NO_ROW), ws.rotA, ws.rotB, ws.half, 0,
-                                          Kn, Kn, row0, mc, 0, ws.out_col, tid, row_of);
+  const rsrc_t rx = make_rsrc(c.act, DB_NO_ROW);
+  auto row_of = [&](const int row) { return sh ? row : nth_token<4 * TPW>(tokmask, row); };
+#define DBR_PASS(NT_, D_) db_pass<true, HV, NT_, D_>(c, (float *)smem, ws.rwA, ws.rwB, rx, ws.rotA, ws.rotB, ws.half, 0, Kn, Kn, row0, mc, \
+                                                     0, ws.out_col, tid, row_of)
+  if (TPW < 8 || mc <= 16) DBR_PASS(1, HV == 2 ? 4 : 6);
+  else DBR_PASS(2, 3);
+#undef DBR_PASS
 }
 
 // ---------------------------------------------------------------------------
@@ -3586,7 +3591,7 @@ static int launch_gemv_mfma_kc_route(const GemvArgs &a_in, int units, hipStream_
   const int grid = a.g_nblk + 1 + a.n_sh_blocks + units * a.cls[1].nblk;
   a.g_cache_from = 256 * 2 + a.g_nblk;  // two workgroups per compute unit at a time
   const size_t lds = gemv_mfma_kc_lds(1, 8);
-  static_assert(RB_PUBLISH_LDS <= 64 * 1024, "the publishing workgroup's LDS");
+  static_assert(RB_PUBLISH_LDS(16) <= 64 * 1024, "the publishing workgroup's LDS");
   static bool attr_set = false;
   if (!attr_set) {
     // (the kernel also has a few hundred bytes of static LDS: dynamic + static must stay within 160 KB)
@@ -3612,7 +3617,7 @@ static bool batch_route_whole_rows(int T, int H) {
 
 // whether moe_decode_batch_int4_gate takes a batch of T tokens of this shape
 extern "C" int moe_decode_batch_int4_gate_fits(int T, int E, int k, int H, int I, int I_sh, int n_gate_rows) {
-  if (T < 2 || T > RB_MAXT || E <= 0 || E > 256 || k <= 0 || k > 32 || k > E || T * k > ROUTE_MAXP || H <= 0 || H % 128 ||
+  if (T < 2 || T > 16 || E <= 0 || E > 256 || k <= 0 || k > 32 || k > E || T * k > ROUTE_MAXP || H <= 0 || H % 128 ||
       I <= 0 || I % 128 || I_sh < 0 || I_sh % 128 || n_gate_rows < E || n_gate_rows > E + 1)
     return 0;
   return 1;
@@ -3719,7 +3724,7 @@ static int decode_batch_gate(bool q4k, const void *x, int T, const void *gate_w,
       int tb = 1;
       while (tb < T) tb <<= 1;
       size_t lds = gemv_mfma_lds(tb, H, 2);
-      if (lds < RB_PUBLISH_LDS) lds = RB_PUBLISH_LDS;
+      if (lds < (size_t)RB_PUBLISH_LDS(T)) lds = RB_PUBLISH_LDS(T);
       const int gpw = (H / 128 + 3) / 4;
       int ch = gpw >= 4 ? ((gpw % 4 == 0) ? 4 : (gpw % 3 == 0 ? 3 : 4)) : gpw;
       if (ch < 1) ch = 1;
@@ -3744,8 +3749,9 @@ static int decode_batch_gate(bool q4k, const void *x, int T, const void *gate_w,
 
 template <int HV, int TPW>
 static int launch_decode_bf16_route(const DbRouteArgs &ra, int grid, hipStream_t s) {
-  size_t lds = (size_t)4 * 2 * HV * 64 * 16;
-  if (lds < RB_PUBLISH_LDS) lds = RB_PUBLISH_LDS;
+  const int T = ra.g.T;
+  size_t lds = (size_t)4 * 2 * HV * (T > 16 ? 2 : 1) * 64 * 16;
+  if (lds < (size_t)RB_PUBLISH_LDS(T)) lds = RB_PUBLISH_LDS(T);
   moe_ktimer_begin(MOE_K_PREFILL_W13, s);
   hipLaunchKernelGGL((k_decode_bf16_route<HV, TPW>), dim3(grid), dim3(256), lds, s, ra);
   moe_ktimer_end(MOE_K_PREFILL_W13, s);
@@ -3760,7 +3766,8 @@ extern "C" int moe_decode_batch_bf16_gate(const void *x, int T, const void *gate
                                           int *n_active, int64_t *active_ids, int max_units, void *h_r, void *h_s, int *err,
                                           moe_unit *units_host_out, int *n_active_host_out, int *seq_host_out, int seq_value,
                                           void *stream) {
-  if (T < 1 || !moe_decode_batch_int4_gate_fits(T < 2 ? 2 : T, E, k, H, I, I_sh, n_gate_rows) || H % 256) {
+  if (T < 1 || T > RB_MAXT || T * k > ROUTE_MAXP || E > 256 || H % 256 ||
+      !moe_decode_batch_int4_gate_fits(2, E, k, H, I, I_sh, n_gate_rows)) {
     moe_set_error("moe_decode_batch_bf16_gate: shape not taken (T=%d E=%d k=%d H=%d I=%d I_sh=%d rows=%d)", T, E, k, H, I, I_sh,
                   n_gate_rows);
     return MOE_EINVAL;
@@ -3805,11 +3812,11 @@ extern "C" int moe_decode_batch_bf16_gate(const void *x, int T, const void *gate
   a.g_nblk = a.g_parts * ((T + tg - 1) / tg) * ((n_gate_rows + 3) / 4);
   a.g_cache_from = 256 * 2 + a.g_nblk;  // two workgroups per compute unit at a time
   const int grid = a.g_nblk + 1 + a.n_sh_blocks + max_units * a.cls[1].nblk;
-  if (hv == 1)
-    return T <= 4 ? launch_decode_bf16_route<1, 1>(ra, grid, s)
-                  : (T <= 8 ? launch_decode_bf16_route<1, 2>(ra, grid, s) : launch_decode_bf16_route<1, 4>(ra, grid, s));
-  return T <= 4 ? launch_decode_bf16_route<2, 1>(ra, grid, s)
-                : (T <= 8 ? launch_decode_bf16_route<2, 2>(ra, grid, s) : launch_decode_bf16_route<2, 4>(ra, grid, s));
+#define DBR_LAUNCH(HV_)                                                                                      \
+  (T <= 4 ? launch_decode_bf16_route<HV_, 1>(ra, grid, s) : T <= 8 ? launch_decode_bf16_route<HV_, 2>(ra, grid, s) \
+   : T <= 16 ? launch_decode_bf16_route<HV_, 4>(ra, grid, s) : launch_decode_bf16_route<HV_, 8>(ra, grid, s))
+  return hv == 1 ? DBR_LAUNCH(1) : DBR_LAUNCH(2);
+#undef DBR_LAUNCH
 }
 
 extern "C" int moe_decode_token_late_expert_int4(const void *x, int H, int I, uint64_t slot_addr, int pos, void *h_r,

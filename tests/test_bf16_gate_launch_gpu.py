@@ -1,4 +1,4 @@
-"""bf16 decode batches of 1 to 16 tokens whose w13 launch sums the gate rows and routes by itself."""
+"""bf16 decode batches of 1 to 32 tokens whose w13 launch sums the gate rows and routes by itself."""
 import numpy as np
 import pytest
 import torch
@@ -15,7 +15,9 @@ pytestmark = pytest.mark.gpu
     (2, 512, 256, 8, 2, 2, 0, None, False), (4, 256, 384, 60, 4, 1, 256, 1.1, True),      # one token a gate workgroup, up to 4
     (5, 512, 128, 200, 8, 0, 0, None, False), (8, 2048, 128, 16, 6, 0, 256, 1.2, False),  # two, up to 8; more than 64 experts
     (9, 256, 256, 60, 4, 1, 512, 1.1, True), (16, 256, 128, 256, 32, 0, 0, None, False),
-    (16, 256, 1024, 40, 4, 0, 128, 1.2, True)])                                           # 32-row sets
+    (16, 256, 1024, 40, 4, 0, 128, 1.2, True),                                            # 32-row sets
+    (17, 512, 128, 8, 2, 0, 128, 1.2, False), (25, 256, 256, 100, 4, 2, 0, None, True),   # eight tokens a wave, units of more than
+    (32, 256, 1024, 40, 4, 0, 128, 1.2, True), (32, 2048, 128, 16, 16, 1, 256, 1.2, False)])   # 16 rows, of all 32
 def test_gate_rows_and_routing_in_the_w13_launch(cuda, T, H, I, E, k, mode, I_sh, zipf, gated):
     """Logits, routing arrays and h rows equal those of the gate, routing and w13 launches, bit for bit, on successive calls
     over one hand-over workspace: ordinary logits, ties, and (two tokens and more) fewer finite logits than choices."""
@@ -28,7 +30,7 @@ def test_gate_rows_and_routing_in_the_w13_launch(cuda, T, H, I, E, k, mode, I_sh
     wg = bf16_dev(layer.wg if not gated else np.concatenate([layer.wg, layer.shared_gate[None, :]], axis=0), cuda)
     rows, P = wg.shape[0], T * k
     bias = torch.zeros(E, device=cuda) if layer.bias is None else torch.from_numpy(layer.bias).to(cuda)
-    gws, gws_ref = ops.GateWorkspace(cuda, 16, 257), ops.GateWorkspace(cuda, 16, 257)
+    gws, gws_ref = ops.GateWorkspace(cuda, 32, 257), ops.GateWorkspace(cuda, 32, 257)
     p = L.ptr
     for seed in range(3 if T == 1 else 4):
         x = bf16_dev(O.synth_acts(T, H, seed=seed + 70), cuda)
@@ -79,7 +81,7 @@ def test_gate_rows_and_routing_in_the_w13_launch(cuda, T, H, I, E, k, mode, I_sh
             assert torch.equal(h_s.view(torch.int16), h_s2.view(torch.int16))
 
 
-@pytest.mark.parametrize("T", [1, 3, 16, 17])
+@pytest.mark.parametrize("T", [1, 3, 16, 17, 32, 33])
 def test_layer_forward(cuda, T):
     from tests.test_engine_gpu import build_engine, ref_forward
     print(f"case bf16_gate_layer T={T}", flush=True)

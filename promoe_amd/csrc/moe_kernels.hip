@@ -1266,7 +1266,8 @@ static __device__ __forceinline__ void route_publish_batch(const GemvArgs &a, un
 template <int NR, int TPW>
 static __device__ __forceinline__ GemvWork gemv_resolve_route_batch_n(const GemvArgs &a, const int lane, const int w,
                                                                       const int rr, unsigned &tokmask) {
-  __shared__ unsigned long long s_sel[RB_MAXT][4];
+  constexpr bool WIDE = TPW > 4;   // up to 32 tokens (static LDS and ballots of the others: a 3-token launch of the Mixtral shape 60 -> 66 us)
+  __shared__ unsigned long long s_sel[WIDE ? RB_MAXT : 16][4];
   GemvWork wk;
   wk.c = a.cls[1];
   const int E = a.r_E, k = a.r_k, T = a.T, Erows = a.g_rows;
@@ -1405,7 +1406,7 @@ static __device__ __forceinline__ GemvWork gemv_resolve_route_batch_n(const Gemv
     const unsigned long long actm = __ballot(cnt[r] > 0);
     const unsigned long long b0 = __ballot((cnt[r] & 1) != 0), b1 = __ballot((cnt[r] & 2) != 0),
                              b2 = __ballot((cnt[r] & 4) != 0), b3 = __ballot((cnt[r] & 8) != 0),
-                             b4 = __ballot((cnt[r] & 16) != 0), b5 = __ballot((cnt[r] & 32) != 0);
+                             b4 = __ballot((cnt[r] & 16) != 0), b5 = WIDE ? __ballot((cnt[r] & 32) != 0) : 0ull;
     const int na = __popcll(actm);
     if (!found && u < cum_act + na) {
       unsigned long long mm = actm;

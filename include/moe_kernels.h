@@ -414,7 +414,7 @@ int moe_experts_prefill_publish(const void *x_bf16, int T, int H, int I, int I_s
 /* The same with the routed experts' partial rows of the w2 pass in routed_pieces pieces as well (1 to 8, nibble formats): part_r
  * holds routed_pieces * T * k rows, piece s at part_r + s*T*k*H, each the product over one window of the I columns (whole
  * 64-column slabs, at least two); moe_combine_windows adds them.  The shared expert's pieces of the nibble formats may be any
- * 1, 2, 4 or 8 windows of whole slabs here.  moe_prefill_routed_windows, moe_prefill_shared_windows = the numbers of pieces
+ * 1, 2, 4 or 8 windows of whole slabs here, those of a bf16 batch of more than 64 tokens windows of an even number of slabs.  moe_prefill_routed_windows, moe_prefill_shared_windows = the numbers of pieces
  * worth taking. */
 int moe_prefill_routed_windows(int fmt, int T, int k, int E, int H, int I);
 int moe_prefill_shared_windows(int fmt, int T, int H, int I_sh);

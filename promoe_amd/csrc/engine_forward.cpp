@@ -202,6 +202,7 @@ extern "C" int moe_forward_prepare(moe_engine *eng, int max_tokens) {
     rows_s = std::max(rows_s, (size_t)t * (size_t)moe_prefill_shared_splits(MOE_FMT_Q4K, t, H, I_sh));
     rows_s = std::max(rows_s, (size_t)t * (size_t)moe_prefill_shared_splits(MOE_FMT_BF16, t, H, I_sh));
     rows_s = std::max(rows_s, (size_t)t * (size_t)moe_prefill_shared_windows(MOE_FMT_INT4_G128, t, H, I_sh));
+    rows_s = std::max(rows_s, (size_t)t * (size_t)moe_prefill_shared_windows(MOE_FMT_BF16, t, H, I_sh));
     if (t <= 64) rows_s = std::max(rows_s, (size_t)t * (size_t)moe_decode_shared_splits(MOE_FMT_Q4K, t, H, I_sh));
   }
   rc |= dalloc(s, &s->part_s, rows_s * H);
@@ -308,7 +309,7 @@ static int run_units(moe_engine *eng, const moe_layer_desc &d, LayerState *s, co
     const int rp = routed_pieces(d, T, s), sp = with_shared ? shared_pieces(d, T, s) : 1, phases = d.fmt == MOE_FMT_BF16 ? 3 : 7;
     const int I_sh = with_shared ? d.I_sh : 0;
     const void *shared = with_shared ? d.shared : nullptr;
-    if (d.fmt != MOE_FMT_BF16 && (rp > 1 || sp > 1))
+    if (rp > 1 || (sp > 1 && (d.fmt != MOE_FMT_BF16 || T > 64)))
       return moe_experts_prefill_windows(x, T, d.H, d.I, I_sh, d.top_k, d.fmt, units_dev, n_units, s->sorted_tok, table, shared,
                                          s->h_r, s->h_s, s->part_r, s->part_s, sp, rp, s->tiles_ws, s->err_host + layer, phases,
                                          pub ? &out : nullptr, st);

@@ -109,9 +109,18 @@ extern "C" int moe_prefill_routed_windows(int fmt, int T, int k, int E, int H, i
 // 22 slabs).  us a layer, one piece / two, DeepSeek shape: 65 tokens 85.9 / 73.4, 128 104.2 / 91.2, 200 115.7 / 103.0, 379 145.3 /
 // 133.3, 512 156.3 / 152.8; past 32 tiles the shared expert's workgroups start a full round and the pieces only cost the
 // combine: 1024 tokens 229.9 / 232.4, 2048 367.2 / 374.1.
+// bf16 past 64 tokens (tile kernel, one workgroup per compute unit): from 64 slabs on, windows of an even number, at least 20, until
+// there are 32 workgroups.  Qwen1.5 shape, 128 tokens: 8 workgroups of 88 slabs took 85 us beside two rounds of 33 us of the
+// routed experts' 22 slabs.  us a layer, 1 / 2 / 4 pieces: 65 tokens 222.1 / 213.1 / 210.3, 128 230.4 / 221.3 / 217.2,
+// 256 243.8 / 233.7 / 248.3, 379 255.2 / 256.2 / 261.7, 1024 325.3 / 327.8 / 340.9.  44 slabs beside 22 (2048 x 1408, shared 2816): 65
+// tokens 149.2 / 151.2, 256 180.8 / 183.3.
 extern "C" int moe_prefill_shared_windows(int fmt, int T, int H, int I_sh) {
-  const int s = moe_prefill_shared_splits(fmt, T, H, I_sh);
-  if (s > 1 || fmt != MOE_FMT_INT4_G128 || T <= 0 || H <= 0 || I_sh <= 0) return s;
+  int s = moe_prefill_shared_splits(fmt, T, H, I_sh);
   const int tiles = (T + 127) / 128 * (H / 256), nk = I_sh / 64;
+  if (fmt == MOE_FMT_BF16 && T > 64 && H > 0 && I_sh > 0) {
+    while (s < 4 && tiles * s <= 16 && nk % (4 * s) == 0 && nk >= 64 && nk / (2 * s) >= 20) s *= 2;
+    return s;
+  }
+  if (s > 1 || fmt != MOE_FMT_INT4_G128 || T <= 0 || H <= 0 || I_sh <= 0) return s;
   return tiles <= 32 && nk % 2 == 0 && nk >= 32 ? 2 : 1;
 }

@@ -50,7 +50,7 @@ struct PfClass {
   int shared;           // the shared expert's class
   int slab_step;        // storage rotation per 128-row group: smallest odd s >= 3 coprime with K/64
   int n_blocks;         // n_mtiles * n_ntiles * ksplit, padded (pf_padded)
-  int ksplit;           // int4 / q4_K w2 pass: workgroups per tile, each over 1/ksplit of the reduction, partial rows
+  int ksplit;           // w2 pass (bf16: the shared expert's): workgroups per tile, each over 1/ksplit of the reduction, partial rows
                         // to out + split * split_stride (0 or 1: the whole reduction)
   long long split_stride;  // elements between the pieces of out
 };
@@ -158,9 +158,10 @@ typedef __amdgpu_buffer_rsrc_t pf_rsrc_t;
 // NTW: the weight fragments are read with the non-temporal hint (a routed expert's tile is the only reader of
 // its fragments: they only pass through the caches); the shared expert's row tiles all read the same fragments
 // and those are requested with plain loads, so that the second-level cache keeps them for the next row tile
+// nk slabs of a row of Kn; rot0, rot1: the storage positions of the first one in the two column halves
 template <int NB, bool NTW>
 static __device__ __forceinline__ void pf_mainloop(f32x16_t (&acc)[8][2], unsigned lds_base, const pf_i32x4_t ra_rsrc,
-                                                    const int (&a_voff)[8], const pf_rsrc_t rb, int b_delta1, int nk, int rot0,
+                                                    const int (&a_voff)[8], const pf_rsrc_t rb, int b_delta1, int nk, int Kn, int rot0,
                                                     int rot1, int tid) {
   const int lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int fr = lane & 31, q = lane >> 5;
@@ -181,8 +182,8 @@ static __device__ __forceinline__ void pf_mainloop(f32x16_t (&acc)[8][2], unsign
   };
   auto bslab = [&](int kt_, int rot) {
     const int kt = kt_ < nk ? kt_ : nk - 1;  // past the end: the last slab once more (never used)
-    const int k = kt + rot;                  // slab position inside the 128-row group's storage
-    return (k >= nk ? k - nk : k) * 16384;   // bytes
+    const int k = kt + rot;                  // slab position inside the 128-row group's storage of Kn slabs
+    return (k >= Kn ? k - Kn : k) * 16384;   // bytes
   };
   // LDS byte address of the lane's fragment of MFMA step j in row block 0 of slot 0 (chunk 4 q + j of its row)
   unsigned faddr[4];
@@ -265,7 +266,8 @@ __global__ __launch_bounds__(256, 1) void k_prefill_gemm(const PfArgs a) {
   const PfTile tile = c.tiles[mt];
   const int rows = pf_rows(tile);
   if (rows <= 0) return;
-  const int K = c.K;
+  // this workgroup's window of the reduction (only the shared expert's w2 pass is ever split)
+  const int Kn = c.K / PF_BK, nk = SWIGLU || c.ksplit <= 1 ? Kn : Kn / c.ksplit, kt0 = SWIGLU ? 0 : split * nk;
   const int n0 = nt * c.n_cols_per_tile;
   const uint16_t *W = (const uint16_t *)(tile.w_base + c.w_off);
 
@@ -282,20 +284,19 @@ __global__ __launch_bounds__(256, 1) void k_prefill_gemm(const PfArgs a) {
   }
   pf_i32x4_t ra_rsrc;
   {
-    const unsigned long long ab = (unsigned long long)c.act;
+    const unsigned long long ab = (unsigned long long)(c.act + kt0 * PF_BK);
     ra_rsrc.x = __builtin_amdgcn_readfirstlane((int)(unsigned)ab);
     ra_rsrc.y = __builtin_amdgcn_readfirstlane((int)(unsigned)(ab >> 32));
     ra_rsrc.z = 0x7fffffff; ra_rsrc.w = 0x00020000;
   }
   // weight blocks of 32 rows x 64 k (4 KiB); the 4 blocks of a 128-row group are adjacent for each k slab, so
   // one slab of a column half is 16 KiB of contiguous memory; wave w reads block w
-  const int nk = K / PF_BK;
-  const unsigned char *wb = (const unsigned char *)W + ((size_t)(n0 / 128) * nk * 4 + w) * 4096;
+  const unsigned char *wb = (const unsigned char *)W + ((size_t)(n0 / 128) * Kn * 4 + w) * 4096;
   const unsigned long long wbu = (unsigned long long)wb;
   const pf_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(
       (void *)(((unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(wbu >> 32)) << 32) |
                (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)wbu)), 0, 0x7fffffff, 0x00020000);
-  const int b_delta1 = (int)(c.half_delta / 128) * nk * 16384;
+  const int b_delta1 = (int)(c.half_delta / 128) * Kn * 16384;
 
   f32x16_t acc[8][2];
 #pragma unroll
@@ -306,19 +307,19 @@ __global__ __launch_bounds__(256, 1) void k_prefill_gemm(const PfArgs a) {
       for (int e = 0; e < 16; ++e) acc[i][h][e] = 0.f;
 
   const int G0 = n0 / 128, G1 = G0 + (int)(c.half_delta / 128);
-  const int rot0 = (int)((unsigned)(G0 * c.slab_step) % (unsigned)nk), rot1 = (int)((unsigned)(G1 * c.slab_step) % (unsigned)nk);
+  const int rot0 = (int)((unsigned)(G0 * c.slab_step + kt0) % (unsigned)Kn), rot1 = (int)((unsigned)(G1 * c.slab_step + kt0) % (unsigned)Kn);
   const int nb = (rows + 31) >> 5;  // live row blocks (uniform for the workgroup)
   const unsigned lds_base = (unsigned)(uintptr_t)(__attribute__((address_space(3))) uint16_t *)As;
 #define PF_LOOPS(NTW_)                                                                                          \
   switch (nb) {                                                                                             \
-    case 1: pf_mainloop<1, NTW_>(acc, lds_base, ra_rsrc, a_voff, rb, b_delta1, nk, rot0, rot1, tid); break; \
-    case 2: pf_mainloop<2, NTW_>(acc, lds_base, ra_rsrc, a_voff, rb, b_delta1, nk, rot0, rot1, tid); break; \
-    case 3: pf_mainloop<3, NTW_>(acc, lds_base, ra_rsrc, a_voff, rb, b_delta1, nk, rot0, rot1, tid); break; \
-    case 4: pf_mainloop<4, NTW_>(acc, lds_base, ra_rsrc, a_voff, rb, b_delta1, nk, rot0, rot1, tid); break; \
-    case 5: pf_mainloop<5, NTW_>(acc, lds_base, ra_rsrc, a_voff, rb, b_delta1, nk, rot0, rot1, tid); break; \
-    case 6: pf_mainloop<6, NTW_>(acc, lds_base, ra_rsrc, a_voff, rb, b_delta1, nk, rot0, rot1, tid); break; \
-    case 7: pf_mainloop<7, NTW_>(acc, lds_base, ra_rsrc, a_voff, rb, b_delta1, nk, rot0, rot1, tid); break; \
-    default: pf_mainloop<8, NTW_>(acc, lds_base, ra_rsrc, a_voff, rb, b_delta1, nk, rot0, rot1, tid); break; \
+    case 1: pf_mainloop<1, NTW_>(acc, lds_base, ra_rsrc, a_voff, rb, b_delta1, nk, Kn, rot0, rot1, tid); break; \
+    case 2: pf_mainloop<2, NTW_>(acc, lds_base, ra_rsrc, a_voff, rb, b_delta1, nk, Kn, rot0, rot1, tid); break; \
+    case 3: pf_mainloop<3, NTW_>(acc, lds_base, ra_rsrc, a_voff, rb, b_delta1, nk, Kn, rot0, rot1, tid); break; \
+    case 4: pf_mainloop<4, NTW_>(acc, lds_base, ra_rsrc, a_voff, rb, b_delta1, nk, Kn, rot0, rot1, tid); break; \
+    case 5: pf_mainloop<5, NTW_>(acc, lds_base, ra_rsrc, a_voff, rb, b_delta1, nk, Kn, rot0, rot1, tid); break; \
+    case 6: pf_mainloop<6, NTW_>(acc, lds_base, ra_rsrc, a_voff, rb, b_delta1, nk, Kn, rot0, rot1, tid); break; \
+    case 7: pf_mainloop<7, NTW_>(acc, lds_base, ra_rsrc, a_voff, rb, b_delta1, nk, Kn, rot0, rot1, tid); break; \
+    default: pf_mainloop<8, NTW_>(acc, lds_base, ra_rsrc, a_voff, rb, b_delta1, nk, Kn, rot0, rot1, tid); break; \
   }
   if (c.shared) { PF_LOOPS(false) } else { PF_LOOPS(true) }
 #undef PF_LOOPS
@@ -357,7 +358,7 @@ __global__ __launch_bounds__(256, 1) void k_prefill_gemm(const PfArgs a) {
     for (int e = 0; e < 16; ++e) {
       const int row = 32 * i + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3);
       if (row < rows) {
-        float *o = (float *)c.out + (size_t)(tile.row0 + row) * c.out_stride + n0 + col;
+        float *o = (float *)c.out + (size_t)split * c.split_stride + (size_t)(tile.row0 + row) * c.out_stride + n0 + col;
         o[0] = acc[i][0][e];
         o[PF_BNH] = acc[i][1][e];
       }
@@ -931,6 +932,12 @@ static int experts_prefill(bool windows, const void *x_bf16, int T, int H, int I
       moe_set_error("moe_experts_prefill: %d pieces do not divide the bf16 shared expert's I_sh / 64 (I_sh=%d)", shared_pieces, I_sh);
       return MOE_EINVAL;
     }
+  } else if (shared_pieces > 1 && windows && fmt == MOE_FMT_BF16) {
+    if (!shared_ptr || (I_sh / 64) % (shared_pieces * 2) != 0) {   // (the tile kernel's loop takes an even number of slabs)
+      moe_set_error("moe_experts_prefill: %d windows need a bf16 shared expert whose I_sh / 64 is a multiple of %d (I_sh=%d)",
+                    shared_pieces, shared_pieces * 2, I_sh);
+      return MOE_EINVAL;
+    }
   } else if (shared_pieces > 1 && (!shared_ptr || (fmt != MOE_FMT_INT4_G128 && fmt != MOE_FMT_Q4K) ||
                                    (windows ? (I_sh / 64) % shared_pieces || I_sh / 64 / shared_pieces < 2
                                             : (I_sh / 128) % (shared_pieces * 2) != 0))) {
@@ -1039,7 +1046,7 @@ static int experts_prefill(bool windows, const void *x_bf16, int T, int H, int I
           return MOE_EINVAL;
         }
       }
-      c.ksplit = (w2 && int4) ? (shared ? shared_pieces : routed_pieces) : 1;
+      c.ksplit = !w2 ? 1 : (shared ? shared_pieces : routed_pieces);
       c.split_stride = (shared ? (long long)T : P) * H;
       c.n_blocks = pf_padded(!int4, c.n_mtiles * c.n_ntiles * c.ksplit);
       c.slab_step = moe_bf16_slab_step(c.K / PF_BK);

@@ -1,10 +1,10 @@
-"""The w2 pass of the nibble tile kernels with the reduction cut into windows, and the combine that adds the pieces."""
+"""The w2 pass of the tile kernels with the reduction cut into windows, and the combine that adds the pieces."""
 import numpy as np
 import pytest
 import torch
 
 from oracle import moe_oracle as O
-from tests.synth import Int4Layer, Q4KLayer
+from tests.synth import Bf16Layer, Int4Layer, Q4KLayer
 
 pytestmark = pytest.mark.gpu
 
@@ -21,13 +21,13 @@ def _passes(layer, fmt, T, k, dev, routed, shared):
     sh = torch.from_numpy(layer.shared_img).to(dev)
     part_r = torch.full((routed, T * k, H), float("nan"), device=dev)
     part_s = torch.full((shared, T, H), float("nan"), device=dev)
-    h_r = torch.empty(T * k, I, dtype=torch.float16, device=dev)
+    h_r = torch.empty(T * k, I, dtype=torch.float16, device=dev)   # (bf16 layers: bf16 in the same room)
     h_s = torch.empty(T, I_sh, dtype=torch.float16, device=dev)
     err = torch.zeros(1, dtype=torch.int32, device=dev)
     ws = torch.empty(ops.prefill_workspace_bytes(fmt, T, H, k, d.max_units), dtype=torch.uint8, device=dev)
-    p = L.ptr
+    p, phases = L.ptr, 3 if fmt == L.FMT_BF16 else 3 | 4
     L.check(L.lib.moe_experts_prefill_windows(p(x), T, H, I, I_sh, k, fmt, p(d.units), d.max_units, p(d.sorted_tok), p(table),
-                                              p(sh), p(h_r), p(h_s), p(part_r), p(part_s), shared, routed, p(ws), p(err), 3 | 4,
+                                              p(sh), p(h_r), p(h_s), p(part_r), p(part_s), shared, routed, p(ws), p(err), phases,
                                               None, L.cur_stream()), "moe_experts_prefill_windows")
     torch.cuda.synchronize()
     assert int(err.item()) == 0
@@ -40,13 +40,16 @@ def _passes(layer, fmt, T, k, dev, routed, shared):
     (Int4Layer, 2048, 2816, 97, 8, 2),    # the most windows; the shared expert in two windows of eleven groups
     (Q4KLayer, 768, 512, 65, 3, 1),       # windows of four slabs: whole super-blocks
     (Q4KLayer, 512, 512, 200, 4, 2),      # windows of two slabs: half a super-block
+    (Bf16Layer, 128, 512, 65, 1, 4),      # windows of two slabs
+    (Bf16Layer, 256, 2816, 129, 1, 2),    # of 22; a second tile of one row
+    (Bf16Layer, 128, 1024, 300, 1, 8),
 ])
 def test_pieces_add_up_to_the_whole_rows(cuda, cls, I, I_sh, T, routed, shared):
     from promoe_amd import _lib as L
     print(f"case windows {cls.__name__} I={I} I_sh={I_sh} T={T} routed={routed} shared={shared}", flush=True)
     H, k = 512, 2
     layer = cls(H=H, I=I, E=5, I_sh=I_sh, seed=21)
-    fmt = L.FMT_Q4K if cls is Q4KLayer else L.FMT_INT4_G128
+    fmt = {Q4KLayer: L.FMT_Q4K, Int4Layer: L.FMT_INT4_G128, Bf16Layer: L.FMT_BF16}[cls]
     r1, s1, _ = _passes(layer, fmt, T, k, cuda, 1, 1)
     rn, sn, d = _passes(layer, fmt, T, k, cuda, routed, shared)
     # the same products, added in another order: fp32 sums of up to 2816 terms differ by some units of 2^-24 of their norm
@@ -75,6 +78,10 @@ def test_windows_that_do_not_divide_the_reduction_are_refused(cuda):
         rc = L.lib.moe_experts_prefill_windows(p, 70, 256, I, 0, 2, fmt, p, 4, p, p, None, p, None, p, None, 1, routed, p, p, 3,
                                                None, None)
         assert rc != 0 and b"windows" in L.lib.moe_last_error(), (fmt, I, routed)
+    for I_sh, pieces in ((384, 2), (512, 8)):    # bf16: windows of three slabs, of one
+        rc = L.lib.moe_experts_prefill_windows(p, 70, 256, 128, I_sh, 2, L.FMT_BF16, p, 4, p, p, p, p, p, p, p, pieces, 1, p, p, 3,
+                                               None, None)
+        assert rc != 0 and b"windows" in L.lib.moe_last_error(), (I_sh, pieces)
 
 
 @pytest.mark.parametrize("cache_rate", [1.0, 0.5])
@@ -120,6 +127,26 @@ def test_layer_with_a_shared_expert_in_two_windows(cuda, cache_rate):
         y = pm.forward(0, torch.from_numpy(x).to(torch.bfloat16).to(cuda))
         torch.cuda.synchronize()
         ref = ref_forward(layer, x, k, 0)
+        err = float(np.abs(y.float().cpu().numpy() - ref["out"]).max() / np.abs(ref["out"]).max())
+        assert err <= 2e-2, (T, err)
+    pm.close()
+
+
+@pytest.mark.parametrize("T", [65, 128, 129, 257])
+def test_bf16_layer_with_a_long_shared_expert(cuda, T):
+    from promoe_amd import _lib as L
+    from tests.test_engine_gpu import build_engine, ref_forward
+    print(f"case bf16 shared windows T={T}", flush=True)
+    lib, b16 = L.lib, L.FMT_BF16
+    assert [lib.moe_prefill_shared_windows(b16, t, 2048, 5632) for t in (65, 128, 129, 256, 257)] == [4, 4, 2, 2, 1]   # Qwen1.5 shape
+    assert lib.moe_prefill_shared_windows(b16, 128, 2048, 1408) == 1 and lib.moe_prefill_shared_windows(b16, 100, 256, 5120) == 4
+    layer = Bf16Layer(H=256, I=256, E=4, I_sh=5120, seed=7, shared_gate=True)
+    pm = build_engine([layer], 2, cuda, max_tokens=257, cache_rate=1.0, cache_policy="lru")
+    for _ in range(2):
+        x = O.synth_acts(T, 256, seed=T)
+        y = pm.forward(0, torch.from_numpy(x).to(torch.bfloat16).to(cuda))
+        torch.cuda.synchronize()
+        ref = ref_forward(layer, x, 2, 0)
         err = float(np.abs(y.float().cpu().numpy() - ref["out"]).max() / np.abs(ref["out"]).max())
         assert err <= 2e-2, (T, err)
     pm.close()

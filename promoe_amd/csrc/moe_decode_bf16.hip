@@ -66,8 +66,8 @@ __global__ __launch_bounds__(256, 2) void k_decode_bf16(const DbArgs a) {
   const DbSets ws = db_sets<SWIGLU, HV>(c, base, rr);
   const rsrc_t rx = make_rsrc(c.act, DB_NO_ROW);
   const size_t orow0 = (size_t)win * a.T;
-  // A unit has more rows than there are tokens where a token holds its expert more than once (a choice among fewer than
-  // k finite logits repeats one): then in further passes, each of no more rows than the LDS takes.
+  // A unit has more rows than there are tokens where a caller's own choices list its expert more than once for a token (the
+  // top-k never does): then in further passes, each of no more rows than the LDS takes.
   const int mm = __builtin_amdgcn_readfirstlane(m), r_0 = __builtin_amdgcn_readfirstlane(row0);
   for (int p0 = 0; p0 < mm; p0 += a.pass_rows) {
     const int mc = mm - p0 < a.pass_rows ? mm - p0 : a.pass_rows, r0 = r_0 + p0;

@@ -56,13 +56,13 @@ static __device__ __forceinline__ void topk_token(const float *__restrict__ row,
                                                   int *s_idx, unsigned long long *s_mask) {
   const float NEG = -__builtin_inff();
   float v[NR], v0[NR];
-  unsigned long long msel[NR];
+  unsigned long long open[NR];
 #pragma unroll
   for (int r = 0; r < NR; ++r) {
     const int e = lane + 64 * r;
-    v[r] = (e < E) ? (COH ? __hip_atomic_load(row + e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : row[e]) : NEG;
+    v[r] = (e < E) ? (COH ? __hip_atomic_load(row + e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : row[e]) : TOPK_NONE;
     v0[r] = v[r];
-    msel[r] = 0ull;
+    open[r] = topk_column(E, r);
   }
   float my_v = 0.f;  // lane j keeps the j-th selected logit
   for (int j = 0; j < k; ++j) {
@@ -70,21 +70,10 @@ static __device__ __forceinline__ void topk_token(const float *__restrict__ row,
 #pragma unroll
     for (int r = 1; r < NR; ++r) bvl = fmaxf(bvl, v[r]);
     const float bv = wave_max_f32(bvl);
-    int wr = -1, wl = 0;
-#pragma unroll
-    for (int r = 0; r < NR; ++r) {
-      const unsigned long long mr = __ballot(v[r] == bv);
-      if (wr < 0 && mr) { wr = r; wl = (int)__builtin_ctzll(mr); }
-    }
-    if (wr < 0) { wr = 0; wl = j; }  // NaN logits match nothing: stay inside the expert range
-#pragma unroll
-    for (int r = 0; r < NR; ++r)
-      if (r == wr) {
-        if (lane == wl) v[r] = NEG;
-        msel[r] |= 1ull << wl;
-      }
+    int wr, wl;
+    topk_choose(v, open, bv, lane, wr, wl);
     if (lane == j) {
-      my_v = bv;
+      my_v = fmaxf(bv, NEG);   // (a NaN counts as -inf in the weights)
       const int bi = wl + 64 * wr;
       idx[j] = bi;
       if (s_idx) s_idx[j] = bi;
@@ -92,7 +81,7 @@ static __device__ __forceinline__ void topk_token(const float *__restrict__ row,
   }
   if (s_mask && lane == 0) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) s_mask[r] = r < NR ? msel[r < NR ? r : 0] : 0ull;
+    for (int r = 0; r < 4; ++r) s_mask[r] = r < NR ? topk_column(E, r) & ~open[r < NR ? r : 0] : 0ull;
   }
   // weights: the row maximum is the first choice; the softmax denominator over all E per lane in column order, then
   // the xor butterfly; the sum over the choices in choice order
@@ -945,7 +934,7 @@ static __device__ __forceinline__ GemvWork gemv_resolve_route_n(const GemvArgs &
 #pragma unroll
   for (int r = 0; r < NR; ++r) {
     const int e = lane + 64 * r;
-    v[r] = (e < E && a.g_nblk == 0) ? a.r_logits[e] : NEG;
+    v[r] = (e < E && a.g_nblk == 0) ? a.r_logits[e] : TOPK_NONE;
     ptrs[r] = (e < E) ? slot_of(a, e) : 0ull;
   }
   bool gate_timeout = false;
@@ -983,9 +972,9 @@ static __device__ __forceinline__ GemvWork gemv_resolve_route_n(const GemvArgs &
   }
 #pragma unroll
   for (int r = 0; r < NR; ++r) v0[r] = v[r];
-  unsigned long long msel[NR];
+  unsigned long long open[NR], msel[NR];
 #pragma unroll
-  for (int r = 0; r < NR; ++r) msel[r] = 0ull;
+  for (int r = 0; r < NR; ++r) open[r] = topk_column(E, r);
   float mx = 0.f, sum_sel = 0.f, my_v = 0.f;  // the last three only matter to the publisher
   int my_e = 0;
   for (int j = 0; j < k; ++j) {
@@ -993,22 +982,12 @@ static __device__ __forceinline__ GemvWork gemv_resolve_route_n(const GemvArgs &
 #pragma unroll
     for (int r = 1; r < NR; ++r) bv = fmaxf(bv, v[r]);
     const float best = wave_max_f32(bv);
-    // the lowest expert id holding the maximum: lowest column r first, then lowest lane
-    int wr = -1, wl = 0;
-#pragma unroll
-    for (int r = 0; r < NR; ++r) {
-      const unsigned long long mr = __ballot(v[r] == best);
-      if (wr < 0 && mr) { wr = r; wl = (int)__builtin_ctzll(mr); }
-    }
-    if (wr < 0) { wr = 0; wl = j; }  // NaN logits match nothing: stay inside the expert range
-#pragma unroll
-    for (int r = 0; r < NR; ++r)
-      if (r == wr) {
-        if (lane == wl) v[r] = NEG;
-        msel[r] |= 1ull << wl;
-      }
-    if (lane == j) { my_v = best; my_e = wl + 64 * wr; }
+    int wr, wl;
+    topk_choose(v, open, best, lane, wr, wl);
+    if (lane == j) { my_v = fmaxf(best, NEG); my_e = wl + 64 * wr; }
   }
+#pragma unroll
+  for (int r = 0; r < NR; ++r) msel[r] = topk_column(E, r) & ~open[r];
   // unit u = the u-th smallest selected id
   int cum = 0;
   bool found = false;
@@ -1274,7 +1253,6 @@ static __device__ __forceinline__ GemvWork gemv_resolve_route_batch_n(const Gemv
   const int u = rr / wk.c.nblk;
   wk.b = rr - u * wk.c.nblk;
   wk.half = 0;
-  const float NEG = -__builtin_inff();
   // Unit records of this part of the chip: four (value, launch number) words per unit slot (slot address low and
   // high, rows << 16 | first row position, token mask), written through this part's second-level cache by every
   // workgroup that has derived the routing.  A workgroup that starts late (grid index from g_cache_from on: the
@@ -1321,7 +1299,7 @@ static __device__ __forceinline__ GemvWork gemv_resolve_route_batch_n(const Gemv
 #pragma unroll
         for (int r = 0; r < NR; ++r) {
           const int e = lane + 64 * r;
-          v[i][r] = NEG;
+          v[i][r] = TOPK_NONE;
           if (e < E && t < T) {
             u32x2_t word;
             if (spins < local_spins) {
@@ -1340,31 +1318,19 @@ static __device__ __forceinline__ GemvWork gemv_resolve_route_batch_n(const Gemv
       __builtin_amdgcn_s_sleep(2);
     }
   }
-  unsigned long long msel[TPW][NR];
+  unsigned long long open[TPW][NR];
 #pragma unroll
   for (int i = 0; i < TPW; ++i)
 #pragma unroll
-    for (int r = 0; r < NR; ++r) msel[i][r] = 0ull;
+    for (int r = 0; r < NR; ++r) open[i][r] = topk_column(E, r);
   for (int j = 0; j < k; ++j) {
 #pragma unroll
     for (int i = 0; i < TPW; ++i) {
       float bv = v[i][0];
 #pragma unroll
       for (int r = 1; r < NR; ++r) bv = fmaxf(bv, v[i][r]);
-      const float best = wave_max_f32(bv);
-      int wr = -1, wl = 0;
-#pragma unroll
-      for (int r = 0; r < NR; ++r) {
-        const unsigned long long mr = __ballot(v[i][r] == best);
-        if (wr < 0 && mr) { wr = r; wl = (int)__builtin_ctzll(mr); }
-      }
-      if (wr < 0) { wr = 0; wl = j; }  // NaN logits match nothing: stay inside the expert range
-#pragma unroll
-      for (int r = 0; r < NR; ++r)
-        if (r == wr) {
-          if (lane == wl) v[i][r] = NEG;
-          msel[i][r] |= 1ull << wl;
-        }
+      int wr, wl;
+      topk_choose(v[i], open[i], wave_max_f32(bv), lane, wr, wl);
     }
   }
   __shared__ int s_timeout[4];
@@ -1374,7 +1340,7 @@ static __device__ __forceinline__ GemvWork gemv_resolve_route_batch_n(const Gemv
       const int t = w + 4 * i;
       if (t < T) {
 #pragma unroll
-        for (int r = 0; r < NR; ++r) s_sel[t][r] = gate_timeout ? 0ull : msel[i][r];
+        for (int r = 0; r < NR; ++r) s_sel[t][r] = gate_timeout ? 0ull : topk_column(E, r) & ~open[i][r];
       }
     }
     s_timeout[w] = gate_timeout ? 1 : 0;

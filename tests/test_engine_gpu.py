@@ -188,8 +188,8 @@ def test_resident_batches_account_their_hits_without_a_wait(cuda, kind):
 
 @pytest.mark.parametrize("kind", ["int4", "bf16", "q4k"])
 def test_gate_bias_that_leaves_fewer_experts_than_choices(cuda, kind):
-    """A gate bias of -inf for all but two experts, four choices per token: the choices past the second repeat an expert with
-    weight 0, so that from 33 tokens on an expert's unit has more rows than the batch has tokens."""
+    """A gate bias of -inf for all but two experts, four choices per token: the choices past the second are other experts, with
+    weight 0."""
     print(f"case engine_masked_gate kind={kind}", flush=True)
     E, k = 8, 4
     mk = {"int4": Int4Layer, "bf16": Bf16Layer, "q4k": Q4KLayer}[kind]

@@ -12,13 +12,6 @@
 
 #include "engine_internal.h"
 
-// (weak: host-only builds of the engine, over stand-ins for the kernels, may lack them; called where a plan says so only)
-extern "C" {
-extern __attribute__((weak)) decltype(moe_experts_prefill_windows) moe_experts_prefill_windows;
-extern __attribute__((weak)) decltype(moe_combine_windows) moe_combine_windows;
-extern __attribute__((weak)) decltype(moe_decode_batch_bf16_gate) moe_decode_batch_bf16_gate;
-}
-
 struct LayerState {
   int max_tokens = 0, max_k = 0, max_units = 0;
   int E = 0, H = 0, I = 0, I_sh = 0;

@@ -82,7 +82,9 @@ int moe_combine_splits(const float *, const float *, const float *, const int *,
   } while (0)
 
 int main(int argc, char **argv) {
-  const std::string what = argc > 1 ? argv[1] : "table";   // which step of the second forward fails: table | launch
+  // which step of the forward fails: table | launch | windows (an entry point this build has no stand-in for but the stub)
+  const std::string what = argc > 1 ? argv[1] : "table";
+  const bool windows = what == "windows";
   moe_cfg *cfg = moe_cfg_create(1, E);
   const char *names[1] = {"w"};
   CK(moe_cfg_set_params(cfg, names, 1));
@@ -99,12 +101,13 @@ int main(int argc, char **argv) {
     CK(moe_register_param(eng, 0, e, 0, bufs.back().data(), bufs.back().size(), 0));
   }
   CK(moe_init_slots(eng));
-  std::vector<uint16_t> gate((size_t)E * H), x((size_t)64 * H), y((size_t)64 * H);
+  std::vector<uint16_t> gate((size_t)E * H), x((size_t)100 * H), y((size_t)100 * H), shared(windows ? 3 * 5120 * H : 1);
   moe_layer_desc d;
   memset(&d, 0, sizeof d);
   d.H = H; d.I = I; d.top_k = K; d.fmt = MOE_FMT_BF16; d.gate_w = gate.data();
+  if (windows) { d.I_sh = 5120; d.shared = shared.data(); }   // (w2 reduction in windows from 65 tokens on)
   CK(moe_set_layer(eng, 0, &d));
-  CK(moe_forward_prepare(eng, 64));
+  CK(moe_forward_prepare(eng, 100));
   CK(moe_launch(eng));
   // every expert into its slot through the module hooks, which leave the slot table's copy on the device as it was
   std::vector<int64_t> ids(E);
@@ -119,8 +122,9 @@ int main(int argc, char **argv) {
   CK(moe_drain(eng));
   moe_counters c0, c1;
   CK(moe_get_counters(eng, &c0));
-  if (what == "table") g_fail_copies = 1; else g_refuse = 1;
-  if (moe_forward(eng, 0, x.data(), 40, y.data()) == MOE_OK) { printf("the forward that was to fail did not\n"); return 1; }
+  if (what == "table") g_fail_copies = 1;
+  if (what == "launch") g_refuse = 1;
+  if (moe_forward(eng, 0, x.data(), windows ? 100 : 40, y.data()) == MOE_OK) { printf("the forward that was to fail did not\n"); return 1; }
   if (g_fail_copies || g_refuse) { printf("the failure was not met\n"); return 1; }
   const auto t0 = std::chrono::steady_clock::now();
   const int n = 20;   // more than there are slots

@@ -16,6 +16,7 @@ STUB(moe_topk_dispatch)
 STUB(moe_gate_topk_dispatch)
 STUB(moe_decode_batch_int4_gate)
 STUB(moe_decode_batch_q4k_gate)
+STUB(moe_decode_batch_bf16_gate)
 STUB(moe_experts_decode_int4)
 STUB(moe_experts_decode_int4_publish)
 STUB(moe_decode_token_int4)
@@ -26,8 +27,10 @@ STUB(moe_experts_decode_q4k_publish)
 STUB(moe_experts_prefill)
 STUB(moe_experts_prefill_pieces)
 STUB(moe_experts_prefill_publish)
+STUB(moe_experts_prefill_windows)
 STUB(moe_combine)
 STUB(moe_combine_splits)
+STUB(moe_combine_windows)
 extern "C" int moe_decode_shared_splits(...) { return 1; }
 extern "C" int moe_prefill_shared_splits(...) { return 1; }
 extern "C" int64_t moe_prefill_workspace_bytes(...) { return 0; }

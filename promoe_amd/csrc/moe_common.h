@@ -26,6 +26,23 @@ static inline bool moe_publish_ok(const moe_publish *p, int max_units) {
   return p->n_active && p->units_host && p->n_active_host && p->seq_host && p->max_units > 0 && p->max_units <= max_units;
 }
 
+// Sizes past the expert kernels' 32-bit offsets: activation buffers of 2 GiB (x, h, of the routed pairs and of the shared
+// expert), rows of 2^24 columns (bf16: 2^23: offsets inside a 128-row group of a bf16 matrix, 256 bytes per column, and inside 16
+// row blocks of nibbles, 128).  I_sh: 0 without a shared expert.  An error, set, or MOE_OK.
+static inline int moe_check_expert_sizes(const char *who, bool nibbles, int T, int k, int H, int I, int I_sh) {
+  const long long widest = I > H ? I : H, rows = (long long)T * (k > 1 ? k : 1);
+  if (rows * widest * 2 >= (1ll << 31) || (I_sh > 0 && (long long)T * (I_sh > H ? I_sh : H) * 2 >= (1ll << 31))) {
+    moe_set_error("%s: activation buffers of 2 GiB or more are not supported (T=%d k=%d)", who, T, k);
+    return MOE_EINVAL;
+  }
+  const int most = nibbles ? 1 << 24 : 1 << 23;
+  if (H >= most || I >= most || I_sh >= most) {
+    moe_set_error("%s: rows of %d columns and more are not supported (H=%d I=%d I_sh=%d)", who, most, H, I, I_sh);
+    return MOE_EINVAL;
+  }
+  return MOE_OK;
+}
+
 // Storage rotation of a bf16 matrix per 128-row group of nk slabs: smallest odd s >= 3 coprime with nk (the slot layout)
 static inline int moe_bf16_slab_step(int nk) {
   for (int s = 3;; s += 2) {

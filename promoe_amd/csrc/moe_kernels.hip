@@ -3747,6 +3747,7 @@ extern "C" int moe_decode_batch_bf16_gate(const void *x, int T, const void *gate
     moe_set_error("moe_decode_batch_bf16_gate: bad argument (T=%d max_units=%d, %d expected)", T, max_units, mu);
     return MOE_EINVAL;
   }
+  if (int rc = moe_check_expert_sizes("moe_decode_batch_bf16_gate", false, T, k, H, I, shared_ptr ? I_sh : 0)) return rc;
   hipStream_t s = (hipStream_t)stream;
   const bool sh = shared_ptr != nullptr;
   DbRouteArgs ra;

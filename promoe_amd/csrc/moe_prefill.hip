@@ -965,24 +965,11 @@ static int experts_prefill(bool windows, const void *x_bf16, int T, int H, int I
     moe_set_error("moe_experts_prefill: q4_K experts need H, I multiples of 256 (H=%d I=%d I_sh=%d)", H, I, I_sh);
     return MOE_EINVAL;
   }
-  {
-    const long long widest = I > H ? I : H, rows = (long long)T * (k > 1 ? k : 1);
-    if (rows * widest * 2 >= (1ll << 31) || (shared_ptr && (long long)T * (I_sh > H ? I_sh : H) * 2 >= (1ll << 31))) {
-      moe_set_error("moe_experts_prefill: activation buffers of 2 GiB or more are not supported (T=%d k=%d)", T, k);
-      return MOE_EINVAL;
-    }
-  }
   if (H % 256 || I % 128 || (shared_ptr && I_sh % 128)) {
     moe_set_error("moe_experts_prefill: H %% 256 == 0 and I %% 128 == 0 required (H=%d I=%d I_sh=%d)", H, I, I_sh);
     return MOE_EINVAL;
   }
-  {  // offsets inside a 128-row group of a bf16 matrix (256 bytes per column) and inside 16 row blocks of nibbles (128)
-    const int most = int4 ? 1 << 24 : 1 << 23;
-    if (H >= most || I >= most || (shared_ptr && I_sh >= most)) {
-      moe_set_error("moe_experts_prefill: rows of %d columns and more are not supported (H=%d I=%d I_sh=%d)", most, H, I, I_sh);
-      return MOE_EINVAL;
-    }
-  }
+  if (int rc = moe_check_expert_sizes("moe_experts_prefill", int4, T, k, H, I, shared_ptr ? I_sh : 0)) return rc;
   if (bf16_decode)
     return moe_decode_bf16(x_bf16, T, H, I, I_sh, units, max_units, sorted_tok, expert_ptr, shared_ptr, h_r, h_s, part_r, part_s,
                            shared_pieces, err, phases, pub, s);

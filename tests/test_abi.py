@@ -52,3 +52,18 @@ def test_expert_rows_past_the_kernels_addressing_are_refused_on_the_host():
                 continue
             rc = L.lib.moe_experts_prefill(p, T, 256, most, 0, 1, fmt, p, 1, p, p, None, p, None, p, None, p, p, 3, None)
             assert rc != 0 and b"columns and more" in L.lib.moe_last_error(), (fmt, T)
+
+
+def test_the_bf16_routing_launch_refuses_what_its_w2_pass_refuses():
+    """Rows of 2^23 columns and activations of 2 GiB, with every other argument as it should be: an error before the w13 launch (no
+    GPU needed), not only from the w2 launch behind it."""
+    import torch  # noqa: F401
+    from promoe_amd import _lib as L
+    p, E = 4096, 16                              # never read
+    for T, k, H, I, I_sh, said in ((1, 1, 1 << 23, 128, 0, b"columns and more"), (1, 1, 256, 1 << 23, 0, b"columns and more"),
+                                   (1, 1, 256, 128, 1 << 23, b"columns and more"), (32, 16, 256, 1 << 21, 0, b"2 GiB"),
+                                   (32, 1, 256, 128, (1 << 23) * 8, b"2 GiB")):
+        sh = p if I_sh else None
+        rc = L.lib.moe_decode_batch_bf16_gate(p, T, p, p, E, p, 1, p, E, E, k, 0, H, I, I_sh, p, sh, p, p, p, p, p, p, p, p, p, p,
+                                              min(E, T * k), p, sh, p, None, None, None, 0, None)
+        assert rc != 0 and said in L.lib.moe_last_error(), (T, k, H, I, I_sh, L.lib.moe_last_error())

@@ -414,10 +414,12 @@ int moe_experts_prefill_publish(const void *x_bf16, int T, int H, int I, int I_s
 /* The same with the routed experts' partial rows of the w2 pass in routed_pieces pieces as well (1 to 8, nibble formats): part_r
  * holds routed_pieces * T * k rows, piece s at part_r + s*T*k*H, each the product over one window of the I columns (whole
  * 64-column slabs, at least two); moe_combine_windows adds them.  The shared expert's pieces of the nibble formats may be any
- * 1, 2, 4 or 8 windows of whole slabs here, those of a bf16 batch of more than 64 tokens windows of an even number of slabs.  moe_prefill_routed_windows, moe_prefill_shared_windows = the numbers of pieces
- * worth taking. */
+ * 1, 2, 4 or 8 windows of whole slabs here, those of a bf16 batch of more than 64 tokens windows of an even number of slabs.
+ * moe_prefill_routed_windows, moe_prefill_shared_windows_beside (routed experts of I columns) = the numbers of pieces worth
+ * taking; moe_prefill_shared_windows = the most that the latter gives for any I. */
 int moe_prefill_routed_windows(int fmt, int T, int k, int E, int H, int I);
 int moe_prefill_shared_windows(int fmt, int T, int H, int I_sh);
+int moe_prefill_shared_windows_beside(int fmt, int T, int H, int I, int I_sh);
 int moe_experts_prefill_windows(const void *x_bf16, int T, int H, int I, int I_sh, int k, int fmt,
                                 const moe_unit *units, int max_units, const int *sorted_tok,
                                 const uint64_t *expert_ptr, const void *shared_ptr, void *h_r, void *h_s,

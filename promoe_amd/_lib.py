@@ -94,6 +94,7 @@ _sig("moe_experts_prefill_windows", [vp, i32, i32, i32, i32, i32, i32, vp, i32, 
 _sig("moe_experts_prefill_publish", [vp, i32, i32, i32, i32, i32, i32, vp, i32, vp, vp, vp, vp, vp, vp, vp, i32, vp, vp, i32, vp, vp])
 _sig("moe_prefill_routed_windows", [i32, i32, i32, i32, i32, i32])
 _sig("moe_prefill_shared_windows", [i32, i32, i32, i32])
+_sig("moe_prefill_shared_windows_beside", [i32, i32, i32, i32, i32])
 _sig("moe_prefill_shared_splits", [i32, i32, i32, i32])
 _sig("moe_kernel_timing", [i32])
 _sig("moe_kernel_timing_read", [i32, C.POINTER(C.c_double), C.POINTER(i32)])

@@ -334,7 +334,7 @@ static int shared_pieces(const moe_layer_desc &d, int T, const LayerState *s) {
   if (d.I_sh <= 0) return 1;
   if (use_prefill(d, T)) {
     // (what the workspace was sized for; a layer narrower than the widest one could ask for more pieces than fit)
-    const int sp = moe_prefill_shared_windows(d.fmt, T, d.H, d.I_sh);
+    const int sp = moe_prefill_shared_windows_beside(d.fmt, T, d.H, d.I, d.I_sh);
     return (size_t)sp * T * d.H <= s->part_s_elems ? sp : 1;
   }
   return d.fmt == MOE_FMT_Q4K ? moe_decode_shared_splits(MOE_FMT_Q4K, T, d.H, d.I_sh) : 1;

@@ -103,24 +103,32 @@ extern "C" int moe_prefill_routed_windows(int fmt, int T, int k, int E, int H, i
   return s;
 }
 
-// Pieces for the shared expert's partial rows of moe_experts_prefill_windows: those of moe_prefill_shared_splits, and two for an
-// int4 shared expert of 32 slabs and more in a launch of few of its tiles.  There its workgroups, each over a reduction twice as
-// long as the routed experts', are the last to end (DeepSeek shape, 128 tokens: 8 workgroups of 44 slabs, 36 us, beside 280 of
-// 22 slabs).  us a layer, one piece / two, DeepSeek shape: 65 tokens 85.9 / 73.4, 128 104.2 / 91.2, 200 115.7 / 103.0, 379 145.3 /
-// 133.3, 512 156.3 / 152.8; past 32 tiles the shared expert's workgroups start a full round and the pieces only cost the
-// combine: 1024 tokens 229.9 / 232.4, 2048 367.2 / 374.1.
-// bf16 past 64 tokens (tile kernel, one workgroup per compute unit): from 64 slabs on, windows of an even number, at least 20, until
-// there are 32 workgroups.  Qwen1.5 shape, 128 tokens: 8 workgroups of 88 slabs took 85 us beside two rounds of 33 us of the
-// routed experts' 22 slabs.  us a layer, 1 / 2 / 4 pieces: 65 tokens 222.1 / 213.1 / 210.3, 128 230.4 / 221.3 / 217.2,
-// 256 243.8 / 233.7 / 248.3, 379 255.2 / 256.2 / 261.7, 1024 325.3 / 327.8 / 340.9.  44 slabs beside 22 (2048 x 1408, shared 2816): 65
-// tokens 149.2 / 151.2, 256 180.8 / 183.3.
-extern "C" int moe_prefill_shared_windows(int fmt, int T, int H, int I_sh) {
+// Pieces for the shared expert's partial rows of moe_experts_prefill_windows beside routed experts of I columns: those of
+// moe_prefill_shared_splits, and two for an int4 shared expert of 32 slabs and more in a launch of few of its tiles.  There its
+// workgroups, which have every token's row where the routed experts' have a few, are the last to end (DeepSeek shape, 128 tokens: 8
+// workgroups of 44 slabs, 36 us, beside 280 of 22 slabs).  us a layer, one piece / two, DeepSeek shape: 65 tokens 85.9 / 73.4, 128
+// 104.2 / 91.2, 200 115.7 / 103.0, 379 145.3 / 133.3, 512 156.3 / 152.8; past 32 tiles the shared expert's workgroups start a full round and the
+// pieces only cost the combine: 1024 tokens 229.9 / 232.4, 2048 367.2 / 374.1.  It pays beside routed experts of the same length too (w13
+// and w2 passes and combine, 65 / 128 / 512 tokens): 2048 columns both, 16 experts top-2 63.0 / 57.0, 66.6 / 59.7, 81.1 / 78.3; 2816 both
+// 71.6 / 64.2, 76.7 / 67.3, 94.5 / 91.6; with 64 experts top-6, whose launches fill the chip, within 3 % (2816 both 163.4 / 159.5, 162.6 /
+// 165.1, 208.8 / 206.4) but where the launch just fits it at once without them (2048 both, 65 tokens: 120 / 127).
+// bf16 past 64 tokens (tile kernel, one workgroup per compute unit): from 64 slabs on, windows of an even number, at least 20, while
+// there are at most 16 workgroups and one of them has a longer reduction than the routed experts'.  Qwen1.5 shape, 128 tokens: 8
+// workgroups of 88 slabs took 85 us beside two rounds of 33 us of the routed experts' 22 slabs.  us a layer, 1 / 2 / 4 pieces: 65
+// tokens 222.1 / 213.1 / 210.3, 128 230.4 / 221.3 / 217.2, 256 243.8 / 233.7 / 248.3, 379 255.2 / 256.2 / 261.7, 1024 325.3 / 327.8 / 340.9.  44 slabs beside 22
+// (2048 x 1408, shared 2816): 65 tokens 149.2 / 151.2, 256 180.8 / 183.3.  128 tokens, passes and combine, 60 experts top-4, shared beside
+// routed columns: 5632 beside 2816 387.2 / 368.5 / 370.4, beside 4096 505.5 / 499.1 / 501.7, beside 5632 675.5 / 676.1 / 684.1; 4096 beside
+// 2048 280.8 / 267.8 / 268.5, beside 4096 493.9 / 494.2 / 499.6.
+extern "C" int moe_prefill_shared_windows_beside(int fmt, int T, int H, int I, int I_sh) {
   int s = moe_prefill_shared_splits(fmt, T, H, I_sh);
   const int tiles = (T + 127) / 128 * (H / 256), nk = I_sh / 64;
   if (fmt == MOE_FMT_BF16 && T > 64 && H > 0 && I_sh > 0) {
-    while (s < 4 && tiles * s <= 16 && nk % (4 * s) == 0 && nk >= 64 && nk / (2 * s) >= 20) s *= 2;
+    while (s < 4 && tiles * s <= 16 && nk % (4 * s) == 0 && nk >= 64 && nk / (2 * s) >= 20 && I_sh / s > I) s *= 2;
     return s;
   }
   if (s > 1 || fmt != MOE_FMT_INT4_G128 || T <= 0 || H <= 0 || I_sh <= 0) return s;
   return tiles <= 32 && nk % 2 == 0 && nk >= 32 ? 2 : 1;
 }
+
+// the most of them, whatever the routed experts
+extern "C" int moe_prefill_shared_windows(int fmt, int T, int H, int I_sh) { return moe_prefill_shared_windows_beside(fmt, T, H, 0, I_sh); }

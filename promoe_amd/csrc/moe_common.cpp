@@ -88,18 +88,24 @@ extern "C" int moe_kernel_timing_read(int kernel_id, double *total_ms, int *call
 
 // Pieces the w2 pass leaves the routed experts' partial rows in (moe_experts_prefill_windows).  A few wide experts have few
 // tiles of a long reduction (Mixtral shape, 256 tokens: 128 workgroups over 224 slabs, half the chip idle for 190 us; 2048
-// tokens: 592 workgroups for 512 places, 80 of them in a second round of 290 us).  Windows of at least 32 slabs, until the
-// launch has about three workgroups per compute unit (an expert has at least one tile, and one more per 128 rows); the rows
-// of more pieces cost the launch and the combine more than the last round has left.  us a layer, 1 / 2 / 4 / 8 pieces, Mixtral
-// shape: 128 tokens 272 / 230 / 224 / 230, 379 tokens 382 / 333 / 328 / 343, 512 470 / 453 / 446 / 456, 1024 777 / 744 / 744 / 778,
-// 2048 1454 / 1427 / 1431 / 1504, 4096 2589 / 2569 / 2627 / 2778.  Short reductions lose: DeepSeek shape (22 slabs) 128 tokens 91.1 /
-// 93.8, 2048 367 / 392; Qwen2-57B shape (40 slabs) 128 tokens 312 / 312 / 322, 512 610 / 620 / 663.
+// tokens: 592 workgroups for 512 places, 80 of them in a second round of 290 us).  Windows of at least 32 slabs while the launch
+// has no more workgroups than the chip has places (two per compute unit; an expert has at least one tile, and one more per 128
+// rows); past that only windows of 96 slabs and more, up to three per compute unit: the rows of more pieces cost the launch and the
+// combine more than the last round has left.  us a layer, 1 / 2 / 4 / 8 pieces, Mixtral shape int4: 128 tokens 272 / 230 / 224 / 230, 379
+// 382 / 333 / 328 / 343, 512 470 / 453 / 446 / 456, 1024 777 / 744 / 744 / 778, 2048 1454 / 1427 / 1431 / 1504, 4096 2589 / 2569 / 2627 / 2778.  q4_K,
+// passes and combine, 1 / 2 / 4: the same shape 65 tokens 247 / 190 / 193, 128 276 / 225 / 229, 512 464 / 440 / 433, 1024 758 / 730 / 721, 2048 1380 /
+// 1337 / 1358; 2048 x 8192, 16 experts top-2 128 tokens 141 / 117 / 115, 512 189 / 154 / 156; 32 experts top-4 65 tokens 217 / 208 / 216, 1024
+// 506 / 497 / 503.  A chip that is full already loses: 2048 x 4096, 64 experts top-6 q4_K 65 tokens 207 / 213, 128 205 / 210, 512 260 / 274;
+// 4096 x 4096, 32 experts top-4 65 tokens int4 202 / 207, q4_K 206 / 214; 2048 x 8192, 64 experts 512 tokens int4 513 / 527, q4_K 533 / 539, 32
+// experts 1536 tokens 648 / 654, 660 / 671 (16 experts 4096 tokens, left whole as well, would gain: 825 / 812, 834 / 818).  So do short
+// reductions: DeepSeek shape (22 slabs) 128 tokens 91.1 / 93.8, 2048 367 / 392; Qwen2-57B shape (40 slabs) 128 tokens 312 / 312 / 322,
+// 512 610 / 620 / 663.
 extern "C" int moe_prefill_routed_windows(int fmt, int T, int k, int E, int H, int I) {
   if ((fmt != MOE_FMT_INT4_G128 && fmt != MOE_FMT_Q4K) || T <= 0 || k <= 0 || E <= 0 || H <= 0 || I <= 0) return 1;
   const long long P = (long long)T * k, wgs = ((P < E ? P : E) + P / 128) * (H / 256);
   const int nk = I / 64;
   int s = 1;
-  while (s < 4 && wgs * s < 768 && nk % (s * 2) == 0 && nk / (s * 2) >= 32) s *= 2;
+  while (s < 4 && nk % (s * 2) == 0 && nk / (s * 2) >= 32 && wgs * s <= (nk / (s * 2) >= 96 ? 767 : 512)) s *= 2;
   return s;
 }
 

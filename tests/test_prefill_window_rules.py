@@ -25,3 +25,17 @@ def test_shared_windows(fmt, H):
                     assert I_sh // 64 % s == 0 and per >= 2, (T, I, I_sh, s)
                     if fmt == L.FMT_BF16 and T > 64:
                         assert per % 2 == 0 and I_sh > I, (T, I, I_sh, s)
+
+
+@pytest.mark.parametrize("fmt", FMTS)
+def test_routed_windows(fmt):
+    """Whole windows of at least 32 slabs, bf16 none; a launch that has a workgroup for every place of the chip (512) is cut only
+    where the windows stay long."""
+    for T in TOKENS:
+        for E, k in ((4, 2), (8, 2), (16, 2), (32, 4), (64, 6), (128, 8)):
+            for H in (256, 2048, 4096):
+                for I in (128, 1408, 4096, 6144, 8192, 14336):
+                    s, nk = L.lib.moe_prefill_routed_windows(fmt, T, k, E, H, I), I // 64
+                    assert s in (1, 2, 4) and (s == 1 or (fmt != L.FMT_BF16 and nk % s == 0 and nk // s >= 32)), (T, E, H, I)
+                    if s > 1 and nk // s < 96:
+                        assert (min(T * k, E) + T * k // 128) * (H // 256) * s // 2 <= 512, (T, E, H, I, s)

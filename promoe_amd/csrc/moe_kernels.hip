@@ -3243,6 +3243,16 @@ static size_t gemv_mfma_kc_lds(int nt, int cg) {
   return (size_t)2 * 16 * nt * (cg * 256 + 16) + (size_t)2 * 16 * nt * cg * 4 + (size_t)4 * 2 * cg * 32 * 4;
 }
 
+// Whether a launch can give the units of more than rs rows a second workgroup per group of block pairs: a device list that a
+// wave can rank, or units by value with room for the halves.
+static bool gemv_can_split(const GemvArgs &a, int units, int rs) {
+  if (a.kunits_dev || units <= 0 || units > GEMV_MAX_KUNITS) return false;
+  if (a.units) return a.pairs > 0;
+  int n = units;
+  for (int u = 0; u < units; ++u) n += a.ku[u].m > rs;
+  return n <= GEMV_MAX_KUNITS;
+}
+
 // chunked-K form: a workgroup takes 4 / KS block pairs of a unit (both classes' pair counts are
 // multiples of four: I and H are multiples of 128)
 template <bool SW, int NTMAX, int KS, bool Q4K = false, int KSS = KS, int RS = (!SW && NTMAX >= 4 ? 32 : 0)>
@@ -3269,16 +3279,14 @@ static int launch_gemv_mfma_kc_ks(const GemvArgs &a_in, int grid_in, hipStream_t
   // second workgroup per group of block pairs for the rows from RS on.  At most pairs / (RS + 1) units can have more than
   // RS rows.  The weights of such a unit are streamed twice (few units, from the caches the second time).
   int units_grid = units;
-  if (RS > 0 && a.unit_slots > 0 && a.pairs > 0 && !a.kunits_dev) {
+  if (RS > 0 && gemv_can_split(a, units, RS)) {
     a.row_split = RS;
-    const int extra = a.pairs / (RS + 1) < units ? a.pairs / (RS + 1) : units;
-    units_grid = units + extra;
     a.n_sh_blocks *= 2;
-  } else if (RS > 0 && !a.units && !a.kunits_dev && units > 0 && units <= GEMV_MAX_KUNITS) {
-    // the same split for units that travel by value: the halves become entries of their own, most rows first
-    int heavy = 0;
-    for (int u = 0; u < units; ++u) heavy += a.ku[u].m > RS;
-    if (units + heavy <= GEMV_MAX_KUNITS) {
+    if (a.units) {
+      const int extra = a.pairs / (RS + 1) < units ? a.pairs / (RS + 1) : units;
+      units_grid = units + extra;
+    } else {
+      // units that travel by value: the halves become entries of their own, most rows first
       KUnit out[GEMV_MAX_KUNITS];
       int n = 0;
       for (int u = 0; u < units; ++u)
@@ -3289,9 +3297,7 @@ static int launch_gemv_mfma_kc_ks(const GemvArgs &a_in, int grid_in, hipStream_t
       for (int u = 0; u < units; ++u)
         if (a.ku[u].m <= RS) out[n++] = a.ku[u];
       for (int u = 0; u < n; ++u) a.ku[u] = out[u];
-      a.row_split = RS;
       units_grid = n;
-      a.n_sh_blocks *= 2;
     }
   }
   const int grid = a.n_sh_blocks + units_grid * a.cls[1].nblk + (SW && a.units && a.p_host_units ? 1 : 0);
@@ -3332,7 +3338,11 @@ static int launch_gemv_mfma_kc(const GemvArgs &a, int grid, hipStream_t s) {
 // Up to 16 tokens the shared expert's workgroups of the w2 pass give two waves to a block pair where its reduction is the
 // longer one (KSS = 2): they are the last to end (DeepSeek shape, 22 groups beside 11).  From 17 to 32 tokens that pass splits
 // units at 16 rows, from 33 to 48 both passes at 32 (BY_ROWS; a unit list of more than 64 slots is not ranked, its units take
-// passes of up to 32 and 64 rows as before).  us a layer, DeepSeek shape, before / now: 9 tokens 42.3 / 40.5, 12 44.0 / 42.0,
+// passes of up to 32 and 64 rows as before).  Units by value whose halves find no room (gemv_can_split) keep the passes of up to 32
+// rows up to 32 tokens (64 units, 5 of them of more than 16 rows, w2 at 24 tokens: 2048 x 1408 with a shared expert of 2816 in passes of 16
+// rows 33.4, of 32 31.8; 2048 x 2560 50.3 / 44.3) and the forms below from 33 on (40 tokens, against passes of up to 64 rows: 35.4 / 39.9,
+// 50.6 / 51.0; the shared
+// expert alone, whose two passes of 32 rows and fewer read its weights twice, 54.0 / 58.9).  us a layer, DeepSeek shape, before / now: 9 tokens 42.3 / 40.5, 12 44.0 / 42.0,
 // 16 45.6 / 44.4, 17 61.2 / 53.5, 24 64.6 / 56.9, 32 67.9 / 63.3, 33 74.2 / 69.8, 48 75.1 / 70.9; Mixtral shape (no shared expert,
 // units of equal size) within 1 %.  Past 48 tokens the splits gain nothing (64: 77.5 / 77.8 to 78.6).  Other splits: w13 at 16 rows
 // for 17 to 32 tokens 54.2 -> 56.5, 63.3 -> 64.6; w2 at 16 rows with KSS = 2 53.4, 55.7 and 66.0 at 17, 24 and 32 tokens.
@@ -3348,7 +3358,8 @@ static int launch_gemv_int4_kc(const GemvArgs &a, int grid, int T, hipStream_t s
     return launch_gemv_mfma_kc<SW, 1>(a, grid, s);
   }
   if (T > 48) return launch_gemv_mfma_kc<SW, 4>(a, grid, s);
-  if (units > 64) return T > 32 ? launch_gemv_mfma_kc<SW, 4>(a, grid, s) : launch_gemv_mfma_kc<SW, 2>(a, grid, s);
+  if (T <= 32 && !gemv_can_split(a, units, 16)) return launch_gemv_mfma_kc<SW, 2>(a, grid, s);
+  if (units > GEMV_MAX_KUNITS) return launch_gemv_mfma_kc<SW, 4>(a, grid, s);
   if (T <= 32) {
     if constexpr (!SW) {
       if (one) return launch_gemv_mfma_kc_ks<SW, 1, 1, false, 1, 16>(a, grid, s);

@@ -45,3 +45,43 @@ def test_units_of_more_than_twice_the_split(cuda, T):
         assert np.isfinite(got).all()
         # h in bf16 between the passes: 2^-9 of each of 128 terms
         assert np.abs(got - want[tok]).max() <= 2e-2 * np.abs(want).max(), host_units
+
+
+def _swiglu_rows(layer, x, idx, d):
+    """Every routed partial row as the oracle's expert gives it, in the order of the dispatch."""
+    T, k = idx.shape
+    want = np.empty((T * k, layer.H), np.float32)
+    pos = d.pos_of_pair.cpu().numpy()[: T * k].reshape(T, k)
+    for e in np.unique(idx):
+        t, j = np.nonzero(idx == e)
+        want[pos[t, j]] = O.swiglu_expert(torch.from_numpy(x[t]), *[torch.from_numpy(w) for w in layer.experts_fp32[e]]).numpy()
+    return want
+
+
+# 24 tokens: units split at 16 rows, 40: at 32.  (60 used experts and 5 of more rows than that: one more half than travels by value)
+@pytest.mark.parametrize("T", [24, 40])
+@pytest.mark.parametrize("used,heavy", [(59, 5), (60, 5), (64, 0), (64, 1)])
+def test_units_by_value_at_the_room_for_their_halves(cuda, T, used, heavy):
+    from promoe_amd import ops
+    print(f"case decode_row_splits by value T={T} used={used} heavy={heavy}", flush=True)
+    H, I, k = 2048, 128, 8
+    layer = Int4Layer(H=H, I=I, E=64, I_sh=256, seed=33)
+    light = np.arange(T * (k - heavy)).reshape(T, k - heavy) % (used - heavy) + heavy
+    idx = np.concatenate([np.tile(np.arange(heavy), (T, 1)), light], axis=1).astype(np.int32)
+    counts = np.bincount(idx.reshape(-1), minlength=64)
+    assert (counts > 0).sum() == used and (counts > (16 if T <= 32 else 32)).sum() == heavy
+    x = O.synth_acts(T, H, seed=6)
+    xd = torch.from_numpy(x).to(torch.bfloat16).to(cuda)
+    d = ops.dispatch(torch.from_numpy(idx).to(cuda), 64, max_units=used)
+    slots = [torch.from_numpy(s).to(cuda) for s in layer.slots]
+    table = torch.tensor([s.data_ptr() for s in slots], dtype=torch.int64, device=cuda)
+    shared = torch.from_numpy(layer.shared_img).to(cuda)
+    want = _swiglu_rows(layer, x, idx, d)
+    sh = O.swiglu_expert(torch.from_numpy(x), *[torch.from_numpy(w) for w in layer.shared_fp32]).numpy()
+    for host_units in (True, False):
+        part_r, part_s, err, _, _ = ops.experts_decode_int4(xd, d, table, shared, H, I, 256, host_units=host_units)
+        torch.cuda.synchronize()
+        assert int(err.item()) == 0
+        # h in bf16 between the passes: 2^-9 of each of 128 and 256 terms
+        assert np.abs(part_r.cpu().numpy() - want).max() <= 2e-2 * np.abs(want).max(), host_units
+        assert np.abs(part_s.cpu().numpy() - sh).max() <= 2e-2 * np.abs(sh).max(), host_units

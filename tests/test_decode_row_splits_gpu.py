@@ -85,3 +85,38 @@ def test_units_by_value_at_the_room_for_their_halves(cuda, T, used, heavy):
         # h in bf16 between the passes: 2^-9 of each of 128 and 256 terms
         assert np.abs(part_r.cpu().numpy() - want).max() <= 2e-2 * np.abs(want).max(), host_units
         assert np.abs(part_s.cpu().numpy() - sh).max() <= 2e-2 * np.abs(sh).max(), host_units
+
+
+@pytest.fixture(scope="module")
+def long_shared():
+    """24 experts of 11 groups in w2 beside a shared expert of 22: several chunks of every pass width, in launches of at least
+    1536 block pairs with all units in use."""
+    return Int4Layer(H=2048, I=1408, E=24, I_sh=2816, seed=34)
+
+
+@pytest.mark.parametrize("T", [9, 12, 16, 17, 32, 33, 40, 48])
+def test_shared_expert_with_more_waves_over_several_chunks(cuda, long_shared, T):
+    """The shared expert's w2 with two waves a block pair (9 to 16 and 33 to 48 tokens), whose sums each have groups of every
+    chunk, and the split at 16 rows; units from the device list and by value."""
+    from promoe_amd import ops
+    layer, H, k = long_shared, 2048, 6
+    print(f"case decode_row_splits long shared T={T}", flush=True)
+    x = O.synth_acts(T, H, seed=7)
+    xd = torch.from_numpy(x).to(torch.bfloat16).to(cuda)
+    rng = np.random.default_rng(T)
+    # five popular experts for half of the choices, the others in turn: every expert in use, units of a few and of many rows
+    idx = np.stack([np.concatenate([rng.permutation(5)[:3], 5 + (np.arange(3) + 3 * t) % 19]) for t in range(T)]).astype(np.int32)
+    d = ops.dispatch(torch.from_numpy(idx).to(cuda), 24)
+    assert int(d.n_active.item()) == 24
+    slots = [torch.from_numpy(s).to(cuda) for s in layer.slots]
+    table = torch.tensor([s.data_ptr() for s in slots], dtype=torch.int64, device=cuda)
+    shared = torch.from_numpy(layer.shared_img).to(cuda)
+    want = _swiglu_rows(layer, x, idx, d)
+    sh = O.swiglu_expert(torch.from_numpy(x), *[torch.from_numpy(w) for w in layer.shared_fp32]).numpy()
+    for host_units in (False, True):
+        part_r, part_s, err, _, _ = ops.experts_decode_int4(xd, d, table, shared, H, 1408, 2816, host_units=host_units)
+        torch.cuda.synchronize()
+        assert int(err.item()) == 0
+        # h in bf16 between the passes: relative 2^-9 a term, sums of 1408 and 2816 terms of random sign
+        assert np.abs(part_r.cpu().numpy() - want).max() <= 2e-2 * np.abs(want).max(), host_units
+        assert np.abs(part_s.cpu().numpy() - sh).max() <= 2e-2 * np.abs(sh).max(), host_units

@@ -71,17 +71,29 @@ def test_pieces_add_up_to_the_whole_rows(cuda, cls, I, I_sh, T, routed, shared):
 
 
 def test_windows_that_do_not_divide_the_reduction_are_refused(cuda):
+    """(Every buffer is real and large enough for the sizes as given, and no unit has rows: a call that was taken after all would
+    only fail the assertion.)"""
     from promoe_amd import _lib as L
-    p = 4096                                     # never read
+    T, H, k, p = 70, 256, 2, L.ptr
+    x = torch.zeros(T, H, dtype=torch.bfloat16, device=cuda)
+    units, tok = torch.zeros(4, 4, dtype=torch.int32, device=cuda), torch.zeros(T * k, dtype=torch.int32, device=cuda)
+    table, err = torch.zeros(4, dtype=torch.int64, device=cuda), torch.zeros(1, dtype=torch.int32, device=cuda)
+    shared = torch.zeros(3 * 512 * H * 2, dtype=torch.uint8, device=cuda)
+    h_r, h_s = torch.zeros(T * k, 1024, dtype=torch.float16, device=cuda), torch.zeros(T, 512, dtype=torch.float16, device=cuda)
+    part_r, part_s = torch.zeros(9 * T * k, H, device=cuda), torch.zeros(8 * T, H, device=cuda)
+    ws = torch.zeros(1 << 20, dtype=torch.uint8, device=cuda)
+
+    def call(fmt, I, I_sh, pieces, routed):
+        sh = I_sh > 0
+        return L.lib.moe_experts_prefill_windows(p(x), T, H, I, I_sh, k, fmt, p(units), 4, p(tok), p(table), p(shared) if sh else None,
+                                                 p(h_r), p(h_s) if sh else None, p(part_r), p(part_s) if sh else None, pieces, routed,
+                                                 p(ws), p(err), 3, None, L.cur_stream())
     for fmt, I, routed in ((L.FMT_INT4_G128, 384, 4), (L.FMT_INT4_G128, 128, 2), (L.FMT_BF16, 512, 2), (L.FMT_INT4_G128, 1024, 9),
                            (L.FMT_INT4_G128, 1024, 0)):
-        rc = L.lib.moe_experts_prefill_windows(p, 70, 256, I, 0, 2, fmt, p, 4, p, p, None, p, None, p, None, 1, routed, p, p, 3,
-                                               None, None)
-        assert rc != 0 and b"windows" in L.lib.moe_last_error(), (fmt, I, routed)
+        assert call(fmt, I, 0, 1, routed) != 0 and b"windows" in L.lib.moe_last_error(), (fmt, I, routed)
     for I_sh, pieces in ((384, 2), (512, 8)):    # bf16: windows of three slabs, of one
-        rc = L.lib.moe_experts_prefill_windows(p, 70, 256, 128, I_sh, 2, L.FMT_BF16, p, 4, p, p, p, p, p, p, p, pieces, 1, p, p, 3,
-                                               None, None)
-        assert rc != 0 and b"windows" in L.lib.moe_last_error(), (I_sh, pieces)
+        assert call(L.FMT_BF16, 128, I_sh, pieces, 1) != 0 and b"windows" in L.lib.moe_last_error(), (I_sh, pieces)
+    torch.cuda.synchronize()
 
 
 @pytest.mark.parametrize("cache_rate", [1.0, 0.5])

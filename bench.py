@@ -194,6 +194,7 @@ def prefill_leg(torch, name, T, H, E, I, k, I_sh, fmt, gated, mode, steps=20):
     y = torch.empty(T, H, dtype=torch.bfloat16, device=dev)
     logits = torch.empty(T, wg.shape[0], dtype=torch.float32, device=dev)
     d = ops.Dispatch(T, k, E, min(E, T * k), dev)
+    rp = ops.prefill_windows(fmt, T, k, E, H, I, I_sh)[0]   # (the launches of moe_forward)
     ws = None
 
     def layer():
@@ -201,8 +202,8 @@ def prefill_leg(torch, name, T, H, E, I, k, I_sh, fmt, gated, mode, steps=20):
         ops.gate_logits(x, wg, None, out=logits)
         idx, w = ops.topk(logits, k, mode, E=E)
         ops.dispatch(idx, E, out=d)
-        ws = ops.experts_prefill(x, d, table, sh, H, I, I_sh, fmt, ws=ws)
-        ops.combine(ws[0], ws[1], w, d.pos_of_pair, logits[:, E] if gated else None, T, H, k, out=y)
+        ws = ops.experts_prefill(x, d, table, sh, H, I, I_sh, fmt, ws=ws, windows=True)
+        ops.combine(ws[0], ws[1], w, d.pos_of_pair, logits[:, E] if gated else None, T, H, k, out=y, routed_pieces=rp)
 
     def timed(fn, n):
         fn(); fn()
@@ -217,8 +218,8 @@ def prefill_leg(torch, name, T, H, E, I, k, I_sh, fmt, gated, mode, steps=20):
 
     t_layer = timed(layer, steps)
     assert int(ws[2].cpu()[0]) == 0
-    t_w13 = timed(lambda: ops.experts_prefill(x, d, table, sh, H, I, I_sh, fmt, phases=1, ws=ws), steps)
-    t_w2 = timed(lambda: ops.experts_prefill(x, d, table, sh, H, I, I_sh, fmt, phases=2, ws=ws), steps)
+    t_w13 = timed(lambda: ops.experts_prefill(x, d, table, sh, H, I, I_sh, fmt, phases=1, ws=ws, windows=True), steps)
+    t_w2 = timed(lambda: ops.experts_prefill(x, d, table, sh, H, I, I_sh, fmt, phases=2, ws=ws, windows=True), steps)
     flops = 2.0 * T * k * 3 * I * H + 2.0 * T * 3 * I_sh * H
     ach = flops * 2 / 3 / t_w13 / 1e12
     tag = name.split("-")[0].split(".")[0].lower() + ("_q4k" if fmt == L.FMT_Q4K else ("_bf16" if fmt == L.FMT_BF16 else "_int4"))
@@ -247,9 +248,10 @@ def decode_leg(torch, name, fmt, T, H, E, I, k, I_sh, gated, mode, layers, zipf,
     mk = synth.random_q4k_images if q4k else synth.random_int4_images
     lay = LY.q4k_layout if q4k else LY.int4_layout
     tiles = T > ops.gemv_max_tokens(fmt)   # the rule of moe_forward: larger token groups take the matrix-core tile kernels
+    rp = ops.prefill_windows(fmt, T, k, E, H, I, I_sh)[0] if tiles else 1
     if tiles:
         def run_experts(x, d_, table, sh, H_, I_, I_sh_, phases=3, ws=None):
-            return ops.experts_prefill(x, d_, table, sh, H_, I_, I_sh_, fmt, phases=phases, ws=ws)
+            return ops.experts_prefill(x, d_, table, sh, H_, I_, I_sh_, fmt, phases=phases, ws=ws, windows=True)
     else:
         run_experts = ops.experts_decode_q4k if q4k else ops.experts_decode_int4
     imgs, shs, gws, biases, tables = [], [], [], [], []
@@ -300,7 +302,7 @@ def decode_leg(torch, name, fmt, T, H, E, I, k, I_sh, gated, mode, layers, zipf,
             step.w = w
         ws = run_experts(x, d, tables[l], shs[l], H, I, I_sh, phases=phases, ws=ws)
         if phases == 3:
-            ops.combine(ws[0], ws[1], step.w, d.pos_of_pair, logits[:, E] if gated else None, T, H, k, out=y)
+            ops.combine(ws[0], ws[1], step.w, d.pos_of_pair, logits[:, E] if gated else None, T, H, k, out=y, routed_pieces=rp)
 
     def timed(fn, n):
         for i in range(min(n, 2 * layers)):

@@ -332,37 +332,49 @@ def prefill_workspace_bytes(fmt: int, T: int, H: int, k: int, max_units: int) ->
     return n if fmt == L.FMT_BF16 else ((n + 255) & ~255) + T * H * 2
 
 
+def prefill_windows(fmt: int, T: int, k: int, E: int, H: int, I: int, I_sh: int) -> tuple[int, int]:
+    """Pieces moe_forward's tile launches leave the routed experts' and the shared expert's partial rows in."""
+    return (int(lib.moe_prefill_routed_windows(fmt, T, k, E, H, I)),
+            int(lib.moe_prefill_shared_windows_beside(fmt, T, H, I, I_sh)) if I_sh else 1)
+
+
 def experts_prefill(x, d: Dispatch, expert_ptr: torch.Tensor, shared: torch.Tensor | None,
-                    H: int, I: int, I_sh: int, fmt: int = L.FMT_BF16, phases: int = 3, ws=None):
+                    H: int, I: int, I_sh: int, fmt: int = L.FMT_BF16, phases: int = 3, ws=None, windows: bool = False):
     """MFMA grouped expert product.  Returns (part_r, part_s, err, h_r, h_s, tiles).  part_s has S*T rows, S =
-    moe_prefill_shared_splits pieces of the shared expert's w2 product (combine adds them; S = 1 mostly)."""
+    moe_prefill_shared_splits pieces of the shared expert's w2 product (combine adds them; S = 1 mostly).
+    windows: the launches of moe_forward, part_r with R*T*k rows and part_s with S*T, R and S of prefill_windows (combine takes
+    R as routed_pieces)."""
     T, k = d.T, d.k
     P = T * k
     dev = x.device
+    has_s = shared is not None or (ws is not None and ws[1] is not None)
+    R, S = prefill_windows(fmt, T, k, d.E, H, I, I_sh if has_s else 0) if windows else (
+        1, int(lib.moe_prefill_shared_splits(fmt, T, H, I_sh)) if has_s else 1)
     if ws is not None:
         part_r, part_s, err, h_r, h_s, tiles = ws
     else:
         h_r = torch.empty(max(P, 1), max(I, 1), dtype=torch.bfloat16, device=dev)
-        part_r = torch.empty(max(P, 1), H, dtype=torch.float32, device=dev)
+        part_r = torch.empty(max(R * P, 1), H, dtype=torch.float32, device=dev)
         h_s = part_s = None
         if shared is not None:
             h_s = torch.empty(T, I_sh, dtype=torch.bfloat16, device=dev)
-            part_s = torch.empty(int(lib.moe_prefill_shared_splits(fmt, T, H, I_sh)) * T, H, dtype=torch.float32, device=dev)
+            part_s = torch.empty(S * T, H, dtype=torch.float32, device=dev)
         err = torch.zeros(1, dtype=torch.int32, device=dev)
         # (nibble formats: behind the tile list, room for the fp16 copy of the activations)
         tiles = torch.empty(prefill_workspace_bytes(fmt, T, H, k, d.max_units), dtype=torch.uint8, device=dev)
     if fmt != L.FMT_BF16 and tiles.numel() >= prefill_workspace_bytes(fmt, T, H, k, d.max_units):
         phases |= 4
-    pieces = 1
-    if part_s is not None:
-        pieces = int(lib.moe_prefill_shared_splits(fmt, T, H, I_sh))
-        if part_s.shape[0] != pieces * T:   # a workspace made for another batch size or format
-            part_s = torch.empty(pieces * T, H, dtype=torch.float32, device=dev)
-    check(lib.moe_experts_prefill_pieces(ptr(_dev(x)), T, H, I, I_sh if shared is not None else 0, k, fmt,
-                                         ptr(d.units), d.max_units, ptr(d.sorted_tok), ptr(expert_ptr),
-                                         ptr(shared), ptr(h_r), ptr(h_s), ptr(part_r), ptr(part_s),
-                                         pieces if shared is not None else 1, ptr(tiles),
-                                         ptr(err), phases, cur_stream()), "moe_experts_prefill")
+    if part_s is not None and part_s.shape[0] != S * T:   # a workspace made for another batch size or format
+        part_s = torch.empty(S * T, H, dtype=torch.float32, device=dev)
+    if windows and part_r.shape[0] < R * P:
+        part_r = torch.empty(R * P, H, dtype=torch.float32, device=dev)
+    args = (ptr(_dev(x)), T, H, I, I_sh if shared is not None else 0, k, fmt, ptr(d.units), d.max_units, ptr(d.sorted_tok),
+            ptr(expert_ptr), ptr(shared), ptr(h_r), ptr(h_s), ptr(part_r), ptr(part_s),
+            S if shared is not None else 1)
+    if windows:
+        check(lib.moe_experts_prefill_windows(*args, R, ptr(tiles), ptr(err), phases, None, cur_stream()), "moe_experts_prefill")
+    else:
+        check(lib.moe_experts_prefill_pieces(*args, ptr(tiles), ptr(err), phases, cur_stream()), "moe_experts_prefill")
     return part_r, part_s, err, h_r, h_s, tiles
 
 
@@ -372,8 +384,9 @@ def shared_splits(fmt: int, T: int, H: int, I_sh: int) -> int:
 
 
 def combine(part_r, part_s, topk_w, pos_of_pair, shared_gate_logit, T: int, H: int, k: int,
-            out: torch.Tensor | None = None, pieces: int | None = None):
+            out: torch.Tensor | None = None, pieces: int | None = None, routed_pieces: int = 1):
     """part_s [S*T, H]: S > 1 when the shared expert's reduction was split (piece s = rows s*T .. s*T+T-1).
+    routed_pieces: the same of part_r [R*T*k, H].
     pieces: S as the expert launch left it (shared_splits / moe_prefill_shared_splits); inferred from the rows of
     part_s when not given, which is only right for a part_s made for exactly this T."""
     dev = (part_r if part_r is not None else part_s).device
@@ -388,7 +401,8 @@ def combine(part_r, part_s, topk_w, pos_of_pair, shared_gate_logit, T: int, H: i
     else:
         assert part_s.shape[0] % max(T, 1) == 0, "part_s was made for another batch size: pass pieces"
         n_splits = max(1, part_s.shape[0] // max(T, 1))
-    check(lib.moe_combine_splits(ptr(part_r), ptr(part_s), ptr(topk_w), ptr(pos_of_pair),
-                                 ptr(shared_gate_logit), sg_stride, ptr(out), T, H, k, n_splits, cur_stream()),
+    assert routed_pieces == 1 or part_r.shape[0] >= routed_pieces * T * k, "part_r holds fewer rows than pieces x pairs"
+    check(lib.moe_combine_windows(ptr(part_r), ptr(part_s), ptr(topk_w), ptr(pos_of_pair),
+                                  ptr(shared_gate_logit), sg_stride, ptr(out), T, H, k, routed_pieces, n_splits, cur_stream()),
           "moe_combine")
     return out

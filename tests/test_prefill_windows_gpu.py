@@ -162,3 +162,30 @@ def test_bf16_layer_with_a_long_shared_expert(cuda, T):
         err = float(np.abs(y.float().cpu().numpy() - ref["out"]).max() / np.abs(ref["out"]).max())
         assert err <= 2e-2, (T, err)
     pm.close()
+
+
+@pytest.mark.parametrize("cls,I,I_sh,T", [(Int4Layer, 4096, 2304, 70), (Q4KLayer, 4096, 256, 70), (Bf16Layer, 256, 5120, 100)])
+def test_the_operators_with_windows_are_the_layer_forward(cuda, cls, I, I_sh, T):
+    """ops.experts_prefill with windows, and combine: the launches of the engine's forward, bit for bit."""
+    from promoe_amd import ops, _lib as L
+    from tests.test_engine_gpu import build_engine
+    print(f"case windows ops {cls.__name__} T={T}", flush=True)
+    H, E, k = 256, 4, 2
+    fmt = {Q4KLayer: L.FMT_Q4K, Int4Layer: L.FMT_INT4_G128, Bf16Layer: L.FMT_BF16}[cls]
+    R, S = ops.prefill_windows(fmt, T, k, E, H, I, I_sh)
+    assert R * S > 1
+    layer = cls(H=H, I=I, E=E, I_sh=I_sh, seed=8)
+    pm = build_engine([layer], k, cuda, max_tokens=T, cache_rate=1.0, cache_policy="lru")
+    x = torch.from_numpy(O.synth_acts(T, H, seed=T)).to(torch.bfloat16).to(cuda)
+    y = pm.forward(0, x)
+    torch.cuda.synchronize()
+    lg = ops.gate_logits(x, torch.from_numpy(layer.wg).to(torch.bfloat16).to(cuda), None)
+    idx, w = ops.topk(lg, k, 0, E=E)
+    d = ops.dispatch(idx, E)
+    slots = [torch.from_numpy(s).to(cuda) for s in layer.slots]
+    table = torch.tensor([s.data_ptr() for s in slots], dtype=torch.int64, device=cuda)
+    ws = ops.experts_prefill(x, d, table, torch.from_numpy(layer.shared_img).to(cuda), H, I, I_sh, fmt, windows=True)
+    assert ws[0].shape[0] == R * T * k and ws[1].shape[0] == S * T and int(ws[2].item()) == 0
+    y2 = ops.combine(ws[0], ws[1], w, d.pos_of_pair, None, T, H, k, routed_pieces=R)
+    assert torch.equal(y.view(torch.int16), y2.view(torch.int16))
+    pm.close()

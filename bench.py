@@ -99,9 +99,10 @@ def launches_timed(torch, launch_n, n, replay_once=False):
 
 
 PROFILE_DIR = os.path.join(os.path.dirname(os.path.abspath(__file__)), "profiles")
-DECODE_SOURCES = ["promoe_amd/csrc/" + f for f in ("moe_kernels.hip", "moe_decode_bf16.hip", "moe_device.h", "moe_common.h")]
-PREFILL_SOURCES = ["promoe_amd/csrc/" + f for f in ("moe_prefill.hip", "moe_gate.hip", "moe_decode_bf16.hip", "moe_device.h",
-                                                    "moe_common.h")]
+DECODE_SOURCES = ["promoe_amd/csrc/" + f for f in ("moe_kernels.hip", "moe_decode_bf16.hip", "moe_decode_bf16.h", "moe_device.h",
+                                                   "moe_common.h")]
+PREFILL_SOURCES = ["promoe_amd/csrc/" + f for f in ("moe_prefill.hip", "moe_gate.hip", "moe_decode_bf16.hip", "moe_decode_bf16.h",
+                                                    "moe_device.h", "moe_common.h")]
 
 
 def source_hash(sources):

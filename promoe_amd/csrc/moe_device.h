@@ -97,37 +97,30 @@ static __device__ __forceinline__ float wave_max_f32(float x) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), 63));
 }
 
-// One choice of a token's top-k by a wave whose lane l holds the logits l, l + 64, ...: the lowest expert that holds `best` (the
-// wave's maximum), or the lowest one still open where none does.  A chosen expert's logit and the lanes past the last expert
-// are NaN (TOPK_NONE), which fmaxf passes over and nothing equals, so whatever a token's logits are it holds k different experts
-// of the layer, as the dispatch counts on: numbers first, then -inf, then NaN.  open: the experts of a column that have not been
-// chosen (topk_column at first).  No branches: the choices of several tokens are interleaved.
-#define TOPK_NONE __builtin_nanf("")
-static __device__ __forceinline__ unsigned long long topk_column(const int E, const int r) {
-  const int n = E - 64 * r;
-  return n >= 64 ? ~0ull : n > 0 ? (1ull << n) - 1ull : 0ull;
+// Top-k of a token by a wave whose lane l holds the logits l, l + 64, ...  topk_logit: what a lane holds at first: a NaN counts as
+// -inf, and a lane past the last expert holds a NaN, which fmaxf passes over and nothing equals.  topk_choose: one choice, the lowest
+// expert that holds `best` (the wave's maximum); the lane then holds a NaN as well.  Whatever the logits are, k rounds (k <= E) so
+// choose k different experts of the layer, as the dispatch counts on: a row of NaN used to choose the lane past the last expert,
+// and a row with fewer finite logits than choices one expert twice.
+static __device__ __forceinline__ float topk_logit(const float x, const bool is_expert) {
+  return is_expert ? fmaxf(x, -__builtin_inff()) : __builtin_nanf("");
 }
 template <int NR>
-static __device__ __forceinline__ void topk_choose(float (&v)[NR], unsigned long long (&open)[NR], const float best, const int lane,
+static __device__ __forceinline__ void topk_choose(float (&v)[NR], unsigned long long (&msel)[NR], const float best, const int lane,
                                                    int &wr, int &wl) {
-  unsigned long long c[NR], any = 0ull;
+  unsigned long long c = __ballot(v[NR - 1] == best);
+  wr = NR - 1; wl = (int)__builtin_ctzll(c);
 #pragma unroll
-  for (int r = 0; r < NR; ++r) {
-    c[r] = __ballot(v[r] == best);
-    any |= c[r];
-  }
-  wr = 0; wl = 0;
-#pragma unroll
-  for (int r = NR - 1; r >= 0; --r) {
-    c[r] = any ? c[r] : open[r];
-    wl = c[r] ? (int)__builtin_ctzll(c[r]) : wl;
-    wr = c[r] ? r : wr;
+  for (int r = NR - 2; r >= 0; --r) {
+    c = __ballot(v[r] == best);
+    wl = c ? (int)__builtin_ctzll(c) : wl;
+    wr = c ? r : wr;
   }
 #pragma unroll
   for (int r = 0; r < NR; ++r)
     if (r == wr) {
-      if (lane == wl) v[r] = TOPK_NONE;
-      open[r] &= ~(1ull << wl);
+      if (lane == wl) v[r] = __builtin_nanf("");
+      msel[r] |= 1ull << wl;
     }
 }
 

@@ -54,15 +54,14 @@ template <int NR, bool COH>
 static __device__ __forceinline__ void topk_token(const float *__restrict__ row, const int E, const int k, const int mode,
                                                   const int lane, int *__restrict__ idx, float *__restrict__ wout,
                                                   int *s_idx, unsigned long long *s_mask) {
-  const float NEG = -__builtin_inff();
   float v[NR], v0[NR];
-  unsigned long long open[NR];
+  unsigned long long msel[NR];
 #pragma unroll
   for (int r = 0; r < NR; ++r) {
     const int e = lane + 64 * r;
-    v[r] = (e < E) ? (COH ? __hip_atomic_load(row + e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : row[e]) : TOPK_NONE;
-    v0[r] = v[r];
-    open[r] = topk_column(E, r);
+    v0[r] = (e < E) ? (COH ? __hip_atomic_load(row + e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : row[e]) : 0.f;
+    v[r] = topk_logit(v0[r], e < E);
+    msel[r] = 0ull;
   }
   float my_v = 0.f;  // lane j keeps the j-th selected logit
   for (int j = 0; j < k; ++j) {
@@ -71,9 +70,9 @@ static __device__ __forceinline__ void topk_token(const float *__restrict__ row,
     for (int r = 1; r < NR; ++r) bvl = fmaxf(bvl, v[r]);
     const float bv = wave_max_f32(bvl);
     int wr, wl;
-    topk_choose(v, open, bv, lane, wr, wl);
+    topk_choose(v, msel, bv, lane, wr, wl);
     if (lane == j) {
-      my_v = fmaxf(bv, NEG);   // (a NaN counts as -inf in the weights)
+      my_v = bv;
       const int bi = wl + 64 * wr;
       idx[j] = bi;
       if (s_idx) s_idx[j] = bi;
@@ -81,7 +80,7 @@ static __device__ __forceinline__ void topk_token(const float *__restrict__ row,
   }
   if (s_mask && lane == 0) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) s_mask[r] = r < NR ? topk_column(E, r) & ~open[r < NR ? r : 0] : 0ull;
+    for (int r = 0; r < 4; ++r) s_mask[r] = r < NR ? msel[r < NR ? r : 0] : 0ull;
   }
   // weights: the row maximum is the first choice; the softmax denominator over all E per lane in column order, then
   // the xor butterfly; the sum over the choices in choice order
@@ -928,13 +927,12 @@ static __device__ __forceinline__ GemvWork gemv_resolve_route_n(const GemvArgs &
   const int rw = publisher ? 0 : ((bx >> 8) & 3);
   wk.m = publisher ? 0 : 1; wk.row0 = u;
   if (w == rw) {
-  const float NEG = -__builtin_inff();
   float v[NR], v0[NR];
   unsigned long long ptrs[NR];  // slot addresses of the lane's candidates, fetched alongside the logits
 #pragma unroll
   for (int r = 0; r < NR; ++r) {
     const int e = lane + 64 * r;
-    v[r] = (e < E && a.g_nblk == 0) ? a.r_logits[e] : TOPK_NONE;
+    v[r] = (e < E && a.g_nblk == 0) ? a.r_logits[e] : 0.f;
     ptrs[r] = (e < E) ? slot_of(a, e) : 0ull;
   }
   bool gate_timeout = false;
@@ -971,10 +969,13 @@ static __device__ __forceinline__ GemvWork gemv_resolve_route_n(const GemvArgs &
     STAMP(2); STAMPV(3, spins);
   }
 #pragma unroll
-  for (int r = 0; r < NR; ++r) v0[r] = v[r];
-  unsigned long long open[NR], msel[NR];
+  for (int r = 0; r < NR; ++r) {
+    v0[r] = v[r];
+    v[r] = topk_logit(v[r], lane + 64 * r < E);
+  }
+  unsigned long long msel[NR];
 #pragma unroll
-  for (int r = 0; r < NR; ++r) open[r] = topk_column(E, r);
+  for (int r = 0; r < NR; ++r) msel[r] = 0ull;
   float mx = 0.f, sum_sel = 0.f, my_v = 0.f;  // the last three only matter to the publisher
   int my_e = 0;
   for (int j = 0; j < k; ++j) {
@@ -983,11 +984,9 @@ static __device__ __forceinline__ GemvWork gemv_resolve_route_n(const GemvArgs &
     for (int r = 1; r < NR; ++r) bv = fmaxf(bv, v[r]);
     const float best = wave_max_f32(bv);
     int wr, wl;
-    topk_choose(v, open, best, lane, wr, wl);
-    if (lane == j) { my_v = fmaxf(best, NEG); my_e = wl + 64 * wr; }
+    topk_choose(v, msel, best, lane, wr, wl);
+    if (lane == j) { my_v = best; my_e = wl + 64 * wr; }
   }
-#pragma unroll
-  for (int r = 0; r < NR; ++r) msel[r] = topk_column(E, r) & ~open[r];
   // unit u = the u-th smallest selected id
   int cum = 0;
   bool found = false;
@@ -1299,7 +1298,7 @@ static __device__ __forceinline__ GemvWork gemv_resolve_route_batch_n(const Gemv
 #pragma unroll
         for (int r = 0; r < NR; ++r) {
           const int e = lane + 64 * r;
-          v[i][r] = TOPK_NONE;
+          v[i][r] = 0.f;
           if (e < E && t < T) {
             u32x2_t word;
             if (spins < local_spins) {
@@ -1318,11 +1317,14 @@ static __device__ __forceinline__ GemvWork gemv_resolve_route_batch_n(const Gemv
       __builtin_amdgcn_s_sleep(2);
     }
   }
-  unsigned long long open[TPW][NR];
+  unsigned long long msel[TPW][NR];
 #pragma unroll
   for (int i = 0; i < TPW; ++i)
 #pragma unroll
-    for (int r = 0; r < NR; ++r) open[i][r] = topk_column(E, r);
+    for (int r = 0; r < NR; ++r) {
+      v[i][r] = topk_logit(v[i][r], lane + 64 * r < E);
+      msel[i][r] = 0ull;
+    }
   for (int j = 0; j < k; ++j) {
 #pragma unroll
     for (int i = 0; i < TPW; ++i) {
@@ -1330,7 +1332,7 @@ static __device__ __forceinline__ GemvWork gemv_resolve_route_batch_n(const Gemv
 #pragma unroll
       for (int r = 1; r < NR; ++r) bv = fmaxf(bv, v[i][r]);
       int wr, wl;
-      topk_choose(v[i], open[i], wave_max_f32(bv), lane, wr, wl);
+      topk_choose(v[i], msel[i], wave_max_f32(bv), lane, wr, wl);
     }
   }
   __shared__ int s_timeout[4];
@@ -1340,7 +1342,7 @@ static __device__ __forceinline__ GemvWork gemv_resolve_route_batch_n(const Gemv
       const int t = w + 4 * i;
       if (t < T) {
 #pragma unroll
-        for (int r = 0; r < NR; ++r) s_sel[t][r] = gate_timeout ? 0ull : topk_column(E, r) & ~open[i][r];
+        for (int r = 0; r < NR; ++r) s_sel[t][r] = gate_timeout ? 0ull : msel[i][r];
       }
     }
     s_timeout[w] = gate_timeout ? 1 : 0;

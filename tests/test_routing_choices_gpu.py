@@ -1,4 +1,4 @@
-"""Top-k of rows without k ordinary logits (NaN, -inf): k different experts of the layer on every route, and a layer forward that
+"""Top-k of rows without k ordinary logits (NaN, which counts as -inf, and -inf): k different experts of the layer on every route, and a layer forward that
 keeps the other tokens' results and goes on."""
 import numpy as np
 import pytest
@@ -24,7 +24,7 @@ def _logits(T, E, k, seed):
 
 
 def _check(idx, d, lg, k, E):
-    want, _ = O.topk_route(lg, k, 0)      # descending, -inf behind the numbers, NaN last; the lower expert among equals
+    want, _ = O.topk_route(np.where(np.isnan(lg), -np.inf, lg), k, 0)      # (a NaN counts as -inf; the lower expert among equals)
     assert np.array_equal(idx.cpu().numpy(), want)
     T = lg.shape[0]
     counts, offsets, sp, pp = O.dispatch(want, E)

@@ -805,7 +805,7 @@ static void gemv_set_table(GemvArgs &a, const uint64_t *expert_ptr, const uint64
 
 // bx: the workgroup's index among the working ones (launches with a publishing workgroup put that one first)
 // BY_ROWS (device-built unit list of at most 64 slots, a.unit_slots > 0): position u of the grid takes the unit of
-// rank u when the units are ordered by the passes they need (more than 32 rows, 17 to 32, 1 to 16, none; list
+// rank u when the units are ordered by the passes they need (more than row_split or 32 rows, from 17 on, 1 to 16, none; list
 // order inside a class).  The workgroups of the units with the most rows then start first and those of the unused
 // slots last, instead of a popular expert starting when the first round of workgroups has finished.
 template <bool DEVUNITS, bool BY_ROWS = false>
@@ -1085,7 +1085,7 @@ static __device__ __forceinline__ GemvWork gemv_resolve_route(const GemvArgs &a,
 }
 
 // ---------------------------------------------------------------------------
-// Decode batches of 2 to 8 tokens whose w13 launch sums the gate rows and routes by itself (the step is then
+// Decode batches (nibble formats 2 to 16 tokens, bf16 1 to 32) whose w13 launch sums the gate rows and routes by itself (the step is then
 // three launches: this one, w2, combine).  Grid: the gate workgroups (a token and four gate rows each, a wave per
 // row, once per part of the chip: see gate_rows_stamped), ONE workgroup that publishes the routing for the later
 // launches and the host (the routing workgroup of k_gate_route), the shared expert's workgroups, then one set of

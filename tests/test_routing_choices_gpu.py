@@ -1,4 +1,5 @@
-"""Top-k of rows without k ordinary logits (NaN, which counts as -inf, and -inf): k different experts of the layer on every route, and a layer forward that
+"""Top-k of rows without k ordinary logits (NaN, which counts as -inf, and -inf): k different experts of the layer on every
+route, and a layer forward that
 keeps the other tokens' results and goes on."""
 import numpy as np
 import pytest
